@@ -619,6 +619,43 @@ def test_compaction_when_few_tokens_are_dropped_and_budgets_differ(shared):
     _compact_case(small(seq_lens=(2176,), budget=2048, num_layers=1, num_q_heads=8, num_kv_heads=8), 1, shared, False, False)
 
 
+@pytest.mark.parametrize("layers,heads,dim,tokens,budget", [
+    (1, 8, 128, 4300, 2049),      # 16 chains: two workgroups per row, one slot beyond an address segment
+    (1, 8, 64, 2100, 2048),       # 16 chains of 128-byte rows: whole rows
+    (8, 8, 128, 700, 513),        # 128 chains: the last with half rows, one slot beyond a tile
+    (16, 8, 256, 300, 100),       # 256 chains: the last with the longest tile
+    (17, 8, 128, 2300, 2048),     # 272 chains: 32 KB tiles
+    (64, 8, 64, 120, 97),         # 1024 chains: the last of those
+    (65, 8, 64, 120, 97),         # 1040 chains: workgroups of 512
+    (32, 8, 64, 600, 120),        # 512 chains of a sparse list: still one launch
+    (33, 8, 64, 600, 120),        # 528 chains of a sparse list: ordered pass and bulk pass
+])
+@pytest.mark.parametrize("in_place", [0, 1, -1])
+def test_compaction_on_both_sides_of_every_launch_rule(layers, heads, dim, tokens, budget, in_place):
+    """The launch depends on how many chains (sequence, layer, K or V, head) there are and on how sparse
+    the lists are; rows already in place (a prefix of the list: none, one, all but one) are not touched.
+    Rows are copies of bytes: exact."""
+    fixed = in_place if in_place >= 0 else budget - 1
+    print(f"compact rules {layers}x{heads}x{dim} {tokens}->{budget} fixed={fixed}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    nb = (tokens + 15) // 16
+    cache = torch.randint(-2**15, 2**15, (layers, 2, nb, 16, heads, dim), dtype=torch.int16, device=DEV, generator=g)
+    kv_cache = cache.view(torch.bfloat16)
+    kv = ops.PagedKV([c[0] for c in kv_cache], [c[1] for c in kv_cache])
+    table = torch.randperm(nb, generator=g, device=DEV)
+    batch = ops.StepBatch(DEV, [tokens], budgets=budget, block_tables=[table.tolist()])
+    tail = torch.rand(heads, tokens - fixed - 1, generator=g, device=DEV).topk(budget - fixed, 1).indices.sort(1).values
+    keep = torch.cat([torch.arange(fixed, device=DEV).expand(heads, fixed), tail + fixed + 1], 1).int().contiguous()
+    want = cache.clone()
+    slot = lambda t: (table[t // 16], t % 16)
+    head = torch.arange(heads, device=DEV).unsqueeze(1).expand(heads, budget)
+    (sb, so), (db, do) = slot(keep.long()), slot(torch.arange(budget, device=DEV).expand(heads, budget))
+    want[:, :, db, do, head] = cache[:, :, sb, so, head]
+    ops.compact(kv, batch, keep)
+    torch.cuda.synchronize()
+    assert torch.equal(cache, want)
+
+
 @pytest.mark.parametrize("axis", [0, 1])
 def test_compaction_matches_reference_golden(axis):
     """Full-permutation output written by the reference's compact_request_kv_in_place(_per_head)."""

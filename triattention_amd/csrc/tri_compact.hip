@@ -1,27 +1,24 @@
 // In-place, order-preserving paged K/V compaction for gfx950.
 //
 // keep[] is strictly ascending, so keep[j] >= j: destination slot j always lies at
-// or below its source.  One workgroup owns one (sequence, layer, K or V, head) and walks the
-// destination slots in ascending tiles.  Every tile is read completely
+// or below its source.  One workgroup owns one (sequence, layer, K or V, head), or half of such a
+// head's row, and walks the destination slots in ascending tiles.  Every tile is read completely
 // into registers, the workgroup synchronises, then the tile is written: a tile's writes
 // land below the next tile's first slot while every later source lies at or above
 // it, so nothing that is still to be read is ever overwritten and no staging copy
 // of the cache is needed.  The reference gathers all T rows of K and V into
 // temporaries and scatters them back (runtime/kv_compaction.py:529-546).
 #include "tri_common.h"
-#include <cstdlib>
+#include <climits>
 #include <mutex>
 
 namespace tri {
 namespace {
 
 constexpr int kCompactThreads = 256;
-constexpr int kChunksPerThread = 4;                                  // 16-byte chunks held per thread
-static_assert(kChunksPerThread == 4, "compact_kernel spells out four chunk registers");
+constexpr int kChunksPerThread = 4;                                  // bulk pass: 16-byte chunks held per thread
 constexpr int kTileChunks = kCompactThreads * kChunksPerThread;      // 16 KiB per tile
-constexpr int kOrderedThreads = 256;                                 // ordered pass: 4 waves, 16 KiB per tile; a whole batch of streams fits the chip at once
-constexpr int kOrderedTileChunks = kOrderedThreads * kChunksPerThread;
-constexpr int kSegEntries = 2048;                                    // (slot, list) addresses staged in LDS at a time
+constexpr int kSegSlots = 2048;                                      // ordered pass: slot addresses staged in LDS at a time
 
 // The per-layer pointers come out of a device-side table and are generic to the compiler;
 // these casts tell it they are global memory, so it emits global (not flat) loads and
@@ -53,8 +50,7 @@ struct CompactArgs {
   uint32_t block_units, token_units, head_units;           // the same strides in 16-byte units
   int B, L, Hkv, block_size, bs_shift, block_table_pitch, max_budget;
   int keep_per_layer, shared;
-  int lists_per_wg;        // keep lists (heads) one workgroup of the ordered pass moves together
-  int split_bulk;          // 1: the ordered kernel stops at the first source >= budget
+  int cols;                // ordered pass: workgroups that share a head's row, each moving chunks_per_row / cols chunks of it
   int chunks_per_row;      // 16-byte chunks of one head row (D * elem_bytes / 16)
   int heads_per_slot;      // shared ? Hkv : 1
   int streams_per_layer;   // 2 * (shared ? 1 : Hkv)
@@ -73,8 +69,6 @@ __device__ __forceinline__ uint32_t slot_units(const CompactArgs& a, const int32
   const int in_off = tok - lb * a.block_size;
   return (uint32_t)bt[lb] * a.block_units + (uint32_t)in_off * a.token_units;
 }
-
-constexpr uint32_t kNoSource = 0xffffffffu;
 
 // Which (sequence, layer, K or V) the unit with this index is.  Units that run at the same time
 // (neighbouring indices) are spread over the whole cache: the layer runs fastest, in steps of
@@ -103,25 +97,28 @@ __device__ __forceinline__ bool guard_raised(const uint32_t* guard) {
 
 // Ordered pass: the slots whose source token lies inside the kept prefix [0, k).  With keep
 // ascending they form a prefix of every list, and only they can be overwritten before they
-// are read.  One workgroup owns one (sequence, layer, K or V, group of keep lists) and moves
-// a tile of destination slots of its lists together.  A tile is read completely, the
+// are read.  One workgroup owns one (sequence, layer, K or V, head, columns of the head's row)
+// and walks its destination slots in ascending tiles.  A tile is read completely, the
 // workgroup synchronises, the tile is written: a tile's writes land below the next tile's
-// first slot while every later source lies at or above it, for every list, so nothing that
-// is still to be read is overwritten.  Slots whose source lies at or beyond k are left to
-// compact_bulk_kernel.
-__global__ __launch_bounds__(kOrderedThreads) void compact_kernel(CompactArgs a) {
-  __shared__ uint32_t src_units[kSegEntries];   // [slot][list], kNoSource: not this pass's
-  __shared__ uint32_t dst_units[kSegEntries];   // [slot]
-  __shared__ int prefix_len[256];
+// first slot while every later source lies at or above it, so nothing that is still to be
+// read is overwritten.
+// Rows that are already in place (keep[j] == j) form a prefix of the list as well (keep[j] >= j
+// everywhere, so a later row can not be in place after an earlier one has moved): the walk
+// starts behind it.
+// kAll = false: slots whose source lies at or beyond k are left to compact_bulk_kernel;
+// kAll = true: the walk goes on over the whole list and is the only launch.
+template <int kThreads, int kChunks, bool kAll>
+__global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs a) {
+  static_assert(kChunks <= 15, "the wait below counts the stores of a tile in four bits");
+  __shared__ uint32_t src_units[kSegSlots];
+  __shared__ uint32_t dst_units[kSegSlots];
+  __shared__ int sh_fixed, sh_below;
   if (guard_raised(a.guard)) return;
 
-  // workgroup -> (sequence, layer, K or V, group of lists)
-  const int all_lists = a.shared ? 1 : a.Hkv;
-  const int lists = a.lists_per_wg;
-  const int groups = all_lists / lists;
-  int sidx = blockIdx.x;
-  const int list0 = (sidx % groups) * lists; sidx /= groups;
-  const Unit unit = unit_of(a, sidx);
+  int idx = blockIdx.x;
+  const int col = idx % a.cols; idx /= a.cols;
+  const int head = idx % a.Hkv;
+  const Unit unit = unit_of(a, idx / a.Hkv);
   const int kv = unit.kv, l = unit.l, b = unit.b;
 
   int k = a.budgets[b];
@@ -129,113 +126,91 @@ __global__ __launch_bounds__(kOrderedThreads) void compact_kernel(CompactArgs a)
   if (k > T) k = T;
   if (k > a.max_budget) k = a.max_budget;   // keep rows hold max_budget entries, whatever the device array says
   if (k <= 0) return;
+  const int lists = a.shared ? 1 : a.Hkv;
   const int32_t* keep =
-      a.keep + ((int64_t)(a.keep_per_layer ? (b * a.L + l) : b) * all_lists + list0) * a.max_budget;
+      a.keep + ((int64_t)(a.keep_per_layer ? (b * a.L + l) : b) * lists + (a.shared ? 0 : head)) * a.max_budget;
   const int32_t* bt = a.block_table + (int64_t)b * a.block_table_pitch;
   char* base = reinterpret_cast<char*>(const_cast<void*>(kv ? a.v_layers[l] : a.k_layers[l]));
 
-  // Length of the prefix of every list (entries below k), and the longest one.
-  for (int h = threadIdx.x; h < lists; h += kOrderedThreads) prefix_len[h] = 0;
+  // Length of the prefix that is in place, and of the prefix whose sources lie below k.
+  if (threadIdx.x == 0) { sh_fixed = 0; sh_below = 0; }
   __syncthreads();
-  for (int h = 0; h < lists; ++h) {
-    int below = 0;
-    for (int j = threadIdx.x; j < k; j += kOrderedThreads) below += keep[(int64_t)h * a.max_budget + j] < k;
-    if (below) atomicAdd(&prefix_len[h], below);
+  {
+    int fixed = 0, below = 0;
+    for (int j0 = 0; j0 < k; j0 += kThreads) {
+      const int j = j0 + threadIdx.x;
+      const int src = j < k ? keep[j] : INT_MAX;
+      fixed += __popcll(__ballot(src == j));
+      below += __popcll(__ballot(src < k));
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+      atomicAdd(&sh_fixed, fixed);
+      atomicAdd(&sh_below, below);
+    }
   }
   __syncthreads();
-  int J = 0;
-  for (int h = 0; h < lists; ++h) J = max(J, prefix_len[h]);
-  if (J <= 0) return;
+  const int J = kAll ? k : sh_below;
 
-  const int row_chunks = a.heads_per_slot * a.chunks_per_row;       // chunks one list moves per slot
-  const int slot_chunks = lists * row_chunks;                       // chunks of a whole token row
-  const int slots_per_tile = max(kOrderedTileChunks / slot_chunks, 1);
-  const int seg_slots = max(kSegEntries / lists / slots_per_tile, 1) * slots_per_tile;
+  // A thread moves the same 16-byte column of every kThreads / row_chunks-th slot of a tile.
+  const int row_chunks = a.chunks_per_row / a.cols;                 // a power of two, at most kThreads
+  const int slot_step = kThreads / row_chunks;
+  const int slots_per_tile = slot_step * kChunks;
+  const int slot0 = threadIdx.x / row_chunks;
+  const uint32_t inner = (uint32_t)head * a.head_units + (uint32_t)(col * row_chunks + threadIdx.x % row_chunks);
 
-  for (int seg = 0; seg < J; seg += seg_slots) {
-    const int nseg = min(seg_slots, J - seg);
+  for (int seg = sh_fixed; seg < J; seg += kSegSlots) {
+    const int nseg = min(kSegSlots, J - seg);
     __syncthreads();   // previous segment's LDS no longer in use
-    for (int i = threadIdx.x; i < nseg * lists; i += kOrderedThreads) {
-      const int sl = i / lists, h = i - sl * lists;
-      const int j = seg + sl;
-      const int src = keep[(int64_t)h * a.max_budget + j];
-      const bool mine = j < prefix_len[h] && src != j;             // source below k, row not already in place
-      src_units[i] = mine ? slot_units(a, bt, src) : kNoSource;
-      if (h == 0) dst_units[sl] = slot_units(a, bt, j);
+    for (int i = threadIdx.x; i < nseg; i += kThreads) {
+      src_units[i] = slot_units(a, bt, keep[seg + i]);
+      dst_units[i] = slot_units(a, bt, seg + i);
     }
     __syncthreads();
 
-    // Units of work: tiles of slots, or, when a token row is wider than a tile, the passes
-    // over one row.  The loads of unit u+1 are issued before the stores of unit u (their
-    // sources lie at or above the first slot of unit u+1, beyond everything unit u writes;
-    // passes of one row touch disjoint chunks), so a load batch and a store batch are
-    // always in flight together; a barrier between the loads of a unit and its stores
-    // orders them across the workgroup.
-    const int passes = max(ceil_div(slot_chunks, kOrderedTileChunks), 1);
+    // The loads of tile t+1 are issued before the stores of tile t (their sources lie at or
+    // above the first slot of tile t+1, beyond everything tile t writes), so a load batch and
+    // a store batch are always in flight together; a barrier between the loads of a tile and
+    // its stores orders them across the workgroup.
     const int tiles = ceil_div(nseg, slots_per_tile);
-    const int units = tiles * passes;
-    uint32_t dsto[kChunksPerThread];
-    bool live[kChunksPerThread];
-    uint4 r0, r1, r2, r3;
-    auto issue = [&](int u) __attribute__((always_inline)) {
-      const int t0 = (u / passes) * slots_per_tile, c0 = (u % passes) * kOrderedTileChunks;
-      const int nchunks = min(slots_per_tile, nseg - t0) * slot_chunks;
-      uint32_t so[kChunksPerThread];
+    uint32_t dsto[kChunks];
+    uint4 r[kChunks];
+    auto issue = [&](int t) __attribute__((always_inline)) {
+      uint32_t so[kChunks];
 #pragma unroll
-      for (int c = 0; c < kChunksPerThread; ++c) {
-        // Branch-free: a chunk index beyond the tile (a token row whose chunk count does not
-        // divide the tile) repeats the pass's first chunk, load and store alike, so what it
-        // writes is what that chunk writes.
-        const int ci = c0 + c * kOrderedThreads + threadIdx.x;
-        const bool in = ci < nchunks;
-        const int cic = in ? ci : c0;
-        const int sl = t0 + cic / slot_chunks;
-        const int within = cic % slot_chunks;
-        const int h = within / row_chunks, rem = within - h * row_chunks;
-        const int hh = rem / a.chunks_per_row, cc = rem - hh * a.chunks_per_row;
-        const uint32_t inner = (uint32_t)((a.shared ? 0 : list0 + h) + hh) * a.head_units + (uint32_t)cc;
-        const uint32_t su = src_units[sl * lists + h];
+      for (int c = 0; c < kChunks; ++c) {
+        // Branch-free: a slot beyond the segment repeats the last one, load and store alike.
+        const int sl = min(t * slots_per_tile + c * slot_step + slot0, nseg - 1);
+        so[c] = src_units[sl] + inner;
         dsto[c] = dst_units[sl] + inner;
-        live[c] = su != kNoSource;
-        so[c] = live[c] ? su + inner : dsto[c];
       }
-      r0 = load_chunk(base + ((uint64_t)so[0] << 4));
-      r1 = load_chunk(base + ((uint64_t)so[1] << 4));
-      r2 = load_chunk(base + ((uint64_t)so[2] << 4));
-      r3 = load_chunk(base + ((uint64_t)so[3] << 4));
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c) r[c] = load_chunk(base + ((uint64_t)so[c] << 4));
     };
     issue(0);
-    __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): this thread's loads of unit 0 have arrived
+    __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): this thread's loads of tile 0 have arrived
     __syncthreads();                       // ... and every other thread's
-    uint4 w0 = r0, w1 = r1, w2 = r2, w3 = r3;
-    uint32_t d0 = dsto[0], d1 = dsto[1], d2 = dsto[2], d3 = dsto[3];
-    bool l0 = live[0], l1 = live[1], l2 = live[2], l3 = live[3];
-    for (int u = 0; u + 1 < units; ++u) {
-      // Unit u is a full tile (only the last unit of a segment can be partial): every chunk
-      // stores, a chunk that is not this pass's writes back what it read from its own
-      // destination.  Exactly four stores follow the four loads of unit u+1, and vector
-      // memory operations complete in issue order, so "at most four outstanding" means the
-      // loads of unit u+1 have arrived; the wave does not wait for its stores to be
+    uint4 w[kChunks];
+    uint32_t d[kChunks];
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) { w[c] = r[c]; d[c] = dsto[c]; }
+    for (int t = 0; t + 1 < tiles; ++t) {
+      // Exactly kChunks stores follow the kChunks loads of tile t+1, and vector memory
+      // operations complete in issue order, so "at most kChunks outstanding" means the
+      // loads of tile t+1 have arrived; the wave does not wait for its stores to be
       // acknowledged.  The loaded registers are copied right after that wait, so nothing at
       // the top of the loop depends on a load.
-      issue(u + 1);
-      store_chunk(base + ((uint64_t)d0 << 4), w0);
-      store_chunk(base + ((uint64_t)d1 << 4), w1);
-      store_chunk(base + ((uint64_t)d2 << 4), w2);
-      store_chunk(base + ((uint64_t)d3 << 4), w3);
+      issue(t + 1);
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c) store_chunk(base + ((uint64_t)d[c] << 4), w[c]);
       asm volatile("" ::: "memory");            // keep the compiler from moving memory operations across
-      __builtin_amdgcn_s_waitcnt(0x0074);       // vmcnt(4) lgkmcnt(0)
-      w0 = r0; w1 = r1; w2 = r2; w3 = r3;
-      d0 = dsto[0]; d1 = dsto[1]; d2 = dsto[2]; d3 = dsto[3];
-      l0 = live[0]; l1 = live[1]; l2 = live[2]; l3 = live[3];
+      __builtin_amdgcn_s_waitcnt(0x0070 | kChunks);   // vmcnt(kChunks) lgkmcnt(0)
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c) { w[c] = r[c]; d[c] = dsto[c]; }
       __builtin_amdgcn_s_barrier();             // ... in every thread of the workgroup
       asm volatile("" ::: "memory");
     }
-    // Last unit of the segment: its loads have arrived in every thread.
-    if (l0) store_chunk(base + ((uint64_t)d0 << 4), w0);
-    if (l1) store_chunk(base + ((uint64_t)d1 << 4), w1);
-    if (l2) store_chunk(base + ((uint64_t)d2 << 4), w2);
-    if (l3) store_chunk(base + ((uint64_t)d3 << 4), w3);
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) store_chunk(base + ((uint64_t)d[c] << 4), w[c]);
   }
 }
 
@@ -493,7 +468,6 @@ CompactArgs make_args(const CompactLaunch& a) {
   c.max_budget = a.max_budget;
   c.keep_per_layer = a.keep_per_layer;
   c.shared = a.shared;
-  c.split_bulk = 1;
   // One list per workgroup: the ordered pass is a chain of dependent tiles per workgroup, so
   // with few sequences its run time is the chain length, and a chain over one head is
   // Hkv times shorter than one over whole token rows; with many sequences it is bound by
@@ -512,7 +486,7 @@ CompactArgs make_args(const CompactLaunch& a) {
   // What does move these figures is where the cache lies physically: the same virtual range freed
   // and allocated again runs the same compaction in 1.69 to 1.98 ms (one box, one process), and
   // physically contiguous allocations (hipDeviceMallocContiguous) show the same spread.
-  c.lists_per_wg = 1;
+  c.cols = 1;
   // Smallest stride of at least 0.3 L that is coprime to L (a permutation of the layers): 11 of 36, 11 of 32, 21 of 64.
   c.layer_stride = 1;
   for (int st = (3 * a.L + 9) / 10; st < a.L; ++st) {
@@ -593,12 +567,37 @@ hipError_t launch_compact(const CompactLaunch& a, hipStream_t s) {
       forked = true;
     }
   }
-  // Ordered pass over the slots whose sources lie inside the kept prefix, then the
-  // unordered bulk pass over the rest; the first must finish reading before the second
-  // writes, which stream order guarantees.
-  const int ordered_groups = (a.shared ? 1 : a.Hkv) / c.lists_per_wg;
-  hipLaunchKernelGGL(compact_kernel, dim3(a.B * a.L * 2 * ordered_groups), dim3(kOrderedThreads), 0, s, c);
-  if (c.split_bulk) {
+  // How the rows are moved (compaction alone, keep lists spread over the context, budget 2048 and 8 heads
+  // of 256-byte rows unless noted; us by the rule below / by the ordered pass of 256 threads plus the
+  // bulk pass, which served every shape before):
+  //  - sparse lists (a fifth of the context or less) of more than a few heads: two passes.  The bulk
+  //    pass writes whole token rows for all heads together, which pays where most sources lie
+  //    beyond the budget: 36 layers x 16384 tokens 133 against 142 us in one launch, 16 such
+  //    requests 1953 against 1969, with 128-byte rows (8 x 8192 -> 1024) 262 against 275; at a quarter
+  //    of the context the two are level (989 / 991).
+  //  - otherwise one launch of the ordered pass over the whole list.  Its time is the chain of
+  //    tiles of one workgroup until the memory system is full, so the fewer chains there are the
+  //    longer the tile: up to 256 chains a tile of 128 KB (one layer x 4096 tokens 9.9 / 19.1 us, 16
+  //    layers 43.1 / 54.1; up to 128 chains two workgroups take half of every row each, 8 layers
+  //    24.3 / 37.1), up to 1024 chains 32 KB (36 layers x 2176 tokens 120.6 / 135.8; 36 layers x 1000 ->
+  //    600 31.2 / 38.0, where 128 KB overshoot the list: 37.5), beyond that 32 KB in workgroups of 512
+  //    (16 requests x 2176 tokens 1997 / 2035; 256 threads 2007).
+  const int chains = a.B * a.L * 2 * a.Hkv;
+  if ((int64_t)5 * a.max_budget > a.Tmax || chains <= 512) {
+    CompactArgs one = c;
+    if (chains <= 256) {
+      if (chains <= 128 && c.chunks_per_row >= 16) one.cols = 2;     // (pieces of 128 bytes: a cache line)
+      hipLaunchKernelGGL((compact_kernel<1024, 8, true>), dim3(chains * one.cols), dim3(1024), 0, s, one);
+    } else if (chains <= 1024) {
+      hipLaunchKernelGGL((compact_kernel<256, 8, true>), dim3(chains), dim3(256), 0, s, one);
+    } else {
+      hipLaunchKernelGGL((compact_kernel<512, 4, true>), dim3(chains), dim3(512), 0, s, one);
+    }
+  } else {
+    // Ordered pass over the slots whose sources lie inside the kept prefix, then the
+    // unordered bulk pass over the rest; the first must finish reading before the second
+    // writes, which stream order guarantees.
+    hipLaunchKernelGGL((compact_kernel<256, 4, false>), dim3(chains), dim3(256), 0, s, c);
     hipError_t e0 = hipGetLastError();
     if (e0 != hipSuccess) return e0;
     const int lists = a.shared ? 1 : a.Hkv;
