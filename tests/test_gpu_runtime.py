@@ -294,6 +294,52 @@ def test_batch_hook_equals_the_hook_called_request_by_request(tmp_path, monkeypa
     assert all(not r.applied and r.reason == "under_budget" for r in again.values())
 
 
+@pytest.mark.parametrize("kw", [dict(pruning_mode="per_layer_per_head"),
+                                dict(pruning_mode="per_layer_per_head", layer_perhead_aggregation="mean"),
+                                dict(pruning_mode="per_layer", allow_per_layer_mode=True),
+                                dict(per_head_selection_semantics="legacy_layer_local")], ids=["max", "mean", "shared", "legacy"])
+@pytest.mark.parametrize("runs", [False, True])
+def test_layer_local_modes_in_one_call_equal_the_layer_by_layer_path(tmp_path, monkeypatch, kw, runs):
+    """The modes in which every layer keeps its own set: all layers and requests in one launch sequence (three
+    times over, the later ones from a captured graph; ``runs``: in runs of layers whose scratch is bounded) give
+    the caches, block lists and result dictionaries of the layer-by-layer path, bit for bit (the same kernels)."""
+    from helpers import build_inputs
+    from triattention_amd import synth
+    from triattention_amd.runtime import hook as hook_mod, selector as selector_mod
+    w = synth.Workload(name="t", num_layers=5, num_q_heads=8, num_kv_heads=2, head_dim=128, seq_lens=(700, 515),
+                       budget=96, block_size=16, window_size=12, rope_theta=1e6, index=33)
+    inp = build_inputs(w)
+    kw = dict(kw, fail_on_effective_len_regression=False)           # (the turns reset the block lists)
+    one, two = _fake_runner(w, inp, tmp_path, **kw), _fake_runner(w, inp, tmp_path, **kw)
+    start = [c.clone() for c in one[2]]
+    if runs:        # two layers a run
+        monkeypatch.setattr(selector_mod, "LAYER_RUN_MAX_SCRATCH_BYTES", 2 * 4 * 2 * (700 * (8 + 2) + 8 * 3 * 64))
+    moved = []
+    monkeypatch.setattr(hook_mod, "run_group_compaction_pipeline", lambda **k: moved.append(k["req_id"]) or pipeline(**k))
+    from triattention_amd.runtime.pipeline import run_group_compaction_pipeline as pipeline
+    for turn in range(3):
+        print(f"layer-local {kw} runs={runs} turn={turn}", flush=True)
+        got = {}
+        for which, (runner, reqs, caches, sched, _) in ((False, one), (True, two)):
+            monkeypatch.setattr(hook_mod, "SINGLE_REQUEST_IN_ONE_CALL", which)
+            for c, c0 in zip(caches, start):
+                c.copy_(c0)
+            for b, t in enumerate(w.seq_lens):
+                reqs[f"r{b}"].num_computed_tokens = t + 50 * turn
+                reqs[f"r{b}"].block_ids = ([int(x) for x in inp["tables"][b]],)
+            sig = {f"r{b}": _signal(req_id=f"r{b}", estimated_cache_len=t + 1, prefill_len=20, protect_prefill=b == 1)
+                   for b, t in enumerate(w.seq_lens)}
+            ex = RunnerHookCompressionExecutor(runner)
+            got[which] = (ex.execute_batch(sig, sched) if which else {r: ex.execute(r, s, sched) for r, s in sig.items()})
+            torch.cuda.synchronize()
+        assert got[True] == got[False] and all(r.applied for r in got[True].values())
+        assert [two[1][r].block_ids for r in got[True]] == [one[1][r].block_ids for r in got[True]]
+        for a, b, c0 in zip(one[2], two[2], start):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+            assert not torch.equal(a.view(torch.int16), c0.view(torch.int16))
+    assert moved == ["r0", "r1"] * 3            # only the one-by-one runner took the layer-by-layer path
+
+
 def test_batch_hook_on_the_resident_kernel(tmp_path, monkeypatch):
     """Sixteen requests of 3072 tokens fill the chip: the batch hook runs the resident kernel;
     result equal to the library calls on the same batch, and, when the resident launch is made to

@@ -19,9 +19,9 @@ from typing import Any, Callable
 import torch
 
 from .config import TriAttentionRuntimeConfig
-from .kv_compaction import (build_keep_token_indices, compact_request_kv_in_place,
+from .kv_compaction import (_debug_validate_compaction_content, build_keep_token_indices, compact_request_kv_in_place,
                             compact_request_kv_in_place_per_head, gather_request_k_dense,
-                            register_kv_layout_axis_hint)
+                            kv_axis_hint, register_kv_layout_axis_hint)
 from .models import TRITON_SCORING_REQUIRED_MARKER as MARK, CompressionSignal
 from .pipeline import (GroupPipelineOutcome, finalize_hook_placement_result, normalize_mutable_block_ids_by_group,
                        num_required_blocks, run_group_compaction_pipeline, truncate_tail_reclaim_group)
@@ -434,6 +434,16 @@ def _debug_env_active() -> bool:
         os.environ.get("TRIATTN_DEBUG_FORCE_PRESERVE_DROPPED", "0").strip().lower() in on
 
 
+def _same_geometry(caches: list, block_size: int) -> bool:
+    """Can the layers be described by one set of strides (and are they blocks of the engine's size)?"""
+    c0 = caches[0]
+    shape, stride, dtype, device, hint = c0.shape, c0.stride(), c0.dtype, c0.device, kv_axis_hint(c0)
+    if c0.ndim != 5 or shape[2] != block_size:
+        return False
+    return all(t.shape == shape and t.stride() == stride and t.dtype == dtype and t.device == device
+               and kv_axis_hint(t) == hint for t in caches[1:])
+
+
 # ------------------------------------------------------------------- the hook
 def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeConfig) -> Callable[..., dict]:
     """runtime/hook_impl.py:30-165."""
@@ -444,6 +454,7 @@ def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeCo
     group_tensors: dict | None = None
     compressed_once: set = set()
     compress_batch = getattr(select_group, "_compress_batch", None) if select_group is not None else None
+    layer_local = bool(getattr(select_group, "_layer_local", False))
 
     def _prepare(req_id: str, signal: CompressionSignal, scheduler_output: Any):
         """Everything before the kernels: a result dictionary when the request is skipped,
@@ -526,10 +537,14 @@ def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeCo
         return _run_single(ready)
 
     def _batchable(r: "_Ready") -> bool:
-        """True when the one-by-one path would take the group selector and the ordered
-        per-head compaction for every KV-cache group of this request, with nothing that only
-        that path knows how to do (debug overrides, the keep-everything and prefill early outs)."""
+        """True when the one-by-one path would take the selector and the ordered compaction
+        for every KV-cache group of this request, with nothing that only
+        that path knows how to do (debug overrides, the keep-everything and prefill early outs; in the
+        layer-local modes, which it walks layer by layer, also the compaction's self-check and layers of
+        different geometry)."""
         if compress_batch is None or _debug_env_active():
+            return False
+        if layer_local and _debug_validate_compaction_content():
             return False
         sig = r.signal
         groups = 0
@@ -543,6 +558,8 @@ def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeCo
             if budget <= 0 or total <= budget:
                 return False
             if sig.protect_prefill and config.include_prefill_in_budget and min(int(sig.prefill_len), total) > budget:
+                return False
+            if layer_local and not _same_geometry([t for _, t in group_tensors[gid]], r.block_size):
                 return False
             groups += 1
         return groups > 0
@@ -582,6 +599,8 @@ def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeCo
             except Exception as exc:
                 raise RuntimeError(f"{MARK}:batch:gid={gid}:global_per_head:{type(exc).__name__}") from exc
             for (r, ids, total), res in zip(members, selected):
+                semantic = res.get("semantic")
+                label = f"{res['mode']}:{semantic}" if semantic else res["mode"]
                 after = int(res["indices"].shape[1])
                 if cache_len[r.req_id] is not None and cache_len[r.req_id] != after:
                     raise RuntimeError(f"{MARK}:inconsistent_cache_len_after:req={r.req_id}:gid={gid}:"
@@ -609,7 +628,7 @@ def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeCo
                 out[r.req_id] = {"applied": False, "reason": "no_compactable_groups"}
                 continue
             out[r.req_id] = _finish(r, GroupPipelineOutcome(
-                cache_len_after=int(cache_len[r.req_id]), selection_mode="per_head:hf_aligned_global_per_head",
+                cache_len_after=int(cache_len[r.req_id]), selection_mode=label,
                 block_reclaim_groups=reclaim[r.req_id], mutable_block_ids_by_group=r.mutable_ids))
         return out
 

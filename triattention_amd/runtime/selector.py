@@ -88,6 +88,9 @@ GRAPH_MAX_SHAPES = 8
 GRAPH_MAX_TOTAL_BYTES = 256 << 20
 GRAPH_MAX_SEEN = 64
 GRAPH_COUNTS = {"captured": 0, "replayed": 0}     # process-wide, for tests and diagnostics
+# The layer-local modes score all layers of a group in one launch sequence as long as its scratch (raw
+# scores of every layer) stays below this many bytes; longer requests go in runs of layers that do.
+LAYER_RUN_MAX_SCRATCH_BYTES = 256 << 20
 
 
 class ResidentLaunchFailed(RuntimeError):
@@ -291,31 +294,60 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
                 "group_agg_mode": agg, "debug_group_layer_indices": list(layer_ids),
                 "debug_recent_count": _recent_count(total_tokens)}
 
+    # Every layer keeps its own set (per_layer: one list for all heads of a layer).
+    layer_local = mode in {"per_layer", "per_layer_per_head"} or semantics != "hf_aligned_global_per_head"
+
     def _compress_group_batch(*, layer_kv: list, block_size: int, requests: list,
                               allow_resident: bool = True) -> list:
         """Selection **and** compaction of several requests of one KV-cache group in one launch
         sequence (no counterpart in the reference, which walks the requests one by one,
         runner_compression_actions.py:24; per request the result equals what
-        ``_select_keep_indices_for_group_per_head`` followed by the per-head compaction gives).
+        ``_select_keep_indices_for_group_per_head`` -- in the layer-local modes ``_select_keep_indices`` of
+        every layer -- followed by the compaction gives).
 
         ``layer_kv``: [(layer_idx, kv_cache)] of the group; ``requests``: one dict per request
         with ``block_ids, total_tokens, prefill_len, protect_prefill, round_start, budget_total``
         and ``total_tokens > budget_total > 0``.  Returns the selector result dictionaries in
-        request order (``indices``: int32, valid until this selector's next step); the caches then hold
+        request order (``indices``: int32, valid until this selector's next step; one row per KV head, in the
+        layer-local modes per layer and KV head or, with one list per layer, per layer); the caches then hold
         the kept rows in slots ``0..k-1``.  Raises
         ``ResidentLaunchFailed`` with the caches of this group untouched when a wait inside the
         resident kernel expired; the caller repeats the call with ``allow_resident=False``, which
         takes the kernels that do not wait for each other."""
-        if mode != "per_head" or semantics != "hf_aligned_global_per_head":
-            raise RuntimeError("batched compression serves the per_head / hf_aligned_global_per_head mode only")
+        if layer_local and len(layer_kv) > 1:
+            run = _layers_per_run(layer_kv, requests)
+            if run < len(layer_kv):
+                parts = []
+                for i in range(0, len(layer_kv), run):
+                    part = _compress_layers(layer_kv[i:i + run], block_size, requests, False)
+                    parts.append([r["indices"].clone() for r in part])        # (the next run writes the same buffer)
+                return [dict(r, indices=torch.cat(rows)) for r, rows in zip(part, zip(*parts))]
+        return _compress_layers(layer_kv, block_size, requests, allow_resident)
+
+    def _layers_per_run(layer_kv: list, requests: list) -> int:
+        kv = _paged_kv([c for _, c in layer_kv])
+        score_heads, _ = _head_layout(kv.num_kv_heads)
+        longest = max(int(r["total_tokens"]) for r in requests)
+        # raw scores, selection scores and the folded coefficients of one layer
+        per_layer = 4 * len(requests) * (longest * (score_heads + kv.num_kv_heads) + score_heads * 3 * kv.head_dim // 2)
+        return max(1, min(len(layer_kv), LAYER_RUN_MAX_SCRATCH_BYTES // per_layer))
+
+    def _compress_layers(layer_kv: list, block_size: int, requests: list, allow_resident: bool) -> list:
         agg = os.environ.get("TRIATTN_RUNTIME_DEBUG_GROUP_PERHEAD_AGG_MODE", "mean").strip().lower()
         if agg not in {"mean", "max"}:
             agg = "mean"
+        shared = mode == "per_layer"
         layer_ids = tuple(int(li) for li, _ in layer_kv)
         kv = _paged_kv([c for _, c in layer_kv])
         if int(kv.block_size) != int(block_size):
             raise RuntimeError("layers of one KV-cache group must share one block size")
-        score_heads, _ = _head_layout(kv.num_kv_heads)
+        score_heads, group_reduce = _head_layout(kv.num_kv_heads)
+        if layer_local:
+            # One launch sequence whose layers are independent: the score-then-select kernels spread it
+            # over the chip, and no status word has to be waited for.
+            agg, allow_resident = None, False
+        else:
+            group_reduce = "max"
         st = _stats()
         omega, offsets = st.vectors(kv.device)
         sc = ops.ScoreConfig(st.folded(layer_ids, score_heads, kv.device), omega, offsets,
@@ -328,7 +360,8 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
         rounds = [int(r["round_start"]) for r in requests]
         tables = [[int(x) for x in r["block_ids"]] for r in requests]
         use_resident = bool(allow_resident) and holder.get("resident_ok", True)
-        rows = len(requests) * kv.num_kv_heads
+        rows_per_request = (len(layer_ids) if layer_local else 1) * (1 if shared else kv.num_kv_heads)
+        rows = len(requests) * rows_per_request
         # A long generation repeats one shape (budget + divide_length tokens down to budget) every
         # divide_length tokens.  The second time a shape is seen its launch sequence is captured into
         # a HIP graph over device arrays that stay put; from then on a step is one small pinned copy
@@ -356,8 +389,8 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
                 batch = ops.StepBatch(kv.device, totals, round_start=rounds, budgets=ks, block_tables=tables,
                                       prefill_lens=guards)
                 sel = ops.SelectConfig(normalize=config.sparse_normalize_scores, window_size=config.window_size,
-                                       protect_prefill=any(g > 0 for g in guards), group_reduce="max", layer_reduce=agg,
-                                       allow_resident=use_resident)
+                                       protect_prefill=any(g > 0 for g in guards), group_reduce=group_reduce,
+                                       layer_reduce=agg, shared=shared, allow_resident=use_resident)
                 resident = ops.select_path(kv, batch, sc, sel) != "two_pass"
                 if not (GRAPH_REPLAY and key in seen):
                     # Scratch and keep rows of the previous step are reused when they fit; the results
@@ -396,16 +429,18 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
             raise RuntimeError(f"{MARK}:score_failed:{type(exc).__name__}") from exc
         if resident and _resident_failed(ws.status()):
             raise ResidentLaunchFailed("a wait inside the resident kernel expired; the caches were left untouched")
-        h = kv.num_kv_heads
         # The per-request indices are int32 views of a buffer this selector writes again at its next
         # step (the hook reads their shape only; a caller that keeps them copies them).
-        return [{"mode": "per_head", "indices": keep[b * h:(b + 1) * h, :k],
+        kept = [keep[b * rows_per_request:(b + 1) * rows_per_request, :k] for b, k in enumerate(ks)]
+        if layer_local:
+            return [{"mode": "shared" if shared else "per_head", "indices": idx} for idx in kept]
+        return [{"mode": "per_head", "indices": idx,
                  "semantic": "hf_aligned_global_per_head", "group_agg_mode": agg,
                  "debug_group_layer_indices": list(layer_ids), "debug_recent_count": _recent_count(t)}
-                for b, (k, t) in enumerate(zip(ks, totals))]
+                for idx, t in zip(kept, totals)]
 
     setattr(_select_keep_indices, "_supports_paged", True)
     setattr(_select_keep_indices_for_group_per_head, "_supports_paged_group", True)
-    if mode == "per_head" and semantics == "hf_aligned_global_per_head":
-        setattr(_select_keep_indices_for_group_per_head, "_compress_batch", _compress_group_batch)
+    setattr(_select_keep_indices_for_group_per_head, "_compress_batch", _compress_group_batch)
+    setattr(_select_keep_indices_for_group_per_head, "_layer_local", layer_local)
     return _select_keep_indices, _select_keep_indices_for_group_per_head, "enabled"
