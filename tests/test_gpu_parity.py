@@ -485,7 +485,7 @@ def test_one_layer_of_a_per_layer_selection_takes_the_resident_kernel(tag, kw, f
 
 @pytest.mark.parametrize("width", [3000, 8192, 16384, 20001, 32768, 40000])
 def test_topk_rows_by_width(width):
-    """Rows up to 8192 / 16384 / 32768 elements are selected from registers (three kernel
+    """Rows up to 4096 / 8192 / 16384 / 32768 elements are selected from registers (four kernel
     instances), longer ones by the streaming kernel; ties keep the lowest index."""
     g = torch.Generator().manual_seed(width)
     x = torch.randn(6, width, generator=g)
@@ -506,6 +506,27 @@ def test_topk_rows_by_width(width):
         kk = min(k, n)
         if kk:
             assert torch.equal(got[r, :kk], osel.topk_ascending(x[r:r + 1, :n], kk)[0])
+
+
+@pytest.mark.parametrize("width", [1025, 4096, 4097, 16385, 32768])
+def test_topk_rows_bin_edges(width):
+    """The histogram pass cuts [min, max] of a row's finite scores into 2048 bins; rows where one bin
+    holds nearly everything (an outlier far away, a range beyond the largest float, subnormal steps),
+    more guarded tokens than the budget, and scores on both sides of zero."""
+    g = torch.Generator().manual_seed(width)
+    x = torch.randn(8, width, generator=g)
+    x[0, 7] = 3.0e38                              # one outlier: the rest shares the lowest bin
+    x[1, 3], x[1, 9] = 3.4e38, -3.4e38            # max - min is not a float
+    x[2] = torch.randint(0, 1 << 20, (width,), generator=g).float() * 1.4e-45   # subnormal spacing
+    x[3] = 1.0 + torch.randint(0, 3, (width,), generator=g).float() * 1.1920929e-07
+    x[4, : width // 2] = float("inf")             # more +inf than most budgets below
+    x[5, ::2] = float("-inf")
+    x[6] = -x[6].abs() * 1e-30
+    x[7, : width - 2] = float("-inf")
+    xd = x.to(DEV)
+    for k in (1, 2, width // 4, width // 2 + 1, width - 1):
+        got = ops.topk_rows(xd, k).cpu().long()
+        assert torch.equal(got[:, :k], osel.topk_ascending(x, k)), k
 
 
 def test_topk_rows_ties_and_order():

@@ -9,9 +9,10 @@
 //                          a KV head first, then normalise per (layer, KV head) with
 //                          core/utils.py:466-480 (torch mean / unbiased std).
 //  topk_rows_kernel      : order-preserving radix select on the monotone integer
-//                          image of the float, then an ordered compaction that emits
-//                          the kept token indices ascending; ties at the threshold
-//                          keep the lowest index (replaces torch.topk + chunk merge +
+//                          image of the float (rows held in registers: one histogram pass
+//                          over equal bins of the scores, then exact ranks inside one bin), then
+//                          an ordered compaction that emits the kept token indices ascending;
+//                          ties at the threshold keep the lowest index (replaces torch.topk + chunk merge +
 //                          torch.sort, runtime/selector_hf.py:990-1025).
 #include "tri_common.h"
 
@@ -427,20 +428,54 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_kernel(const float* sc
   }
 }
 
+// Wave-wide reductions (every lane gets the result).
+__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, off));
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
+  return v;
+}
+// Inverse of float_key.
+__device__ __forceinline__ float key_float(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+constexpr uint32_t kKeyInf = 0xff800000u;        // float_key(+inf); NaNs of positive sign lie above
+constexpr uint32_t kKeyFiniteMin = 0x00800000u;  // float_key(-FLT_MAX); -inf and NaNs of negative sign lie below
+constexpr int kTopkBins = 2048;
+constexpr int kTopkCand = kTopkThreads;          // candidates ranked by counting, one thread each
+
 // The same selection for rows of at most VPT * 1024 elements: the row is read once into
-// registers (thread t owns the contiguous elements [t*VPT, (t+1)*VPT), so the ordered
-// emission needs no second pass over memory), the 256-bin suffix sums of a radix pass are
-// taken by one wave with shuffles, and the final scan over threads is a wave scan plus 16
-// wave totals: 3 barriers per radix pass instead of 19.
+// registers.  A wave owns 64 * VPT consecutive elements, 64 at a time: loads are whole lines, and the
+// ascending emission counts with ballots (a lane's place is the number of kept lanes below it) and
+// writes runs of consecutive indices.  (With a thread owning VPT consecutive elements every store of the
+// emission went to 64 different lines.)
+//
+// A few rows on a few CUs: the time is the chain of barriers and LDS round trips, not the
+// bytes.  The threshold is found in one histogram pass: the finite scores are
+// cut into 2048 bins of equal width between their minimum and maximum ((x - lo) * scale,
+// rounded, is monotone in x, so the bins are ordered as the scores are), a scan over all
+// threads finds the bin of the k-th largest, and the few scores of that bin are ranked
+// against each other, one thread per candidate, on their exact keys.  Guarded tokens (+inf)
+// are counted apart, they would stretch the bins.  A bin of more than 1024 scores (rows with
+// many equal scores, or a few outliers far away) falls back to radix passes of 8 bits over its keys.
+// Seven barriers; with radix passes alone it was thirteen, around scans by a single wave.
+// 8 rows of 4096: 13.1 -> 6.9 us; 8 rows of 2176 added up from 36 groups: 21.7 -> 14.3; 192 rows
+// of up to 12001: 24.7 -> 12.3; 8 rows of 32768: 47.8 -> 25.3 (there the instructions of one CU bound it).
 template <int VPT>
 __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float* scores, int64_t row_pitch,
                                                                     const int32_t* row_lens,
                                                                     const int32_t* row_ks, int rows_per_entry,
                                                                     int32_t* keep, int keep_pitch, int max_len,
                                                                     int groups, int64_t group_stride, int group_max) {
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t sh_prefix, sh_remaining;
-  __shared__ uint32_t wave_tot[kTopkThreads / 64];
+  constexpr int kWaves = kTopkThreads / 64;
+  __shared__ uint32_t hist[kTopkBins];
+  __shared__ __align__(16) uint32_t cand[kTopkCand];
+  __shared__ uint32_t wave_lo[kWaves], wave_hi[kWaves], wave_tot[kWaves];
+  __shared__ uint32_t sh_high, sh_ncand, sh_prefix, sh_remaining, sh_count;
 
   const int row = blockIdx.x;
   const int entry = row / rows_per_entry;
@@ -459,8 +494,11 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
     return;
   }
 
-  const int c0 = tid * VPT;
-  const int nvalid = min(max(T - c0, 0), VPT);
+  const int e0 = wave * (64 * VPT) + lane;        // element i of this thread: e0 + 64 * i
+  const int nvalid = min(max((T - e0 + 63) / 64, 0), VPT);
+  // Key 0 is "no element" (the one NaN pattern whose key it would be shares the next key), so nothing below
+  // asks for an element's place in the row again.
+  auto row_key = [](float f) __attribute__((always_inline)) { return max(float_key(f), 1u); };
   uint32_t key[VPT];
   if (groups > 1) {
     // The row arrives as `groups` partial rows `group_stride` floats apart (a resident launch cut
@@ -468,69 +506,163 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
     // fused_layer_reduce_kernel does; the division by the layer count that turns the sum into a
     // mean does not change the order of the scores and is left out.
     // The rows of several groups are requested before the first is added (a thread's loads of one
-    // group after the other, each waited for, made 36 groups of a single request take 30 us).
-    constexpr int U = VPT >= 32 ? 1 : (VPT >= 16 ? 2 : 4);            // groups in flight per round
-    const bool vec = nvalid == VPT && (reinterpret_cast<uintptr_t>(x + c0) & 15) == 0 && (group_stride & 3) == 0;
+    // group after the other, each waited for, made 36 groups of a single request take 30 us); the last
+    // round repeats the last group where there is none left and leaves it out of the sum.
+    constexpr int U = VPT >= 32 ? 1 : (VPT >= 16 ? 3 : (VPT >= 8 ? 6 : 12));   // groups in flight per round
     auto load_row = [&](int g, float (&y)[VPT]) __attribute__((always_inline)) {
-      const float* p = x + (int64_t)g * group_stride + c0;
-      if (vec) {
+      const float* p = x + (int64_t)g * group_stride;
 #pragma unroll
-        for (int i = 0; i < VPT; i += 4) {
-          const float4 q = *reinterpret_cast<const float4*>(p + i);
-          y[i] = q.x; y[i + 1] = q.y; y[i + 2] = q.z; y[i + 3] = q.w;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) y[i] = i < nvalid ? p[i] : 0.f;
-      }
+      for (int i = 0; i < VPT; ++i) y[i] = p[min(e0 + 64 * i, T - 1)];
     };
     float v[VPT];
     load_row(0, v);
-    int g = 1;
-    for (; g + U <= groups; g += U) {
+    for (int g = 1; g < groups; g += U) {
       float y[U][VPT];
 #pragma unroll
-      for (int u = 0; u < U; ++u) load_row(g + u, y[u]);
+      for (int u = 0; u < U; ++u) load_row(min(g + u, groups - 1), y[u]);
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+      for (int u = 0; u < U; ++u) {
+        if (g + u >= groups) continue;
 #pragma unroll
         for (int i = 0; i < VPT; ++i) v[i] = group_max ? fmaxf(v[i], y[u][i]) : __fadd_rn(v[i], y[u][i]);
-    }
-    for (; g < groups; ++g) {
-      float y[VPT];
-      load_row(g, y);
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) v[i] = group_max ? fmaxf(v[i], y[i]) : __fadd_rn(v[i], y[i]);
+      }
     }
 #pragma unroll
-    for (int i = 0; i < VPT; ++i) key[i] = i < nvalid ? float_key(v[i]) : 0u;
-  } else if (nvalid == VPT && (reinterpret_cast<uintptr_t>(x + c0) & 15) == 0) {
-#pragma unroll
-    for (int i = 0; i < VPT; i += 4) {
-      const float4 v = *reinterpret_cast<const float4*>(x + c0 + i);
-      key[i] = float_key(v.x); key[i + 1] = float_key(v.y); key[i + 2] = float_key(v.z); key[i + 3] = float_key(v.w);
-    }
+    for (int i = 0; i < VPT; ++i) key[i] = i < nvalid ? row_key(v[i]) : 0u;
   } else {
 #pragma unroll
-    for (int i = 0; i < VPT; ++i) key[i] = i < nvalid ? float_key(x[c0 + i]) : 0u;
+    for (int i = 0; i < VPT; ++i) key[i] = __float_as_uint(x[min(e0 + 64 * i, T - 1)]);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) key[i] = i < nvalid ? row_key(__uint_as_float(key[i])) : 0u;
   }
 
-  // ---- radix select of the k-th largest key, 8 bits per pass from the top.
-  uint32_t prefix = 0, mask = 0, remaining = (uint32_t)k;
-  for (int shift = 24; shift >= 0; shift -= 8) {
-    if (tid < 256) hist[tid] = 0;
-    __syncthreads();
-    // Selection scores are sums of z-scores of similar size, so the leading digit (sign and the top
-    // exponent bits) takes three or four values in a whole row and the first pass would send all 64
-    // lanes of every atomic to the same few counters, one after the other.  The lanes of a wave that
-    // hold the same digit are counted with a ballot and added once (up to four distinct digits per
-    // round; what is left, and the later passes, whose digits are spread, take the plain atomics).
+  // ---- range of the finite scores, number of scores at or above +inf.
+  uint32_t lo_key = 0xffffffffu, hi_key = 0u;
+  int high = 0;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const bool fin = key[i] - kKeyFiniteMin < kKeyInf - kKeyFiniteMin;
+    lo_key = min(lo_key, fin ? key[i] : 0xffffffffu);
+    hi_key = max(hi_key, fin ? key[i] : 0u);
+    high += __popcll(__ballot(key[i] >= kKeyInf));
+  }
+  lo_key = wave_min(lo_key);
+  hi_key = wave_max(hi_key);
+  if (lane == 0) {
+    wave_lo[wave] = lo_key;
+    wave_hi[wave] = hi_key;
+    wave_tot[wave] = (uint32_t)high;
+  }
+  for (int i = tid; i < kTopkBins; i += kTopkThreads) hist[i] = 0;
+  if (tid == 0) sh_ncand = 0;
+  __syncthreads();
+  uint32_t above = 0;                            // scores at or above +inf in the row
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    lo_key = min(lo_key, wave_lo[w]);
+    hi_key = max(hi_key, wave_hi[w]);
+    above += wave_tot[w];
+  }
+  // A row without a finite score has lo_key > hi_key: everything else then falls into bin 0.
+  const float lo = lo_key <= hi_key ? key_float(lo_key) : 0.f;
+  const float width = lo_key <= hi_key ? __fsub_rn(key_float(hi_key), lo) : 0.f;
+  // (a width beyond the largest float is +inf and puts everything into bin 0 as well)
+  const float scale = width > 0.f ? fminf(__fdiv_rn((float)kTopkBins, width), 3.0e38f) : 0.f;
+  auto bin_of = [&](uint32_t kk) __attribute__((always_inline)) {
+    const float t = __fmul_rn(__fsub_rn(key_float(kk), lo), scale);
+    const int b = kk < kKeyFiniteMin ? 0 : (int)fminf(t, (float)(kTopkBins - 1));
+    return (uint32_t)b;
+  };
+
+  // ---- which scores the k-th largest is among, and how many of those are kept.
+  uint32_t remaining = (uint32_t)k, count;
+  uint32_t cmask = 0;                            // bit i: element i is a candidate
+  if (above >= (uint32_t)k) {                    // (the same for the whole workgroup)
+    count = above;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) cmask |= (uint32_t)(key[i] >= kKeyInf) << i;
+  } else {
+    remaining -= above;
+    uint32_t bins[VPT / 2];                      // two per register; 0xffff: none
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const bool part = i < nvalid && (key[i] & mask) == prefix;
-      const uint32_t digit = (key[i] >> shift) & 255u;
-      unsigned long long todo = __ballot(part);
-      if (shift == 24) {
+      const bool ok = key[i] - 1u < kKeyInf - 1u;
+      const uint32_t b = ok ? bin_of(key[i]) : 0xffffu;
+      if (ok) atomicAdd(&hist[b], 1u);
+      bins[i / 2] = (i & 1) ? bins[i / 2] | (b << 16) : b;
+    }
+    __syncthreads();
+    constexpr int BPT = kTopkBins / kTopkThreads;   // bins per thread
+    uint32_t h[BPT], own = 0;
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) { h[j] = hist[tid * BPT + j]; own += h[j]; }
+    uint32_t suffix = own;                         // scores in the bins of lanes >= this one
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t v = __shfl_down(suffix, off);
+      if (lane + off < 64) suffix += v;
+    }
+    if (lane == 0) wave_lo[wave] = suffix;         // (read by everyone before the barrier above)
+    __syncthreads();
+    uint32_t gt = suffix - own;
+    for (int w = wave + 1; w < kWaves; ++w) gt += wave_lo[w];
+#pragma unroll
+    for (int j = BPT - 1; j >= 0; --j) {
+      const uint32_t ge = gt + h[j];
+      if (gt < remaining && remaining <= ge) {     // exactly one bin satisfies this
+        sh_prefix = (uint32_t)(tid * BPT + j);
+        sh_remaining = remaining - gt;
+        sh_count = h[j];
+      }
+      gt = ge;
+    }
+    __syncthreads();
+    const uint32_t bin = sh_prefix;
+    remaining = sh_remaining;
+    count = sh_count;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+      cmask |= (uint32_t)(((bins[i / 2] >> (16 * (i & 1))) & 0xffffu) == bin) << i;
+  }
+
+  // ---- the k-th largest among the candidates.
+  if (count <= (uint32_t)kTopkCand) {
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+      if ((cmask >> i) & 1u) cand[atomicAdd(&sh_ncand, 1u)] = key[i];
+    __syncthreads();
+    if ((uint32_t)tid < count) {
+      const uint32_t mine = cand[tid];
+      uint32_t gt = 0, ge = 0;
+      uint32_t i = 0;
+      for (; i + 4 <= count; i += 4) {
+        const uint4 c = *reinterpret_cast<const uint4*>(&cand[i]);
+        gt += (c.x > mine) + (c.y > mine) + (c.z > mine) + (c.w > mine);
+        ge += (c.x >= mine) + (c.y >= mine) + (c.z >= mine) + (c.w >= mine);
+      }
+      for (; i < count; ++i) { gt += cand[i] > mine; ge += cand[i] >= mine; }
+      if (gt < remaining && remaining <= ge) {     // candidates with this very key, and only they
+        sh_high = mine;
+        sh_count = remaining - gt;
+      }
+    }
+    __syncthreads();
+  } else {
+    // Radix select over the candidates' keys, 8 bits per pass from the top.
+    uint32_t prefix = 0, mask = 0;
+    for (int shift = 24; shift >= 0; shift -= 8) {
+      __syncthreads();
+      if (tid < 256) hist[tid] = 0;
+      __syncthreads();
+      // Keys of one bin are close together, so the leading digits take one or two values and the plain
+      // atomics of a wave would go to the same counter one after the other: the lanes that hold
+      // the same digit are counted with a ballot and added once (up to four distinct digits per
+      // round; what is left takes the plain atomics).
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) {
+        const bool part = ((cmask >> i) & 1u) && (key[i] & mask) == prefix;
+        const uint32_t digit = (key[i] >> shift) & 255u;
+        unsigned long long todo = __ballot(part);
         for (int it = 0; it < 4 && todo; ++it) {
           const int leader = __builtin_amdgcn_readfirstlane(__ffsll((long long)todo) - 1);
           const uint32_t dl = (uint32_t)__builtin_amdgcn_readlane((int)digit, leader);
@@ -538,75 +670,69 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
           if (lane == leader) atomicAdd(&hist[dl], (uint32_t)__popcll(same));
           todo &= ~same;
         }
+        if ((todo >> lane) & 1ull) atomicAdd(&hist[digit], 1u);
       }
-      if ((todo >> lane) & 1ull) atomicAdd(&hist[digit], 1u);
-    }
-    __syncthreads();
-    if (wave == 0) {
-      // lane owns bins 4*lane .. 4*lane+3; ge[j] = candidates whose digit is >= that bin
-      uint32_t h[4];
+      __syncthreads();
+      if (wave == 0) {
+        // lane owns bins 4*lane .. 4*lane+3
+        uint32_t h[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) h[j] = hist[4 * lane + j];
-      const uint32_t own = h[0] + h[1] + h[2] + h[3];
-      uint32_t suffix = own;                         // sum over lanes >= lane
+        for (int j = 0; j < 4; ++j) h[j] = hist[4 * lane + j];
+        const uint32_t own = h[0] + h[1] + h[2] + h[3];
+        uint32_t suffix = own;                         // sum over lanes >= lane
 #pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t v = __shfl_down(suffix, off);
-        if (lane + off < 64) suffix += v;
-      }
-      uint32_t gt = suffix - own;                    // digits above this lane's bins
-#pragma unroll
-      for (int j = 3; j >= 0; --j) {
-        const uint32_t ge = gt + h[j];
-        if (gt < remaining && remaining <= ge) {     // exactly one bin satisfies this
-          sh_prefix = prefix | ((uint32_t)(4 * lane + j) << shift);
-          sh_remaining = remaining - gt;
+        for (int off = 1; off < 64; off <<= 1) {
+          const uint32_t v = __shfl_down(suffix, off);
+          if (lane + off < 64) suffix += v;
         }
-        gt = ge;
+        uint32_t gt = suffix - own;                    // digits above this lane's bins
+#pragma unroll
+        for (int j = 3; j >= 0; --j) {
+          const uint32_t ge = gt + h[j];
+          if (gt < remaining && remaining <= ge) {     // exactly one bin satisfies this
+            sh_high = prefix | ((uint32_t)(4 * lane + j) << shift);
+            sh_count = remaining - gt;
+          }
+          gt = ge;
+        }
       }
+      __syncthreads();
+      prefix = sh_high;
+      remaining = sh_count;
+      mask |= 255u << shift;
     }
-    __syncthreads();
-    prefix = sh_prefix;
-    remaining = sh_remaining;
-    mask |= 255u << shift;
   }
-  const uint32_t thr = prefix;        // key of the k-th largest element
-  const uint32_t need_eq = remaining; // how many elements equal to it are kept (lowest index first)
+  const uint32_t thr = sh_high;        // key of the k-th largest element
+  const uint32_t need_eq = sh_count;   // how many elements equal to it are kept (lowest index first)
 
-  // ---- ordered compaction.  Counts of (greater, equal) packed as (g << 16) | e: a row has
-  // at most 32768 elements, so neither half overflows.
-  uint32_t g = 0, e = 0;
+  // ---- ordered compaction.  Counts of (greater, equal) of the wave packed as (g << 16) | e: a row has
+  // at most 32768 elements.  Elements beyond the row hold key 0, which the threshold never is.
+  uint32_t mine = 0;
 #pragma unroll
-  for (int i = 0; i < VPT; ++i) {
-    if (i < nvalid) {
-      g += key[i] > thr;
-      e += key[i] == thr;
-    }
-  }
-  const uint32_t mine = (g << 16) | e;
-  uint32_t incl = mine;                              // inclusive scan inside the wave
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t v = __shfl_up(incl, off);
-    if (lane >= off) incl += v;
-  }
-  if (lane == 63) wave_tot[wave] = incl;
+  for (int i = 0; i < VPT; ++i)
+    mine += ((uint32_t)__popcll(__ballot(key[i] > thr)) << 16) + (uint32_t)__popcll(__ballot(key[i] == thr));
+  if (lane == 0) wave_tot[wave] = mine;
   __syncthreads();
-  uint32_t before = incl - mine;
+  uint32_t before = 0;
   for (int w = 0; w < wave; ++w) before += wave_tot[w];
-  const uint32_t gt_before = before >> 16;
   uint32_t eq_before = before & 0xffffu;
-  uint32_t pos = gt_before + min(eq_before, need_eq);
+  uint32_t pos = (before >> 16) + min(eq_before, need_eq);
+  auto lanes_below = [](unsigned long long m) __attribute__((always_inline)) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+  };
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    if (i < nvalid) {
-      if (key[i] > thr) {
-        out[pos++] = c0 + i;
-      } else if (key[i] == thr) {
-        if (eq_before < need_eq) out[pos++] = c0 + i;
-        ++eq_before;
-      }
+    unsigned long long km = __ballot(key[i] > thr);
+    bool kept = key[i] > thr;
+    const unsigned long long em = __ballot(key[i] == thr);
+    if (em != 0) {                               // (wave-uniform, rarely taken)
+      const bool eq = key[i] == thr && eq_before + lanes_below(em) < need_eq;
+      kept = kept || eq;
+      km |= __ballot(eq);
+      eq_before += (uint32_t)__popcll(em);
     }
+    if (kept) out[pos + lanes_below(km)] = e0 + 64 * i;
+    pos += (uint32_t)__popcll(km);
   }
 }
 
@@ -617,7 +743,10 @@ hipError_t launch_topk_rows(const float* scores, int64_t row_pitch, int num_rows
                             int32_t* keep, int keep_pitch, hipStream_t s, int groups, int64_t group_stride,
                             int group_max) {
   if (num_rows <= 0) return hipSuccess;
-  if (max_len > 0 && max_len <= 8 * kTopkThreads)
+  if (max_len > 0 && max_len <= 4 * kTopkThreads)
+    hipLaunchKernelGGL(topk_rows_reg_kernel<4>, dim3(num_rows), dim3(kTopkThreads), 0, s, scores, row_pitch, row_lens,
+                       row_ks, rows_per_entry, keep, keep_pitch, max_len, groups, group_stride, group_max);
+  else if (max_len > 0 && max_len <= 8 * kTopkThreads)
     hipLaunchKernelGGL(topk_rows_reg_kernel<8>, dim3(num_rows), dim3(kTopkThreads), 0, s, scores, row_pitch, row_lens,
                        row_ks, rows_per_entry, keep, keep_pitch, max_len, groups, group_stride, group_max);
   else if (max_len > 0 && max_len <= 16 * kTopkThreads)
