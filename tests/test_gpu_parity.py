@@ -1356,6 +1356,30 @@ def test_resident_path_falls_back_when_shape_has_no_kernel(monkeypatch):
         assert torch.equal(keep_a, keep_b) and torch.equal(fin_a[:, :300], fin_b[:, :300])
 
 
+@pytest.mark.parametrize("kw", [
+    dict(num_q_heads=32, num_kv_heads=8),
+    dict(num_q_heads=24, num_kv_heads=8, block_size=1),
+    dict(num_q_heads=10, num_kv_heads=5, head_dim=128, kv_dtype="fp8"),
+    dict(num_q_heads=24, num_kv_heads=3, head_dim=256),
+], ids=["gqa4", "token_blocks", "five_heads_fp8", "d256_gqa8"])
+@pytest.mark.parametrize("lens", [(1,), (127, 2), (128, 129), (513, 31, 4), (511, 1025)])
+def test_quarter_tile_scores_give_the_sums_of_whole_tiles(kw, lens):
+    """A small launch that scores and selects in one call cuts its tiles in four; scored and selected by
+    two calls it walks whole tiles.  The statistics, and so the selection scores, are the same bits."""
+    w = small(seq_lens=lens, budget=1, window_size=0, **kw)
+    inp = build_inputs(w)
+    caches, kv, batch, sc = device_objects(w, inp, DEV)
+    sel = ops.SelectConfig(window_size=0, allow_resident=False)
+    print(f"quarter tiles {kw} {lens}", flush=True)
+    keep_a, fin_a, _ = ops.select_paged(kv, batch, sc, sel, want_scores=True)
+    raw, ws = ops.score_paged(kv, batch, sc)
+    keep_b, fin_b = ops.select(kv, batch, sc, sel, raw, ws, want_scores=True)
+    h = w.num_kv_heads
+    assert torch.equal(keep_a, keep_b)
+    for b, t in enumerate(lens):
+        assert torch.equal(fin_a[b * h:(b + 1) * h, :t], fin_b[b * h:(b + 1) * h, :t]), (b, t)
+
+
 def test_fp8_every_code_decodes_like_torch():
     """All 254 finite e4m3 codes through the scorer: with one non-zero coefficient the
     score is code_value * scale * coefficient, which pins the decoder against torch's

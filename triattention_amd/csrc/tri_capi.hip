@@ -203,23 +203,23 @@ T* at(void* ws, int64_t off) { return reinterpret_cast<T*>(reinterpret_cast<char
 
 int do_score(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp, float* raw,
              int64_t rs_layer, int64_t rs_token, int64_t rs_head, void* ws, const tri::Workspace& w,
-             hipStream_t s) {
+             hipStream_t s, int fine, float* partial, uint32_t* status) {
   const int F = kv->head_dim / 2;
   hipError_t e = tri::launch_prepare(sp->folded, sp->omega, sp->offsets, sp->num_offsets, batch->round_start,
                                      batch->num_seqs, kv->num_layers, sp->num_score_heads, F, sp->aggregation,
-                                     at<float>(ws, w.coef), at<float>(ws, w.trig), s);
+                                     at<float>(ws, w.coef), at<float>(ws, w.trig), status, s);
   if (e != hipSuccess) return launch_status(e, "prepare");
   tri::ScoreLaunch a{};
   a.B = batch->num_seqs; a.L = kv->num_layers; a.Hkv = kv->num_kv_heads; a.D = kv->head_dim;
   a.block_size = kv->block_size; a.kv_dtype = kv->kv_dtype; a.rope_style = kv->rope_style;
   a.A = sp->num_score_heads; a.G = sp->num_score_heads / kv->num_kv_heads; a.NO = sp->num_offsets;
   a.aggregation = sp->aggregation;
-  a.Tmax = batch->max_seq_len; a.num_tiles = w.num_tiles;
+  a.Tmax = batch->max_seq_len; a.fine = fine;
   a.stride_block = kv->stride_block; a.stride_token = kv->stride_token; a.stride_head = kv->stride_head;
   a.k_layers = kv->k_layers; a.k_scale_layers = kv->k_scale_layers;
   a.block_table = batch->block_table; a.block_table_pitch = batch->block_table_pitch;
   a.seq_lens = batch->seq_lens;
-  a.coef = at<float>(ws, w.coef); a.trig = at<float>(ws, w.trig); a.partial = at<float>(ws, w.partial);
+  a.coef = at<float>(ws, w.coef); a.trig = at<float>(ws, w.trig); a.partial = partial;
   a.raw = raw; a.raw_stride_layer = rs_layer; a.raw_stride_token = rs_token; a.raw_stride_head = rs_head;
   return launch_status(tri::launch_score(a, s), "score");
 }
@@ -239,16 +239,17 @@ int check_select(const tri_select_params* sel) {
 
 int do_select(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
               const tri_select_params* sel, const float* raw, int64_t rs_layer, int64_t rs_token,
-              int64_t rs_head, float* fin, int32_t* keep, void* ws, const tri::Workspace& w, hipStream_t s) {
+              int64_t rs_head, float* fin, int32_t* keep, void* ws, const tri::Workspace& w, hipStream_t s,
+              int fine, const float* partial) {
   tri::SelectLaunch a{};
   a.B = batch->num_seqs; a.L = kv->num_layers; a.Hkv = kv->num_kv_heads; a.A = sp->num_score_heads;
-  a.G = sp->num_score_heads / kv->num_kv_heads; a.Tmax = batch->max_seq_len; a.num_tiles = w.num_tiles;
+  a.G = sp->num_score_heads / kv->num_kv_heads; a.Tmax = batch->max_seq_len; a.fine = fine;
   a.max_budget = batch->max_budget;
   a.normalize = sel->normalize; a.window_size = sel->window_size; a.protect_prefill = sel->protect_prefill;
   a.group_reduce = sel->group_reduce; a.layer_reduce = sel->layer_reduce; a.shared = sel->shared;
   a.group_first = sel->group_first ? 1 : 0;
   a.seq_lens = batch->seq_lens; a.prefill_lens = batch->prefill_lens; a.budgets = batch->budgets;
-  a.partial = at<float>(ws, w.partial); a.mustd = at<float>(ws, w.mustd);
+  a.partial = partial; a.mustd = at<float>(ws, w.mustd);
   a.raw = raw; a.raw_stride_layer = rs_layer; a.raw_stride_token = rs_token; a.raw_stride_head = rs_head;
   a.fin = fin ? fin : at<float>(ws, w.fin);
   a.keep = keep;
@@ -275,22 +276,28 @@ int do_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_s
                     hipStream_t s) {
   const bool fused = takes_resident(w, kv, sel);
   if (!fused) {
-    // The status word belongs to the resident kernel; on this path it just reads "fine".
-    const hipError_t ce = tri::launch_clear_status(at<uint32_t>(ws, w.status), s);
-    if (ce != hipSuccess) return launch_status(ce, "clear_status");
     float* raw = at<float>(ws, w.raw);
     const int64_t A = sp->num_score_heads;
     const int64_t rs_layer = (int64_t)batch->max_seq_len * A;
-    const int rc = do_score(kv, batch, sp, raw, rs_layer, A, 1, ws, w, s);
+    // Sums per quarter tile take more room than the workspace plans; they go where the selection scores
+    // are written later (the statistics are finished by then).
+    const int64_t sums = (int64_t)batch->num_seqs * kv->num_layers * A *
+                         tri::ceil_div(batch->max_seq_len, tri::kScoreFineTokens) * 4 * 4;
+    const int fine = sums <= w.xchg - w.fin &&
+                     tri::score_takes_fine(batch->num_seqs, kv->num_layers, kv->num_kv_heads, kv->head_dim,
+                                           (int)A / kv->num_kv_heads, batch->max_seq_len, sp->aggregation);
+    float* partial = at<float>(ws, fine ? w.fin : w.partial);
+    // The status word belongs to the resident kernel; on this path it just reads "fine".
+    const int rc = do_score(kv, batch, sp, raw, rs_layer, A, 1, ws, w, s, fine, partial, at<uint32_t>(ws, w.status));
     if (rc) return rc;
-    return do_select(kv, batch, sp, sel, raw, rs_layer, A, 1, fin, keep, ws, w, s);
+    return do_select(kv, batch, sp, sel, raw, rs_layer, A, 1, fin, keep, ws, w, s, fine, partial);
   }
   const int F = kv->head_dim / 2;
   hipError_t e = hipSuccess;
   if (w.fused.eligible != 2) {   // the matrix-core kernel has a preparation launch of its own
     e = tri::launch_prepare(sp->folded, sp->omega, sp->offsets, sp->num_offsets, batch->round_start,
                             batch->num_seqs, kv->num_layers, sp->num_score_heads, F, sp->aggregation,
-                            at<float>(ws, w.coef), at<float>(ws, w.trig), s);
+                            at<float>(ws, w.coef), at<float>(ws, w.trig), nullptr, s);
     if (e != hipSuccess) return launch_status(e, "prepare");
   }
   tri::FusedLaunch a{};
@@ -482,7 +489,7 @@ int tri_score_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_s
   rc = check_workspace(w, workspace, workspace_bytes);
   if (rc) return rc;
   return do_score(kv, batch, sp, raw, raw_stride_layer, raw_stride_token, raw_stride_head, workspace, w,
-                  (hipStream_t)stream);
+                  (hipStream_t)stream, 0, at<float>(workspace, w.partial), nullptr);
 }
 
 int tri_select(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
@@ -502,7 +509,7 @@ int tri_select(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_
   rc = check_workspace(w, workspace, workspace_bytes);
   if (rc) return rc;
   return do_select(kv, batch, sp, sel, raw, raw_stride_layer, raw_stride_token, raw_stride_head, final_scores,
-                   keep, workspace, w, (hipStream_t)stream);
+                   keep, workspace, w, (hipStream_t)stream, 0, at<float>(workspace, w.partial));
 }
 
 int tri_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,

@@ -11,6 +11,7 @@ namespace tri {
 constexpr int kWave = 64;
 constexpr int kScoreThreads = 256;      // 4 waves per scorer workgroup
 constexpr int kScoreTileTokens = 512;   // tokens of one (sequence, layer) per scorer workgroup
+constexpr int kScoreFineTokens = 128;   // of a small launch: one wave's part of a tile
 constexpr int kQPerPass = 4;            // query heads scored per wave pass
 constexpr int kPairsPerLane = 8;        // frequency pairs held by one lane
 constexpr int kMaxOffsets = 32;
@@ -96,7 +97,7 @@ inline Workspace plan_workspace(int B, int L, int A, int F, int NO, int Hkv, int
 struct ScoreLaunch {
   // geometry
   int B, L, Hkv, D, block_size, kv_dtype, rope_style, A, G, NO, aggregation;
-  int Tmax, num_tiles;
+  int Tmax, fine;       // fine: quarter tiles (score_takes_fine)
   int64_t stride_block, stride_token, stride_head;
   const void* const* k_layers;
   const float* const* k_scale_layers;
@@ -105,7 +106,7 @@ struct ScoreLaunch {
   const int32_t* seq_lens;
   const float* coef;     // workspace
   const float* trig;     // workspace
-  float* partial;        // workspace
+  float* partial;        // workspace: [B][L][tiles][A][2]; fine: [B][L][quarter tiles][A][4]
   float* raw;
   int64_t raw_stride_layer, raw_stride_token, raw_stride_head;
 };
@@ -115,11 +116,12 @@ hipError_t launch_fold_stats(const float* qr, const float* qi, const float* qabs
                              hipStream_t s);
 hipError_t launch_prepare(const float* folded, const float* omega, const float* offsets, int NO,
                           const int32_t* round_start, int B, int L, int A, int F, int aggregation,
-                          float* coef, float* trig, hipStream_t s);
+                          float* coef, float* trig, uint32_t* status, hipStream_t s);
+bool score_takes_fine(int B, int L, int Hkv, int D, int G, int Tmax, int aggregation);
 hipError_t launch_score(const ScoreLaunch& a, hipStream_t s);
 
 struct SelectLaunch {
-  int B, L, Hkv, A, G, Tmax, num_tiles, max_budget;
+  int B, L, Hkv, A, G, Tmax, fine, max_budget;
   int normalize, window_size, protect_prefill, group_reduce, layer_reduce, shared, group_first;
   const int32_t* seq_lens;
   const int32_t* prefill_lens;
@@ -136,7 +138,6 @@ struct SelectLaunch {
   int64_t group_scratch_bytes;
 };
 hipError_t launch_select(const SelectLaunch& a, hipStream_t s);
-hipError_t launch_clear_status(uint32_t* status, hipStream_t s);
 // groups > 1: row r is the sum (group_max: maximum) of `groups` partial rows group_stride floats apart,
 // added while loading (rows of at most topk_register_row_limit() elements).
 hipError_t launch_topk_rows(const float* scores, int64_t row_pitch, int num_rows,

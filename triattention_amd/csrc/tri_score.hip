@@ -113,10 +113,18 @@ __device__ __forceinline__ RowData load_row(const ScoreArgs& a, const char* kbas
 // ------------------------------------------------------------------ mean
 // UNI: one token per wave iteration (the KV heads fill the wave's rows) and the tokens
 // of a stage share a block (or the keys are dense): scalar addressing, buffer loads.
-template <int LPH, int DT, bool IL, int SP, bool UNI>
+// FINE (LPH >= 8, one token per wave iteration): a workgroup takes 128 tokens, a quarter of a tile, which is
+// what one wave of a whole-tile workgroup walks alone; its four waves leave their scores in LDS and one of
+// them adds those up in that wave's order, so the sums are the same to the last bit whichever form runs.  A
+// launch of few workgroups is bound by the instructions of one wave's walk (~180 per token) while most of the chip
+// idles: 36 layers x 2176 tokens 58 -> 43 us (every token still costs its ~180 instructions, on 256 CUs that get two or three workgroups each).
+template <int LPH, int DT, bool IL, int SP, bool UNI, bool FINE>
 __global__ __launch_bounds__(kScoreThreads) void score_mean_kernel(ScoreArgs a) {
+  static_assert(!FINE || LPH >= 8, "quarter tiles need one score per lane and token pair");
   constexpr int F = LPH * kPairsPerLane;
-  __shared__ int lds_blk[kScoreTileTokens + 2];
+  constexpr int kTile = FINE ? kScoreFineTokens : kScoreTileTokens;
+  __shared__ float lds_v[FINE ? kTile / 2 : 1][kWave];
+  __shared__ int lds_blk[kTile + 2];
   __shared__ float lds_s1[kScoreThreads];
   __shared__ float lds_s2[kScoreThreads];
 
@@ -125,9 +133,9 @@ __global__ __launch_bounds__(kScoreThreads) void score_mean_kernel(ScoreArgs a) 
   const int tile = blockIdx.x, sib = blockIdx.y;
   const int b = blockIdx.z / a.L, l = blockIdx.z % a.L;
   const int seq_len = a.seq_lens[b];
-  const int n0 = tile * kScoreTileTokens;
+  const int n0 = tile * kTile;
   if (n0 >= seq_len) return;
-  const int n1 = min(n0 + kScoreTileTokens, seq_len);
+  const int n1 = min(n0 + kTile, seq_len);
 
   int lb0 = 0;
   if (a.block_table_pitch >= 0) {
@@ -168,7 +176,7 @@ __global__ __launch_bounds__(kScoreThreads) void score_mean_kernel(ScoreArgs a) 
   const uint32_t lane_off_bytes = (uint32_t)(lane_off * ES);
 
   // This wave's tokens: a quarter of the tile, walked in stages of SP token pairs.
-  constexpr int TW = kScoreTileTokens / 4;
+  constexpr int TW = kTile / 4;
   const int wstart = n0 + wave * TW;
   const int wend = min(wstart + TW, n1);
   const int tok_per_pair = UNI ? 2 : 2 * lm.tpi;
@@ -267,8 +275,10 @@ __global__ __launch_bounds__(kScoreThreads) void score_mean_kernel(ScoreArgs a) 
           const float v = lm.slot_b ? rb : ra;
           float* row = raw_bl + (int64_t)ta * a.raw_stride_token;
           const bool ok = (ta + 1 < wend) ? out_ok : out_ok_a;
-          if (ok) {
-            row[store_off] = v;
+          if (ok) row[store_off] = v;
+          if constexpr (FINE) {
+            lds_v[(ta - n0) >> 1][lane] = ok ? v : 0.f;
+          } else if (ok) {
             s1 += v;
             s2 = fmaf(v, v, s2);
           }
@@ -280,8 +290,11 @@ __global__ __launch_bounds__(kScoreThreads) void score_mean_kernel(ScoreArgs a) 
       if (LPH >= 8) {
         const float v = lm.slot_b ? rb : ra;
         const int t = lm.slot_b ? tb : ta;
-        if (out_ok && t < wend) {
-          raw_row[(int64_t)t * a.raw_stride_token] = v;
+        const bool ok = out_ok && t < wend;
+        if (ok) raw_row[(int64_t)t * a.raw_stride_token] = v;
+        if constexpr (FINE) {          // (one token per wave iteration: token pairs as above)
+          if (base + p * 2 < wend) lds_v[(base + p * 2 - n0) >> 1][lane] = ok ? v : 0.f;
+        } else if (ok) {
           s1 += v;
           s2 = fmaf(v, v, s2);
         }
@@ -315,6 +328,40 @@ __global__ __launch_bounds__(kScoreThreads) void score_mean_kernel(ScoreArgs a) 
     }
   }
 
+  if constexpr (FINE) {
+    // The quarter's sums, in the order in which one wave alone accumulates them (a zero where a lane stored
+    // nothing changes no sum): [quarter][score head] (sum of A, sum of B, squares of A, squares of B).
+    __syncthreads();
+    if (wave == 0) {
+      const int pairs = (n1 - n0 + 1) >> 1;
+      for (int i = 0; i < pairs; i += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = lds_v[min(i + u, pairs - 1)][lane];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if (i + u >= pairs) continue;
+          s1 += v[u];
+          s2 = fmaf(v[u], v[u], s2);
+        }
+      }
+      lds_s1[lane] = s1;
+      lds_s2[lane] = s2;
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < (kWave / LPH) * kQPerPass) {
+      const int hl = threadIdx.x / kQPerPass, q = threadIdx.x % kQPerPass;
+      const int head = (sib / a.QC) * (kWave / LPH) + hl, qq = (sib % a.QC) * kQPerPass + q;
+      if (head < a.Hkv && qq < a.G) {
+        const int la = hl * LPH + ((q >> 1) | ((q & 1) << 1));
+        const int lb = hl * LPH + 4 + (1 - (q >> 1)) + 2 * (1 - (q & 1));
+        float4* out = reinterpret_cast<float4*>(a.partial) +
+                      ((int64_t)(b * a.L + l) * a.num_tiles + tile) * a.A + head * a.G + qq;
+        *out = float4{lds_s1[la], lds_s1[lb], lds_s2[la], lds_s2[lb]};
+      }
+    }
+    return;
+  }
   // Per-tile sum and sum of squares of every (head, query head) of this pass, in
   // a fixed order so that the statistics are reproducible run to run.
   lds_s1[threadIdx.x] = s1;
@@ -357,6 +404,7 @@ __global__ __launch_bounds__(kScoreThreads) void score_mean_kernel(ScoreArgs a) 
 template <int LPH, int DT, bool IL>
 __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
   constexpr int F = LPH * kPairsPerLane;
+  constexpr int kTile = kScoreTileTokens;
   __shared__ int lds_blk[kScoreTileTokens + 2];
   __shared__ float lds_s1[kScoreThreads];
   __shared__ float lds_s2[kScoreThreads];
@@ -367,9 +415,9 @@ __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
   const int tile = blockIdx.x, sib = blockIdx.y;
   const int b = blockIdx.z / a.L, l = blockIdx.z % a.L;
   const int seq_len = a.seq_lens[b];
-  const int n0 = tile * kScoreTileTokens;
+  const int n0 = tile * kTile;
   if (n0 >= seq_len) return;
-  const int n1 = min(n0 + kScoreTileTokens, seq_len);
+  const int n1 = min(n0 + kTile, seq_len);
 
   int lb0 = 0;
   if (a.block_table_pitch >= 0) {
@@ -407,7 +455,7 @@ __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
   const char* kbase = reinterpret_cast<const char*>(a.k_layers[l]);
   const float* kscale = FP8 ? a.k_scale_layers[l] : nullptr;
   const int64_t lane_off = (int64_t)head_c * a.stride_head + (IL ? lm.m * 16 : lm.m * 8);
-  constexpr int TW = kScoreTileTokens / 4;
+  constexpr int TW = kTile / 4;
   const int wstart = n0 + wave * TW;
   const int wend = min(wstart + TW, n1);
   const int a_out = head_c * a.G + lm.q0 + lm.qsel;
@@ -935,76 +983,111 @@ __global__ void fold_stats_kernel(const float* qr, const float* qi, const float*
   o[2 * F + f] = s * coef;
 }
 
-// cos/sin of the fp32-rounded phase t*w per offset (phase_cos_sin) and their means over the offsets.
-__global__ void trig_kernel(const float* omega, const float* offsets, int NO, const int32_t* round_start,
-                            int F, float* trig, float* mean_cs) {
-  const int b = blockIdx.x, f = threadIdx.x;
-  if (f >= F) return;
-  const float w = omega[f];
-  const float rs = (float)round_start[b];
-  double sc = 0.0, ss = 0.0;
-  for (int j = 0; j < NO; ++j) {
-    const float t = __fadd_rn(rs, offsets[j]);
-    float c, s;
-    phase_cos_sin(__fmul_rn(t, w), c, s);
-    if (trig) {
-      trig[((int64_t)(b * NO + j) * 2 + 0) * F + f] = c;
-      trig[((int64_t)(b * NO + j) * 2 + 1) * F + f] = s;
-    }
-    sc += c;
-    ss += s;
-  }
-  mean_cs[(int64_t)b * 2 * F + f] = (float)(sc / NO);
-  mean_cs[(int64_t)b * 2 * F + F + f] = (float)(ss / NO);
-}
-
-__global__ void coef_kernel(const float* folded, const float* mean_cs, int LA, int F, int mean_mode,
-                            float* coef) {
+// Everything the two-pass scorer needs before it starts, in one launch.  Workgroup (x, b): cos / sin of the
+// fp32-rounded phase (round_start + offset) * omega (phase_cos_sin) of every offset and their means over the
+// offsets (summed in offset order in double), then kPrepareRows rows [P | R | E][F] of the (layer, score
+// head) coefficients of sequence b.  The phases cost each workgroup ~1 us again; as a launch of their own (one thread
+// per pair, 17 phases one after the other: 5-7 us) plus one for the coefficients and one for the status
+// word the same took 12 us.
+// tables != NULL (max aggregation): the coefficients stay A1, A2, E and workgroup (0, b) leaves the
+// per-offset values there.
+constexpr int kPrepareThreads = 256;
+constexpr int kPrepareRows = 16;
+template <int F>
+__global__ __launch_bounds__(kPrepareThreads) void prepare_kernel(const float* folded, const float* omega,
+                                                                  const float* offsets, int NO,
+                                                                  const int32_t* round_start, int LA, float* coef,
+                                                                  float* tables, uint32_t* status) {
+  __shared__ float trig[2][kMaxOffsets][F];
+  __shared__ float mean_cs[2][F];
   const int b = blockIdx.y;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= LA * F) return;
-  const int la = idx / F, f = idx % F;
-  const float* in = folded + (int64_t)la * 3 * F;
-  float* o = coef + ((int64_t)b * LA + la) * 3 * F;
-  const float a1 = in[f], a2 = in[F + f], e = in[2 * F + f];
-  if (mean_mode) {
-    const float c = mean_cs[(int64_t)b * 2 * F + f], s = mean_cs[(int64_t)b * 2 * F + F + f];
-    o[f] = fmaf(a1, c, -a2 * s);
-    o[F + f] = fmaf(a2, c, a1 * s);
-  } else {
-    o[f] = a1;
-    o[F + f] = a2;
+  const bool mean_mode = tables == nullptr;
+  if (status && blockIdx.x == 0 && b == 0 && threadIdx.x == 0) *status = 0u;
+  // The rows' statistics are requested first: nothing of them depends on the phases.
+  constexpr int NI = kPrepareRows * F / kPrepareThreads;
+  const int row0 = blockIdx.x * kPrepareRows;
+  const int f = threadIdx.x % F;
+  float in[NI][3];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = min(row0 + (int)threadIdx.x / F + i * (kPrepareThreads / F), LA - 1);
+    const float* p = folded + (int64_t)r * 3 * F + f;
+    in[i][0] = p[0]; in[i][1] = p[F]; in[i][2] = p[2 * F];
   }
-  o[2 * F + f] = e;
+  if (mean_mode || blockIdx.x == 0) {
+    const float rs = (float)round_start[b], w = omega[f];
+    for (int j = threadIdx.x / F; j < NO; j += kPrepareThreads / F) {
+      float c, s;
+      phase_cos_sin(__fmul_rn(__fadd_rn(rs, offsets[j]), w), c, s);
+      if (mean_mode) {
+        trig[0][j][f] = c;
+        trig[1][j][f] = s;
+      } else {
+        tables[((int64_t)(b * NO + j) * 2 + 0) * F + f] = c;
+        tables[((int64_t)(b * NO + j) * 2 + 1) * F + f] = s;
+      }
+    }
+  }
+  float c = 0.f, sn = 0.f;
+  if (mean_mode) {
+    __syncthreads();
+    if ((int)threadIdx.x < 2 * F) {
+      const int which = threadIdx.x / F;
+      double sum = 0.0;
+      for (int j = 0; j < NO; ++j) sum += trig[which][j][f];
+      mean_cs[which][f] = (float)(sum / NO);
+    }
+    __syncthreads();
+    c = mean_cs[0][f];
+    sn = mean_cs[1][f];
+  }
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = row0 + (int)threadIdx.x / F + i * (kPrepareThreads / F);
+    if (r >= LA) continue;
+    float* o = coef + ((int64_t)b * LA + r) * 3 * F + f;
+    const float a1 = in[i][0], a2 = in[i][1];
+    o[0] = mean_mode ? fmaf(a1, c, -a2 * sn) : a1;
+    o[F] = mean_mode ? fmaf(a2, c, a1 * sn) : a2;
+    o[2 * F] = in[i][2];
+  }
 }
 
 template <int LPH, int DT, bool IL>
-hipError_t launch_score_t(const ScoreArgs& args, dim3 grid, int aggregation, hipStream_t s) {
+hipError_t launch_score_t(const ScoreArgs& args, dim3 grid, int aggregation, bool fine, hipStream_t s) {
   // Scalar addressing needs one token per wave iteration (the padded KV heads fill the
   // wave's rows) and a stage of 4 tokens inside one block (or dense keys).
   const bool uni = args.Hpad >= kWave / LPH &&
                    (args.block_table_pitch < 0 || (args.bs_shift >= 2));
   if (aggregation == TRI_REDUCE_MEAN) {
-    if (uni)
-      hipLaunchKernelGGL((score_mean_kernel<LPH, DT, IL, 2, true>), grid, dim3(kScoreThreads), 0, s, args);
+    if (fine) {
+      if constexpr (LPH >= 8) {
+        if (uni)
+          hipLaunchKernelGGL((score_mean_kernel<LPH, DT, IL, 1, true, true>), grid, dim3(kScoreThreads), 0, s, args);
+        else
+          hipLaunchKernelGGL((score_mean_kernel<LPH, DT, IL, 1, false, true>), grid, dim3(kScoreThreads), 0, s, args);
+      } else
+        return hipErrorInvalidValue;
+    } else if (uni)
+      hipLaunchKernelGGL((score_mean_kernel<LPH, DT, IL, 2, true, false>), grid, dim3(kScoreThreads), 0, s, args);
     else
-      hipLaunchKernelGGL((score_mean_kernel<LPH, DT, IL, 2, false>), grid, dim3(kScoreThreads), 0, s, args);
+      hipLaunchKernelGGL((score_mean_kernel<LPH, DT, IL, 2, false, false>), grid, dim3(kScoreThreads), 0, s, args);
   } else
     hipLaunchKernelGGL((score_max_kernel<LPH, DT, IL>), grid, dim3(kScoreThreads), 0, s, args);
   return hipGetLastError();
 }
 
 template <int LPH>
-hipError_t launch_score_lph(const ScoreArgs& args, dim3 grid, int dt, int il, int aggregation, hipStream_t s) {
+hipError_t launch_score_lph(const ScoreArgs& args, dim3 grid, int dt, int il, int aggregation, bool fine, hipStream_t s) {
   if (dt == TRI_KV_BF16)
-    return il ? launch_score_t<LPH, TRI_KV_BF16, true>(args, grid, aggregation, s)
-              : launch_score_t<LPH, TRI_KV_BF16, false>(args, grid, aggregation, s);
+    return il ? launch_score_t<LPH, TRI_KV_BF16, true>(args, grid, aggregation, fine, s)
+              : launch_score_t<LPH, TRI_KV_BF16, false>(args, grid, aggregation, fine, s);
   if (dt == TRI_KV_FP16)
-    return il ? launch_score_t<LPH, TRI_KV_FP16, true>(args, grid, aggregation, s)
-              : launch_score_t<LPH, TRI_KV_FP16, false>(args, grid, aggregation, s);
+    return il ? launch_score_t<LPH, TRI_KV_FP16, true>(args, grid, aggregation, fine, s)
+              : launch_score_t<LPH, TRI_KV_FP16, false>(args, grid, aggregation, fine, s);
   if (dt == TRI_KV_FP8_E4M3)
-    return il ? launch_score_t<LPH, TRI_KV_FP8_E4M3, true>(args, grid, aggregation, s)
-              : launch_score_t<LPH, TRI_KV_FP8_E4M3, false>(args, grid, aggregation, s);
+    return il ? launch_score_t<LPH, TRI_KV_FP8_E4M3, true>(args, grid, aggregation, fine, s)
+              : launch_score_t<LPH, TRI_KV_FP8_E4M3, false>(args, grid, aggregation, fine, s);
   return hipErrorInvalidValue;
 }
 
@@ -1021,21 +1104,34 @@ hipError_t launch_fold_stats(const float* qr, const float* qi, const float* qabs
 
 hipError_t launch_prepare(const float* folded, const float* omega, const float* offsets, int NO,
                           const int32_t* round_start, int B, int L, int A, int F, int aggregation,
-                          float* coef, float* trig, hipStream_t s) {
-  // The first 2*F floats per sequence of the trig area hold the offset means; the
-  // per-offset tables (max aggregation) follow the means of all sequences.
-  float* mean_cs = trig;
+                          float* coef, float* trig, uint32_t* status, hipStream_t s) {
+  // The per-offset tables (max aggregation) follow 2*F floats per sequence in the trig area.
   float* tables = (aggregation == TRI_REDUCE_MAX) ? trig + (int64_t)B * 2 * F : nullptr;
-  hipLaunchKernelGGL(trig_kernel, dim3(B), dim3(F), 0, s, omega, offsets, NO, round_start, F, tables, mean_cs);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(coef_kernel, dim3(ceil_div(L * A * F, 256), B), dim3(256), 0, s, folded, mean_cs, L * A, F,
-                     aggregation == TRI_REDUCE_MEAN ? 1 : 0, coef);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(ceil_div(L * A, kPrepareRows), B), dim3(kPrepareThreads), 0, s, folded, omega, offsets,
+                       NO, round_start, L * A, coef, tables, status);
+  };
+  switch (F) {
+    case 32: launch(prepare_kernel<32>); break;
+    case 64: launch(prepare_kernel<64>); break;
+    case 128: launch(prepare_kernel<128>); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
 // TRI_TUNE_MAX_KERNEL = 1 keeps max aggregation on the vector-unit kernel (comparison runs).
 static bool max_on_vector_unit() { return tuning(TRI_TUNE_MAX_KERNEL) == 1; }
+
+// Quarter tiles (score_mean_kernel, FINE) for launches that give less than half of the CUs' room (two
+// workgroups each, by registers) a whole tile: mean aggregation, head dimensions 128 and 256, KV heads that
+// fill a wave.
+bool score_takes_fine(int B, int L, int Hkv, int D, int G, int Tmax, int aggregation) {
+  if (aggregation != TRI_REDUCE_MEAN || D < 128) return false;
+  const int upw = kWave / (D / 16);
+  if (Hkv * 2 <= upw) return false;                 // (padded to a power of two the heads do not fill a wave)
+  return (int64_t)ceil_div(Hkv, upw) * ceil_div(G, kQPerPass) * B * L * ceil_div(Tmax, kScoreTileTokens) < 256;
+}
 
 hipError_t launch_score(const ScoreLaunch& a, hipStream_t s) {
   ScoreArgs k{};
@@ -1059,24 +1155,25 @@ hipError_t launch_score(const ScoreLaunch& a, hipStream_t s) {
   for (int sft = 0; sft < 31; ++sft)
     if ((1 << sft) == a.block_size) k.bs_shift = sft;
   k.block_table_pitch = a.block_table ? a.block_table_pitch : -1;
-  k.num_tiles = a.num_tiles;
+  k.num_tiles = ceil_div(a.Tmax, a.fine ? kScoreFineTokens : kScoreTileTokens);
   k.QC = ceil_div(a.G, kQPerPass);
   int hpad = 1;
   while (hpad < a.Hkv) hpad <<= 1;
   k.Hpad = hpad;
   const int il_max = a.rope_style == TRI_ROPE_INTERLEAVED;
+  if (a.fine && !score_takes_fine(a.B, a.L, a.Hkv, a.D, a.G, a.Tmax, a.aggregation)) return hipErrorInvalidValue;
   if (a.aggregation == TRI_REDUCE_MAX && a.kv_dtype == TRI_KV_BF16 && a.D == 128 && a.NO <= kMaxOffsets &&
       !max_on_vector_unit())
     return launch_max_mfma(k, a.B, il_max, s);
   const int lph = a.D / 16;
   const int upw = kWave / lph;
   const int HC = hpad >= upw ? hpad / upw : 1;
-  dim3 grid(a.num_tiles, HC * k.QC, a.B * a.L);
+  dim3 grid(k.num_tiles, HC * k.QC, a.B * a.L);
   const int il = a.rope_style == TRI_ROPE_INTERLEAVED;
   switch (lph) {
-    case 4: return launch_score_lph<4>(k, grid, a.kv_dtype, il, a.aggregation, s);
-    case 8: return launch_score_lph<8>(k, grid, a.kv_dtype, il, a.aggregation, s);
-    case 16: return launch_score_lph<16>(k, grid, a.kv_dtype, il, a.aggregation, s);
+    case 4: return launch_score_lph<4>(k, grid, a.kv_dtype, il, a.aggregation, a.fine != 0, s);
+    case 8: return launch_score_lph<8>(k, grid, a.kv_dtype, il, a.aggregation, a.fine != 0, s);
+    case 16: return launch_score_lph<16>(k, grid, a.kv_dtype, il, a.aggregation, a.fine != 0, s);
     default: return hipErrorInvalidValue;
   }
 }

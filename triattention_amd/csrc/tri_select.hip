@@ -19,8 +19,10 @@
 namespace tri {
 namespace {
 
+// fine: the sums come per quarter of a tile as (sum of A, sum of B, squares of A, squares of B) and are
+// added here in the order in which a whole-tile workgroup adds those of its four waves.
 __global__ void finalize_stats_kernel(const float* partial, const int32_t* seq_lens, int B, int L, int A,
-                                      int num_tiles, int normalize, float* mustd) {
+                                      int num_tiles, int fine, int normalize, float* mustd) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= B * L * A) return;
   const int a = idx % A, bl = idx / A, b = bl / L;
@@ -29,11 +31,38 @@ __global__ void finalize_stats_kernel(const float* partial, const int32_t* seq_l
     const int T = seq_lens[b];
     const int nt = ceil_div(T, kScoreTileTokens);
     double s = 0.0, q = 0.0;
-    for (int t = 0; t < nt; ++t) {
-      const float* p = partial + (((int64_t)bl * num_tiles + t) * A + a) * 2;
-      s += (double)p[0];
-      q += (double)p[1];
-    }
+    if (fine) {
+      const int nq = ceil_div(T, kScoreFineTokens);
+      const float4* p = reinterpret_cast<const float4*>(partial) + (int64_t)bl * num_tiles * A + a;
+      for (int t = 0; t < nq; t += 4) {
+        float4 x[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) x[w] = p[(int64_t)min(t + w, nq - 1) * A];
+        float t1 = 0.f, t2 = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+          if (t + w < nq) {
+            t1 += x[w].x;
+            t2 += x[w].z;
+            t1 += x[w].y;
+            t2 += x[w].w;
+          }
+        s += (double)t1;
+        q += (double)t2;
+      }
+    } else
+      for (int t = 0; t < nt; t += 8) {              // eight tiles requested before the first is added
+        const float2* p = reinterpret_cast<const float2*>(partial) + (int64_t)bl * num_tiles * A + a;
+        float2 x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = p[(int64_t)min(t + u, nt - 1) * A];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (t + u < nt) {
+            s += (double)x[u].x;
+            q += (double)x[u].y;
+          }
+      }
     // The reference's formula on fp32 sums (runtime/selector_hf.py:902-909).
     const float sum = (float)s, sumsq = (float)q, cnt = (float)T;
     mean = __fdiv_rn(sum, cnt);
@@ -111,19 +140,22 @@ __global__ __launch_bounds__(256) void group_stats_kernel(const float* raw, int6
 // KV head), so a wave reads 1 KB of consecutive memory per load where the kernel above reads 16 bytes
 // of every 128-byte row eight times over (one request of 16384 tokens x 36 layers: 117 -> 30 us), and
 // leaves the chunk's sums in double; the second launch adds the chunks in order.
-constexpr int kGroupStatsChunk = 2048;
+// A few requests take chunks of down to 256 tokens: one of 2176 tokens x 36 layers is 72 workgroups of 2048
+// tokens (27 us) or 324 of 256.
+constexpr int kGroupStatsChunk = 2048, kGroupStatsChunkMin = 256;
 __global__ __launch_bounds__(256) void group_stats_partial_kernel(const float* raw, int64_t stride_layer,
                                                                   int64_t stride_token, const int32_t* seq_lens, int L,
-                                                                  int Hkv, int chunks, int group_reduce,
+                                                                  int Hkv, int chunk, int chunks, int group_reduce,
                                                                   double* partial) {
   __shared__ double red[256][2];
   const int c = blockIdx.x, bl = blockIdx.y, b = bl / L;
   const int T = seq_lens[b];
   const int h = threadIdx.x % Hkv, tn = threadIdx.x / Hkv, tstep = 256 / Hkv;
-  const int n_end = min(T, (c + 1) * kGroupStatsChunk);
+  const int n_end = min(T, (c + 1) * chunk);
   const float* base = raw + (int64_t)bl * stride_layer + h * 4;
   double s = 0.0, q = 0.0;
-  for (int n = c * kGroupStatsChunk + tn; n < n_end; n += tstep) {
+#pragma unroll 4
+  for (int n = c * chunk + tn; n < n_end; n += tstep) {
     const float4 x = *reinterpret_cast<const float4*>(base + (int64_t)n * stride_token);
     float m;
     if (group_reduce == TRI_REDUCE_MAX) m = fmaxf(fmaxf(x.x, x.y), fmaxf(x.z, x.w));
@@ -149,12 +181,12 @@ __global__ __launch_bounds__(256) void group_stats_partial_kernel(const float* r
 }
 
 __global__ void group_stats_finish_kernel(const double* partial, const int32_t* seq_lens, int BL, int L, int Hkv, int A,
-                                          int chunks, float* mustd) {
+                                          int chunk, int chunks, float* mustd) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= BL * Hkv) return;
   const int h = idx % Hkv, bl = idx / Hkv, b = bl / L;
   const int T = seq_lens[b];
-  const int nc = ceil_div(T, kGroupStatsChunk);
+  const int nc = ceil_div(T, chunk);
   double s = 0.0, q = 0.0;
   for (int c = 0; c < nc; ++c) {
     const double* p = partial + (((int64_t)bl * chunks + c) * Hkv + h) * 2;
@@ -180,9 +212,8 @@ struct CombineArgs {
   int64_t raw_stride_layer, raw_stride_token, raw_stride_head;
   int B, L, Hkv, A, G, Tmax;
   int window_size, protect_prefill, group_reduce, layer_reduce, shared;
-  int group_first;    // 1: reduce over the query heads of a KV head before normalising (mustd is per KV head)
   int rows_per_seq;   // rows per (sequence[, layer]): shared ? 1 : Hkv
-  int tokens_per_wg;  // 256 / rows_per_seq
+  int tokens_per_wg;  // threads / rows_per_seq
 };
 
 // z-score of one raw value with the reference's operation order: (x - mean) / std.
@@ -193,7 +224,9 @@ __device__ __forceinline__ float zscore(float x, float mean, float sd) {
 // One thread per (token, output row).  Grid: (token tiles, layers or 1, B).
 // NV > 0: groups of 4 * NV query heads (4 or 8), raw scores head-contiguous and 16-byte aligned, read as
 // NV 16-byte loads per layer; NV = 0: any layout, one score at a time.
-template <int NV>
+// U (NV > 0): layers a thread requests before it uses the first; GF: group_first, a constant there because a
+// branch between the loads made every one of them wait for the one before.
+template <int NV, int U, bool GF>
 __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
   extern __shared__ float tile[];  // [rows_per_seq][tokens_per_wg]
   const int b = blockIdx.z;
@@ -219,33 +252,32 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
       // flight per thread.
       constexpr int NVV = NV > 0 ? NV : 1;
       constexpr int GQ = 4 * NVV;                  // query heads per KV head
-      constexpr int U = NVV == 1 ? 4 : 2;          // layers in flight
       const float* raw0 = a.raw + (int64_t)b * a.L * a.raw_stride_layer + (int64_t)n * a.raw_stride_token + r * GQ;
       // Reduce-first order (group_first): the statistics are those of the KV head's reduced score and
-      // sit in entry r of the layer's table; they arrive in m[0].x / m[0].y (the rest unused).
-      const float* ms0 = a.mustd + ((int64_t)b * a.L * a.A + (a.group_first ? r : r * GQ)) * 2;
-      struct LayerIn { float4 x[NVV]; float4 m[2 * NVV]; };
-      auto load_layer = [&](int l, LayerIn& in) {
+      // sit in entry r of the layer's table; they arrive in m[0].x / m[0].y.
+      const float* ms0 = a.mustd + ((int64_t)b * a.L * a.A + (GF ? r : r * GQ)) * 2;
+      constexpr int NM = GF ? 1 : 2 * NVV;
+      struct LayerIn { float4 x[NVV]; float4 m[NM]; };
+      auto load_layer = [&](int l, LayerIn& in) __attribute__((always_inline)) {
         const float* rl = raw0 + (int64_t)l * a.raw_stride_layer;
         const float* ms = ms0 + (int64_t)l * a.A * 2;
 #pragma unroll
         for (int i = 0; i < NVV; ++i) in.x[i] = *reinterpret_cast<const float4*>(rl + 4 * i);
-        if (a.group_first) {
+        if constexpr (GF) {
           const float2 m = *reinterpret_cast<const float2*>(ms);
-#pragma unroll
-          for (int i = 0; i < 2 * NVV; ++i) in.m[i] = float4{m.x, m.y, 0.f, 0.f};
+          in.m[0] = float4{m.x, m.y, 0.f, 0.f};
         } else {
           // mustd is [head][mean, std]: m[2 i] = (mean, std) of query heads 4 i and 4 i + 1, m[2 i + 1] of the next two.
 #pragma unroll
-          for (int i = 0; i < 2 * NVV; ++i) in.m[i] = *reinterpret_cast<const float4*>(ms + 4 * i);
+          for (int i = 0; i < NM; ++i) in.m[i] = *reinterpret_cast<const float4*>(ms + 4 * i);
         }
       };
-      auto layer_value = [&](const LayerIn& in) {
+      auto layer_value = [&](const LayerIn& in) __attribute__((always_inline)) {
         float xs[GQ];
 #pragma unroll
         for (int i = 0; i < NVV; ++i) { xs[4 * i] = in.x[i].x; xs[4 * i + 1] = in.x[i].y; xs[4 * i + 2] = in.x[i].z; xs[4 * i + 3] = in.x[i].w; }
         float v;
-        if (a.group_first) {
+        if constexpr (GF) {
           // (the order of the scalar path below: query heads one after the other)
           float m = xs[0];
 #pragma unroll
@@ -255,7 +287,7 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
         } else {
           float z[GQ];
 #pragma unroll
-          for (int i = 0; i < 2 * NVV; ++i) {
+          for (int i = 0; i < NM; ++i) {
             z[2 * i] = zscore(xs[2 * i], in.m[i].x, in.m[i].y);
             z[2 * i + 1] = zscore(xs[2 * i + 1], in.m[i].z, in.m[i].w);
           }
@@ -266,24 +298,17 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
         }
         return guard ? INFINITY : v;
       };
-      int l = l_begin;
-      for (; l + U <= l_end; l += U) {
+      for (int l = l_begin; l < l_end; l += U) {
         LayerIn in[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) load_layer(l + u, in[u]);
+        for (int u = 0; u < U; ++u) load_layer(min(l + u, l_end - 1), in[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+          if (l + u >= l_end) continue;
           const float v = layer_value(in[u]);
           if (l + u == l_begin) acc = v;
           else acc = (a.layer_reduce == TRI_REDUCE_MAX) ? fmaxf(acc, v) : __fadd_rn(acc, v);
         }
-      }
-      for (; l < l_end; ++l) {
-        LayerIn in;
-        load_layer(l, in);
-        const float v = layer_value(in);
-        if (l == l_begin) acc = v;
-        else acc = (a.layer_reduce == TRI_REDUCE_MAX) ? fmaxf(acc, v) : __fadd_rn(acc, v);
       }
     } else {
       for (int l = l_begin; l < l_end; ++l) {
@@ -295,11 +320,11 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
           for (int q = 0; q < a.G; ++q) {
             const int ah = h * a.G + q;
             const float x = raw_l[(int64_t)ah * a.raw_stride_head];
-            const float z = a.group_first ? x : zscore(x, ms[ah * 2], ms[ah * 2 + 1]);
+            const float z = GF ? x : zscore(x, ms[ah * 2], ms[ah * 2 + 1]);
             gv = (a.group_reduce == TRI_REDUCE_MAX) ? fmaxf(gv, z) : __fadd_rn(gv, z);
           }
           if (a.group_reduce != TRI_REDUCE_MAX) gv = __fdiv_rn(gv, (float)a.G);
-          if (a.group_first) gv = zscore(gv, ms[h * 2], ms[h * 2 + 1]);
+          if (GF) gv = zscore(gv, ms[h * 2], ms[h * 2 + 1]);
           v = fmaxf(v, gv);
         }
         if (guard) v = INFINITY;
@@ -314,7 +339,7 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
   // Coalesced write of the [rows][tokens] tile.
   const int nvalid = min(a.tokens_per_wg, T - n0);
   const int64_t row0 = per_layer ? ((int64_t)(b * a.L + blockIdx.y) * R) : ((int64_t)b * R);
-  for (int i = threadIdx.x; i < R * a.tokens_per_wg; i += 256) {
+  for (int i = threadIdx.x; i < R * a.tokens_per_wg; i += (int)blockDim.x) {
     const int rr = i / a.tokens_per_wg, tt = i % a.tokens_per_wg;
     if (tt < nvalid) a.fin[(row0 + rr) * a.Tmax + n0 + tt] = tile[i];
   }
@@ -766,18 +791,15 @@ hipError_t launch_topk_rows(const float* scores, int64_t row_pitch, int num_rows
 // Longest row the register top-k kernels take (they can also add partial rows while loading).
 int topk_register_row_limit() { return 32 * kTopkThreads; }
 
-__global__ void clear_word_kernel(uint32_t* word) { *word = 0u; }
-
-hipError_t launch_clear_status(uint32_t* status, hipStream_t s) {
-  hipLaunchKernelGGL(clear_word_kernel, dim3(1), dim3(1), 0, s, status);
-  return hipGetLastError();
-}
-
 hipError_t launch_select(const SelectLaunch& a, hipStream_t s) {
   const int n = a.B * a.L * a.A;
-  // Whole token rows for the usual layout; the chunk sums ([B][L][chunks of 2048][Hkv][2] doubles) go
+  // Whole token rows for the usual layout; the chunk sums ([B][L][chunks][Hkv][2] doubles) go
   // into scratch the caller names.
-  const int chunks = ceil_div(a.Tmax, kGroupStatsChunk);
+  int chunk = kGroupStatsChunk;
+  while (chunk > kGroupStatsChunkMin && (int64_t)ceil_div(a.Tmax, chunk) * a.B * a.L < 1024 &&
+         (int64_t)a.B * a.L * ceil_div(a.Tmax, chunk / 2) * a.Hkv * 16 <= a.group_scratch_bytes)
+    chunk /= 2;
+  const int chunks = ceil_div(a.Tmax, chunk);
   const bool rows = a.group_first && a.normalize && a.G == 4 && a.A == a.Hkv * 4 && a.raw_stride_head == 1 &&
                     a.raw_stride_token % 4 == 0 && a.raw_stride_layer % 4 == 0 &&
                     (reinterpret_cast<uintptr_t>(a.raw) % 16) == 0 && a.Hkv <= 128 && (a.Hkv & (a.Hkv - 1)) == 0 &&
@@ -786,16 +808,16 @@ hipError_t launch_select(const SelectLaunch& a, hipStream_t s) {
   if (rows) {
     double* part = a.group_scratch;
     hipLaunchKernelGGL(group_stats_partial_kernel, dim3(chunks, a.B * a.L), dim3(256), 0, s, a.raw, a.raw_stride_layer,
-                       a.raw_stride_token, a.seq_lens, a.L, a.Hkv, chunks, a.group_reduce, part);
+                       a.raw_stride_token, a.seq_lens, a.L, a.Hkv, chunk, chunks, a.group_reduce, part);
     hipLaunchKernelGGL(group_stats_finish_kernel, dim3(ceil_div(a.B * a.L * a.Hkv, 256)), dim3(256), 0, s, part,
-                       a.seq_lens, a.B * a.L, a.L, a.Hkv, a.A, chunks, a.mustd);
+                       a.seq_lens, a.B * a.L, a.L, a.Hkv, a.A, chunk, chunks, a.mustd);
   } else if (a.group_first)
     hipLaunchKernelGGL(group_stats_kernel, dim3(a.B * a.L * a.Hkv), dim3(256), 0, s, a.raw, a.raw_stride_layer,
                        a.raw_stride_token, a.raw_stride_head, a.seq_lens, a.L, a.Hkv, a.A, a.G, a.group_reduce,
                        a.normalize, a.mustd);
   else
     hipLaunchKernelGGL(finalize_stats_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, a.partial, a.seq_lens,
-                       a.B, a.L, a.A, a.num_tiles, a.normalize, a.mustd);
+                       a.B, a.L, a.A, ceil_div(a.Tmax, a.fine ? kScoreFineTokens : kScoreTileTokens), a.fine, a.normalize, a.mustd);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
 
@@ -814,21 +836,34 @@ hipError_t launch_select(const SelectLaunch& a, hipStream_t s) {
   c.group_reduce = a.group_reduce;
   c.layer_reduce = a.layer_reduce;
   c.shared = a.shared;
-  c.group_first = a.group_first;
   c.rows_per_seq = a.shared ? 1 : a.Hkv;
-  c.tokens_per_wg = 256 / c.rows_per_seq;
   const bool per_layer = a.layer_reduce < 0;
-  dim3 grid(ceil_div(a.Tmax, c.tokens_per_wg), per_layer ? a.L : 1, a.B);
-  const size_t smem = (size_t)c.rows_per_seq * c.tokens_per_wg * sizeof(float);
+  // Reducing over the layers, a thread's time is its rounds of loads.  Where few workgroups share the chip
+  // nothing hides them: one wave per workgroup (four times as many of them) and three times as many
+  // layers requested at once (one request of 2176 tokens x 36 layers, 68 workgroups: 19 -> 8 us; 2 x 8192
+  // tokens 32 -> 23).  One layer per thread (a keep set per layer) has nothing to batch.
   const bool vec = (a.G == 4 || a.G == 8) && a.raw_stride_head == 1 && a.raw_stride_token % 4 == 0 &&
                    a.raw_stride_layer % 4 == 0 && (reinterpret_cast<uintptr_t>(a.raw) % 16) == 0 &&
                    (reinterpret_cast<uintptr_t>(a.mustd) % 16) == 0;
-  if (vec && a.G == 4)
-    hipLaunchKernelGGL(combine_kernel<1>, grid, dim3(256), smem, s, c);
-  else if (vec)
-    hipLaunchKernelGGL(combine_kernel<2>, grid, dim3(256), smem, s, c);
-  else
-    hipLaunchKernelGGL(combine_kernel<0>, grid, dim3(256), smem, s, c);
+  const bool few = vec && !per_layer && c.rows_per_seq <= 64 &&
+                   (int64_t)ceil_div(a.Tmax, 256 / c.rows_per_seq) * a.B < 1024;
+  const int threads = few ? 64 : 256;
+  c.tokens_per_wg = threads / c.rows_per_seq;
+  dim3 grid(ceil_div(a.Tmax, c.tokens_per_wg), per_layer ? a.L : 1, a.B);
+  const size_t smem = (size_t)c.rows_per_seq * c.tokens_per_wg * sizeof(float);
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(threads), smem, s, c); };
+  if (!vec) {
+    if (a.group_first) launch(combine_kernel<0, 1, true>);
+    else launch(combine_kernel<0, 1, false>);
+  } else if (a.G == 4) {
+    if (per_layer) { if (a.group_first) launch(combine_kernel<1, 1, true>); else launch(combine_kernel<1, 1, false>); }
+    else if (few) { if (a.group_first) launch(combine_kernel<1, 12, true>); else launch(combine_kernel<1, 12, false>); }
+    else { if (a.group_first) launch(combine_kernel<1, 4, true>); else launch(combine_kernel<1, 4, false>); }
+  } else {
+    if (per_layer) { if (a.group_first) launch(combine_kernel<2, 1, true>); else launch(combine_kernel<2, 1, false>); }
+    else if (few) { if (a.group_first) launch(combine_kernel<2, 6, true>); else launch(combine_kernel<2, 6, false>); }
+    else { if (a.group_first) launch(combine_kernel<2, 2, true>); else launch(combine_kernel<2, 2, false>); }
+  }
   e = hipGetLastError();
   if (e != hipSuccess) return e;
 
