@@ -265,6 +265,33 @@ int tri_topk_rows(const float* scores, int64_t row_pitch, int32_t num_rows, cons
                   const int32_t* row_ks, int32_t rows_per_entry, int32_t max_len, int32_t* keep,
                   int32_t keep_pitch, void* stream);
 
+/* Compression of one layer of a dense cache into new tensors, everything the dense compressor
+ * launches after its trigger (core/compressor.py:279-346): score every key [H][T][D] against one
+ * score head per KV head, normalise over the tokens (mean and unbiased standard deviation, core/utils.py:466-480),
+ * guard the last window_size tokens, keep the budget largest per head, gather.  Strides and row sizes
+ * of K and V in bytes, multiples of 16, bases 16-byte aligned; V rows may hold any type.  0 < budget <= T.
+ * out_k [H][budget][D], out_v [H][budget][v row], out_keep [H][budget] ascending.  Scratch as
+ * tri_dense_workspace_bytes says (0: not supported), 256-byte aligned.  Nothing waits; capturable. */
+typedef struct tri_dense_params {
+  int32_t num_heads, num_tokens, head_dim, kv_dtype, rope_style;     /* bf16 or fp16 keys */
+  int32_t budget, window_size, normalize, round_start;
+  int32_t num_offsets, aggregation, disable_mlr, disable_trig;
+  int32_t v_row_bytes;
+  const void* k;
+  const void* v;
+  int64_t k_stride_head, k_stride_token, v_stride_head, v_stride_token;
+  const float* q_mean_complex;  /* [H][D/2][2] */
+  const float* q_abs_mean;      /* [H][D/2] */
+  const float* freq_scale_sq;   /* [H][D/2] */
+  const float* omega;           /* [D/2] */
+  const float* offsets;         /* [num_offsets] */
+  void* out_k;
+  void* out_v;
+  int64_t* out_keep;
+} tri_dense_params;
+uint64_t tri_dense_workspace_bytes(const tri_dense_params* params);
+int tri_dense_compress(const tri_dense_params* params, void* workspace, uint64_t workspace_bytes, void* stream);
+
 /* In-place, order-preserving compaction of K and V of every layer: slot j of
  * (seq b, head h) receives the row of token keep[...][j], for j < budget_b;
  * replaces compact_request_kv_in_place(_per_head) per layer

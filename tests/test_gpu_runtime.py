@@ -520,6 +520,84 @@ def test_dense_compressor_against_oracle(tmp_path):
                                              torch.zeros(2, h, 600, d, dtype=torch.bfloat16, device=DEV))
 
 
+@pytest.mark.parametrize("case", [
+    dict(), dict(t=600, budget=584, window_size=0), dict(h=1, d=64, t=130, budget=1, window_size=0),
+    dict(h=3, d=256, t=4097, budget=1000), dict(h=8, t=513, budget=300, token_major=True), dict(dtype=torch.float16),
+    dict(score_aggregation="max"), dict(sparse_normalize_scores=False), dict(v_dim=24, v_dtype=torch.float32)], ids=str)
+def test_dense_compressor_in_one_call_equals_its_parts(tmp_path, case):
+    """The one library call against the general way of the same object (scorer, torch's normalisation,
+    top-k, torch.gather): the two statistics differ in their last bits (double sums here, fp32 Welford there), so
+    an index may change places with another within 1e-5 of the scores' scale."""
+    case = dict(case)
+    g = torch.Generator().manual_seed(23)
+    h, t, d, budget = case.pop("h", 4), case.pop("t", 1000), case.pop("d", 128), case.pop("budget", 128)
+    dtype, v_dim = case.pop("dtype", torch.bfloat16), case.pop("v_dim", None)
+    v_dtype, token_major = case.pop("v_dtype", dtype), case.pop("token_major", False)
+    omega = 1.0 / (1e6 ** (torch.arange(0, d, 2, dtype=torch.float32) / d))
+    qc = torch.randn(1, h, d // 2, 2, generator=g)
+    qa = qc.pow(2).sum(-1).sqrt() + torch.randn(1, h, d // 2, generator=g).abs()
+    _write_stats(tmp_path / "s.pt", qc, qa, omega, d)
+    shape = (1, t, h, d) if token_major else (1, h, t, d)
+    keys = (torch.randn(shape, generator=g) + 1.0).to(dtype).to(DEV)
+    vals = torch.randn(*shape[:3], v_dim or d, generator=g).to(v_dtype).to(DEV)
+    if token_major:
+        keys, vals = keys.transpose(1, 2), vals.transpose(1, 2)
+    cfg = TriAttentionConfig(**dict(dict(device=torch.device(DEV), stats_path=tmp_path / "s.pt", kv_budget=budget,
+                                         divide_length=16, window_size=16, protect_prefill=False,
+                                         compute_dtype=torch.float32), **case))
+    comp = TriAttentionCompressor(cfg)
+    comp._lazy_init()
+    assert comp._one_call_args(keys, vals, 0) is not None
+    k2, v2, keep = comp.compress(keys, vals)
+    index = keep.unsqueeze(-1)
+    assert k2.is_contiguous() and v2.is_contiguous() and keep.dtype == torch.long and keep.shape == (1, h, budget)
+    assert torch.equal(k2, torch.gather(keys, 2, index.expand(*keep.shape, d)))
+    assert torch.equal(v2, torch.gather(vals, 2, index.expand(*keep.shape, vals.shape[3])))
+    parts = TriAttentionCompressor(cfg)
+    parts._one_call_args = lambda *a: None
+    k3, v3, keep_parts = parts.compress(keys, vals)
+    parts.state.reset()
+    parts.state.should_compress(t)
+    fin = parts._compute_scores(keys, 0)[0]
+    if cfg.sparse_normalize_scores:
+        fin = (fin - fin.mean(-1, keepdim=True)) / fin.std(-1, keepdim=True)
+    scale = float(fin.abs().max())
+    if cfg.window_size:
+        fin[:, -cfg.window_size:] = float("inf")
+    assert_keep_matches(keep[0].cpu(), keep_parts[0].cpu(), fin.cpu(), budget, 1e-5 * scale)
+    assert k3.stride() == k2.stride() and v3.stride() == v2.stride()
+
+
+def test_dense_compressor_leaves_other_calls_to_its_parts(tmp_path):
+    """Gradients, forward-mode tangents, vmapped values and rows that are not multiples of 16 bytes."""
+    g = torch.Generator().manual_seed(29)
+    h, t, d, budget = 2, 200, 64, 32
+    omega = 1.0 / (1e6 ** (torch.arange(0, d, 2, dtype=torch.float32) / d))
+    qc = torch.randn(1, h, d // 2, 2, generator=g)
+    _write_stats(tmp_path / "s.pt", qc, qc.pow(2).sum(-1).sqrt(), omega, d)
+    cfg = TriAttentionConfig(device=torch.device(DEV), stats_path=tmp_path / "s.pt", kv_budget=budget, divide_length=16,
+                             window_size=4, protect_prefill=False, compute_dtype=torch.float32)
+    keys = torch.randn(1, h, t, d, generator=g).to(torch.bfloat16).to(DEV)
+    vals = torch.randn(1, h, t, d, generator=g).to(DEV)
+
+    def run(k, v):
+        return TriAttentionCompressor(cfg).compress(k, v)
+
+    _, plain, keep = run(keys, vals)
+    wanted = vals.clone().requires_grad_(True)
+    out = run(keys, wanted)[1]
+    out.sum().backward()
+    assert torch.equal(out.detach(), plain) and float(wanted.grad.sum()) == h * budget * d
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(vals, torch.ones_like(vals))
+        tangent = torch.autograd.forward_ad.unpack_dual(run(keys, dual)[1]).tangent
+        assert tangent is not None and bool((tangent == 1).all())
+    stacked = torch.func.vmap(lambda v: run(keys, v)[1])(torch.stack([vals, vals + 1]))
+    assert torch.equal(stacked[0], plain) and torch.equal(stacked[1], plain + 1)
+    _, odd, keep_odd = run(keys, vals[..., :3])
+    assert torch.equal(odd, plain[..., :3]) and torch.equal(keep_odd, keep)
+
+
 def test_scheduler_and_worker_bookkeeping_around_the_hook_over_a_decode_loop(tmp_path):
     """A stand-in engine (block pool, per-group block manager, worker block table) drives the hook
     through ``engine_glue`` for 80 decode steps of two requests: the scheduler's and the worker's

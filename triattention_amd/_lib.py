@@ -33,7 +33,8 @@ EXPORTS = (
     "tri_abi_version", "tri_last_error", "tri_source_digest", "tri_set_tuning", "tri_get_tuning", "tri_resident_gate_enter",
     "tri_resident_gate_leave", "tri_fold_stats", "tri_workspace_bytes", "tri_workspace_status_offset",
     "tri_score_paged",
-    "tri_select", "tri_select_paged", "tri_select_path", "tri_describe_plan", "tri_topk_rows", "tri_compact_paged", "tri_compact_full_staging_bytes",
+    "tri_select", "tri_select_paged", "tri_select_path", "tri_describe_plan", "tri_topk_rows", "tri_dense_workspace_bytes", "tri_dense_compress",
+    "tri_compact_paged", "tri_compact_full_staging_bytes",
     "tri_compact_paged_full", "tri_compress_step", "tri_compress_step_static", "tri_qstats_workspace_bytes", "tri_qstats",
 )
 
@@ -80,6 +81,17 @@ class SelectParams(C.Structure):
     ]
 
 
+class DenseParams(C.Structure):
+    _fields_ = (
+        [(n, C.c_int32) for n in ("num_heads", "num_tokens", "head_dim", "kv_dtype", "rope_style", "budget", "window_size",
+                                  "normalize", "round_start", "num_offsets", "aggregation", "disable_mlr", "disable_trig",
+                                  "v_row_bytes")]
+        + [(n, C.c_void_p) for n in ("k", "v")]
+        + [(n, C.c_int64) for n in ("k_stride_head", "k_stride_token", "v_stride_head", "v_stride_token")]
+        + [(n, C.c_void_p) for n in ("q_mean_complex", "q_abs_mean", "freq_scale_sq", "omega", "offsets", "out_k", "out_v",
+                                     "out_keep")])
+
+
 class TriError(RuntimeError):
     def __init__(self, code: int, message: str):
         super().__init__(f"libtriattention_hip error {code}: {message}")
@@ -117,6 +129,9 @@ def load() -> C.CDLL:
                                     P, I64, I64, I64, P, U64, P]
     lib.tri_select.argtypes = [C.POINTER(KvLayout), C.POINTER(Batch), C.POINTER(ScoreParams),
                                C.POINTER(SelectParams), P, I64, I64, I64, P, P, P, U64, P]
+    lib.tri_dense_workspace_bytes.argtypes = [C.POINTER(DenseParams)]
+    lib.tri_dense_workspace_bytes.restype = U64
+    lib.tri_dense_compress.argtypes = [C.POINTER(DenseParams), P, U64, P]
     lib.tri_select_paged.argtypes = [C.POINTER(KvLayout), C.POINTER(Batch), C.POINTER(ScoreParams),
                                      C.POINTER(SelectParams), P, P, P, U64, P]
     lib.tri_select_path.argtypes = [C.POINTER(KvLayout), C.POINTER(Batch), C.POINTER(ScoreParams),

@@ -2,9 +2,10 @@
 
 The reference's ``TriAttentionCompressor`` (triattention/vllm/core/compressor.py:27-421)
 with ``CompressionState`` (core/state.py:23-196) and the dense helpers of
-core/utils.py:433-502.  Scoring, normalisation, window guard and top-k run in the HIP
-kernels; only the final gather into NEW dense tensors uses ``torch.gather`` (this API
-returns fresh tensors, it does not touch a paged cache).
+core/utils.py:433-502.  Ordinary device tensors go through one library call from the scores
+to the gathered rows (``ops.dense_compress``); what that call does not take (gradients wanted,
+a scoring mode or dtype of its own, rows that are not 16-byte multiples) is put together from the
+scoring and top-k kernels and torch's normalisation and gather.
 """
 from __future__ import annotations
 
@@ -157,6 +158,47 @@ class TriAttentionCompressor:
         keep = ops.topk_rows(flat, k)[:, :k].to(torch.long)
         return keep.reshape(*scores.shape[:-1], k)
 
+    def _one_call_args(self, keys: torch.Tensor, values: torch.Tensor, layer_idx: int):
+        """The fp32 statistics (q_mean_complex, q_abs_mean, freq_scale_sq) for ``ops.dense_compress``, or None
+        where the step has to take the general way: everything that call would not do in the same way --
+        gradients, forward-mode tangents, transformed or traced tensors, which only torch's gather carries; scores
+        per layer or of a narrower type; a layout or a budget outside the kernels' range -- and every
+        argument that the general way refuses."""
+        cfg = self.config
+        h, t, d = keys.shape[1:]
+        if type(self) is not TriAttentionCompressor or not self.__dict__.keys().isdisjoint(("_compute_scores", "_select_topk")):
+            return None                       # (a step of its own in a subclass or on the instance)
+        if (type(keys) is not torch.Tensor or type(values) is not torch.Tensor or values.ndim != 4
+                or not keys.is_cuda or values.device != keys.device or keys.device.index != torch.cuda.current_device()
+                or keys.dtype not in (torch.bfloat16, torch.float16) or values.shape[:3] != keys.shape[:3]
+                or keys.shape[0] != 1 or d not in (64, 128, 256) or h > 256):
+            return None
+        if ((torch.is_grad_enabled() and (keys.requires_grad or values.requires_grad))
+                or torch.autograd.forward_ad._current_level >= 0 or torch.jit.is_tracing()
+                or torch._C._functorch.is_functorch_wrapped_tensor(keys)
+                or torch._C._functorch.is_functorch_wrapped_tensor(values)
+                or values.is_conj() or values.is_neg()):
+            return None
+        if (cfg.topk_dtype != torch.float32 or cfg.pruning_mode == "per_layer" or cfg.score_aggregation not in ("mean", "max")
+                or cfg.rope_style not in ("half", "interleaved") or not 0 < cfg.kv_budget <= t or t < 2):
+            return None
+        ks, vs, row = keys.stride(), values.stride(), values.shape[3] * values.element_size()
+        if (ks[3] != 1 or vs[3] != 1 or ks[1] % 8 or ks[2] % 8 or ks[1] < d or row == 0 or row % 16
+                or (vs[1] * values.element_size()) % 16 or (vs[2] * values.element_size()) % 16
+                or keys.data_ptr() % 16 or values.data_ptr() % 16):
+            return None
+        entry = self.head_stats.get(layer_idx)
+        if entry is None or "q_abs_mean" not in entry:
+            return None
+        stats = (entry["q_mean_complex"], entry["q_abs_mean"], self.freq_scale_sq[layer_idx])
+        f = d // 2
+        if tuple(stats[0].shape) != (h, f, 2) or tuple(stats[1].shape) != (h, f) or tuple(stats[2].shape) != (h, f):
+            return None
+        if self.omega.numel() != f or self.offsets.numel() > 32:
+            return None
+        return tuple(x.to(device=keys.device, dtype=torch.float32).contiguous()
+                     for x in (*stats, self.omega, self.offsets))
+
     def compress(self, key_states: torch.Tensor, value_states: torch.Tensor,
                  cache_positions: Optional[torch.Tensor] = None, layer_idx: int = 0
                  ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -167,6 +209,16 @@ class TriAttentionCompressor:
             raise ValueError(f"TriAttention currently only supports batch_size=1 for compression. Got batch_size={b}.")
         if not self.state.should_compress(t):
             return key_states, value_states, torch.arange(t, device=key_states.device)
+        one_call = self._one_call_args(key_states, value_states, layer_idx)
+        if one_call is not None:
+            cfg = self.config
+            keys, values, keep = ops.dense_compress(
+                key_states, value_states, *one_call, budget=cfg.kv_budget, round_start=int(self.state.get_round_start()),
+                window_size=cfg.window_size, normalize=bool(cfg.sparse_normalize_scores),
+                aggregation=cfg.score_aggregation, rope_style=cfg.rope_style, disable_mlr=bool(cfg.disable_mlr),
+                disable_trig=bool(cfg.disable_trig))
+            self.state.update_after_compression(keys.shape[2])
+            return keys, values, keep
         scores = self._compute_scores(key_states, layer_idx)
         if self.config.sparse_normalize_scores:
             scores = normalize_scores(scores)

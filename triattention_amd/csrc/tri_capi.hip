@@ -580,6 +580,100 @@ int tri_topk_rows(const float* scores, int64_t row_pitch, int32_t num_rows, cons
                        "topk_rows");
 }
 
+namespace {
+
+// A dense call as the general layout, batch and parameters, on a workspace whose last part holds what those
+// point to.
+struct DensePlan {
+  tri_kv_layout kv{};
+  tri_batch batch{};
+  tri_score_params sp{};
+  tri_select_params sel{};
+  tri::Workspace w{};
+  int64_t arg_key, arg_words, folded, keep32, total;
+};
+
+int plan_dense(const tri_dense_params* p, DensePlan& d) {
+  if (!p) return fail(TRI_ERR_INVALID_ARGUMENT, "dense params are NULL");
+  if (p->kv_dtype != TRI_KV_BF16 && p->kv_dtype != TRI_KV_FP16)
+    return fail(TRI_ERR_UNSUPPORTED, "tri_dense_compress takes two-byte keys, got kv_dtype %d", p->kv_dtype);
+  if (p->num_tokens <= 0 || p->budget <= 0 || p->budget > p->num_tokens)
+    return fail(TRI_ERR_INVALID_ARGUMENT, "budget %d of %d tokens", p->budget, p->num_tokens);
+  if (p->k_stride_head % 2 || p->k_stride_token % 2)
+    return fail(TRI_ERR_INVALID_ARGUMENT, "key strides must be whole elements");
+  d.kv.num_layers = 1; d.kv.num_kv_heads = p->num_heads; d.kv.head_dim = p->head_dim; d.kv.block_size = p->num_tokens;
+  d.kv.kv_dtype = p->kv_dtype; d.kv.rope_style = p->rope_style;
+  d.kv.stride_block = p->k_stride_head / 2 * p->num_heads;          // one sequence: never used as a distance
+  d.kv.stride_token = p->k_stride_token / 2; d.kv.stride_head = p->k_stride_head / 2;
+  d.batch.num_seqs = 1; d.batch.max_seq_len = p->num_tokens; d.batch.max_budget = p->budget;
+  d.sp.num_score_heads = p->num_heads; d.sp.num_offsets = p->num_offsets; d.sp.aggregation = p->aggregation;
+  d.sel.normalize = p->normalize ? 1 : 0; d.sel.window_size = p->window_size;
+  d.sel.group_reduce = TRI_REDUCE_MAX; d.sel.layer_reduce = TRI_REDUCE_MEAN;
+  d.sel.group_first = 1; d.sel.no_resident = 1;
+  if (p->num_heads <= 0 || p->num_heads > 256 ||
+      (p->head_dim != 64 && p->head_dim != 128 && p->head_dim != 256) || p->num_offsets <= 0)
+    return fail(TRI_ERR_UNSUPPORTED, "%d heads of %d, %d offsets", p->num_heads, p->head_dim, p->num_offsets);
+  d.w = plan(&d.kv, &d.batch, &d.sp, 0, false);
+  int64_t off = d.w.total;
+  auto take = [&](int64_t bytes) { const int64_t o = off; off = tri::align_up(off + bytes, 256); return o; };
+  d.arg_key = take(8);
+  d.arg_words = take(12);
+  d.folded = take((int64_t)p->num_heads * 3 * (p->head_dim / 2) * 4);
+  d.keep32 = take((int64_t)p->num_heads * p->budget * 4);
+  d.total = off;
+  return TRI_OK;
+}
+
+}  // namespace
+
+uint64_t tri_dense_workspace_bytes(const tri_dense_params* params) {
+  DensePlan d;
+  return plan_dense(params, d) ? 0 : (uint64_t)d.total;
+}
+
+int tri_dense_compress(const tri_dense_params* p, void* ws, uint64_t ws_bytes, void* stream) {
+  DensePlan d;
+  int rc = plan_dense(p, d);
+  if (rc) return rc;
+  tri::Workspace need = d.w;
+  need.total = d.total;
+  rc = check_workspace(need, ws, ws_bytes);
+  if (rc) return rc;
+  if (!p->k || !p->v || !p->q_mean_complex || !p->q_abs_mean || !p->freq_scale_sq || !p->out_k || !p->out_v || !p->out_keep)
+    return fail(TRI_ERR_INVALID_ARGUMENT, "tri_dense_compress: NULL pointer");
+  if (!is_aligned(p->k, 16) || !is_aligned(p->v, 16) || !is_aligned(p->out_k, 16) || !is_aligned(p->out_v, 16))
+    return fail(TRI_ERR_INVALID_ARGUMENT, "tri_dense_compress: bases must be 16-byte aligned");
+  if (p->v_row_bytes <= 0 || p->v_row_bytes % 16 || p->v_stride_head % 16 || p->v_stride_token % 16 ||
+      p->k_stride_head % 16 || p->k_stride_token % 16)
+    return fail(TRI_ERR_INVALID_ARGUMENT, "tri_dense_compress: rows and strides must be multiples of 16 bytes");
+  d.kv.k_layers = at<const void*>(ws, d.arg_key);
+  int32_t* words = at<int32_t>(ws, d.arg_words);
+  d.batch.seq_lens = words; d.batch.round_start = words + 1; d.batch.budgets = words + 2;
+  d.sp.folded = at<float>(ws, d.folded); d.sp.omega = p->omega; d.sp.offsets = p->offsets;
+  rc = check_layout(&d.kv, false);
+  if (!rc) rc = check_batch(&d.batch, true);
+  if (!rc) rc = check_score(&d.kv, &d.sp);
+  if (!rc) rc = check_select(&d.sel);
+  if (rc) return rc;
+  tri::DenseLaunch l{};
+  l.k = p->k; l.v = p->v;
+  l.k_stride_head = p->k_stride_head; l.k_stride_token = p->k_stride_token;
+  l.v_stride_head = p->v_stride_head; l.v_stride_token = p->v_stride_token;
+  l.k_row_bytes = p->head_dim * 2; l.v_row_bytes = p->v_row_bytes;
+  l.H = p->num_heads; l.T = p->num_tokens; l.D = p->head_dim; l.budget = p->budget; l.round_start = p->round_start;
+  l.disable_mlr = p->disable_mlr; l.disable_trig = p->disable_trig;
+  l.q_mean = p->q_mean_complex; l.q_abs = p->q_abs_mean; l.freq_scale = p->freq_scale_sq;
+  l.out_k = p->out_k; l.out_v = p->out_v; l.out_keep = p->out_keep;
+  l.folded = at<float>(ws, d.folded); l.arg_key = at<const void*>(ws, d.arg_key); l.arg_words = words;
+  l.keep32 = at<int32_t>(ws, d.keep32);
+  hipStream_t s = (hipStream_t)stream;
+  rc = launch_status(tri::launch_dense_prologue(l, s), "dense prologue");
+  if (rc) return rc;
+  rc = do_select_paged(&d.kv, &d.batch, &d.sp, &d.sel, nullptr, at<int32_t>(ws, d.keep32), ws, d.w, s);
+  if (rc) return rc;
+  return launch_status(tri::launch_dense_gather(l, s), "dense gather");
+}
+
 int tri_compact_paged(const tri_kv_layout* kv, const tri_batch* batch, const int32_t* keep,
                       int32_t keep_per_layer, int32_t shared, void* stream) {
   tri::CompactLaunch a{};

@@ -197,6 +197,24 @@ struct CompactLaunch {
 };
 hipError_t launch_compact(const CompactLaunch& a, hipStream_t s);
 
+// One layer of a dense cache into new tensors (tri_dense.hip).  Strides of K and V in bytes.
+struct DenseLaunch {
+  const void* k; const void* v;
+  int64_t k_stride_head, k_stride_token, v_stride_head, v_stride_token;
+  int k_row_bytes, v_row_bytes;
+  int H, T, D, budget, round_start, disable_mlr, disable_trig;
+  const float* q_mean; const float* q_abs; const float* freq_scale;
+  void* out_k; void* out_v;
+  int64_t* out_keep;
+  // workspace
+  float* folded;           // [H][3][D/2]
+  const void** arg_key;    // the layer table of one entry
+  int32_t* arg_words;      // sequence length, round start, budget
+  const int32_t* keep32;   // [H][budget]
+};
+hipError_t launch_dense_prologue(const DenseLaunch& d, hipStream_t s);
+hipError_t launch_dense_gather(const DenseLaunch& d, hipStream_t s);
+
 // Calibration statistics of one layer's captured queries (tri_calib.hip).
 struct QStatsLaunch {
   const void* q_rot;      // [H][T][D] through (stride_head, stride_token), 16-bit elements

@@ -528,6 +528,37 @@ def topk_rows(scores: torch.Tensor, k: int | Sequence[int], lens: Sequence[int] 
     return keep
 
 
+def dense_compress(keys: torch.Tensor, values: torch.Tensor, q_mean_complex: torch.Tensor, q_abs_mean: torch.Tensor,
+                   freq_scale_sq: torch.Tensor, omega: torch.Tensor, offsets: torch.Tensor, *, budget: int,
+                   round_start: int, window_size: int, normalize: bool, aggregation: str = "mean",
+                   rope_style: str = "half", disable_mlr: bool = False, disable_trig: bool = False):
+    """One layer of a dense cache, keys [1, H, T, D] and values [1, H, T, *], compressed into new tensors by one
+    library call (``tri_dense_compress``).  Returns (keys, values, keep int64 [1, H, budget])."""
+    lib = _lib.load()
+    _, h, t, d = keys.shape
+    ks, vs = keys.stride(), values.stride()
+    k_es, v_es = keys.element_size(), values.element_size()
+    out_k = torch.empty((1, h, budget, d), dtype=keys.dtype, device=keys.device)
+    out_v = torch.empty((1, h, budget, values.shape[3]), dtype=values.dtype, device=values.device)
+    keep = torch.empty((1, h, budget), dtype=torch.int64, device=keys.device)
+    p = _lib.DenseParams(
+        num_heads=h, num_tokens=t, head_dim=d, kv_dtype=_DTYPES[keys.dtype],
+        rope_style=ROPE_INTERLEAVED if rope_style == "interleaved" else ROPE_HALF, budget=budget,
+        window_size=window_size, normalize=int(normalize), round_start=round_start, num_offsets=offsets.numel(),
+        aggregation=REDUCE_MAX if aggregation == "max" else REDUCE_MEAN, disable_mlr=int(disable_mlr),
+        disable_trig=int(disable_trig), v_row_bytes=values.shape[3] * v_es, k=_ptr(keys), v=_ptr(values),
+        k_stride_head=ks[1] * k_es, k_stride_token=ks[2] * k_es, v_stride_head=vs[1] * v_es, v_stride_token=vs[2] * v_es,
+        q_mean_complex=_ptr(q_mean_complex), q_abs_mean=_ptr(q_abs_mean), freq_scale_sq=_ptr(freq_scale_sq),
+        omega=_ptr(omega), offsets=_ptr(offsets), out_k=_ptr(out_k), out_v=_ptr(out_v), out_keep=_ptr(keep))
+    need = int(lib.tri_dense_workspace_bytes(C.byref(p)))
+    if need == 0:
+        raise ValueError("invalid dense call: " + lib.tri_last_error().decode("utf-8", "replace"))
+    buf = torch.empty(need + 256, dtype=torch.uint8, device=keys.device)
+    at = buf.data_ptr()
+    _lib.check(lib.tri_dense_compress(C.byref(p), at + (-at) % 256, need, _stream()))
+    return out_k, out_v, keep
+
+
 def query_stats(q_rot: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, scale: float = 1.0,
                 rope_style: str = "half"):
     """Frequency statistics of one layer's captured query states (scripts/calibrate.py:196-224).
