@@ -23,7 +23,7 @@ struct FusedArgs {
   int64_t stride_block, stride_token, stride_head;
   int L, Hkv, A, G, HC;
   int block_size, bs_shift, block_table_pitch;
-  int tiles_per_seq, tile_tokens, seq_base, num_seqs, Tmax;
+  int tiles_per_seq, tile_tokens, ring_stride, seq_base, num_seqs, Tmax;
   int normalize, window_size, protect_prefill, group_reduce, layer_reduce;
   long long spin_ticks;
   // Several launches (more workgroups than the device holds at once): which launch a

@@ -273,6 +273,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   constexpr int NS = HD / 32;            // key slabs (MFMAs) per step
   constexpr int NSO = NS + NS / 2;       // operands per query-head group
   static_assert(SL % (16 * NB) == 0, "the slack must hold whole rotations of the step buffers");
+  // Token t of layer l sits at (l * ring_stride + t) % RING, ring_stride the tokens of this launch's tiles (at
+  // most TW): what a tile leaves free of the ring is slack, down to SL for a whole tile.
   constexpr int RING = TW + SL;
   constexpr int RQ = 4 * QG;                                   // ring floats per token
   extern __shared__ __align__(16) float lds[];
@@ -546,7 +548,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     const int tl = t + 4 * kb + rsel;
     // first ring slot of the step (scalar; a step never straddles the wrap: t and RING are
     // multiples of 16)
-    const uint32_t slot0 = (uint32_t)(l * TW + t) % RING;
+    const uint32_t slot0 = (uint32_t)(l * a.ring_stride + t) % RING;
 #pragma unroll
     for (int g = 0; g < QG; ++g) {
       float v = 0.f;
@@ -671,7 +673,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       // This lane's entry of chunk 0 inside the wave's ring; chunk k lies 64 k entries further on, or
       // RING entries back once that passes the ring's end (one compare and one select per chunk, the
       // distance itself goes into the LDS instruction's offset field).
-      const uint32_t lane_pos = (uint32_t)(l * TW) % RING + (uint32_t)lane;          // below 2 * RING
+      const uint32_t lane_pos = (uint32_t)(l * a.ring_stride) % RING + (uint32_t)lane;          // below 2 * RING
       uint32_t at = lane_pos * 4, at_wrapped = (lane_pos - RING) * 4;               // in floats
       asm volatile("" : "+v"(at), "+v"(at_wrapped));     // (keeps both in vector registers)
       struct Entry { float4 x[QG]; };
@@ -722,7 +724,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       float xs[RQ];
 #pragma unroll
       for (int g = 0; g < QG; ++g) {
-        const float4 x = *reinterpret_cast<const float4*>(&ring[(uint32_t)g * (RING * 4) + ((uint32_t)(l * TW + tl) % RING) * 4]);
+        const float4 x = *reinterpret_cast<const float4*>(&ring[(uint32_t)g * (RING * 4) + ((uint32_t)(l * a.ring_stride + tl) % RING) * 4]);
         xs[4 * g] = x.x; xs[4 * g + 1] = x.y; xs[4 * g + 2] = x.z; xs[4 * g + 3] = x.w;
       }
       float v;
@@ -754,7 +756,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // but key loads and scoring, and the work at layer boundaries sits between them.
   const int nsteps = (ntok + 15) >> 4;
   const int rotations = (nsteps + NB - 1) / NB;
-  const int rot_before_consume = min(SL / (16 * NB), rotations);
+  const int rot_before_consume = min((RING - a.ring_stride) / (16 * NB), rotations);
   auto score = [&](const StepData<DT, HD>& d, int l, int slot, int which) __attribute__((always_inline)) {
     if (slot < nsteps) compute_step(d, l, slot * 16, which);
   };
@@ -959,7 +961,7 @@ hipError_t launch_mfma_tw(FusedArgs& k, const uint4* bmat, int tw, int waves, in
   if (k.G > 4) {
     switch (tw) {   // eight query heads per KV head: 32 bytes of ring per token
       case 512: return launch_mfma_t<DT, IL, 512, 64, 2, 4>(k, bmat, shape, s);
-      case 256: return launch_mfma_t<DT, IL, 256, 64, 2, 4>(k, bmat, shape, s);
+      case 256: return launch_mfma_t<DT, IL, 256, 320, 2, 4>(k, bmat, shape, s);
       default: return hipErrorInvalidValue;
     }
   }
@@ -967,11 +969,12 @@ hipError_t launch_mfma_tw(FusedArgs& k, const uint4* bmat, int tw, int waves, in
   constexpr int NB = DT == TRI_KV_FP8_E4M3 ? 8 : 4;
   // Slack: as much as LDS allows beside the ring of a 1024-token tile, in whole rotations
   // (16 x 16384 tokens x 36 layers, bf16, warm GPU: 3.54 ms with 64, 3.49 with 128, 3.45 with 192).
+  // The instances of shorter tiles keep the same ring (one workgroup has the CU's LDS to itself).
   constexpr int SL = DT == TRI_KV_FP8_E4M3 ? 128 : 192;
   switch (tw) {
     case 1024: return launch_mfma_t<DT, IL, 1024, SL, 1, NB>(k, bmat, shape, s);
-    case 512: return launch_mfma_t<DT, IL, 512, SL, 1, NB>(k, bmat, shape, s);
-    case 256: return launch_mfma_t<DT, IL, 256, SL, 1, NB>(k, bmat, shape, s);
+    case 512: return launch_mfma_t<DT, IL, 512, SL + 512, 1, NB>(k, bmat, shape, s);
+    case 256: return launch_mfma_t<DT, IL, 256, SL + 768, 1, NB>(k, bmat, shape, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1154,6 +1157,8 @@ hipError_t launch_fused_mfma(const FusedLaunch& a, hipStream_t s) {
   k.block_size = a.block_size; k.bs_shift = a.plan.bs_shift;
   k.block_table_pitch = a.block_table ? a.block_table_pitch : -1;
   k.tiles_per_seq = a.plan.tiles_per_seq; k.tile_tokens = a.plan.tile_tokens;
+  k.ring_stride = (int)align_up(k.tile_tokens, 16);
+  if (k.ring_stride > a.plan.tw) return hipErrorInvalidValue;
   k.layer_groups = a.plan.layer_groups > 1 ? a.plan.layer_groups : 1;
   k.layers_per_group = k.layer_groups > 1 ? a.plan.layers_per_group : a.L;
   k.fin_part = a.fin_part;
