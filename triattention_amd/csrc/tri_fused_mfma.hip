@@ -140,13 +140,13 @@ __device__ __forceinline__ float coefficient_piece(float x, int pieces) {
   return x;
 }
 
-// Everything the resident kernel needs before it starts, in one launch: workgroup (l, b)
-//  - clears its share of the exchange words (and workgroup (0, 0) the status word);
+// Everything the resident kernel needs before it starts, in one launch: workgroup (l, b, z)
+//  - clears its share of the exchange words (and workgroup (0, 0, 0) the status word);
 //  - evaluates cos / sin of (round_start[b] + offset_j) * omega_f for all offsets and their
-//    means over the offsets, the way trig_kernel does (phase_cos_sin, means summed in offset
+//    means over the offsets, the way prepare_kernel does (phase_cos_sin, means summed in offset
 //    order in double);
-//  - combines the means with the folded statistics of layer l into P = a1*C - a2*S,
-//    R = a2*C + a1*S, E (as coef_kernel) and writes them as MFMA B operands:
+//  - combines the means with the folded statistics of its KV heads of layer l (heads z * heads_per_wg
+//    and up) into P = a1*C - a2*S, R = a2*C + a1*S, E and writes them as MFMA B operands:
 // bmat[(((b*L + l)*Hkv + head)*QG + g)*6 + o][lane][8] bf16.  Group g holds query heads
 // 4g..4g+3 of the KV head.  Operand o: 0..3 the key slabs of MFMA o, 4 and 5 the magnitudes
 // of pair sets 0 and 1.  Lane (j = lane % 16, kb): column j = (query head 4g + j % 4, split
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
                                                                  const int32_t* round_start, int L, int Hkv, int G,
                                                                  int A, int QG, uint4* bmat,
                                                                  unsigned long long* xchg, int64_t words,
-                                                                 uint32_t* status) {
+                                                                 uint32_t* status, int heads_per_wg) {
   // One buffer, used twice: the per-offset cos / sin values, then the coefficients of up to
   // kPrepHeads query heads as [head][P | R | E][F] with a row pitch of 3F + 1 floats.
   constexpr int F = HD / 2;              // frequency pairs
@@ -177,7 +177,14 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
   static_assert(kPrepHeads * kPrepPitch >= 2 * kMaxOffsets * F, "the trig values must fit the buffer");
   float (*part)[kMaxOffsets][F] = reinterpret_cast<float (*)[kMaxOffsets][F]>(buf);
   const int l = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-  const int64_t wg = (int64_t)b * gridDim.x + l, nwg = (int64_t)gridDim.x * gridDim.y;
+  const int h_begin = blockIdx.z * heads_per_wg, h_end = min(Hkv, h_begin + heads_per_wg);
+  const int64_t wg = ((int64_t)blockIdx.z * gridDim.y + b) * gridDim.x + l;
+  const int64_t nwg = (int64_t)gridDim.x * gridDim.y * gridDim.z;
+  // The first statistics are requested before the phases, on which they do not depend.
+  const float* in = folded + ((int64_t)l * A + (int64_t)h_begin * G) * 3 * F;   // [head][a1 | a2 | e][F]
+  const int first = min(tid, (h_end - h_begin) * G * F - 1);
+  const float* in0 = in + first / F * 3 * F + first % F;
+  const float first_a1 = in0[0], first_a2 = in0[F], first_e = in0[2 * F];
   for (int64_t i = wg * kPrepThreads + tid; i < words; i += nwg * kPrepThreads) xchg[i] = 0ull;
   if (wg == 0 && tid == 0) *status = 0u;
 
@@ -195,14 +202,17 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
   }
 
   const int heads_per_pass = max(1, kPrepHeads / G);        // whole KV heads
-  for (int head0 = 0; head0 < Hkv; head0 += heads_per_pass) {
-    const int nh = min(heads_per_pass, Hkv - head0);
+  for (int head0 = h_begin; head0 < h_end; head0 += heads_per_pass) {
+    const int nh = min(heads_per_pass, h_end - head0);
     __syncthreads();                                        // means written; buffer free
     // P = a1*C - a2*S, R = a2*C + a1*S, E, of query heads head0*G .. (head0 + nh)*G - 1
-    const float* in = folded + ((int64_t)l * A + (int64_t)head0 * G) * 3 * F;   // [head][a1 | a2 | e][F]
     for (int i = tid; i < nh * G * F; i += kPrepThreads) {
       const int q = i / F, f = i % F;
-      const float a1 = in[q * 3 * F + f], a2 = in[q * 3 * F + F + f], e = in[q * 3 * F + 2 * F + f];
+      float a1 = first_a1, a2 = first_a2, e = first_e;
+      if (head0 > h_begin || i >= kPrepThreads) {
+        const float* p = in + ((int64_t)(head0 - h_begin) * G + q) * 3 * F + f;
+        a1 = p[0]; a2 = p[F]; e = p[2 * F];
+      }
       const float c = mean_cs[0][f], sn = mean_cs[1][f];
       buf[q * kPrepPitch + f] = fmaf(a1, c, -a2 * sn);
       buf[q * kPrepPitch + F + f] = fmaf(a2, c, a1 * sn);
@@ -1179,9 +1189,16 @@ hipError_t launch_fused_mfma(const FusedLaunch& a, hipStream_t s) {
   if (a.kv_dtype != TRI_KV_BF16 && !fp8 && !fp16) return hipErrorInvalidValue;
   if (a.NO <= 0 || a.NO > kMaxOffsets || (a.D != 128 && a.D != 64 && a.D != 256)) return hipErrorInvalidValue;
   if (a.D != 128 && fp8) return hipErrorInvalidValue;
+  // A workgroup takes all KV heads of a layer and request, which evaluates the phases least often, unless that
+  // leaves CUs without one: then the heads are halved until there are 256 workgroups.  The launch is a chain of
+  // latencies (statistics, phases, slabs), not bytes: the whole step of one layer x 4096 tokens 56.6 -> 53.0 us with eight
+  // workgroups in place of one and the statistics requested first; 36 layers x 2176 tokens 267 -> 265 (a hook call).
+  int heads_per_wg = a.Hkv;
+  while (heads_per_wg > 1 && (int64_t)a.L * a.B * ceil_div(a.Hkv, heads_per_wg) < 256) heads_per_wg = ceil_div(heads_per_wg, 2);
   auto prep_launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)a.L, (unsigned)a.B), dim3(kPrepThreads), 0, s, a.folded, a.omega,
-                       a.offsets, a.NO, a.round_start, a.L, a.Hkv, a.G, a.A, QG, bmat, a.xchg, words, a.status);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)a.L, (unsigned)a.B, (unsigned)ceil_div(a.Hkv, heads_per_wg)),
+                       dim3(kPrepThreads), 0, s, a.folded, a.omega, a.offsets, a.NO, a.round_start, a.L, a.Hkv, a.G, a.A,
+                       QG, bmat, a.xchg, words, a.status, heads_per_wg);
   };
   if (fp8) {
     if (il) prep_launch(prep_mfma_kernel<TRI_KV_FP8_E4M3, true, 128>);
