@@ -382,6 +382,30 @@ def test_batch_hook_on_the_resident_kernel(tmp_path, monkeypatch):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("tokens,kv_heads,two_pass", [(1185, 8, True), (3072, 6, True), (3072, 2, False)])
+def test_hook_call_for_one_small_request_takes_the_kernels_that_do_not_wait(tmp_path, monkeypatch, tokens, kv_heads, two_pass):
+    """A single request below the selector's limit gives, through the hook, the bits of the score-then-select
+    kernels; a shape without quarter tiles keeps the library's own choice."""
+    from helpers import build_inputs
+    from triattention_amd import ops, synth
+    w = synth.Workload(name="t", num_layers=3, num_q_heads=4 * kv_heads, num_kv_heads=kv_heads, head_dim=128,
+                       seq_lens=(tokens,), budget=256, block_size=16, window_size=12, rope_theta=1e6, index=33)
+    inp = build_inputs(w)
+    runner, reqs, caches, sched, signals = _fake_runner(w, inp, tmp_path)
+    got = RunnerHookCompressionExecutor(runner).execute("r0", signals["r0"], sched)
+    torch.cuda.synchronize()
+    assert got.applied and got.cache_len_after == 256
+    ref = [c.to(DEV) for c in inp["caches"]]
+    batch = ops.StepBatch(DEV, w.seq_lens, round_start=w.seq_lens, budgets=w.budget, block_tables=inp["tables"],
+                          prefill_lens=[0])
+    sc = ops.ScoreConfig(ops.fold_stats(inp["qc"].to(DEV), inp["qa"].to(DEV), inp["fs"].to(DEV)),
+                         inp["omega"].to(DEV), inp["offsets"].to(DEV))
+    ops.compress_step(ops.PagedKV.from_kv_caches(ref), batch, sc,
+                      ops.SelectConfig(window_size=w.window_size, allow_resident=not two_pass))
+    for a, b in zip(caches, ref):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 @pytest.mark.parametrize("resident", [False, True])
 def test_repeated_shape_replays_a_graph_with_the_same_results(tmp_path, monkeypatch, resident):
     """A decoding request comes back to the hook with the same lengths every ``divide_length``

@@ -16,7 +16,7 @@ from typing import Any, Callable, Iterable
 
 import torch
 
-from .. import ops
+from .. import _lib, ops
 from ..core import stats as stats_mod
 from .config import TriAttentionRuntimeConfig
 from .kv_compaction import kv_axis_hint, mark_keep_validated
@@ -332,6 +332,21 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
         per_layer = 4 * len(requests) * (longest * (score_heads + kv.num_kv_heads) + score_heads * 3 * kv.head_dim // 2)
         return max(1, min(len(layer_kv), LAYER_RUN_MAX_SCRATCH_BYTES // per_layer))
 
+    def _small_step(kv: Any, layers: int, score_heads: int, tokens: int) -> bool:
+        # One request whose keys the score-then-select kernels read in quarter tiles (fewer than 256 workgroups
+        # of 512 tokens, head dimension 128 or 256, KV heads that fill a wave).  Their GPU time equals the
+        # resident kernel's there and they cannot fail, so the call does not end in a wait for the status
+        # word: 36 layers x 2176 tokens 266 -> 184 us a call among others, 270 -> 238 with a synchronisation
+        # after each.  (Sixteen such requests gain nothing where each call is waited for, 2786 against
+        # 2796 us, and keep the resident kernel.)  A resident kernel asked for by name is taken.
+        if _lib.get_tuning(_lib.TUNE_RESIDENT_KERNEL) != 0:
+            return False
+        wave_heads = 1024 // kv.head_dim                  # KV heads a wave of the scorer reads at once
+        if kv.head_dim < 128 or kv.dtype not in (torch.bfloat16, torch.float16) or 2 * kv.num_kv_heads <= wave_heads:
+            return False
+        heads = -(-kv.num_kv_heads // wave_heads) * -(-(score_heads // kv.num_kv_heads) // 4)
+        return heads * layers * -(-tokens // 512) < 256
+
     def _compress_layers(layer_kv: list, block_size: int, requests: list, allow_resident: bool) -> list:
         agg = os.environ.get("TRIATTN_RUNTIME_DEBUG_GROUP_PERHEAD_AGG_MODE", "mean").strip().lower()
         if agg not in {"mean", "max"}:
@@ -359,6 +374,8 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
         guards = [int(r["prefill_len"]) if r["protect_prefill"] and int(r["prefill_len"]) > 0 else 0 for r in requests]
         rounds = [int(r["round_start"]) for r in requests]
         tables = [[int(x) for x in r["block_ids"]] for r in requests]
+        if len(requests) == 1 and _small_step(kv, len(layer_ids), score_heads, totals[0]):
+            allow_resident = False
         use_resident = bool(allow_resident) and holder.get("resident_ok", True)
         rows_per_request = (len(layer_ids) if layer_local else 1) * (1 if shared else kv.num_kv_heads)
         rows = len(requests) * rows_per_request
