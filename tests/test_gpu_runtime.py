@@ -406,6 +406,65 @@ def test_hook_call_for_one_small_request_takes_the_kernels_that_do_not_wait(tmp_
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("kw", [dict(), dict(pruning_mode="per_layer_per_head")], ids=["small_step", "layer_local"])
+@pytest.mark.parametrize("replay", [False, True], ids=["eager", "replay"])
+@pytest.mark.parametrize("threads", [False, True, "external"], ids=["one_thread", "two_threads", "external_streams"])
+def test_hook_calls_on_two_streams_do_not_share_what_is_in_flight(tmp_path, monkeypatch, kw, replay, threads):
+    """Calls that return with their work queued: a second request on another stream, while the first one's work is
+    still held back behind a delay on its own, must not touch the block table, scratch, keep rows or graph
+    that work reads.  Four turns (a shape is captured on its second visit) against a runner that is waited for
+    after every call, with the requests handed over by one thread or by one each, on torch's streams or on streams it only wraps."""
+    import threading
+
+    from helpers import build_inputs
+    from triattention_amd import synth
+    from triattention_amd.runtime import selector as selector_mod
+    monkeypatch.setattr(selector_mod, "GRAPH_REPLAY", replay)
+    w = synth.Workload(name="t", num_layers=3, num_q_heads=32, num_kv_heads=8, head_dim=128, seq_lens=(1185, 1185),
+                       budget=256, block_size=16, window_size=12, rope_theta=1e6, index=37)
+    inp = build_inputs(w)
+    kw = dict(kw, fail_on_effective_len_regression=False)
+    want, got = _fake_runner(w, inp, tmp_path, **kw), _fake_runner(w, inp, tmp_path, **kw)
+    start = [c.clone() for c in want[2]]
+    own = [torch.cuda.Stream(), torch.cuda.Stream()]
+    streams = [torch.cuda.ExternalStream(s.cuda_stream) for s in own] if threads == "external" else own
+    for turn in range(4):
+        print(f"two streams {kw} replay={replay} threads={threads} turn={turn}", flush=True)
+        for runner, reqs, caches, _, _ in (want, got):
+            for c, c0 in zip(caches, start):
+                c.copy_(c0)
+            for b, rid in enumerate(reqs):
+                reqs[rid].num_computed_tokens = 1185 + 40 * turn + b
+                reqs[rid].block_ids = ([int(x) for x in inp["tables"][b]],)
+        torch.cuda.synchronize()
+        for rid in want[1]:
+            want[0].triattention_apply_compression(req_id=rid, signal=want[4][rid], scheduler_output=want[3])
+            torch.cuda.synchronize()
+        results = {}
+
+        def call(b):
+            with torch.cuda.stream(streams[(b + turn) % 2]):
+                if b == 0:
+                    torch.cuda._sleep(20_000_000)
+                results[b] = got[0].triattention_apply_compression(req_id=f"r{b}", signal=got[4][f"r{b}"],
+                                                                   scheduler_output=got[3])
+
+        if threads is True:
+            workers = [threading.Thread(target=call, args=(b,)) for b in (0, 1)]
+            for t in workers:
+                t.start()
+            for t in workers:
+                t.join()
+        else:
+            call(0)
+            call(1)
+        torch.cuda.synchronize()
+        assert sorted(results) == [0, 1] and all(r["applied"] for r in results.values())
+        for a, b, c0 in zip(want[2], got[2], start):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)), f"turn {turn}"
+            assert not torch.equal(a.view(torch.int16), c0.view(torch.int16))
+
+
 @pytest.mark.parametrize("resident", [False, True])
 def test_repeated_shape_replays_a_graph_with_the_same_results(tmp_path, monkeypatch, resident):
     """A decoding request comes back to the hook with the same lengths every ``divide_length``

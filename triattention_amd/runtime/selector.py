@@ -11,6 +11,7 @@ index (the reference's ``torch.topk`` leaves them undefined).
 from __future__ import annotations
 
 import os
+import threading
 from pathlib import Path
 from typing import Any, Callable, Iterable
 
@@ -98,6 +99,62 @@ class ResidentLaunchFailed(RuntimeError):
     another workload for seconds); nothing was compacted, the step can be repeated."""
 
 
+class _Turn:
+    """One call at a time on what a selector keeps for all of its calls: captured graphs, scratch, keep rows,
+    the step's integers, the folded statistics.  A call may return with its kernels still queued, so
+    threads take turns on the host (the lock is held until the call's work is queued) and a call on another
+    stream than the one before it waits, on the device, for an event behind that one's work.  The event is recorded when
+    that other stream turns up (behind every call it costs 5 of 182 us: a barrier on the GPU); only a stream that may be
+    destroyed meanwhile, one made outside torch, gets it at once.  A call
+    under an outer stream capture can neither wait for such an event nor leave one; it uses buffers of
+    its own (``capturing``)."""
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._stream = self._event = None
+        self._several = False             # calls have come on more than one stream
+        self.capturing = False
+
+    def __enter__(self):
+        self._lock.acquire()
+        try:
+            self.capturing = torch.cuda.is_current_stream_capturing()
+            if not self.capturing:
+                stream = torch.cuda.current_stream()
+                if self._stream is not None and stream != self._stream:
+                    self._several = True
+                    self._wait_for_last(stream)
+                self._stream, self._event = stream, None
+            return self
+        except BaseException:
+            self._lock.release()
+            raise
+
+    def _wait_for_last(self, stream) -> None:
+        if self._event is None:
+            with torch.cuda.stream(self._stream):
+                if torch.cuda.is_current_stream_capturing():
+                    raise RuntimeError("the stream of the previous call is being captured")
+                self._event = self._stream.record_event()
+        stream.wait_event(self._event)
+
+    def uses(self, *tensors) -> None:
+        """Memory of one stream that this call uses on another: not handed out again before that is done."""
+        if self._several and not self.capturing:
+            for t in tensors:
+                if t is not None:
+                    t.record_stream(self._stream)
+
+    def __exit__(self, *exc):
+        try:
+            # torch's own streams (id 0, odd ids) live as long as the process; the id of any other is its address
+            if not self.capturing and self._stream.stream_id != 0 and self._stream.stream_id % 2 == 0:
+                self._event = self._stream.record_event()
+        finally:
+            self._lock.release()
+        return False
+
+
 def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: Any | None = None):
     """(select_keep_indices, select_keep_indices_for_group, status)."""
     mode = config.pruning_mode
@@ -134,6 +191,7 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
                 break
 
     holder: dict = {}
+    turn = _Turn()
 
     def _stats() -> _DeviceStats:
         if "s" not in holder:
@@ -313,7 +371,14 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
         the kept rows in slots ``0..k-1``.  Raises
         ``ResidentLaunchFailed`` with the caches of this group untouched when a wait inside the
         resident kernel expired; the caller repeats the call with ``allow_resident=False``, which
-        takes the kernels that do not wait for each other."""
+        takes the kernels that do not wait for each other.
+
+        The caches are compacted in the order of the current stream; a call that took no resident kernel
+        returns with the work queued there.  Calls may come from several threads and on several streams."""
+        with turn:
+            return _compress_in_turn(layer_kv, block_size, requests, allow_resident)
+
+    def _compress_in_turn(layer_kv: list, block_size: int, requests: list, allow_resident: bool) -> list:
         if layer_local and len(layer_kv) > 1:
             run = _layers_per_run(layer_kv, requests)
             if run < len(layer_kv):
@@ -374,7 +439,7 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
         guards = [int(r["prefill_len"]) if r["protect_prefill"] and int(r["prefill_len"]) > 0 else 0 for r in requests]
         rounds = [int(r["round_start"]) for r in requests]
         tables = [[int(x) for x in r["block_ids"]] for r in requests]
-        if len(requests) == 1 and _small_step(kv, len(layer_ids), score_heads, totals[0]):
+        if not turn.capturing and len(requests) == 1 and _small_step(kv, len(layer_ids), score_heads, totals[0]):
             allow_resident = False
         use_resident = bool(allow_resident) and holder.get("resident_ok", True)
         rows_per_request = (len(layer_ids) if layer_local else 1) * (1 if shared else kv.num_kv_heads)
@@ -388,11 +453,14 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
                agg, use_resident)
         graphs = holder.setdefault("graphs", {})       # captured shapes, least recently used first
         seen = holder.setdefault("seen", {})           # keys of shapes that ran once, oldest first
-        entry = graphs.get(key) if GRAPH_REPLAY else None
+        replay = GRAPH_REPLAY and not turn.capturing
+        entry = graphs.get(key) if replay else None
+        turn.uses(sc.folded, omega, offsets, kv.k_ptrs, kv.v_ptrs, kv.ks_ptrs, kv.vs_ptrs)
         try:
             if entry is not None:
                 graphs[key] = graphs.pop(key)          # most recently used
                 batch, ws, keep, resident = entry["batch"], entry["ws"], entry["keep"], entry["resident"]
+                turn.uses(batch._flat, ws.buf, keep)
                 batch.refill(rounds, tables, guards)
                 if resident:
                     # A graph holds neither the wait on the process's previous resident launch nor the
@@ -409,7 +477,9 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
                                        protect_prefill=any(g > 0 for g in guards), group_reduce=group_reduce,
                                        layer_reduce=agg, shared=shared, allow_resident=use_resident)
                 resident = ops.select_path(kv, batch, sc, sel) != "two_pass"
-                if not (GRAPH_REPLAY and key in seen):
+                if turn.capturing:
+                    keep, ws = ops.compress_step(kv, batch, sc, sel)
+                elif not (replay and key in seen):
                     # Scratch and keep rows of the previous step are reused when they fit; the results
                     # handed out below are fresh tensors.
                     keep_buf = holder.get("keep")
@@ -419,7 +489,8 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
                     keep, ws = ops.compress_step(kv, batch, sc, sel, holder.get("ws"),
                                                  keep_buf[:rows * batch.max_budget].view(rows, batch.max_budget))
                     holder["ws"] = ws
-                    if GRAPH_REPLAY and ws.bytes <= GRAPH_MAX_SCRATCH_BYTES:
+                    turn.uses(ws.buf, keep_buf)
+                    if replay and ws.bytes <= GRAPH_MAX_SCRATCH_BYTES:
                         if len(seen) >= GRAPH_MAX_SEEN:
                             seen.pop(next(iter(seen)))
                         seen[key] = True
