@@ -651,6 +651,41 @@ def test_dense_compressor_in_one_call_equals_its_parts(tmp_path, case):
     assert k3.stride() == k2.stride() and v3.stride() == v2.stride()
 
 
+@pytest.mark.parametrize("normalize", [True, False])
+@pytest.mark.parametrize("window", [16, 0])
+@pytest.mark.parametrize("bad", ["nan", "-nan", "inf", "-inf"])
+def test_dense_compressor_in_one_call_treats_scores_that_are_no_numbers_like_its_parts(tmp_path, bad, window, normalize):
+    """Keys that make a score NaN or infinite: through torch's normalisation and the top-k a NaN is the largest score
+    of its row (with the sign set the smallest) and turns a normalised row into NaN of that sign throughout.  Heads 1
+    and 2 hold such keys, in and before the protected window; without normalisation the scores of the two ways are the
+    same bits and a normalised row is all ties, so the lists are equal.  In a normalised row with infinite scores and no NaN
+    the sign is an accident of torch's reduction; one call gives the window and the first tokens."""
+    g = torch.Generator().manual_seed(31)
+    h, t, d, budget = 4, 600, 128, 128
+    omega = 1.0 / (1e6 ** (torch.arange(0, d, 2, dtype=torch.float32) / d))
+    qc = torch.randn(1, h, d // 2, 2, generator=g)
+    _write_stats(tmp_path / "s.pt", qc, qc.pow(2).sum(-1).sqrt() + 1, omega, d)
+    bits = {"nan": 0x7fc0, "-nan": 0xffc0 - 0x10000, "inf": 0x7f80, "-inf": 0xff80 - 0x10000}[bad]
+    keys = torch.randn(1, h, t, d, generator=g).to(torch.bfloat16)
+    for head, token, lane in ((1, 77, 5), (2, 300, 70), (2, 590, 3)):
+        keys.view(torch.int16)[0, head, token, lane] = bits
+    keys = keys.to(DEV)
+    cfg = TriAttentionConfig(device=torch.device(DEV), stats_path=tmp_path / "s.pt", kv_budget=budget, divide_length=16,
+                             window_size=window, protect_prefill=False, compute_dtype=torch.float32,
+                             sparse_normalize_scores=normalize)
+    one, parts = TriAttentionCompressor(cfg), TriAttentionCompressor(cfg)
+    parts._one_call_args = lambda *a: None
+    keep, keep_parts = one.compress(keys, keys)[2], parts.compress(keys, keys)[2]
+    raw = parts._compute_scores(keys, 0)[0]
+    first = torch.cat([torch.arange(budget - window), torch.arange(t - window, t)]).to(DEV)
+    for head in (1, 2):
+        assert not raw[head].isfinite().all()
+        if raw[head].isnan().any() or not normalize:
+            assert torch.equal(keep[0, head], keep_parts[0, head]), head
+        else:
+            assert torch.equal(keep[0, head], first), head
+
+
 def test_dense_compressor_leaves_other_calls_to_its_parts(tmp_path):
     """Gradients, forward-mode tangents, vmapped values and rows that are not multiples of 16 bytes."""
     g = torch.Generator().manual_seed(29)

@@ -5,7 +5,9 @@ with ``CompressionState`` (core/state.py:23-196) and the dense helpers of
 core/utils.py:433-502.  Ordinary device tensors go through one library call from the scores
 to the gathered rows (``ops.dense_compress``); what that call does not take (gradients wanted,
 a scoring mode or dtype of its own, rows that are not 16-byte multiples) is put together from the
-scoring and top-k kernels and torch's normalisation and gather.
+scoring and top-k kernels and torch's normalisation and gather.  NaN scores rank alike both ways (above
++inf, or lowest with the sign set); only the sign of the NaN that a normalised row with infinite scores and
+no NaN, or with NaN of both signs, turns into differs: there torch's depends on the order of its reduction.
 """
 from __future__ import annotations
 

@@ -240,7 +240,7 @@ int check_select(const tri_select_params* sel) {
 int do_select(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
               const tri_select_params* sel, const float* raw, int64_t rs_layer, int64_t rs_token,
               int64_t rs_head, float* fin, int32_t* keep, void* ws, const tri::Workspace& w, hipStream_t s,
-              int fine, const float* partial) {
+              int fine, const float* partial, int pass_nan) {
   tri::SelectLaunch a{};
   a.B = batch->num_seqs; a.L = kv->num_layers; a.Hkv = kv->num_kv_heads; a.A = sp->num_score_heads;
   a.G = sp->num_score_heads / kv->num_kv_heads; a.Tmax = batch->max_seq_len; a.fine = fine;
@@ -248,6 +248,7 @@ int do_select(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_p
   a.normalize = sel->normalize; a.window_size = sel->window_size; a.protect_prefill = sel->protect_prefill;
   a.group_reduce = sel->group_reduce; a.layer_reduce = sel->layer_reduce; a.shared = sel->shared;
   a.group_first = sel->group_first ? 1 : 0;
+  a.pass_nan = pass_nan;
   a.seq_lens = batch->seq_lens; a.prefill_lens = batch->prefill_lens; a.budgets = batch->budgets;
   a.partial = partial; a.mustd = at<float>(ws, w.mustd);
   a.raw = raw; a.raw_stride_layer = rs_layer; a.raw_stride_token = rs_token; a.raw_stride_head = rs_head;
@@ -273,7 +274,7 @@ bool takes_resident(const tri::Workspace& w, const tri_kv_layout* kv, const tri_
 // else score into the workspace and select from there.
 int do_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
                     const tri_select_params* sel, float* fin, int32_t* keep, void* ws, const tri::Workspace& w,
-                    hipStream_t s) {
+                    hipStream_t s, int pass_nan = 0) {
   const bool fused = takes_resident(w, kv, sel);
   if (!fused) {
     float* raw = at<float>(ws, w.raw);
@@ -290,7 +291,7 @@ int do_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_s
     // The status word belongs to the resident kernel; on this path it just reads "fine".
     const int rc = do_score(kv, batch, sp, raw, rs_layer, A, 1, ws, w, s, fine, partial, at<uint32_t>(ws, w.status));
     if (rc) return rc;
-    return do_select(kv, batch, sp, sel, raw, rs_layer, A, 1, fin, keep, ws, w, s, fine, partial);
+    return do_select(kv, batch, sp, sel, raw, rs_layer, A, 1, fin, keep, ws, w, s, fine, partial, pass_nan);
   }
   const int F = kv->head_dim / 2;
   hipError_t e = hipSuccess;
@@ -509,7 +510,7 @@ int tri_select(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_
   rc = check_workspace(w, workspace, workspace_bytes);
   if (rc) return rc;
   return do_select(kv, batch, sp, sel, raw, raw_stride_layer, raw_stride_token, raw_stride_head, final_scores,
-                   keep, workspace, w, (hipStream_t)stream, 0, at<float>(workspace, w.partial));
+                   keep, workspace, w, (hipStream_t)stream, 0, at<float>(workspace, w.partial), 0);
 }
 
 int tri_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
@@ -669,7 +670,9 @@ int tri_dense_compress(const tri_dense_params* p, void* ws, uint64_t ws_bytes, v
   hipStream_t s = (hipStream_t)stream;
   rc = launch_status(tri::launch_dense_prologue(l, s), "dense prologue");
   if (rc) return rc;
-  rc = do_select_paged(&d.kv, &d.batch, &d.sp, &d.sel, nullptr, at<int32_t>(ws, d.keep32), ws, d.w, s);
+  // (NaN scores stay NaN, the largest of a row or, with the sign set, the smallest: torch's normalisation and
+  // tri_topk_rows, which this call stands for, treat them so)
+  rc = do_select_paged(&d.kv, &d.batch, &d.sp, &d.sel, nullptr, at<int32_t>(ws, d.keep32), ws, d.w, s, 1);
   if (rc) return rc;
   return launch_status(tri::launch_dense_gather(l, s), "dense gather");
 }

@@ -123,6 +123,7 @@ hipError_t launch_score(const ScoreLaunch& a, hipStream_t s);
 struct SelectLaunch {
   int B, L, Hkv, A, G, Tmax, fine, max_budget;
   int normalize, window_size, protect_prefill, group_reduce, layer_reduce, shared, group_first;
+  int pass_nan;         // one query head per KV head and a row of its own: its score passes as it is, NaN included
   const int32_t* seq_lens;
   const int32_t* prefill_lens;
   const int32_t* budgets;

@@ -90,7 +90,8 @@ __global__ void finalize_stats_kernel(const float* partial, const int32_t* seq_l
 // workgroup per (sequence, layer, KV head).  mustd[(b*L + l)*A*2 + h*2] = (mean, std).
 __global__ __launch_bounds__(256) void group_stats_kernel(const float* raw, int64_t stride_layer, int64_t stride_token,
                                                           int64_t stride_head, const int32_t* seq_lens, int L, int Hkv,
-                                                          int A, int G, int group_reduce, int normalize, float* mustd) {
+                                                          int A, int G, int group_reduce, int normalize, int pass_nan,
+                                                          float* mustd) {
   __shared__ double red[256][2];
   const int h = blockIdx.x % Hkv;
   const int bl = blockIdx.x / Hkv, b = bl / L;
@@ -104,12 +105,15 @@ __global__ __launch_bounds__(256) void group_stats_kernel(const float* raw, int6
   double s = 0.0, q = 0.0;
   for (int n = threadIdx.x; n < T; n += 256) {
     const float* p = base + (int64_t)n * stride_token;
-    float m = (group_reduce == TRI_REDUCE_MAX) ? -INFINITY : 0.f;
-    for (int g = 0; g < G; ++g) {
-      const float x = p[(int64_t)g * stride_head];
-      m = (group_reduce == TRI_REDUCE_MAX) ? fmaxf(m, x) : __fadd_rn(m, x);
+    float m = p[0];
+    if (!pass_nan) {
+      m = (group_reduce == TRI_REDUCE_MAX) ? -INFINITY : 0.f;
+      for (int g = 0; g < G; ++g) {
+        const float x = p[(int64_t)g * stride_head];
+        m = (group_reduce == TRI_REDUCE_MAX) ? fmaxf(m, x) : __fadd_rn(m, x);
+      }
+      if (group_reduce != TRI_REDUCE_MAX) m = __fdiv_rn(m, (float)G);
     }
-    if (group_reduce != TRI_REDUCE_MAX) m = __fdiv_rn(m, (float)G);
     s += (double)m;
     q += (double)m * (double)m;
   }
@@ -211,7 +215,7 @@ struct CombineArgs {
   float* fin;
   int64_t raw_stride_layer, raw_stride_token, raw_stride_head;
   int B, L, Hkv, A, G, Tmax;
-  int window_size, protect_prefill, group_reduce, layer_reduce, shared;
+  int window_size, protect_prefill, group_reduce, layer_reduce, shared, pass_nan;
   int rows_per_seq;   // rows per (sequence[, layer]): shared ? 1 : Hkv
   int tokens_per_wg;  // threads / rows_per_seq
 };
@@ -219,6 +223,16 @@ struct CombineArgs {
 // z-score of one raw value with the reference's operation order: (x - mean) / std.
 __device__ __forceinline__ float zscore(float x, float mean, float sd) {
   return __fdiv_rn(__fsub_rn(x, mean), sd);
+}
+
+// The same where a NaN is a score like another (SelectLaunch::pass_nan); its sign says at which end of the order
+// it lies, and is kept: that of the score itself, else of the row's mean (the subtraction above would turn it).
+// A row with infinite scores and no NaN is NaN throughout too, by inf - inf, with a sign that in torch's reduction
+// depends on where the score stood; here it is negative, below the guarded tokens.
+__device__ __forceinline__ float passed_zscore(float x, float mean, float sd) {
+  const float z = zscore(x, mean, sd);
+  if (!__builtin_isnan(z)) return z;
+  return __builtin_isnan(x) ? x : (__builtin_isnan(mean) ? mean : __uint_as_float(0xffc00000u));
 }
 
 // One thread per (token, output row).  Grid: (token tiles, layers or 1, B).
@@ -316,6 +330,10 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a) {
         const float* ms = a.mustd + (int64_t)(b * a.L + l) * a.A * 2;
         float v = -INFINITY;
         for (int h = h_begin; h < h_end; ++h) {
+          if (a.pass_nan) {      // (the maxima below drop a NaN)
+            v = passed_zscore(raw_l[(int64_t)h * a.raw_stride_head], ms[h * 2], ms[h * 2 + 1]);
+            continue;
+          }
           float gv = (a.group_reduce == TRI_REDUCE_MAX) ? -INFINITY : 0.f;
           for (int q = 0; q < a.G; ++q) {
             const int ah = h * a.G + q;
@@ -814,7 +832,7 @@ hipError_t launch_select(const SelectLaunch& a, hipStream_t s) {
   } else if (a.group_first)
     hipLaunchKernelGGL(group_stats_kernel, dim3(a.B * a.L * a.Hkv), dim3(256), 0, s, a.raw, a.raw_stride_layer,
                        a.raw_stride_token, a.raw_stride_head, a.seq_lens, a.L, a.Hkv, a.A, a.G, a.group_reduce,
-                       a.normalize, a.mustd);
+                       a.normalize, a.pass_nan, a.mustd);
   else
     hipLaunchKernelGGL(finalize_stats_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, a.partial, a.seq_lens,
                        a.B, a.L, a.A, ceil_div(a.Tmax, a.fine ? kScoreFineTokens : kScoreTileTokens), a.fine, a.normalize, a.mustd);
@@ -836,6 +854,8 @@ hipError_t launch_select(const SelectLaunch& a, hipStream_t s) {
   c.group_reduce = a.group_reduce;
   c.layer_reduce = a.layer_reduce;
   c.shared = a.shared;
+  c.pass_nan = a.pass_nan;
+  if (a.pass_nan && (a.G != 1 || a.shared)) return hipErrorInvalidValue;
   c.rows_per_seq = a.shared ? 1 : a.Hkv;
   const bool per_layer = a.layer_reduce < 0;
   // Reducing over the layers, a thread's time is its rounds of loads.  Where few workgroups share the chip
