@@ -716,6 +716,23 @@ def test_dense_compressor_leaves_other_calls_to_its_parts(tmp_path):
     assert torch.equal(odd, plain[..., :3]) and torch.equal(keep_odd, keep)
 
 
+def test_dense_compressor_refuses_a_position_that_is_no_32_bit_integer(tmp_path):
+    """The kernels take the position as a 32-bit integer; one beyond is an error, as in the general way, not cut off."""
+    h, t, d, budget = 2, 200, 64, 32
+    _write_stats(tmp_path / "s.pt", torch.ones(1, h, d // 2, 2), 2 * torch.ones(1, h, d // 2), torch.ones(d // 2), d)
+    comp = TriAttentionCompressor(TriAttentionConfig(
+        device=torch.device(DEV), stats_path=tmp_path / "s.pt", kv_budget=budget, divide_length=16, window_size=4,
+        protect_prefill=False, compute_dtype=torch.float32))
+    keys = torch.randn(1, h, t, d, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).to(DEV)
+    for position in (2**31 - 1, 2**31):
+        comp.state.absolute_position, comp.state.current_cache_len = position, t
+        if position < 2**31:
+            assert comp.compress(keys, keys)[2].shape == (1, h, budget)
+        else:
+            with pytest.raises((RuntimeError, OverflowError)):
+                comp.compress(keys, keys)
+
+
 def test_scheduler_and_worker_bookkeeping_around_the_hook_over_a_decode_loop(tmp_path):
     """A stand-in engine (block pool, per-group block manager, worker block table) drives the hook
     through ``engine_glue`` for 80 decode steps of two requests: the scheduler's and the worker's

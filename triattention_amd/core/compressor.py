@@ -196,7 +196,7 @@ class TriAttentionCompressor:
         f = d // 2
         if tuple(stats[0].shape) != (h, f, 2) or tuple(stats[1].shape) != (h, f) or tuple(stats[2].shape) != (h, f):
             return None
-        if self.omega.numel() != f or self.offsets.numel() > 32:
+        if self.omega.numel() != f or self.offsets.numel() > 32 or not -2**31 <= self.state.get_round_start() < 2**31:
             return None
         return tuple(x.to(device=keys.device, dtype=torch.float32).contiguous()
                      for x in (*stats, self.omega, self.offsets))
