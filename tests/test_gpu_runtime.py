@@ -340,6 +340,41 @@ def test_layer_local_modes_in_one_call_equal_the_layer_by_layer_path(tmp_path, m
     assert moved == ["r0", "r1"] * 3            # only the one-by-one runner took the layer-by-layer path
 
 
+@pytest.mark.parametrize("requests,layers", [(3, 1), (2, 1), (1, 1)])
+def test_layer_local_scratch_is_bounded_in_requests_too(tmp_path, monkeypatch, requests, layers):
+    """A scheduler step whose one layer of all requests exceeds the limit goes in groups of requests: no workspace
+    is larger than that of the group that fits (and one layer of one request is the least), caches, results and block
+    lists are those of a step without a limit."""
+    from helpers import build_inputs
+    from triattention_amd import ops, synth
+    from triattention_amd.runtime import selector as selector_mod
+    w = synth.Workload(name="t", num_layers=3, num_q_heads=8, num_kv_heads=2, head_dim=128, seq_lens=(700, 515, 300, 640, 128),
+                       budget=96, block_size=16, window_size=12, rope_theta=1e6, index=35)
+    inp = build_inputs(w)
+    kw = dict(pruning_mode="per_layer_per_head")
+    got = []
+    sizes = []
+    real = ops.Workspace.__init__
+    monkeypatch.setattr(ops.Workspace, "__init__", lambda self, *a: (real(self, *a), sizes.append(self.bytes))[0])
+    for limit in (1 << 40, requests * layers * 4 * (700 * (8 + 2) + 8 * 3 * 64)):
+        print(f"bounded layer-local scratch {limit}", flush=True)
+        monkeypatch.setattr(selector_mod, "LAYER_RUN_MAX_SCRATCH_BYTES", limit)
+        sizes.clear()
+        runner, reqs, caches, sched, signals = _fake_runner(w, inp, tmp_path, **kw)
+        out = RunnerHookCompressionExecutor(runner).execute_batch(signals, sched)
+        torch.cuda.synchronize()
+        got.append((out, [reqs[r].block_ids for r in out], [c.view(torch.int16).clone() for c in caches]))
+        largest = max(sizes)
+    kv = ops.PagedKV.from_kv_caches([c.to(DEV) for c in inp["caches"][:layers]])
+    batch = ops.StepBatch(DEV, [700] * requests, round_start=700, budgets=96, block_tables=[[0] * 44] * requests)
+    sc = ops.ScoreConfig(torch.zeros(layers, 8, 3, 64, device=DEV), inp["omega"].to(DEV), inp["offsets"].to(DEV))
+    bound = ops.Workspace(kv, batch, sc).bytes
+    assert largest <= bound
+    assert got[0][:2] == got[1][:2] and all(r.applied for r in got[0][0].values())
+    for a, b in zip(got[0][2], got[1][2]):
+        assert torch.equal(a, b)
+
+
 def test_batch_hook_on_the_resident_kernel(tmp_path, monkeypatch):
     """Sixteen requests of 3072 tokens fill the chip: the batch hook runs the resident kernel;
     result equal to the library calls on the same batch, and, when the resident launch is made to

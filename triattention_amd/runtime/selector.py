@@ -90,7 +90,8 @@ GRAPH_MAX_TOTAL_BYTES = 256 << 20
 GRAPH_MAX_SEEN = 64
 GRAPH_COUNTS = {"captured": 0, "replayed": 0}     # process-wide, for tests and diagnostics
 # The layer-local modes score all layers of a group in one launch sequence as long as its scratch (raw
-# scores of every layer) stays below this many bytes; longer requests go in runs of layers that do.
+# scores of every layer and request) stays below this many bytes; more of it goes in runs of layers and, where one
+# layer of all requests is too much, in groups of requests (one layer of one request is the least).
 LAYER_RUN_MAX_SCRATCH_BYTES = 256 << 20
 
 
@@ -379,23 +380,32 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
             return _compress_in_turn(layer_kv, block_size, requests, allow_resident)
 
     def _compress_in_turn(layer_kv: list, block_size: int, requests: list, allow_resident: bool) -> list:
-        if layer_local and len(layer_kv) > 1:
-            run = _layers_per_run(layer_kv, requests)
-            if run < len(layer_kv):
-                parts = []
-                for i in range(0, len(layer_kv), run):
-                    part = _compress_layers(layer_kv[i:i + run], block_size, requests, False)
-                    parts.append([r["indices"].clone() for r in part])        # (the next run writes the same buffer)
-                return [dict(r, indices=torch.cat(rows)) for r, rows in zip(part, zip(*parts))]
+        if layer_local:
+            at_once, run = _scratch_split(layer_kv, requests)
+            if at_once < len(requests) or run < len(layer_kv):
+                runs = [layer_kv[i:i + run] for i in range(0, len(layer_kv), run)]
+                kv = _paged_kv([c for _, c in layer_kv])
+                for part in runs:            # (a layer without statistics fails before the first one is compacted)
+                    _stats().folded(tuple(int(li) for li, _ in part), _head_layout(kv.num_kv_heads)[0], kv.device)
+                out = []
+                for first in range(0, len(requests), at_once):
+                    some, rows = requests[first:first + at_once], []
+                    for part in runs:
+                        kept = _compress_layers(part, block_size, some, False)
+                        rows.append([r["indices"].clone() for r in kept])     # (the next run writes the same buffer)
+                    out += [dict(r, indices=torch.cat(per_run)) for r, per_run in zip(kept, zip(*rows))]
+                return out
         return _compress_layers(layer_kv, block_size, requests, allow_resident)
 
-    def _layers_per_run(layer_kv: list, requests: list) -> int:
+    def _scratch_split(layer_kv: list, requests: list) -> tuple:
+        """(requests, layers) of one launch sequence whose scratch stays below LAYER_RUN_MAX_SCRATCH_BYTES,
+        at least one of each: the raw scores, the selection scores and the folded coefficients."""
         kv = _paged_kv([c for _, c in layer_kv])
         score_heads, _ = _head_layout(kv.num_kv_heads)
         longest = max(int(r["total_tokens"]) for r in requests)
-        # raw scores, selection scores and the folded coefficients of one layer
-        per_layer = 4 * len(requests) * (longest * (score_heads + kv.num_kv_heads) + score_heads * 3 * kv.head_dim // 2)
-        return max(1, min(len(layer_kv), LAYER_RUN_MAX_SCRATCH_BYTES // per_layer))
+        one = 4 * (longest * (score_heads + kv.num_kv_heads) + score_heads * 3 * kv.head_dim // 2)
+        at_once = max(1, min(len(requests), LAYER_RUN_MAX_SCRATCH_BYTES // one))
+        return at_once, max(1, min(len(layer_kv), LAYER_RUN_MAX_SCRATCH_BYTES // (one * at_once)))
 
     def _small_step(kv: Any, layers: int, score_heads: int, tokens: int) -> bool:
         # One request whose keys the score-then-select kernels read in quarter tiles (fewer than 256 workgroups
