@@ -586,6 +586,25 @@ def test_batch_hook_groups_requests_and_falls_back(monkeypatch):
     assert set(res) == {"a", "b"} and all(r.applied for r in res.values())
 
 
+@pytest.mark.parametrize("layer_local,label", [(False, "global_per_head"), (True, "layer_local")])
+def test_batched_failure_names_the_mode_that_failed(monkeypatch, layer_local, label):
+    def compress_batch(**kw):
+        raise ValueError("forced")
+
+    select_group = lambda **kw: None
+    select_group._supports_paged_group, select_group._compress_batch, select_group._layer_local = True, compress_batch, layer_local
+    select_layer = lambda **kw: None
+    select_layer._supports_paged = True
+    monkeypatch.setattr(hook_mod, "_build_triattention_selector",
+                        lambda config, base_runner=None: (select_layer, select_group, "enabled"))
+    runner, _ = _fake_runner()
+    install_runner_compression_hook(runner, TriAttentionRuntimeConfig(
+        kv_budget=8, divide_length=2, window_size=2, sparse_stats_path=GOLDEN / "qwen3_8b_stats_slice.pt"))
+    sched = types.SimpleNamespace(num_scheduled_tokens={"r": 1})
+    with pytest.raises(RuntimeError, match=f":batch:gid=0:{label}:ValueError"):
+        runner.triattention_apply_compression(req_id="r", signal=_signal(), scheduler_output=sched)
+
+
 def test_verify_rope_alignment():
     a = rope.default_inv_freq(128, 1e6)
     rope.verify_rope_alignment(a, types.SimpleNamespace(inv_freq=a.clone()))

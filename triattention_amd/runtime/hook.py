@@ -597,7 +597,8 @@ def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeCo
                     selected = compress_batch(layer_kv=group_tensors[gid], block_size=batch[0].block_size,
                                               requests=requests, allow_resident=False)
             except Exception as exc:
-                raise RuntimeError(f"{MARK}:batch:gid={gid}:global_per_head:{type(exc).__name__}") from exc
+                what = "layer_local" if layer_local else "global_per_head"
+                raise RuntimeError(f"{MARK}:batch:gid={gid}:{what}:{type(exc).__name__}") from exc
             for (r, ids, total), res in zip(members, selected):
                 semantic = res.get("semantic")
                 label = f"{res['mode']}:{semantic}" if semantic else res["mode"]
