@@ -259,6 +259,12 @@ typedef struct tri_plan_info {
 int tri_describe_plan(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
                       const tri_select_params* sel, int32_t assume_resident_workgroups, tri_plan_info* out);
 
+/* Tokens a workgroup of the score-then-select kernels takes in one call that scores and selects: 512, or 128
+ * (quarter tiles, the same bits) for a launch that would leave most CUs idle; 0 for invalid arguments.
+ * Host-only.  No counterpart in the reference. */
+int32_t tri_score_tile_tokens(const tri_kv_layout* kv, int32_t num_seqs, int32_t max_seq_len, int32_t num_score_heads,
+                              int32_t aggregation);
+
 /* Top-k of arbitrary fp32 rows (core/compressor.py:388-409): keep[r][0..k_r) =
  * ascending indices of the k_r largest of scores[r][0..len_r). */
 int tri_topk_rows(const float* scores, int64_t row_pitch, int32_t num_rows, const int32_t* row_lens,

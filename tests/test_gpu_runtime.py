@@ -441,6 +441,37 @@ def test_hook_call_for_one_small_request_takes_the_kernels_that_do_not_wait(tmp_
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("tile,kernel,requests,waits", [(None, "auto", 1, False), (512, "auto", 1, True), (None, "mfma", 1, True),
+                                                        (None, "auto", 2, True)],
+                         ids=["small", "whole_tiles", "kernel_by_name", "two_requests"])
+def test_hook_waits_for_the_status_word_only_where_it_takes_a_resident_kernel(tmp_path, monkeypatch, tile, kernel, requests, waits):
+    """The rule for one small request: the library's quarter tiles (where its answer is whole tiles, the resident
+    kernel), no kernel asked for by name, one request.  Eager, captured and replayed calls alike."""
+    from helpers import build_inputs
+    from triattention_amd import ops, synth
+    if kernel != "auto":
+        tune(resident_kernel=kernel)
+    w = synth.Workload(name="t", num_layers=3, num_q_heads=32, num_kv_heads=8, head_dim=128, seq_lens=(1185,) * requests,
+                       budget=256, block_size=16, window_size=12, rope_theta=1e6, index=39)
+    inp = build_inputs(w)
+    paths, reads, asked = [], [], []
+    select_path, status, tokens = ops.select_path, ops.Workspace.status, ops.score_tile_tokens
+    monkeypatch.setattr(ops, "select_path", lambda *a: paths.append(select_path(*a)) or paths[-1])
+    monkeypatch.setattr(ops.Workspace, "status", lambda self: reads.append(status(self)) or reads[-1])
+    monkeypatch.setattr(ops, "score_tile_tokens", lambda *a: asked.append(a[1:]) or (tokens(*a) if tile is None else tile))
+    runner, reqs, caches, sched, signals = _fake_runner(w, inp, tmp_path, fail_on_effective_len_regression=False)
+    for turn in range(3):
+        for b, rid in enumerate(reqs):
+            reqs[rid].num_computed_tokens = 1185
+            reqs[rid].block_ids = ([int(x) for x in inp["tables"][b]],)
+        out = RunnerHookCompressionExecutor(runner).execute_batch(signals, sched)
+        torch.cuda.synchronize()
+        assert all(r.applied for r in out.values())
+    assert set(paths) == {"resident_mfma" if waits else "two_pass"}
+    assert reads == ([0] * 3 if waits else [])
+    assert asked == ([(1, 1185, 32, "mean")] * 3 if requests == 1 and kernel == "auto" else [])
+
+
 @pytest.mark.parametrize("kw", [dict(), dict(pruning_mode="per_layer_per_head")], ids=["small_step", "layer_local"])
 @pytest.mark.parametrize("replay", [False, True], ids=["eager", "replay"])
 @pytest.mark.parametrize("threads", [False, True, "external"], ids=["one_thread", "two_threads", "external_streams"])

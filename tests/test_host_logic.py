@@ -879,3 +879,28 @@ def test_planner_cuts_the_benchmarked_shapes_as_documented():
     assert path == 2 and groups == 1 and launches * 64 >= 16 * tiles
     import ctypes as C
     assert _lib.load().tri_describe_plan(None, None, None, None, 0, None) == _lib.TRI_ERR_INVALID_ARGUMENT
+
+
+def test_quarter_tiles_are_for_launches_that_leave_most_of_the_chip_idle():
+    """``tri_score_tile_tokens`` on both sides of its rule: fewer than 256 workgroups of 512 tokens, head dimension
+    128 or 256, KV heads that fill a wave of the scorer, mean aggregation."""
+    import ctypes as C
+    lib = _lib.load()
+
+    def tile(layers, q, kv, d, tokens, seqs=1, aggregation=_lib.REDUCE_MEAN, dtype=0):
+        layout = _lib.KvLayout(num_layers=layers, num_kv_heads=kv, head_dim=d, block_size=16, kv_dtype=dtype, rope_style=0,
+                               stride_block=16 * kv * d, stride_token=kv * d, stride_head=d, k_layers=4096,
+                               v_layers=4096, k_scale_layers=4096, v_scale_layers=4096)
+        return lib.tri_score_tile_tokens(C.byref(layout), seqs, tokens, q, aggregation)
+
+    assert tile(36, 32, 8, 128, 3584) == 128 and tile(36, 32, 8, 128, 3585) == 512       # 252 | 288 workgroups
+    assert tile(3, 32, 8, 128, 85 * 512) == 128 and tile(3, 32, 8, 128, 85 * 512 + 1) == 512
+    assert tile(1, 32, 8, 128, 255 * 512) == 128 and tile(1, 32, 8, 128, 255 * 512 + 1) == 512
+    assert tile(16, 64, 8, 128, 7 * 512) == 128 and tile(16, 64, 8, 128, 7 * 512 + 1) == 512   # two passes of query heads
+    assert tile(18, 32, 8, 256, 7 * 512) == 128 and tile(18, 32, 8, 256, 7 * 512 + 1) == 512   # two waves of KV heads
+    assert tile(36, 32, 8, 128, 2176, seqs=2) == 512 and tile(3, 32, 8, 128, 2176, seqs=16) == 128
+    assert tile(3, 20, 5, 128, 2176) == 128 and tile(3, 16, 4, 128, 2176) == 512         # five of eight heads | padded to four
+    assert tile(3, 32, 8, 64, 2176) == 512 and tile(3, 32, 8, 128, 2176, aggregation=_lib.REDUCE_MAX) == 512
+    assert tile(3, 32, 8, 128, 2176, dtype=2) == 128
+    assert tile(3, 64, 8, 128, 29) == 512 and tile(3, 64, 8, 128, 30) == 128             # room for the sums
+    assert tile(3, 31, 8, 128, 2176) == 0 and tile(3, 32, 8, 100, 2176) == 0 and tile(3, 32, 8, 128, 0) == 0

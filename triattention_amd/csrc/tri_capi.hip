@@ -270,6 +270,15 @@ bool takes_resident(const tri::Workspace& w, const tri_kv_layout* kv, const tri_
   return w.fused.eligible && layer_reduce_of(kv, sel) >= 0 && !sel->shared && !sel->group_first && !sel->no_resident;
 }
 
+// Quarter tiles of the two-pass scorer.  Their sums take more room than the workspace plans; they go where the
+// selection scores are written later (the statistics are finished by then).
+bool takes_quarter_tiles(const tri_kv_layout* kv, int B, int Tmax, int A, int aggregation) {
+  const int64_t sums = (int64_t)B * kv->num_layers * A * tri::ceil_div(Tmax, tri::kScoreFineTokens) * 4 * 4;
+  const int64_t room = tri::align_up((int64_t)B * kv->num_layers * kv->num_kv_heads * Tmax * 4, 256);   // Workspace::fin
+  return sums <= room && tri::score_takes_fine(B, kv->num_layers, kv->num_kv_heads, kv->head_dim, A / kv->num_kv_heads,
+                                               Tmax, aggregation);
+}
+
 // Selection straight from the paged keys: the resident kernel when the shape has one,
 // else score into the workspace and select from there.
 int do_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
@@ -280,13 +289,7 @@ int do_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_s
     float* raw = at<float>(ws, w.raw);
     const int64_t A = sp->num_score_heads;
     const int64_t rs_layer = (int64_t)batch->max_seq_len * A;
-    // Sums per quarter tile take more room than the workspace plans; they go where the selection scores
-    // are written later (the statistics are finished by then).
-    const int64_t sums = (int64_t)batch->num_seqs * kv->num_layers * A *
-                         tri::ceil_div(batch->max_seq_len, tri::kScoreFineTokens) * 4 * 4;
-    const int fine = sums <= w.xchg - w.fin &&
-                     tri::score_takes_fine(batch->num_seqs, kv->num_layers, kv->num_kv_heads, kv->head_dim,
-                                           (int)A / kv->num_kv_heads, batch->max_seq_len, sp->aggregation);
+    const int fine = takes_quarter_tiles(kv, batch->num_seqs, batch->max_seq_len, (int)A, sp->aggregation);
     float* partial = at<float>(ws, fine ? w.fin : w.partial);
     // The status word belongs to the resident kernel; on this path it just reads "fine".
     const int rc = do_score(kv, batch, sp, raw, rs_layer, A, 1, ws, w, s, fine, partial, at<uint32_t>(ws, w.status));
@@ -568,6 +571,15 @@ int tri_describe_plan(const tri_kv_layout* kv, const tri_batch* batch, const tri
   if (batch->num_seqs <= f.seqs_per_launch) out->launches = 1;
   else out->launches = f.launches;      // > 0: the planner replayed the packing of the host's lengths
   return TRI_OK;
+}
+
+int32_t tri_score_tile_tokens(const tri_kv_layout* kv, int32_t num_seqs, int32_t max_seq_len, int32_t num_score_heads,
+                              int32_t aggregation) {
+  if (check_layout(kv, false) || num_seqs <= 0 || max_seq_len <= 0 || num_score_heads <= 0 ||
+      num_score_heads % kv->num_kv_heads)
+    return 0;
+  return takes_quarter_tiles(kv, num_seqs, max_seq_len, num_score_heads, aggregation) ? tri::kScoreFineTokens
+                                                                                      : tri::kScoreTileTokens;
 }
 
 int tri_topk_rows(const float* scores, int64_t row_pitch, int32_t num_rows, const int32_t* row_lens,

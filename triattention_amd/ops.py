@@ -497,6 +497,13 @@ def select_path(kv: PagedKV, batch: StepBatch, sc: ScoreConfig, sel: SelectConfi
     return {2: "resident_mfma", 1: "resident_valu"}.get(rc, "two_pass")
 
 
+def score_tile_tokens(kv: PagedKV, num_seqs: int, max_seq_len: int, num_score_heads: int, aggregation: str = "mean") -> int:
+    """Tokens a workgroup of the score-then-select kernels takes for a call of this size: 512, or 128 where
+    whole tiles would leave most of the chip idle (``tri_score_tile_tokens``)."""
+    return int(_lib.load().tri_score_tile_tokens(C.byref(kv.struct), num_seqs, max_seq_len, num_score_heads,
+                                                 REDUCE_MAX if aggregation == "max" else REDUCE_MEAN))
+
+
 def describe_plan(kv: PagedKV, batch: StepBatch, sc: ScoreConfig, sel: SelectConfig,
                   assume_resident_workgroups: int = 0) -> dict:
     """How select_paged / compress_step would cut these arguments into workgroups (``tri_describe_plan``):

@@ -407,20 +407,18 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
         at_once = max(1, min(len(requests), LAYER_RUN_MAX_SCRATCH_BYTES // one))
         return at_once, max(1, min(len(layer_kv), LAYER_RUN_MAX_SCRATCH_BYTES // (one * at_once)))
 
-    def _small_step(kv: Any, layers: int, score_heads: int, tokens: int) -> bool:
-        # One request whose keys the score-then-select kernels read in quarter tiles (fewer than 256 workgroups
-        # of 512 tokens, head dimension 128 or 256, KV heads that fill a wave).  Their GPU time equals the
-        # resident kernel's there and they cannot fail, so the call does not end in a wait for the status
-        # word: 36 layers x 2176 tokens 266 -> 184 us a call among others, 270 -> 238 with a synchronisation
-        # after each.  (Sixteen such requests gain nothing where each call is waited for, 2786 against
-        # 2796 us, and keep the resident kernel.)  A resident kernel asked for by name is taken.
-        if _lib.get_tuning(_lib.TUNE_RESIDENT_KERNEL) != 0:
+    def _small_step(kv: ops.PagedKV, score_heads: int, tokens: int) -> bool:
+        # One request of two-byte keys that the score-then-select kernels read in quarter tiles.  They take longer on
+        # the GPU than the resident kernel (36 layers x 2176 tokens 65 against 56 us, 3 x 40000 190 / 161, 64 / 8 heads 16 x
+        # 2176 65 / 44) but can not fail, so the call does not end in a wait for the status word, which costs more, with
+        # calls queued behind each other (with a synchronisation after each): 36 x 2176 204 against 278 us
+        # (264 / 285), 3 x 40000 487 / 511 (508 / 515), 16 x 2176 of 64 / 8 heads 125 / 194 (186 / 194), 18 x 2176 of head
+        # dimension 256 217 / 290 (273 / 297).  Least at the far end of the rule: one layer x 120000 tokens 732 / 909
+        # (921 / 912).  Sixteen requests of 2176 tokens, beyond it, gain nothing where each call is waited for, 2786
+        # against 2796 us.  A resident kernel asked for by name is taken.
+        if _lib.get_tuning(_lib.TUNE_RESIDENT_KERNEL) != 0 or kv.dtype not in (torch.bfloat16, torch.float16):
             return False
-        wave_heads = 1024 // kv.head_dim                  # KV heads a wave of the scorer reads at once
-        if kv.head_dim < 128 or kv.dtype not in (torch.bfloat16, torch.float16) or 2 * kv.num_kv_heads <= wave_heads:
-            return False
-        heads = -(-kv.num_kv_heads // wave_heads) * -(-(score_heads // kv.num_kv_heads) // 4)
-        return heads * layers * -(-tokens // 512) < 256
+        return ops.score_tile_tokens(kv, 1, tokens, score_heads, config.sparse_score_aggregation) < 512
 
     def _compress_layers(layer_kv: list, block_size: int, requests: list, allow_resident: bool) -> list:
         agg = os.environ.get("TRIATTN_RUNTIME_DEBUG_GROUP_PERHEAD_AGG_MODE", "mean").strip().lower()
@@ -449,7 +447,7 @@ def build_triattention_selector(config: TriAttentionRuntimeConfig, base_runner: 
         guards = [int(r["prefill_len"]) if r["protect_prefill"] and int(r["prefill_len"]) > 0 else 0 for r in requests]
         rounds = [int(r["round_start"]) for r in requests]
         tables = [[int(x) for x in r["block_ids"]] for r in requests]
-        if not turn.capturing and len(requests) == 1 and _small_step(kv, len(layer_ids), score_heads, totals[0]):
+        if not turn.capturing and len(requests) == 1 and _small_step(kv, score_heads, totals[0]):
             allow_resident = False
         use_resident = bool(allow_resident) and holder.get("resident_ok", True)
         rows_per_request = (len(layer_ids) if layer_local else 1) * (1 if shared else kv.num_kv_heads)
