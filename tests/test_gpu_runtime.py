@@ -419,10 +419,12 @@ def test_batch_hook_on_the_resident_kernel(tmp_path, monkeypatch):
 
 @pytest.mark.parametrize("tokens,kv_heads,two_pass", [(1185, 8, True), (3072, 6, True), (3072, 2, False)])
 def test_hook_call_for_one_small_request_takes_the_kernels_that_do_not_wait(tmp_path, monkeypatch, tokens, kv_heads, two_pass):
-    """A single request below the selector's limit gives, through the hook, the bits of the score-then-select
-    kernels; a shape without quarter tiles keeps the library's own choice."""
+    """A single request below the selector's limit takes the score-then-select kernels (and gives their bits); a
+    shape without quarter tiles keeps the library's own choice, the resident kernel."""
     from helpers import build_inputs
     from triattention_amd import ops, synth
+    paths, select_path = [], ops.select_path
+    monkeypatch.setattr(ops, "select_path", lambda *a: paths.append(select_path(*a)) or paths[-1])
     w = synth.Workload(name="t", num_layers=3, num_q_heads=4 * kv_heads, num_kv_heads=kv_heads, head_dim=128,
                        seq_lens=(tokens,), budget=256, block_size=16, window_size=12, rope_theta=1e6, index=33)
     inp = build_inputs(w)
@@ -430,6 +432,7 @@ def test_hook_call_for_one_small_request_takes_the_kernels_that_do_not_wait(tmp_
     got = RunnerHookCompressionExecutor(runner).execute("r0", signals["r0"], sched)
     torch.cuda.synchronize()
     assert got.applied and got.cache_len_after == 256
+    assert paths == ["two_pass" if two_pass else "resident_mfma"]
     ref = [c.to(DEV) for c in inp["caches"]]
     batch = ops.StepBatch(DEV, w.seq_lens, round_start=w.seq_lens, budgets=w.budget, block_tables=inp["tables"],
                           prefill_lens=[0])

@@ -54,7 +54,7 @@ FusedPlan plan_fused_mfma(int B, int Hkv, int D, int G, int block_size, bool pag
 // Scratch carved out of the caller's workspace.  All offsets in bytes, 256-aligned.
 struct Workspace {
   int64_t coef;      // [B][L][A][3][F] fp32: P, R, E for mean aggregation; A1, A2, E for max
-  int64_t trig;      // [B][2][F] offset means of cos / sin, then [B][NO][2][F] tables (max aggregation)
+  int64_t trig;      // max aggregation: [B][NO][2][F] tables of cos / sin, behind B*2*F floats that nothing uses
   int64_t partial;   // [B][L][NT][A][2] fp32 per-tile sum / sum of squares
   int64_t mustd;     // [B][L][A][2] fp32 mean / safe std
   int64_t raw;       // [B][L][Tmax][A] fp32 raw scores (tri_compress_step)

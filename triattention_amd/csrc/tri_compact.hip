@@ -574,10 +574,16 @@ hipError_t launch_compact(const CompactLaunch& a, hipStream_t s) {
   //    pass writes whole token rows for all heads together, which pays where most sources lie
   //    beyond the budget: 36 layers x 16384 tokens 133 against 142 us in one launch, 16 such
   //    requests 1953 against 1969, with 128-byte rows (8 x 8192 -> 1024) 262 against 275; at a quarter
-  //    of the context the two are level (989 / 991).
+  //    of the context the two are level (989 / 991).  Up to 512 chains one launch is the faster one for these
+  //    too (budget 2048; against two passes with a chain per head): 1 layer x 32768 tokens 10.2 / 15.4, 16 x 16384
+  //    48.0 / 62.1, 28 x 32768 103.3 / 103.9.
+  //    Shared lists go head by head like the others (against one workgroup that moved whole token rows): one
+  //    layer x 4096 tokens 9.8 / 136, 36 layers x 2176 112.6 / 372, x 8192 139 / 193, x 16384 133 / 167, eight requests x
+  //    2176 1008 / 1182, x 8192 996 / 1030, four x 16384 502 / 508.
   //  - otherwise one launch of the ordered pass over the whole list.  Its time is the chain of
   //    tiles of one workgroup until the memory system is full, so the fewer chains there are the
-  //    longer the tile: up to 256 chains a tile of 128 KB (one layer x 4096 tokens 9.9 / 19.1 us, 16
+  //    longer the tile: up to 256 chains a tile of 128 KB (one layer x 4096 tokens 9.9 / 19.1 us, called over
+  //    and over on one cache; 14.6 behind the scorer of a step, the rows not in L2; 16
   //    layers 43.1 / 54.1; up to 128 chains two workgroups take half of every row each, 8 layers
   //    24.3 / 37.1), up to 1024 chains 32 KB (36 layers x 2176 tokens 120.6 / 135.8; 36 layers x 1000 ->
   //    600 31.2 / 38.0, where 128 KB overshoot the list: 37.5), beyond that 32 KB in workgroups of 512

@@ -1192,7 +1192,7 @@ hipError_t launch_fused_mfma(const FusedLaunch& a, hipStream_t s) {
   // A workgroup takes all KV heads of a layer and request, which evaluates the phases least often, unless that
   // leaves CUs without one: then the heads are halved until there are 256 workgroups.  The launch is a chain of
   // latencies (statistics, phases, slabs), not bytes: the whole step of one layer x 4096 tokens 56.6 -> 53.0 us with eight
-  // workgroups in place of one and the statistics requested first; 36 layers x 2176 tokens 267 -> 265 (a hook call).
+  // workgroups in place of one and the statistics requested first; a call on 36 layers x 2176 tokens 267 -> 265.
   int heads_per_wg = a.Hkv;
   while (heads_per_wg > 1 && (int64_t)a.L * a.B * ceil_div(a.Hkv, heads_per_wg) < 256) heads_per_wg = ceil_div(heads_per_wg, 2);
   auto prep_launch = [&](auto kernel) {

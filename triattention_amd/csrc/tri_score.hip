@@ -404,7 +404,6 @@ __global__ __launch_bounds__(kScoreThreads) void score_mean_kernel(ScoreArgs a) 
 template <int LPH, int DT, bool IL>
 __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
   constexpr int F = LPH * kPairsPerLane;
-  constexpr int kTile = kScoreTileTokens;
   __shared__ int lds_blk[kScoreTileTokens + 2];
   __shared__ float lds_s1[kScoreThreads];
   __shared__ float lds_s2[kScoreThreads];
@@ -415,9 +414,9 @@ __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
   const int tile = blockIdx.x, sib = blockIdx.y;
   const int b = blockIdx.z / a.L, l = blockIdx.z % a.L;
   const int seq_len = a.seq_lens[b];
-  const int n0 = tile * kTile;
+  const int n0 = tile * kScoreTileTokens;
   if (n0 >= seq_len) return;
-  const int n1 = min(n0 + kTile, seq_len);
+  const int n1 = min(n0 + kScoreTileTokens, seq_len);
 
   int lb0 = 0;
   if (a.block_table_pitch >= 0) {
@@ -455,7 +454,7 @@ __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
   const char* kbase = reinterpret_cast<const char*>(a.k_layers[l]);
   const float* kscale = FP8 ? a.k_scale_layers[l] : nullptr;
   const int64_t lane_off = (int64_t)head_c * a.stride_head + (IL ? lm.m * 16 : lm.m * 8);
-  constexpr int TW = kTile / 4;
+  constexpr int TW = kScoreTileTokens / 4;
   const int wstart = n0 + wave * TW;
   const int wend = min(wstart + TW, n1);
   const int a_out = head_c * a.G + lm.q0 + lm.qsel;
@@ -1105,7 +1104,7 @@ hipError_t launch_fold_stats(const float* qr, const float* qi, const float* qabs
 hipError_t launch_prepare(const float* folded, const float* omega, const float* offsets, int NO,
                           const int32_t* round_start, int B, int L, int A, int F, int aggregation,
                           float* coef, float* trig, uint32_t* status, hipStream_t s) {
-  // The per-offset tables (max aggregation) follow 2*F floats per sequence in the trig area.
+  // The per-offset tables (max aggregation) follow 2*F floats per sequence in the trig area that nothing uses.
   float* tables = (aggregation == TRI_REDUCE_MAX) ? trig + (int64_t)B * 2 * F : nullptr;
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(ceil_div(L * A, kPrepareRows), B), dim3(kPrepareThreads), 0, s, folded, omega, offsets,

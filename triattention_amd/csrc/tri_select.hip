@@ -609,7 +609,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
   // A row without a finite score has lo_key > hi_key: everything else then falls into bin 0.
   const float lo = lo_key <= hi_key ? key_float(lo_key) : 0.f;
   const float width = lo_key <= hi_key ? __fsub_rn(key_float(hi_key), lo) : 0.f;
-  // (a width beyond the largest float is +inf and puts everything into bin 0 as well)
+  // (A width beyond the largest float is +inf and makes the scale 0: a score whose distance from lo is still a
+  // number falls into bin 0; the largest ones, whose distance is +inf too, give inf * 0 = NaN, which the fminf
+  // below drops for the last bin.  Two bins, in order.)
   const float scale = width > 0.f ? fminf(__fdiv_rn((float)kTopkBins, width), 3.0e38f) : 0.f;
   auto bin_of = [&](uint32_t kk) __attribute__((always_inline)) {
     const float t = __fmul_rn(__fsub_rn(key_float(kk), lo), scale);

@@ -408,9 +408,9 @@ def build_hook_runtime_context(*, base_runner: Any, config: TriAttentionRuntimeC
                               int(recent) if isinstance(recent, int) else None, bool(defer))
 
 
-# A single request in the default mode goes through the same one-call launch sequence as a batch
+# A single request goes through the same one-call launch sequence as a batch
 # of requests; False sends it through the reference-shaped pipeline (selector callable, then the
-# per-head compaction function), which gives the same result dictionaries and cache contents.
+# compaction function), which gives the same result dictionaries and cache contents.
 SINGLE_REQUEST_IN_ONE_CALL = True
 
 
@@ -530,9 +530,9 @@ def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeCo
         if isinstance(ready, dict):
             return ready
         if SINGLE_REQUEST_IN_ONE_CALL and _batchable(ready):
-            # Default mode, something to drop: score, select and compact in one library call with one
-            # host synchronisation at its end (the layer-by-layer pipeline below waits for the keep
-            # indices on the host before the compaction is launched).
+            # Something to drop: score, select and compact in one library call with at most one
+            # host synchronisation, at its end, where a resident kernel ran (the pipeline below
+            # launches selection and compaction apart, in the layer-local modes layer by layer).
             return _run_batch([ready])[req_id]
         return _run_single(ready)
 
@@ -635,8 +635,8 @@ def make_runner_compression_hook(base_runner: Any, config: TriAttentionRuntimeCo
 
     def _batch_hook(signals: dict, scheduler_output: Any) -> dict:
         """All triggered requests of a scheduler step at once: ``{req_id: result}`` with the
-        result dictionaries the one-by-one hook returns.  Requests that qualify (the default
-        per-head mode, something to drop) are scored, selected and compacted together, one
+        result dictionaries the one-by-one hook returns.  Requests that qualify (something to
+        drop, no debug switch) are scored, selected and compacted together, one
         launch sequence per KV-cache group; the others go through the one-by-one path."""
         results, together = {}, []
         for req_id, signal in signals.items():

@@ -1,7 +1,7 @@
 """Keep-set selection for the runtime hook: the callable pair the reference builds in
 ``build_triattention_selector`` (triattention/vllm/runtime/selector_hf.py:15-1083), same
 keyword signatures, result dictionaries and failure markers, executed by the HIP scorer,
-the combine kernel and the radix top-k.
+the combine kernel and the top-k.
 
 Nothing is chunked and K is neither gathered nor repeated per query head: the scorer
 reads the paged blocks of every layer once and, for shapes that have a resident kernel,
