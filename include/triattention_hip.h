@@ -274,7 +274,8 @@ int tri_topk_rows(const float* scores, int64_t row_pitch, int32_t num_rows, cons
 /* Compression of one layer of a dense cache into new tensors, everything the dense compressor
  * launches after its trigger (core/compressor.py:279-346): score every key [H][T][D] against one
  * score head per KV head, normalise over the tokens (mean and unbiased standard deviation, core/utils.py:466-480),
- * guard the last window_size tokens, keep the budget largest per head, gather.  Strides and row sizes
+ * guard the last window_size tokens, keep the budget largest per head (a NaN above +inf, or below -inf with
+ * its sign set), gather.  Strides and row sizes
  * of K and V in bytes, multiples of 16, bases 16-byte aligned; V rows may hold any type.  0 < budget <= T.
  * out_k [H][budget][D], out_v [H][budget][v row], out_keep [H][budget] ascending.  Scratch as
  * tri_dense_workspace_bytes says (0: not supported), 256-byte aligned.  Nothing waits; capturable. */
