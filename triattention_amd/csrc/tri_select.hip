@@ -88,10 +88,11 @@ __global__ void finalize_stats_kernel(const float* partial, const int32_t* seq_l
 // raw[n][h*G .. h*G+G), per (sequence, layer, KV head), with torch's definitions
 // (core/utils.py:476-479: mean, unbiased std, std < 1e-8 -> 1).  Sums in double; one
 // workgroup per (sequence, layer, KV head).  mustd[(b*L + l)*A*2 + h*2] = (mean, std).
+// kPass (SelectLaunch::pass_nan): the one score of a KV head as it is.
+template <bool kPass>
 __global__ __launch_bounds__(256) void group_stats_kernel(const float* raw, int64_t stride_layer, int64_t stride_token,
                                                           int64_t stride_head, const int32_t* seq_lens, int L, int Hkv,
-                                                          int A, int G, int group_reduce, int normalize, int pass_nan,
-                                                          float* mustd) {
+                                                          int A, int G, int group_reduce, int normalize, float* mustd) {
   __shared__ double red[256][2];
   const int h = blockIdx.x % Hkv;
   const int bl = blockIdx.x / Hkv, b = bl / L;
@@ -105,8 +106,10 @@ __global__ __launch_bounds__(256) void group_stats_kernel(const float* raw, int6
   double s = 0.0, q = 0.0;
   for (int n = threadIdx.x; n < T; n += 256) {
     const float* p = base + (int64_t)n * stride_token;
-    float m = p[0];
-    if (!pass_nan) {
+    float m;
+    if constexpr (kPass) {
+      m = p[0];
+    } else {
       m = (group_reduce == TRI_REDUCE_MAX) ? -INFINITY : 0.f;
       for (int g = 0; g < G; ++g) {
         const float x = p[(int64_t)g * stride_head];
@@ -831,11 +834,14 @@ hipError_t launch_select(const SelectLaunch& a, hipStream_t s) {
                        a.raw_stride_token, a.seq_lens, a.L, a.Hkv, chunk, chunks, a.group_reduce, part);
     hipLaunchKernelGGL(group_stats_finish_kernel, dim3(ceil_div(a.B * a.L * a.Hkv, 256)), dim3(256), 0, s, part,
                        a.seq_lens, a.B * a.L, a.L, a.Hkv, a.A, chunk, chunks, a.mustd);
-  } else if (a.group_first)
-    hipLaunchKernelGGL(group_stats_kernel, dim3(a.B * a.L * a.Hkv), dim3(256), 0, s, a.raw, a.raw_stride_layer,
-                       a.raw_stride_token, a.raw_stride_head, a.seq_lens, a.L, a.Hkv, a.A, a.G, a.group_reduce,
-                       a.normalize, a.pass_nan, a.mustd);
-  else
+  } else if (a.group_first) {
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(a.B * a.L * a.Hkv), dim3(256), 0, s, a.raw, a.raw_stride_layer, a.raw_stride_token,
+                         a.raw_stride_head, a.seq_lens, a.L, a.Hkv, a.A, a.G, a.group_reduce, a.normalize, a.mustd);
+    };
+    if (a.pass_nan) launch(group_stats_kernel<true>);
+    else launch(group_stats_kernel<false>);
+  } else
     hipLaunchKernelGGL(finalize_stats_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, a.partial, a.seq_lens,
                        a.B, a.L, a.A, ceil_div(a.Tmax, a.fine ? kScoreFineTokens : kScoreTileTokens), a.fine, a.normalize, a.mustd);
   hipError_t e = hipGetLastError();
