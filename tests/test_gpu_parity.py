@@ -677,6 +677,48 @@ def test_compaction_on_both_sides_of_every_launch_rule(layers, heads, dim, token
     assert torch.equal(cache, want)
 
 
+@pytest.mark.parametrize("dtype,scales,layers,heads,dim,tokens,budget", [
+    ("bf16", False, 136, 1, 128, 6200, 2048),    # 272 chains, a third of the context: one launch up to 2048 entries,
+    ("bf16", False, 136, 1, 128, 6200, 2049),    # ... two passes beyond
+    ("bf16", False, 129, 8, 64, 300, 100),       # 2064 chains of 128-byte rows: two passes,
+    ("bf16", False, 129, 8, 64, 300, 150),       # ... one launch from half of the context on
+    ("bf16", False, 17, 8, 256, 330, 110),       # 512-byte rows: two passes at a third of the context,
+    ("bf16", False, 17, 8, 256, 330, 111),       # ... one launch above
+    ("fp8", False, 17, 8, 64, 600, 120),         # 64-byte rows, 272 chains: two passes at a fifth,
+    ("fp8", False, 17, 8, 64, 600, 121),         # ... one launch above
+    ("fp8", False, 33, 8, 64, 300, 149),         # 528 chains: two passes below half
+    ("fp8", True, 12, 8, 128, 300, 100),         # 192 chains beside the scales: one launch,
+    ("fp8", True, 13, 8, 128, 300, 209),         # ... 208: two passes below 70 % of the context,
+    ("fp8", True, 13, 8, 128, 300, 210),         # ... one launch from there,
+    ("fp8", True, 26, 4, 128, 300, 149),         # ... with four heads from half of it
+    ("fp8", True, 26, 4, 128, 300, 150),
+])
+def test_compaction_on_both_sides_of_the_rule_for_one_launch(dtype, scales, layers, heads, dim, tokens, budget):
+    """One launch or two passes depends on the chains, the share and the number of rows that stay, the bytes of a row
+    and whether a cache's scales move beside them.  Rows and scales are copies: exact."""
+    print(f"one launch or two {dtype} scales={scales} {layers}x{heads}x{dim} {tokens}->{budget}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(7)
+    nb, size = (tokens + 15) // 16, 1 if dtype == "fp8" else 2
+    raw = torch.randint(0, 256, (layers, 2, nb, 16, heads, dim * size), dtype=torch.uint8, device=DEV, generator=g)
+    cache = raw.view(torch.float8_e4m3fn if dtype == "fp8" else torch.bfloat16)
+    sc = torch.rand(layers, 2, nb * 16, heads, device=DEV, generator=g)
+    sides = [[x[i] for x in sc] if scales else None for i in (0, 1)]
+    kv = ops.PagedKV([c[0] for c in cache], [c[1] for c in cache], "half", *sides)
+    table = torch.randperm(nb, generator=g, device=DEV)
+    batch = ops.StepBatch(DEV, [tokens], budgets=budget, block_tables=[table.tolist()])
+    keep = torch.rand(heads, tokens, generator=g, device=DEV).topk(budget, 1).indices.sort(1).values.int().contiguous()
+    slot = lambda t: (table[t // 16], t % 16)
+    head = torch.arange(heads, device=DEV).unsqueeze(1).expand(heads, budget)
+    (sb, so), (db, do) = slot(keep.long()), slot(torch.arange(budget, device=DEV).expand(heads, budget))
+    want, want_sc = raw.clone(), sc.clone()
+    want[:, :, db, do, head] = raw[:, :, sb, so, head]
+    if scales:
+        want_sc[:, :, db * 16 + do, head] = sc[:, :, sb * 16 + so, head]
+    ops.compact(kv, batch, keep)
+    torch.cuda.synchronize()
+    assert torch.equal(raw, want) and torch.equal(sc, want_sc)
+
+
 @pytest.mark.parametrize("axis", [0, 1])
 def test_compaction_matches_reference_golden(axis):
     """Full-permutation output written by the reference's compact_request_kv_in_place(_per_head)."""

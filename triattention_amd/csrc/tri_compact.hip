@@ -537,6 +537,35 @@ SideStream& side_stream() {
   return s;
 }
 
+// How the rows are moved: one launch of the ordered pass over the whole list, or the ordered pass over the sources
+// inside the kept prefix and the bulk pass over the rest.  One launch is bound by the chain of
+// tiles of a workgroup until the memory system is full; the bulk pass has no chains and writes whole token rows for all heads
+// together, which pays the more the more sources lie beyond the budget, the smaller a row and the longer the list.  Both
+// sides, one launch / two passes, in turn on one cache (compaction alone, lists spread over the context, 8 heads, us):
+//  - few chains: 8 requests x 8192 -> 2048 of one layer, 128 chains, 23 / 32, 256 chains 50 / 60, rows of 64 bytes 20 / 25;
+//  - half of the context or more stays: 36 layers x 2176 -> 2048, 128-byte rows, 46 / 53; 256-byte rows, 32 layers x
+//    20 x 4096 -> 2048 1938 / 2036;
+//  - a list of at most 2048 entries, from 5 k > T (with rows of 512 bytes 3 k > T: 18 layers x 8192 -> 2048 142 / 126), any
+//    k up to 512 chains: 32 layers x 4096 -> 1400 62 / 74, x 8192 -> 1300 60 / 68, 8 x 8192 -> 2048 879 / 878.
+//    Not rows of 64 bytes (36 layers x 8 x 8192 -> 2048 444 / 380; sparse, 512 chains, 46 / 40), nor of 128 bytes beyond
+//    2048 chains (36 layers x 8 x 4096 -> 1400 379 / 363);
+//  - longer lists: two passes (36 layers x 30000 -> 8000, 128-byte rows, 309 / 272; 256-byte rows level).
+// Beside the kernel that moves an fp8 cache's scales on the side stream two passes do better from 192 chains on (32 layers x
+// 8192 -> 2048 95 / 86, 30000 -> 8000 333 / 281; 144 chains of two heads 36 / 42) until most rows stay (1000 -> 700
+// 39 / 41; with fewer than eight heads half of them: 28 layers of four heads x 4 x 4096 -> 2048 101 / 128).
+// Shared lists go head by head like the others (against one workgroup that moved whole token rows): one
+// layer x 4096 tokens 9.8 / 136, 36 layers x 2176 112.6 / 372, x 8192 139 / 193, x 16384 133 / 167.
+bool takes_one_launch(const CompactLaunch& a, int chains, bool beside_scales) {
+  const int64_t k = a.max_budget, T = a.Tmax;
+  if (beside_scales) return chains <= 192 || 10 * k >= 7 * T || (a.Hkv < 8 && 2 * k >= T);
+  if (chains <= 256 || 2 * k >= T) return true;
+  const int row = a.D * a.elem_bytes;
+  if (k > 2048) return false;
+  if (row >= 512) return 3 * k > T;
+  if (chains <= 512) return row >= 128 || 5 * k > T;
+  return 5 * k > T && (row >= 256 || (row >= 128 && chains <= 2048));
+}
+
 }  // namespace
 
 hipError_t launch_compact(const CompactLaunch& a, hipStream_t s) {
@@ -567,29 +596,14 @@ hipError_t launch_compact(const CompactLaunch& a, hipStream_t s) {
       forked = true;
     }
   }
-  // How the rows are moved (compaction alone, keep lists spread over the context, budget 2048 and 8 heads
-  // of 256-byte rows unless noted; us by the rule below / by the ordered pass of 256 threads plus the
-  // bulk pass, which served every shape before):
-  //  - sparse lists (a fifth of the context or less) of more than a few heads: two passes.  The bulk
-  //    pass writes whole token rows for all heads together, which pays where most sources lie
-  //    beyond the budget: 36 layers x 16384 tokens 133 against 142 us in one launch, 16 such
-  //    requests 1953 against 1969, with 128-byte rows (8 x 8192 -> 1024) 262 against 275; at a quarter
-  //    of the context the two are level (989 / 991).  Up to 512 chains one launch is the faster one for these
-  //    too (budget 2048; against two passes with a chain per head): 1 layer x 32768 tokens 10.2 / 15.4, 16 x 16384
-  //    48.0 / 62.1, 28 x 32768 103.3 / 103.9.
-  //    Shared lists go head by head like the others (against one workgroup that moved whole token rows): one
-  //    layer x 4096 tokens 9.8 / 136, 36 layers x 2176 112.6 / 372, x 8192 139 / 193, x 16384 133 / 167, eight requests x
-  //    2176 1008 / 1182, x 8192 996 / 1030, four x 16384 502 / 508.
-  //  - otherwise one launch of the ordered pass over the whole list.  Its time is the chain of
-  //    tiles of one workgroup until the memory system is full, so the fewer chains there are the
-  //    longer the tile: up to 256 chains a tile of 128 KB (one layer x 4096 tokens 9.9 / 19.1 us, called over
-  //    and over on one cache; 14.6 behind the scorer of a step, the rows not in L2; 16
-  //    layers 43.1 / 54.1; up to 128 chains two workgroups take half of every row each, 8 layers
-  //    24.3 / 37.1), up to 1024 chains 32 KB (36 layers x 2176 tokens 120.6 / 135.8; 36 layers x 1000 ->
-  //    600 31.2 / 38.0, where 128 KB overshoot the list: 37.5), beyond that 32 KB in workgroups of 512
-  //    (16 requests x 2176 tokens 1997 / 2035; 256 threads 2007).
   const int chains = a.B * a.L * 2 * a.Hkv;
-  if ((int64_t)5 * a.max_budget > a.Tmax || chains <= 512) {
+  if (takes_one_launch(a, chains, forked)) {
+    // The longer the fewer chains there are: up to 256 a tile of 128 KB (one layer x 4096 tokens 9.9 / 19.1 us, called over
+    // and over on one cache; 14.3 behind the scorer of a step, the rows not in L2; 16
+    // layers 43.1 / 54.1; up to 128 chains two workgroups take half of every row each, 8 layers
+    // 24.3 / 37.1), up to 1024 chains 32 KB (36 layers x 2176 tokens 120.6 / 135.8; 36 layers x 1000 ->
+    // 600 31.2 / 38.0, where 128 KB overshoot the list: 37.5), beyond that 32 KB in workgroups of 512
+    // (16 requests x 2176 tokens 1997 / 2035; 256 threads 2007).
     CompactArgs one = c;
     if (chains <= 256) {
       if (chains <= 128 && c.chunks_per_row >= 16) one.cols = 2;     // (pieces of 128 bytes: a cache line)
