@@ -529,6 +529,36 @@ def test_topk_rows_bin_edges(width):
         assert torch.equal(got[:, :k], osel.topk_ascending(x, k)), k
 
 
+@pytest.mark.parametrize("width", [1026, 4096, 8000, 16384, 32768])
+def test_topk_rows_cut_again_where_many_scores_share_a_bin(width):
+    """Rows in which one of the 2048 equal bins holds more than the 1024 scores that are ranked: outliers, long tails,
+    clusters closer than a bin on both sides of zero, a few values many times over.  One, two and three cuts of the
+    keys, and cuts that end because all that is left is equal."""
+    g = torch.Generator().manual_seed(width + 1)
+    x = torch.randn(9, width, generator=g)
+    step = torch.randint(0, 3000, (width,), generator=g).float() * 2.0 ** -23
+    x[0, 5] = 1e30
+    x[1] = x[1].sign() * (8 * x[1].abs()).exp()
+    x[2] = 1.0 + step
+    x[2, 9] = 1e6
+    x[3, : width // 2] = 1.0 + step[: width // 2]
+    x[3, width // 2:] = -1.0 - step[width // 2:]
+    x[3, 11] = -1e20
+    x[4] = 2.5
+    x[4, 0] = 3e38
+    x[5] = torch.randint(-1, 2, (width,), generator=g).float()
+    x[5, 1], x[5, 2] = 1e35, -1e35
+    x[6, ::3] *= 1e-41
+    x[6, 1::3] *= 1e30
+    x[7] = (30 * x[7]).exp()
+    x[8] = torch.randint(0, 1 << 23, (width,), generator=g).int().view(torch.float32)     # subnormal, any spacing
+    x[8, 3] = 1.0
+    xd = x.to(DEV)
+    for k in (1, 2, width // 4, width // 3 + 1, width // 2, width - 1):
+        got = ops.topk_rows(xd, k).cpu().long()
+        assert torch.equal(got[:, :k], osel.topk_ascending(x, k)), k
+
+
 def test_topk_rows_ties_and_order():
     g = torch.Generator().manual_seed(1)
     x = torch.randn(5, 3000, generator=g)

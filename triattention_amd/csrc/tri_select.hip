@@ -474,17 +474,30 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_kernel(const float* sc
   }
 }
 
-// Wave-wide reductions (every lane gets the result).
-__device__ __forceinline__ uint32_t wave_min(uint32_t v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, off));
-  return v;
+// Reductions over the 16 lanes of a row and over the wave (every lane gets the result): rotations inside a row, then the
+// four rows' results as scalars.
+template <int N>
+__device__ __forceinline__ uint32_t row_rotate(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x120 + N, 0xf, 0xf, true);
 }
-__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off));
-  return v;
+template <typename Op>
+__device__ __forceinline__ uint32_t row_reduce(uint32_t v, Op op) {
+  v = op(v, row_rotate<8>(v));
+  v = op(v, row_rotate<4>(v));
+  v = op(v, row_rotate<2>(v));
+  return op(v, row_rotate<1>(v));
 }
+template <typename Op>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t v, Op op) {
+  v = row_reduce(v, op);
+  const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
+  const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+  return op(op(a, b), op(c, d));
+}
+__device__ __forceinline__ uint32_t scalar_of(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+struct MinOp { __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return min(a, b); } };
+struct MaxOp { __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return max(a, b); } };
+struct SumOp { __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return a + b; } };
 // Inverse of float_key.
 __device__ __forceinline__ float key_float(uint32_t k) {
   return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
@@ -492,7 +505,7 @@ __device__ __forceinline__ float key_float(uint32_t k) {
 constexpr uint32_t kKeyInf = 0xff800000u;        // float_key(+inf); NaNs of positive sign lie above
 constexpr uint32_t kKeyFiniteMin = 0x00800000u;  // float_key(-FLT_MAX); -inf and NaNs of negative sign lie below
 constexpr int kTopkBins = 2048;
-constexpr int kTopkCand = kTopkThreads;          // candidates ranked by counting, one thread each
+constexpr int kTopkCand = 128;                   // candidates ranked by counting, one thread each (their square is the time)
 
 // The same selection for rows of at most VPT * 1024 elements: the row is read once into
 // registers.  A wave owns 64 * VPT consecutive elements, 64 at a time: loads are whole lines, and the
@@ -502,17 +515,20 @@ constexpr int kTopkCand = kTopkThreads;          // candidates ranked by countin
 //
 // A few rows on a few CUs: the time is the chain of barriers and LDS round trips, not the
 // bytes.  The threshold is found in one histogram pass: the finite scores are
-// cut into 2048 bins of equal width between their minimum and maximum ((x - lo) * scale,
+// cut into 2000 bins of equal width between their minimum and maximum ((x - lo) * scale,
 // rounded, is monotone in x, so the bins are ordered as the scores are), a scan over all
 // threads finds the bin of the k-th largest, and the few scores of that bin are ranked
 // against each other, one thread per candidate, on their exact keys.  Guarded tokens (+inf)
-// are counted apart, they would stretch the bins.  A bin of more than 1024 scores (rows with
-// many equal scores, or a few outliers far away) falls back to radix passes of 8 bits over its keys.
-// Seven barriers; with radix passes alone it was thirteen, around scans by a single wave.
-// 8 rows of 4096: 13.1 -> 6.9 us; 8 rows of 2176 added up from 36 groups: 21.7 -> 14.3; 192 rows
-// of up to 12001: 24.7 -> 12.3; 8 rows of 32768: 47.8 -> 25.3 (there the instructions of one CU bound it).
+// are counted apart, they would stretch the bins.  A bin of more than 128 scores (rows with many equal ones) and rows whose
+// range lies far beyond where most scores are (outliers, long tails) are cut by their keys, whose range shrinks by 2^11 a
+// pass: a key is a logarithm of the score, so one or two passes take care of those, and equal scores end it.
+// Seven barriers, five more a further pass; with radix passes of 8 bits alone it was thirteen, around scans by a single wave.
+// us, scores of one size / with an outlier at 1e6, against 27 and 53 of radix passes for the longer ones: 8 rows of 4096
+// 6.6 / 6.2 (12.5), 288 rows of 2176 7.7 / 9.2 (15.8: two workgroups a CU, 64 registers a thread), 128 rows of 16384
+// 11.3 / 13.5, 8 rows of 32768 19.4 / 23.2 (there the instructions of one CU bound it).  Ranking up to 1024
+// candidates took 30 us at 750, radix passes behind the first histogram 57 and 106 with an outlier.
 template <int VPT>
-__global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float* scores, int64_t row_pitch,
+__global__ __launch_bounds__(kTopkThreads, VPT <= 4 ? 8 : 4) void topk_rows_reg_kernel(const float* scores, int64_t row_pitch,
                                                                     const int32_t* row_lens,
                                                                     const int32_t* row_ks, int rows_per_entry,
                                                                     int32_t* keep, int keep_pitch, int max_len,
@@ -592,22 +608,31 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
     hi_key = max(hi_key, fin ? key[i] : 0u);
     high += __popcll(__ballot(key[i] >= kKeyInf));
   }
-  lo_key = wave_min(lo_key);
-  hi_key = wave_max(hi_key);
+  lo_key = wave_reduce(lo_key, MinOp());
+  hi_key = wave_reduce(hi_key, MaxOp());
   if (lane == 0) {
     wave_lo[wave] = lo_key;
     wave_hi[wave] = hi_key;
     wave_tot[wave] = (uint32_t)high;
   }
-  for (int i = tid; i < kTopkBins; i += kTopkThreads) hist[i] = 0;
+  auto clear_hist = [&]() __attribute__((always_inline)) {
+    for (int i = tid; i < kTopkBins; i += kTopkThreads) hist[i] = 0;
+  };
+  clear_hist();
   if (tid == 0) sh_ncand = 0;
   __syncthreads();
-  uint32_t above = 0;                            // scores at or above +inf in the row
-#pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    lo_key = min(lo_key, wave_lo[w]);
-    hi_key = max(hi_key, wave_hi[w]);
-    above += wave_tot[w];
+  static_assert(kWaves == 16, "a lane of a row reads what one wave left");
+  uint32_t above;                                // scores at or above +inf in the row
+  uint32_t core_lo, core_hi;                     // a range that every full wave's finite scores reach beyond
+  {
+    const int w = lane & 15;
+    const uint32_t wl = wave_lo[w], wh = wave_hi[w];
+    const bool full = (w + 1) * (64 * VPT) <= T && wl <= wh;
+    above = scalar_of(row_reduce(wave_tot[w], SumOp()));
+    lo_key = scalar_of(row_reduce(wl, MinOp()));
+    hi_key = scalar_of(row_reduce(wh, MaxOp()));
+    core_lo = scalar_of(row_reduce(full ? wl : 0u, MaxOp()));
+    core_hi = scalar_of(row_reduce(full ? wh : 0xffffffffu, MinOp()));
   }
   // A row without a finite score has lo_key > hi_key: everything else then falls into bin 0.
   const float lo = lo_key <= hi_key ? key_float(lo_key) : 0.f;
@@ -615,31 +640,23 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
   // (A width beyond the largest float is +inf and makes the scale 0: a score whose distance from lo is still a
   // number falls into bin 0; the largest ones, whose distance is +inf too, give inf * 0 = NaN, which the fminf
   // below drops for the last bin.  Two bins, in order.)
-  const float scale = width > 0.f ? fminf(__fdiv_rn((float)kTopkBins, width), 3.0e38f) : 0.f;
+  // (2000 of the 2048 bins: scores on a grid would otherwise fall into bins a power of two apart, counters of one bank)
+  const float scale = width > 0.f ? fminf(__fdiv_rn(2000.f, width), 3.0e38f) : 0.f;
   auto bin_of = [&](uint32_t kk) __attribute__((always_inline)) {
     const float t = __fmul_rn(__fsub_rn(key_float(kk), lo), scale);
     const int b = kk < kKeyFiniteMin ? 0 : (int)fminf(t, (float)(kTopkBins - 1));
     return (uint32_t)b;
   };
+  // A range far beyond what every wave's scores span (outliers, long tails) would leave most scores in a few bins, and the
+  // lanes of a wave adding to one counter one after the other.  Those rows are cut by their keys from the start.  (Scores
+  // of one size span 1.5 times the core.)
+  const bool skewed = core_lo <= core_hi && core_lo != 0u && !(width <= 16.f * __fsub_rn(key_float(core_hi), key_float(core_lo)));
 
   // ---- which scores the k-th largest is among, and how many of those are kept.
-  uint32_t remaining = (uint32_t)k, count;
-  uint32_t cmask = 0;                            // bit i: element i is a candidate
-  if (above >= (uint32_t)k) {                    // (the same for the whole workgroup)
-    count = above;
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) cmask |= (uint32_t)(key[i] >= kKeyInf) << i;
-  } else {
-    remaining -= above;
-    uint32_t bins[VPT / 2];                      // two per register; 0xffff: none
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-      const bool ok = key[i] - 1u < kKeyInf - 1u;
-      const uint32_t b = ok ? bin_of(key[i]) : 0xffffu;
-      if (ok) atomicAdd(&hist[b], 1u);
-      bins[i / 2] = (i & 1) ? bins[i / 2] | (b << 16) : b;
-    }
-    __syncthreads();
+  uint32_t remaining = (uint32_t)k, count = 0;
+  // The bin of the finished histogram that holds the `remaining`-th largest; remaining and count become those of
+  // the bin.  Everyone is past the barrier behind the histogram.
+  auto find_bin = [&]() __attribute__((always_inline)) {
     constexpr int BPT = kTopkBins / kTopkThreads;   // bins per thread
     uint32_t h[BPT], own = 0;
 #pragma unroll
@@ -652,8 +669,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
     }
     if (lane == 0) wave_lo[wave] = suffix;         // (read by everyone before the barrier above)
     __syncthreads();
-    uint32_t gt = suffix - own;
-    for (int w = wave + 1; w < kWaves; ++w) gt += wave_lo[w];
+    uint32_t gt = suffix - own + row_reduce((lane & 15) > wave ? wave_lo[lane & 15] : 0u, SumOp());
 #pragma unroll
     for (int j = BPT - 1; j >= 0; --j) {
       const uint32_t ge = gt + h[j];
@@ -665,16 +681,79 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
       gt = ge;
     }
     __syncthreads();
-    const uint32_t bin = sh_prefix;
     remaining = sh_remaining;
     count = sh_count;
+    return sh_prefix;
+  };
+  // ---- cuts into 2048 bins until few candidates are left or all are equal: the first by score (of a skewed row by the
+  // leading bits of the key), the next ones by the range of the keys that are left.
+  uint32_t cmask = 0;                            // bit i: element i is a candidate
+  if (above >= (uint32_t)k) {                    // (the same for the whole workgroup)
+    count = above;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) cmask |= (uint32_t)(key[i] >= kKeyInf) << i;
+  } else if (skewed) {
+    remaining -= above;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+      if (key[i] - 1u < kKeyInf - 1u) atomicAdd(&hist[key[i] >> 21], 1u);
+    __syncthreads();
+    const uint32_t bin = find_bin();
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) cmask |= (uint32_t)(key[i] - 1u < kKeyInf - 1u && key[i] >> 21 == bin) << i;
+  } else {
+    remaining -= above;
+    uint32_t bins[VPT / 2];                      // two per register; 0xffff: none
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const bool ok = key[i] - 1u < kKeyInf - 1u;
+      const uint32_t b = ok ? bin_of(key[i]) : 0xffffu;
+      if (ok) atomicAdd(&hist[b], 1u);
+      bins[i / 2] = (i & 1) ? bins[i / 2] | (b << 16) : b;
+    }
+    __syncthreads();
+    const uint32_t bin = find_bin();
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
       cmask |= (uint32_t)(((bins[i / 2] >> (16 * (i & 1))) & 0xffffu) == bin) << i;
   }
+  uint32_t thr = 0, need_eq = 0;                 // key of the k-th largest, how many equal to it are kept (lowest index first)
+  bool equal = false;
+  while (count > (uint32_t)kTopkCand) {
+    uint32_t lo_c = 0xffffffffu, hi_c = 0u;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const bool part = (cmask >> i) & 1u;
+      lo_c = min(lo_c, part ? key[i] : 0xffffffffu);
+      hi_c = max(hi_c, part ? key[i] : 0u);
+    }
+    lo_c = wave_reduce(lo_c, MinOp());
+    hi_c = wave_reduce(hi_c, MaxOp());
+    __syncthreads();                             // (wave_lo and hist are read by everyone before they are written again)
+    if (lane == 0) { wave_lo[wave] = lo_c; wave_hi[wave] = hi_c; }
+    clear_hist();
+    __syncthreads();
+    lo_c = scalar_of(row_reduce(wave_lo[lane & 15], MinOp()));
+    hi_c = scalar_of(row_reduce(wave_hi[lane & 15], MaxOp()));
+    if (lo_c == hi_c) {
+      equal = true;
+      thr = lo_c;
+      need_eq = remaining;
+      break;
+    }
+    const int shift = max(32 - __clz((int)(hi_c - lo_c)) - 11, 0);     // 0: a bin is a key
+#pragma unroll
+    for (int i = 0; i < VPT; ++i)
+      if ((cmask >> i) & 1u) atomicAdd(&hist[(key[i] - lo_c) >> shift], 1u);
+    __syncthreads();                             // (wave_lo is free again as well)
+    const uint32_t bin = find_bin();
+    asm volatile("" : "+v"(lo_c));
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) cmask &= ~((uint32_t)((key[i] - lo_c) >> shift != bin) << i);
+  }
 
   // ---- the k-th largest among the candidates.
-  if (count <= (uint32_t)kTopkCand) {
+  if (!equal) {
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
       if ((cmask >> i) & 1u) cand[atomicAdd(&sh_ncand, 1u)] = key[i];
@@ -695,63 +774,9 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
       }
     }
     __syncthreads();
-  } else {
-    // Radix select over the candidates' keys, 8 bits per pass from the top.
-    uint32_t prefix = 0, mask = 0;
-    for (int shift = 24; shift >= 0; shift -= 8) {
-      __syncthreads();
-      if (tid < 256) hist[tid] = 0;
-      __syncthreads();
-      // Keys of one bin are close together, so the leading digits take one or two values and the plain
-      // atomics of a wave would go to the same counter one after the other: the lanes that hold
-      // the same digit are counted with a ballot and added once (up to four distinct digits per
-      // round; what is left takes the plain atomics).
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) {
-        const bool part = ((cmask >> i) & 1u) && (key[i] & mask) == prefix;
-        const uint32_t digit = (key[i] >> shift) & 255u;
-        unsigned long long todo = __ballot(part);
-        for (int it = 0; it < 4 && todo; ++it) {
-          const int leader = __builtin_amdgcn_readfirstlane(__ffsll((long long)todo) - 1);
-          const uint32_t dl = (uint32_t)__builtin_amdgcn_readlane((int)digit, leader);
-          const unsigned long long same = __ballot(part && digit == dl) & todo;
-          if (lane == leader) atomicAdd(&hist[dl], (uint32_t)__popcll(same));
-          todo &= ~same;
-        }
-        if ((todo >> lane) & 1ull) atomicAdd(&hist[digit], 1u);
-      }
-      __syncthreads();
-      if (wave == 0) {
-        // lane owns bins 4*lane .. 4*lane+3
-        uint32_t h[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) h[j] = hist[4 * lane + j];
-        const uint32_t own = h[0] + h[1] + h[2] + h[3];
-        uint32_t suffix = own;                         // sum over lanes >= lane
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const uint32_t v = __shfl_down(suffix, off);
-          if (lane + off < 64) suffix += v;
-        }
-        uint32_t gt = suffix - own;                    // digits above this lane's bins
-#pragma unroll
-        for (int j = 3; j >= 0; --j) {
-          const uint32_t ge = gt + h[j];
-          if (gt < remaining && remaining <= ge) {     // exactly one bin satisfies this
-            sh_high = prefix | ((uint32_t)(4 * lane + j) << shift);
-            sh_count = remaining - gt;
-          }
-          gt = ge;
-        }
-      }
-      __syncthreads();
-      prefix = sh_high;
-      remaining = sh_count;
-      mask |= 255u << shift;
-    }
+    thr = sh_high;
+    need_eq = sh_count;
   }
-  const uint32_t thr = sh_high;        // key of the k-th largest element
-  const uint32_t need_eq = sh_count;   // how many elements equal to it are kept (lowest index first)
 
   // ---- ordered compaction.  Counts of (greater, equal) of the wave packed as (g << 16) | e: a row has
   // at most 32768 elements.  Elements beyond the row hold key 0, which the threshold never is.
@@ -761,8 +786,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_rows_reg_kernel(const float
     mine += ((uint32_t)__popcll(__ballot(key[i] > thr)) << 16) + (uint32_t)__popcll(__ballot(key[i] == thr));
   if (lane == 0) wave_tot[wave] = mine;
   __syncthreads();
-  uint32_t before = 0;
-  for (int w = 0; w < wave; ++w) before += wave_tot[w];
+  const uint32_t before = scalar_of(row_reduce((lane & 15) < wave ? wave_tot[lane & 15] : 0u, SumOp()));
   uint32_t eq_before = before & 0xffffu;
   uint32_t pos = (before >> 16) + min(eq_before, need_eq);
   auto lanes_below = [](unsigned long long m) __attribute__((always_inline)) {
