@@ -720,6 +720,13 @@ def test_dense_compressor_in_one_call_equals_its_parts(tmp_path, case):
     assert k3.stride() == k2.stride() and v3.stride() == v2.stride()
 
 
+@pytest.mark.parametrize("h,t,d", [(3, 16383, 128), (3, 16384, 128), (1, 16385, 64), (8, 20481, 128)])
+def test_dense_compressor_statistics_of_long_rows(tmp_path, h, t, d):
+    """From 16384 tokens on a row's statistics come in chunks of 2048: both sides, a last chunk of one token, heads that
+    are no power of two."""
+    test_dense_compressor_in_one_call_equals_its_parts(tmp_path, dict(h=h, t=t, d=d, budget=t // 5))
+
+
 @pytest.mark.parametrize("normalize", [True, False])
 @pytest.mark.parametrize("window", [16, 0])
 @pytest.mark.parametrize("bad", ["nan", "-nan", "inf", "-inf"])

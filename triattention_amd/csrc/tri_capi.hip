@@ -254,8 +254,10 @@ int do_select(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_p
   a.raw = raw; a.raw_stride_layer = rs_layer; a.raw_stride_token = rs_token; a.raw_stride_head = rs_head;
   a.fin = fin ? fin : at<float>(ws, w.fin);
   a.keep = keep;
-  a.group_scratch = at<double>(ws, w.coef);
-  a.group_scratch_bytes = w.trig - w.coef;
+  // Scratch of the chunked statistics: the coefficients (the scorer is done with them) or, where one score per KV head
+  // needs no sums of the scorer's tiles, the room planned for those.
+  a.group_scratch = at<double>(ws, pass_nan ? w.partial : w.coef);
+  a.group_scratch_bytes = pass_nan ? w.mustd - w.partial : w.trig - w.coef;
   return launch_status(tri::launch_select(a, s), "select");
 }
 
