@@ -531,7 +531,7 @@ def test_topk_rows_bin_edges(width):
 
 @pytest.mark.parametrize("width", [1026, 4096, 8000, 16384, 32768])
 def test_topk_rows_cut_again_where_many_scores_share_a_bin(width):
-    """Rows in which one of the 2048 equal bins holds more than the 1024 scores that are ranked: outliers, long tails,
+    """Rows in which one of the equal bins holds more than the 128 scores that are ranked: outliers, long tails,
     clusters closer than a bin on both sides of zero, a few values many times over.  One, two and three cuts of the
     keys, and cuts that end because all that is left is equal."""
     g = torch.Generator().manual_seed(width + 1)
