@@ -1052,6 +1052,21 @@ def test_matrix_core_scores_carry_every_piece(kv_dtype, head_dim, monkeypatch):
     two-pass kernels' fp32 arithmetic to 5e-6 of the largest score (measured: 2e-7 .. 1.5e-6);
     a dropped second piece of the magnitudes would show as 1e-4 .. 2e-3."""
     w = small(kv_dtype=kv_dtype, head_dim=head_dim, seq_lens=(3000, 1000), index=77)
+    _assert_scores_carry_every_piece(w)
+
+
+@pytest.mark.parametrize("kv_dtype,head_dim,g", [("bf16", 128, 5), ("bf16", 64, 8), ("bf16", 256, 7), ("fp16", 128, 8),
+                                                 ("fp16", 64, 6), ("fp8", 128, 8)])
+def test_every_piece_of_five_to_eight_query_heads(kv_dtype, head_dim, g, monkeypatch):
+    """The operand layout of five to eight query heads per KV head (two pieces side by side, the third in an
+    operand of its own; two pieces of the magnitude coefficients): same bound as with four.  Tiles that end
+    inside a step, one token into it and at its end."""
+    w = small(kv_dtype=kv_dtype, head_dim=head_dim, num_q_heads=3 * g, num_kv_heads=3, seq_lens=(1201, 1000, 33), index=78)
+    _assert_scores_carry_every_piece(w)
+
+
+def _assert_scores_carry_every_piece(w):
+    kv_dtype, head_dim = w.kv_dtype, w.head_dim
     inp = build_inputs(w)
     caches, kv, batch, sc = device_objects(w, inp, DEV)
     sel = ops.SelectConfig(window_size=w.window_size, normalize=False, layer_reduce="max")

@@ -333,10 +333,8 @@ int do_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_s
   a.skip_layer_reduce = split && !fin && keep && batch->max_seq_len <= tri::topk_register_row_limit();
   a.bmat = at<char>(ws, w.bmat);
   if (w.fused.eligible == 2) {
-    // The preparation launch writes one 16-byte entry per (sequence, layer, KV head, group of four
-    // query heads, slab, lane); the region planned for them must hold that.
-    const int64_t groups = a.G > 4 ? 2 : 1, slabs = a.D / 32 + a.D / 64;
-    const int64_t need = (int64_t)a.B * a.L * a.Hkv * groups * slabs * 64 * 16;
+    // The preparation launch writes one 16-byte entry per (sequence, layer, KV head, operand, lane); the region planned for them must hold that.
+    const int64_t need = (int64_t)a.B * a.L * a.Hkv * tri::mfma_operands(F, a.G) * 64 * 16;
     if (need > w.total - w.bmat)
       return fail(TRI_ERR_WORKSPACE, "coefficient slabs need %lld bytes, %lld planned", (long long)need,
                   (long long)(w.total - w.bmat));

@@ -62,11 +62,15 @@ struct Workspace {
   int64_t xchg;      // [B][L][tiles_per_seq][A][2] tagged sums exchanged by the resident kernel
   int64_t status;    // one word: non-zero when a bounded wait of the resident kernel expired
   int64_t pack;      // [2][B] int32: launch of every sequence and its first workgroup there (several launches)
-  int64_t bmat;      // [B][L][Hkv][groups of 4 query heads][slabs][64][8] bf16 coefficient slabs (matrix-core kernel)
+  int64_t bmat;      // [B][L][Hkv][mfma_operands][64][8] coefficient slabs (matrix-core kernel)
   int64_t total;
   int32_t num_tiles; // NT
   FusedPlan fused;
 };
+
+// Coefficient operands of a KV head in the matrix-core resident kernel: key slabs (head_dim / 32; once more for the
+// third pieces of five to eight query heads) and magnitude slabs (head_dim / 64).  F = head_dim / 2.
+__host__ __device__ inline int mfma_operands(int F, int G) { return (G > 4 ? 2 : 1) * (F / 16) + F / 32; }
 
 inline Workspace plan_workspace(int B, int L, int A, int F, int NO, int Hkv, int Tmax, const FusedPlan& fused) {
   Workspace w{};
@@ -85,9 +89,7 @@ inline Workspace plan_workspace(int B, int L, int A, int F, int NO, int Hkv, int
   w.fin = take((int64_t)B * L * Hkv * Tmax * 4);
   w.xchg = take(fused.eligible ? (int64_t)B * L * fused.tiles_per_seq * A * 2 * 8 : 0);
   w.pack = take(fused.eligible ? (int64_t)B * 8 : 0);
-  // key slabs (head_dim / 32) and magnitude slabs (half as many) per group of four query heads
-  const int slabs = max(F / 16 + F / 32, 6);
-  w.bmat = take(fused.eligible == 2 ? (int64_t)B * L * Hkv * (A / Hkv > 4 ? 2 : 1) * slabs * 64 * 16 : 0);
+  w.bmat = take(fused.eligible == 2 ? (int64_t)B * L * Hkv * mfma_operands(F, A / Hkv) * 64 * 16 : 0);
   w.total = off;
   return w;
 }

@@ -47,10 +47,10 @@ constexpr int kDppRor8m = 0x128;  // row_ror:8
 // MFMA s takes half s % 2 of chunk s / 2) and the dequantisation scale of the token this
 // lane will store.
 // HD: head dimension, 128 or (two-byte keys only) 64: half the chunks, MFMAs and pairs.
-template <int DT, int HD>
+template <int DT, int HD, int QG>
 struct StepData {
   uint4 c[DT == TRI_KV_FP8_E4M3 ? 2 : HD / 32];
-  float scale;
+  float scale[QG];      // fp8 only
 };
 
 // Index, inside the 128 elements of a head row, of element e of lane block kb in MFMA s.
@@ -119,6 +119,12 @@ __device__ __forceinline__ uint32_t split_pair_f16(float x0, float x1, float& r0
   return packed;
 }
 
+// Larger halves of two packed fp16 pairs (no quieting of the operands, which costs an instruction each).
+__device__ __forceinline__ f16x2 pk_max_f16(f16x2 a, uint32_t b) {
+  asm("v_pk_max_f16 %0, %0, %1" : "+v"(a) : "v"(b));
+  return a;
+}
+
 // One 16x16x32 matrix-core step in the operand type of the keys (fp8 keys are converted to bf16).
 template <int DT>
 __device__ __forceinline__ f32x4 mfma_step(const uint4& a, const uint4& b, f32x4 c) {
@@ -147,11 +153,12 @@ __device__ __forceinline__ float coefficient_piece(float x, int pieces) {
 //    order in double);
 //  - combines the means with the folded statistics of its KV heads of layer l (heads z * heads_per_wg
 //    and up) into P = a1*C - a2*S, R = a2*C + a1*S, E and writes them as MFMA B operands:
-// bmat[(((b*L + l)*Hkv + head)*QG + g)*6 + o][lane][8] bf16.  Group g holds query heads
-// 4g..4g+3 of the KV head.  Operand o: 0..3 the key slabs of MFMA o, 4 and 5 the magnitudes
-// of pair sets 0 and 1.  Lane (j = lane % 16, kb): column j = (query head 4g + j % 4, split
-// j / 4); element e = k index kb*8 + e of the slab.  Piece `split` of a coefficient x is
-// what is left of x after `split` roundings to bf16 (x = x1 + x2 + x3).
+// bmat[((b*L + l)*Hkv + head)*NSO + o][lane][8] of two bytes.  Lane (j = lane % 16, kb) of an operand holds
+// column j, k indices kb*8 .. + 7 of its slab.  Up to four query heads per KV head: operands 0..NS-1 are the
+// key slabs, NS/2 magnitude slabs follow; column j = (query head j % 4, piece j / 4).  Five to eight: NS key
+// operands with column j = (query head j % 8, piece j / 8), NS more with the third piece in columns 0..7 and
+// zeros beside it, NS/2 magnitude operands (query head j % 8, piece j / 8).  Piece p of a coefficient x is
+// what is left of x after p roundings to the operand type (x = x1 + x2 + x3).
 constexpr int kPrepThreads = 1024;
 // Query heads whose coefficients are staged at a time, and the pitch of a staged head
 // [P | R | E][F] in floats (odd: the four query heads and four k blocks a wave reads at once
@@ -163,14 +170,15 @@ template <int DT, bool IL, int HD>
 __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* folded, const float* omega,
                                                                  const float* offsets, int NO,
                                                                  const int32_t* round_start, int L, int Hkv, int G,
-                                                                 int A, int QG, uint4* bmat,
+                                                                 int A, uint4* bmat,
                                                                  unsigned long long* xchg, int64_t words,
                                                                  uint32_t* status, int heads_per_wg) {
   // One buffer, used twice: the per-offset cos / sin values, then the coefficients of up to
   // kPrepHeads query heads as [head][P | R | E][F] with a row pitch of 3F + 1 floats.
   constexpr int F = HD / 2;              // frequency pairs
-  constexpr int NS = HD / 32;            // key slabs (MFMAs) per step
-  constexpr int NSO = NS + NS / 2;       // operands per query-head group: key slabs, magnitude slabs
+  constexpr int NS = HD / 32;            // key slabs
+  const int NSO = mfma_operands(F, G);   // operands of a KV head
+  const int NK = NSO - NS / 2;           // of them key operands, the magnitude operands follow
   constexpr int kPrepHeads = prep_heads<HD>(), kPrepPitch = prep_pitch<HD>();
   __shared__ float buf[kPrepHeads * kPrepPitch];
   __shared__ float mean_cs[2][F];
@@ -219,15 +227,23 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
       buf[q * kPrepPitch + 2 * F + f] = e;
     }
     __syncthreads();
-    const int items = nh * QG * NSO * 64;                   // (head, group, operand, lane)
-    uint4* out_base = bmat + (((int64_t)b * L + l) * Hkv + head0) * QG * NSO * 64;
+    const int items = nh * NSO * 64;                        // (head, operand, lane)
+    uint4* out_base = bmat + (((int64_t)b * L + l) * Hkv + head0) * NSO * 64;
     for (int idx = tid; idx < items; idx += kPrepThreads) {
       const int lane = idx & 63;
       const int o = (idx >> 6) % NSO;
-      const int g = (idx / (64 * NSO)) % QG;
-      const int head = idx / (64 * NSO * QG);
+      const int head = idx / (64 * NSO);
       const int j = lane & 15, kb = lane >> 4;
-      const int q = 4 * g + (j & 3), sp = j >> 2;
+      const bool mag = o >= NK;
+      const int slab = mag ? o - NK : o % NS;
+      int q, sp;                                            // query head and piece of column j (piece 3: a zero column)
+      if (G > 4) {
+        q = j & 7;
+        sp = !mag && o >= NS ? (j < 8 ? 2 : 3) : j >> 3;
+      } else {
+        q = j & 3;
+        sp = j >> 2;
+      }
       uint32_t out[4] = {0, 0, 0, 0};
       if (q < G && sp < 3) {
         const float* c = buf + (head * G + q) * kPrepPitch;
@@ -236,29 +252,28 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
         for (int e = 0; e < 8; ++e) {
           int which, pair;   // which: 0 = P, 1 = R, 2 = E
           constexpr bool kRegrouped = DT == TRI_KV_FP8_E4M3 && !IL;   // see compute_step
-          if (o < NS) {
-            const int el = slab_elem<DT>(o, kb, e);
-            if (kRegrouped) { which = e & 1; pair = kb * 16 + 4 * o + (e >> 1); }
+          if (!mag) {
+            const int el = slab_elem<DT>(slab, kb, e);
+            if (kRegrouped) { which = e & 1; pair = kb * 16 + 4 * slab + (e >> 1); }
             else if (IL) { which = el & 1; pair = el >> 1; }
             else { which = el >= F ? 1 : 0; pair = el & (F - 1); }
           } else {
             which = 2;
-            const int set = o - NS;
-            // interleaved: pairs of MFMAs 2*set and 2*set + 1; half: real parts of MFMA `set`
-            if (kRegrouped) pair = kb * 16 + 4 * (2 * set + (e >> 2)) + (e & 3);
-            else if (IL) pair = slab_elem<DT>(2 * set + (e >> 2), kb, 2 * (e & 3)) >> 1;
-            else pair = slab_elem<DT>(set, kb, e) & (F - 1);
+            // interleaved: pairs of slabs 2*set and 2*set + 1; half: real parts of slab `set`
+            if (kRegrouped) pair = kb * 16 + 4 * (2 * slab + (e >> 2)) + (e & 3);
+            else if (IL) pair = slab_elem<DT>(2 * slab + (e >> 2), kb, 2 * (e & 3)) >> 1;
+            else pair = slab_elem<DT>(slab, kb, e) & (F - 1);
           }
           // The magnitudes go through the fp16 matrix-core instruction whatever the key type (see
           // compute_step), so the magnitude slabs are fp16 pieces.
-          const bool half_slab = DT == TRI_KV_FP16 || o >= NS;
+          const bool half_slab = DT == TRI_KV_FP16 || mag;
           v[e] = half_slab ? coefficient_piece<TRI_KV_FP16>(c[which * F + pair], sp)
                            : coefficient_piece<TRI_KV_BF16>(c[which * F + pair], sp);
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const f32x2 x = {v[2 * e], v[2 * e + 1]};
-          if (DT == TRI_KV_FP16 || o >= NS)
+          if (DT == TRI_KV_FP16 || mag)
             out[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, f16x2));
           else
             out[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, bf16x2));
@@ -270,6 +285,16 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
 }
 
 // QG: groups of four query heads per KV head (1 or 2).
+//
+// Two groups (five to eight query heads): a second operand set per group of four would leave a quarter of the
+// matrix columns empty twice and every step with two column reductions (three columns per head, four
+// values each, both groups: 34 of its 84 vector instructions at a head dimension of 64).  Instead the
+// columns are (query head, piece 1 | piece 2) and a second operand holds the third pieces beside zeros: one
+// accumulator for all eight heads, one exchange between column halves at the end, and the magnitude
+// coefficients, whose two fp16 pieces carry 24 bits, take one operand in place of two.  Vector / matrix
+// instructions a step: 84 / 8 -> 56 / 6 at a head dimension of 64, 166 / 16 -> 97 / 12 at 128.  24 requests of 1500 to
+// 12001 tokens x 36 layers x 64 query heads of 64: 1316 -> 1166 us; 1 x 32768 x 64 layers x 64 of 128: 824 -> 815 (there
+// the layers' statistics are waited for, not the instructions).
 __device__ __forceinline__ int nsteps_of(int ntok) { return (ntok + 15) >> 4; }
 
 // W: waves per workgroup.  Eight (one workgroup per CU), or four for models with at most four
@@ -280,8 +305,9 @@ template <int DT, bool IL, int TW, int SL, int QG, int NB, int W, int HD>
 __global__ __launch_bounds__(W * kWave) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   static_assert(HD == 128 || ((HD == 64 || HD == 256) && DT != TRI_KV_FP8_E4M3), "head dimensions with a kernel");
-  constexpr int NS = HD / 32;            // key slabs (MFMAs) per step
-  constexpr int NSO = NS + NS / 2;       // operands per query-head group
+  constexpr int NS = HD / 32;            // key slabs per step
+  constexpr int NK = QG * NS;            // key operands (MFMAs) of a KV head
+  constexpr int NSO = NK + NS / 2;       // all operands
   static_assert(SL % (16 * NB) == 0, "the slack must hold whole rotations of the step buffers");
   // Token t of layer l sits at (l * ring_stride + t) % RING, ring_stride the tokens of this launch's tiles (at
   // most TW): what a tile leaves free of the ring is slack, down to SL for a whole tile.
@@ -311,10 +337,10 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int heads_here = min(8, a.Hkv - chunk * 8);
 
   float* ring = lds + wave * (RING * RQ);                      // [QG][RING][4 query heads]
-  float* part = lds + W * (RING * RQ);                         // [waves][64][QG][2]
-  float* stats = part + W * 128 * QG;                          // [2][32*QG score heads][2]
+  float* part = lds + W * (RING * RQ);                         // [waves][64][2]
+  float* stats = part + W * 128;                          // [2][32*QG score heads][2]
   uint32_t* ctl = reinterpret_cast<uint32_t*>(stats + 128 * QG);  // arrive count, claimed, ready; [8..15]: how far each wave is
-  for (int i = threadIdx.x; i < W * 128 * QG; i += W * kWave) part[i] = 0.f;
+  for (int i = threadIdx.x; i < W * 128; i += W * kWave) part[i] = 0.f;
   if (threadIdx.x < 16) ctl[threadIdx.x] = 0;
   __syncthreads();
   // From here on the waves of the workgroup run independently.
@@ -322,16 +348,18 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int head = chunk * 8 + wave;
 
   const int j = lane & 15, kb = lane >> 4;       // MFMA column / k block; also output row block
-  const int q = j & 3, rsel = j >> 2;
+  // What this lane ends up with of a step: one group: the score of query head q = j % 4 for the step's token
+  // 4 kb + j / 4; two: of query head q = j % 8 for the tokens 4 kb + 2 (j / 8) and the one after.
+  const int q = QG == 1 ? j & 3 : j & 7;
+  const int rsel = QG == 1 ? j >> 2 : 2 * (j >> 3);
+  const bool upper = j >= 8;
 
   // Coefficient slabs of the current layer.
-  uint4 B[QG][NSO];
+  uint4 B[NSO];
   auto load_coefs = [&](int l) __attribute__((always_inline)) {
-    const uint4* p = bmat + (((int64_t)(b * a.L + l) * a.Hkv + head) * QG * NSO) * 64 + lane;
+    const uint4* p = bmat + (((int64_t)(b * a.L + l) * a.Hkv + head) * NSO) * 64 + lane;
 #pragma unroll
-    for (int g = 0; g < QG; ++g)
-#pragma unroll
-      for (int o = 0; o < NSO; ++o) B[g][o] = p[(g * NSO + o) * 64];
+    for (int o = 0; o < NSO; ++o) B[o] = p[o * 64];
     {
       // A coefficient beyond fp16's range (65504) arrives as an infinity: the scores of this
       // launch would be meaningless, so the status word is raised (the caller repeats the
@@ -339,14 +367,12 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       // all slabs; otherwise the magnitude slabs.
       uint32_t bad = 0;
 #pragma unroll
-      for (int g = 0; g < QG; ++g)
+      for (int o = (DT == TRI_KV_FP16 ? 0 : NK); o < NSO; ++o) {
+        const uint32_t w4[4] = {B[o].x, B[o].y, B[o].z, B[o].w};
 #pragma unroll
-        for (int o = (DT == TRI_KV_FP16 ? 0 : NS); o < NSO; ++o) {
-          const uint32_t w4[4] = {B[g][o].x, B[g][o].y, B[g][o].z, B[g][o].w};
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            bad |= (uint32_t)((w4[i] & 0x7c00u) == 0x7c00u) | (uint32_t)((w4[i] & 0x7c000000u) == 0x7c000000u);
-        }
+        for (int i = 0; i < 4; ++i)
+          bad |= (uint32_t)((w4[i] & 0x7c00u) == 0x7c00u) | (uint32_t)((w4[i] & 0x7c000000u) == 0x7c000000u);
+      }
       if (__any(bad != 0) && lane == 0) atomicExch(a.status, 2u);
     }
   };
@@ -382,62 +408,40 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       lb.scale = table_entry(reinterpret_cast<const void* const*>(a.k_scale_layers), l) + head * 4;
     return lb;
   };
-  // One-byte keys: with eight step buffers and a scale per row the scalar registers do not
-  // hold the strides, masks and sizes of the address arithmetic any more (the compiler kept
-  // them in lanes of a vector register and fetched 16 of them back per step with v_readlane,
-  // a tenth of the step's vector instructions).  For them the arithmetic is done once per
-  // tile instead: lane i keeps the byte offset of step i's first row from the head's base
-  // (the same in every layer) and the index of its first token slot.
-  uint32_t step_off_lo = 0, step_off_hi = 0;
+  // The address arithmetic of a step is done once per tile: lane i keeps the byte offset of step i's first
+  // row from the head's base (the same in every layer) and, for one-byte keys, the index of its first token
+  // slot.  (Per step it is 25 scalar instructions in the path of every wave; with one-byte keys, eight step
+  // buffers and a scale per row, the compiler kept its operands in lanes of a vector register on top.)
+  uint32_t step_off_lo, step_off_hi;
   int step_slot = 0;
-  if constexpr (FP8) {
+  {
     const int nt = min(n0 + 16 * lane, (nsteps_of(ntok) - 1) * 16 + n0);
     const int in_blk = nt & bs_mask;
     const int64_t off = ((int64_t)step_blk * a.stride_block + (int64_t)in_blk * a.stride_token) * ES;
     step_off_lo = (uint32_t)off;
     step_off_hi = (uint32_t)((uint64_t)off >> 32);
-    step_slot = step_blk * a.block_size + in_blk;
+    if constexpr (FP8) step_slot = step_blk * a.block_size + in_blk;
   }
-  auto load_step = [&](StepData<DT, HD>& d, const LayerBase& lb, int t) __attribute__((always_inline)) {
-    if constexpr (FP8) {
-      const int step = t >> 4;
-      const uint32_t rows_left = (uint32_t)(last_tok - (n0 + t));
-      const uint64_t row_off = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)step_off_hi, step) << 32) |
-                               (uint32_t)__builtin_amdgcn_readlane((int)step_off_lo, step);
-      const char* base = reinterpret_cast<const char*>(uniform_ptr(lb.k + row_off));
-      const uint32_t off = min(lane_row, rows_left * tok_bytes) + lane_col;
-      GlobalBytes p = (GlobalBytes)(uintptr_t)base + off;
-#pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const u32x4 v = *(GlobalU4)(p + s * 64);
-        d.c[s] = uint4{v.x, v.y, v.z, v.w};
-      }
-      const uint32_t hkv4 = (uint32_t)a.Hkv * 4u;
-      const uint64_t slot_off = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(step_slot, step) * hkv4;
-      const char* sc = reinterpret_cast<const char*>(uniform_ptr(lb.scale + slot_off));
-      const uint32_t soff = min(lane_scale_row, rows_left * hkv4);
-      d.scale = *(GlobalF32)((GlobalBytes)(uintptr_t)sc + soff);
-      return;
-    }
-    const int blk = __builtin_amdgcn_readlane(step_blk, t >> 4);
-    const int nt = n0 + t;
-    const int in_blk = nt & bs_mask;
-    const uint32_t rows_left = (uint32_t)(last_tok - nt);
-    const int64_t row0 = (int64_t)blk * a.stride_block + (int64_t)in_blk * a.stride_token;
-    const char* base = reinterpret_cast<const char*>(uniform_ptr(lb.k + row0 * ES));
+  auto load_step = [&](StepData<DT, HD, QG>& d, const LayerBase& lb, int t) __attribute__((always_inline)) {
+    const int step = t >> 4;
+    const uint32_t rows_left = (uint32_t)(last_tok - (n0 + t));
+    const uint64_t row_off = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)step_off_hi, step) << 32) |
+                             (uint32_t)__builtin_amdgcn_readlane((int)step_off_lo, step);
+    const char* base = reinterpret_cast<const char*>(uniform_ptr(lb.k + row_off));
     const uint32_t off = min(lane_row, rows_left * tok_bytes) + lane_col;
     GlobalBytes p = (GlobalBytes)(uintptr_t)base + off;
-    d.scale = 1.f;
 #pragma unroll
     for (int s = 0; s < (FP8 ? 2 : NS); ++s) {
       const u32x4 v = *(GlobalU4)(p + s * 64);
       d.c[s] = uint4{v.x, v.y, v.z, v.w};
     }
     if constexpr (FP8) {
-      const int64_t slot0 = (int64_t)blk * a.block_size + in_blk;
-      const char* sc = reinterpret_cast<const char*>(uniform_ptr(lb.scale + slot0 * a.Hkv * 4));
-      const uint32_t soff = min(lane_scale_row, rows_left * (uint32_t)a.Hkv * 4u);
-      d.scale = *(GlobalF32)((GlobalBytes)(uintptr_t)sc + soff);
+      const uint32_t hkv4 = (uint32_t)a.Hkv * 4u;
+      const uint64_t slot_off = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(step_slot, step) * hkv4;
+      const char* sc = reinterpret_cast<const char*>(uniform_ptr(lb.scale + slot_off));
+#pragma unroll
+      for (int i = 0; i < QG; ++i)
+        d.scale[i] = *(GlobalF32)((GlobalBytes)(uintptr_t)sc + min(lane_scale_row + (uint32_t)i * hkv4, rows_left * hkv4));
     }
   };
 
@@ -445,16 +449,14 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // (16 tokens x 4 heads of one group) cover 64 consecutive words and the 16-byte reads of
   // consecutive tokens are 16 bytes apart, whatever the number of groups (with [RING][8] the stores of
   // one group fell on half the banks; it does not show in the kernel's time).
-  const uint32_t lane_ring = (uint32_t)(4 * kb + rsel) * 4 + q;
-  float s1[QG], s2[QG];
-#pragma unroll
-  for (int g = 0; g < QG; ++g) { s1[g] = 0.f; s2[g] = 0.f; }
+  const uint32_t lane_ring = (uint32_t)(q >> 2) * (RING * 4) + (uint32_t)(4 * kb + rsel) * 4 + (q & 3);
+  float s1 = 0.f, s2 = 0.f;
   // Largest of a sample of the layer's magnitudes (their first fp16 pieces), per lane; see the check
   // after every layer.
   f16x2 mag_seen = {(_Float16)0.f, (_Float16)0.f};
   // Scores of the 16 tokens of a step: MFMAs over keys and magnitudes, split columns added
   // by row rotations; lane (j, kb) ends up with the score of token 4*kb + j/4, query head j%4.
-  auto compute_step = [&](const StepData<DT, HD>& raw, int l, int t, int which) __attribute__((always_inline)) {
+  auto compute_step = [&](const StepData<DT, HD, QG>& raw, int l, int t, int which) __attribute__((always_inline)) {
     // The four bf16 A operands of the step as dwords (two elements each): the loaded
     // registers for bf16 keys, one conversion per dword (exact) for fp8 keys.
     uint32_t w[NS][4];
@@ -497,15 +499,9 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     struct { uint4 c[NS]; } d;
 #pragma unroll
     for (int s = 0; s < NS; ++s) d.c[s] = uint4{w[s][0], w[s][1], w[s][2], w[s][3]};
-    f32x4 acc[QG], acc_e[QG];
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int g = 0; g < QG; ++g) {
-      acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < NS; ++s)
-        acc[g] = mfma_step<DT>(d.c[s], B[g][s], acc[g]);
-      acc_e[g] = acc[g];   // the magnitude MFMAs continue the sum (the key MFMAs are long done by then)
-    }
+    for (int o = 0; o < NK; ++o) acc = mfma_step<DT>(d.c[o % NS], B[o], acc);
 #pragma unroll
     for (int set = 0; set < NS / 2; ++set) {
       // |k_f|^2 = k_r^2 + k_i^2 straight from the bf16 pairs (v_dot2_f32_bf16).
@@ -547,34 +543,47 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
         (&lo.x)[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, f16x2));
       }
       if constexpr (!FP8)   // `which` is the step buffer's number: a constant after unrolling
-        mag_seen = __builtin_elementwise_max(mag_seen, __builtin_bit_cast(f16x2, (&hi.x)[which & 3]));
+        mag_seen = pk_max_f16(mag_seen, (&hi.x)[which & 3]);
       constexpr int MT = TRI_KV_FP16;                // operand type of the magnitude MFMAs
-#pragma unroll
-      for (int g = 0; g < QG; ++g) {
-        acc_e[g] = mfma_step<MT>(hi, B[g][NS + set], acc_e[g]);
-        acc_e[g] = mfma_step<MT>(lo, B[g][NS + set], acc_e[g]);
-      }
+      acc = mfma_step<MT>(hi, B[NK + set], acc);
+      acc = mfma_step<MT>(lo, B[NK + set], acc);
     }
-    const int tl = t + 4 * kb + rsel;
-    // first ring slot of the step (scalar; a step never straddles the wrap: t and RING are
-    // multiples of 16)
-    const uint32_t slot0 = (uint32_t)(l * a.ring_stride + t) % RING;
-#pragma unroll
-    for (int g = 0; g < QG; ++g) {
-      float v = 0.f;
+    // The pieces of a head are added across the columns; v[i] is then the score of this lane's i-th token.
+    float v[QG];
+    if constexpr (QG == 1) {
+      v[0] = 0.f;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        float x = acc_e[g][r];
+        float x = acc[r];
         x += dpp<kDppRor8m>(x);
         x += dpp<kDppRor4>(x);
-        v = (rsel == r) ? x : v;
+        v[0] = (rsel == r) ? x : v[0];
       }
-      if (FP8) v *= raw.scale;
-      if (4 * g + q < a.G && tl < ntok) {
-        ring[(uint32_t)g * (RING * 4) + slot0 * 4 + lane_ring] = v;
-        s1[g] += v;
-        s2[g] = fmaf(v, v, s2[g]);
-      }
+    } else {
+      const float x0 = acc[0], x1 = acc[1], x2 = acc[2], x3 = acc[3];
+      const float send0 = upper ? x0 : x2, send1 = upper ? x1 : x3;
+      v[0] = (upper ? x2 : x0) + dpp<kDppRor8m>(send0);
+      v[1] = (upper ? x3 : x1) + dpp<kDppRor8m>(send1);
+    }
+    if constexpr (FP8) {
+#pragma unroll
+      for (int i = 0; i < QG; ++i) v[i] *= raw.scale[i];
+    }
+    // first ring slot of the step (scalar; a step never straddles the wrap: t and RING are
+    // multiples of 16).  The ring has a place for every row of the step and every head slot: rows past the
+    // tile's last token and slots beyond the last query head (zero columns) are written too and never read.
+    const uint32_t slot0 = (uint32_t)(l * a.ring_stride + t) % RING;
+    if (t + 16 > ntok) {                              // (wave-uniform: the last step of a tile)
+      asm volatile("");
+#pragma unroll
+      for (int i = 0; i < QG; ++i)
+        if (t + 4 * kb + rsel + i >= ntok) v[i] = 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < QG; ++i) {
+      ring[slot0 * 4 + lane_ring + 4 * i] = v[i];
+      s1 += v[i];
+      s2 = fmaf(v[i], v[i], s2);
     }
   };
 
@@ -590,13 +599,10 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // before any wave deposits layer l + 1 (a wave consumes layer l, which needs every
   // deposit of layer l, before it finishes layer l + 1), so the counter never mixes layers.
   auto arrive = [&](int l) __attribute__((always_inline)) {
-#pragma unroll
-    for (int g = 0; g < QG; ++g) {
-      part[((wave * 64 + lane) * QG + g) * 2] = s1[g];
-      part[((wave * 64 + lane) * QG + g) * 2 + 1] = s2[g];
-      s1[g] = 0.f;
-      s2[g] = 0.f;
-    }
+    part[(wave * 64 + lane) * 2] = s1;
+    part[(wave * 64 + lane) * 2 + 1] = s2;
+    s1 = 0.f;
+    s2 = 0.f;
     uint32_t prev = 0;
     if (lane == 0) prev = __hip_atomic_fetch_add(arrive_cnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
     prev = __builtin_amdgcn_readfirstlane(prev);
@@ -606,10 +612,9 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     for (int item = lane; item < items; item += 64) {
       const int ahl = item >> 1, which = item & 1;
       const int w = ahl / a.G, qq = ahl - w * a.G;
-      const int g = qq >> 2, q4 = qq & 3;
+      constexpr int kLanes = 16 / QG;                // lanes that hold scores of one query head
       float t = 0.f;
-      for (int i = 0; i < 16; ++i)
-        t += part[((w * 64 + (i >> 2) * 16 + (i & 3) * 4 + q4) * QG + g) * 2 + which];
+      for (int i = 0; i < kLanes; ++i) t += part[(w * 64 + i * (4 * QG) + qq) * 2 + which];
       xchg_store(out + item, ((unsigned long long)(uint32_t)(l + 1) << 32) | __float_as_uint(t));
     }
   };
@@ -767,10 +772,10 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int nsteps = (ntok + 15) >> 4;
   const int rotations = (nsteps + NB - 1) / NB;
   const int rot_before_consume = min((RING - a.ring_stride) / (16 * NB), rotations);
-  auto score = [&](const StepData<DT, HD>& d, int l, int slot, int which) __attribute__((always_inline)) {
+  auto score = [&](const StepData<DT, HD, QG>& d, int l, int slot, int which) __attribute__((always_inline)) {
     if (slot < nsteps) compute_step(d, l, slot * 16, which);
   };
-  StepData<DT, HD> buf[NB];
+  StepData<DT, HD, QG> buf[NB];
   LayerBase base_cur = layer_base(l_begin), base_next = base_cur;
   // The two waves of a SIMD (waves i and i + 4 of a workgroup of eight) compete for its issue slots and
   // the arbiter prefers the older one: left alone, waves 0..3 of every workgroup run ahead, then wait at
@@ -815,8 +820,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       // A magnitude beyond fp16's range (or a key that is not finite) has left an infinity or a NaN
       // in this layer's sums.
       bool bad = false;
-#pragma unroll
-      for (int g = 0; g < QG; ++g) bad = bad || !(s2[g] < INFINITY);
+      bad = !(s2 < INFINITY);
       // The other end of fp16's range: below 2^-14 the first piece is a subnormal and below 2^-3 the
       // second one is, so magnitudes carry an absolute error of up to 2^-25 whatever their size.
       // Against keys of ordinary size that is nothing (scaled by 2^-10, magnitudes around 2^-9, the
@@ -862,7 +866,7 @@ struct LaunchShape {
 
 template <int TW, int SL, int QG, int W>
 constexpr size_t mfma_lds_bytes() {
-  return ((size_t)W * (TW + SL) * 4 * QG + W * 128 * QG + 128 * QG + 16) * 4;
+  return ((size_t)W * (TW + SL) * 4 * QG + W * 128 + 128 * QG + 16) * 4;
 }
 
 template <int DT, bool IL, int TW, int SL, int QG, int NB, int W = kFusedWaves, int HD = 128>
@@ -1183,7 +1187,6 @@ hipError_t launch_fused_mfma(const FusedLaunch& a, hipStream_t s) {
   const int64_t words = (int64_t)a.B * a.L * k.tiles_per_seq * a.A * 2;
   const bool il = a.rope_style == TRI_ROPE_INTERLEAVED;
   uint4* bmat = reinterpret_cast<uint4*>(a.bmat);
-  const int QG = a.G > 4 ? 2 : 1;
   const bool fp8 = a.kv_dtype == TRI_KV_FP8_E4M3;
   const bool fp16 = a.kv_dtype == TRI_KV_FP16;
   if (a.kv_dtype != TRI_KV_BF16 && !fp8 && !fp16) return hipErrorInvalidValue;
@@ -1198,7 +1201,7 @@ hipError_t launch_fused_mfma(const FusedLaunch& a, hipStream_t s) {
   auto prep_launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)a.L, (unsigned)a.B, (unsigned)ceil_div(a.Hkv, heads_per_wg)),
                        dim3(kPrepThreads), 0, s, a.folded, a.omega, a.offsets, a.NO, a.round_start, a.L, a.Hkv, a.G, a.A,
-                       QG, bmat, a.xchg, words, a.status, heads_per_wg);
+                       bmat, a.xchg, words, a.status, heads_per_wg);
   };
   if (fp8) {
     if (il) prep_launch(prep_mfma_kernel<TRI_KV_FP8_E4M3, true, 128>);
