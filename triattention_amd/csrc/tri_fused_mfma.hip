@@ -108,15 +108,32 @@ __device__ __forceinline__ void magnitudes4(const uint32_t (&x)[4], float* m) {
   }
 }
 
-// Two fp32 values -> packed fp16 and the fp32 remainders, the remainders by the
-// mixed-precision fused multiply-add, which reads the halves of the packed register as they
-// are (x - half is exact): four instructions per two values where a bf16 split needs six.
-__device__ __forceinline__ uint32_t split_pair_f16(float x0, float x1, float& r0, float& r1) {
-  const f32x2 x = {x0, x1};
-  const uint32_t packed = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, f16x2));
-  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(packed), "v"(x0));
-  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(packed), "v"(x1));
-  return packed;
+// Eight fp32 values as two packed fp16 pieces each.  The remainders x - hi are exact in fp32 and rounded to fp16 by
+// the same instruction (the mixed-precision fused multiply-add reads and writes halves of packed
+// registers): three instructions per two values, which used to be four (no case got measurably faster by it alone).  A half written by one instruction is read by the next but three at
+// the earliest: this chip wants one between.
+__device__ __forceinline__ void split8_f16(const float (&x)[8], uint4& hi, uint4& lo) {
+  uint32_t h[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x2 v = {x[2 * i], x[2 * i + 1]};
+    h[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2));
+  }
+  asm("v_fma_mixlo_f16 %0, %4, -1.0, %8 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixlo_f16 %1, %5, -1.0, %9 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixlo_f16 %2, %6, -1.0, %10 op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixlo_f16 %3, %7, -1.0, %11 op_sel_hi:[1,0,0]"
+      : "=&v"(l[0]), "=&v"(l[1]), "=&v"(l[2]), "=&v"(l[3])
+      : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(x[0]), "v"(x[2]), "v"(x[4]), "v"(x[6]));
+  asm("v_fma_mixhi_f16 %0, %4, -1.0, %8 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %1, %5, -1.0, %9 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %2, %6, -1.0, %10 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+      "v_fma_mixhi_f16 %3, %7, -1.0, %11 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+      "s_nop 0"
+      : "+&v"(l[0]), "+&v"(l[1]), "+&v"(l[2]), "+&v"(l[3])
+      : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(x[1]), "v"(x[3]), "v"(x[5]), "v"(x[7]));
+  hi = uint4{h[0], h[1], h[2], h[3]};
+  lo = uint4{l[0], l[1], l[2], l[3]};
 }
 
 // Larger halves of two packed fp16 pairs (no quieting of the operands, which costs an instruction each).
@@ -526,22 +543,13 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
         magnitudes4<DT>(x, &mag[4 * h]);
       }
       uint4 hi, lo;
-      float r[8];
       // The magnitudes are cut into two fp16 pieces (22 bits; two bf16 pieces would carry 16) and
       // go through the fp16 matrix-core instruction whatever the key type: the fp16 split is two
       // instructions per pair cheaper than the bf16 one.  Magnitudes of one-byte codes lie in
       // [2^-9, 634]; a two-byte key beyond fp16's range turns its scores into infinities or NaNs,
       // which the check after every layer finds (status word 2: the caller repeats the step on the
       // vector-unit kernels).
-      hi.x = split_pair_f16(mag[0], mag[1], r[0], r[1]);
-      hi.y = split_pair_f16(mag[2], mag[3], r[2], r[3]);
-      hi.z = split_pair_f16(mag[4], mag[5], r[4], r[5]);
-      hi.w = split_pair_f16(mag[6], mag[7], r[6], r[7]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const f32x2 x = {r[2 * i], r[2 * i + 1]};
-        (&lo.x)[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(x, f16x2));
-      }
+      split8_f16(mag, hi, lo);
       if constexpr (!FP8)   // `which` is the step buffer's number: a constant after unrolling
         mag_seen = pk_max_f16(mag_seen, (&hi.x)[which & 3]);
       constexpr int MT = TRI_KV_FP16;                // operand type of the magnitude MFMAs
@@ -637,14 +645,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
         // (8 x 32768 tokens x 64 layers, 64 query heads: 7.55 -> 6.82 ms).  With up to four query
         // heads the one wave's gather below hides behind the slack and this form is slower (16 x 16384
         // tokens x 36 layers: 3.29 -> 3.30 ms; fp8 keys 1.72 -> 1.80; 16 x 2176 tokens 0.54 -> 0.62).
-        float m8[8], s8[8];
-        gather_head_stats(a, b, l, seq_tiles, T, (chunk * 8 + wave) * a.G, a.G, m8, s8, lane, aborted);
-#pragma unroll
-        for (int qq = 0; qq < RQ; ++qq)
-          if (qq < a.G) {
-            mean[qq] = m8[qq];
-            sd[qq] = __fdiv_rn(1.f, s8[qq]);
-          }
+        gather_head_stats(a, b, l, seq_tiles, T, (chunk * 8 + wave) * a.G, a.G, mean, sd, lane, aborted);
       } else {
       uint32_t won = 0;
       if (lane == 0) {
@@ -676,15 +677,15 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       }
     }
     // The usual mode -- every query-head slot of the group in use, maximum over the group, running sum
-    // over layers, whole chunks of 64 tokens, not the first layer -- without the per-head predicates, the
+    // over layers, not the first layer -- without the per-head predicates, the
     // two reduction variants, the lane masks and the modulo per token of the general loop below: a third
-    // of its instructions.  The guards need no attention here: the first layer of a workgroup goes
+    // of its instructions.  (Lanes past the tile's last token take whatever the ring holds there into a sum that
+    // nobody reads.)  The guards need no attention here: the first layer of a workgroup goes
     // through the general loop, which sets the guarded tokens to +inf, and a finite contribution leaves
     // them there.  This piece of work sits on every wave's path once per layer (removed altogether, for
     // timing only, it is worth 3.4 % of the kernel on 16 x 16384 tokens x 36 layers, 4.2 % with eight
     // query heads per KV head).
-    if (a.G == RQ && a.group_reduce == TRI_REDUCE_MAX && a.layer_reduce == TRI_REDUCE_MEAN && l != l_begin &&
-        (ntok & 63) == 0) {
+    if (a.G == RQ && a.group_reduce == TRI_REDUCE_MAX && a.layer_reduce == TRI_REDUCE_MEAN && l != l_begin) {
       // This lane's entry of chunk 0 inside the wave's ring; chunk k lies 64 k entries further on, or
       // RING entries back once that passes the ring's end (one compare and one select per chunk, the
       // distance itself goes into the LDS instruction's offset field).
