@@ -1467,6 +1467,70 @@ def test_quarter_tile_scores_give_the_sums_of_whole_tiles(kw, lens):
         assert torch.equal(fin_a[b * h:(b + 1) * h, :t], fin_b[b * h:(b + 1) * h, :t]), (b, t)
 
 
+@pytest.mark.parametrize("lens", [(1,), (15, 128, 129), (2049,), (4096,), (4097, 16)])
+@pytest.mark.parametrize("kv_dtype,head_dim,heads,layers,rope", [
+    ("bf16", 128, (32, 8), 1, "half"), ("bf16", 128, (12, 4), 3, "interleaved"), ("fp16", 128, (8, 8), 4, "half"),
+    ("bf16", 64, (24, 3), 2, "half"), ("fp16", 64, (10, 5), 1, "interleaved"), ("bf16", 256, (4, 2), 2, "interleaved"),
+    ("fp16", 256, (14, 2), 1, "half")])
+def test_small_launches_match_the_two_pass_kernels(kv_dtype, head_dim, heads, layers, rope, lens, monkeypatch):
+    """A few layers of a few requests go through kernels of their own (a wave per step, statistics in the selection's
+    workgroups): selection scores and kept sets against the score-then-select kernels, and without
+    normalisation, where the raw scores show, to 5e-6 of the largest (two fp32 evaluations of one sum)."""
+    w = small(kv_dtype=kv_dtype, head_dim=head_dim, num_q_heads=heads[0], num_kv_heads=heads[1], num_layers=layers, rope_style=rope,
+              seq_lens=lens, budget=96, index=91)
+    print(f"small {w}", flush=True)
+    inp = build_inputs(w)
+    caches, kv, batch, sc = device_objects(w, inp, DEV, prefill_lens=[5] * len(lens))
+    h = w.num_kv_heads
+    for kw in (dict(), dict(normalize=False, layer_reduce="max"), dict(group_reduce="mean", protect_prefill=True)):
+        sel = ops.SelectConfig(window_size=w.window_size, **kw)
+        tune(resident_kernel="auto")
+        keep_s, fin_s, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
+        keep_only, _, _ = ops.select_paged(kv, batch, sc, sel)
+        tune(resident_kernel="off")
+        raw, ws2 = ops.score_paged(kv, batch, sc)
+        keep_t, fin_t = ops.select(kv, batch, sc, sel, raw, ws2, want_scores=True)
+        torch.cuda.synchronize()
+        assert ws.status() == 0
+        for b, t in enumerate(lens):
+            k = min(w.budget, t)
+            assert torch.equal(keep_only[b * h:(b + 1) * h, :k], keep_s[b * h:(b + 1) * h, :k])
+            a, c = fin_s[b * h:(b + 1) * h, :t].cpu(), fin_t[b * h:(b + 1) * h, :t].cpu()
+            assert torch.equal(torch.isinf(a), torch.isinf(c))
+            m = torch.isfinite(c)
+            scale = float(c[m].abs().max()) if bool(m.any()) else 1.0
+            tol = selection_score_tol(raw[b, :, :t].transpose(-1, -2).cpu()) if sel.normalize else 5e-6
+            assert float((a[m] - c[m]).abs().max() if bool(m.any()) else 0.0) <= tol * scale, (kw, b)
+            assert_keep_matches(keep_s[b * h:(b + 1) * h, :k].cpu().long(), keep_t[b * h:(b + 1) * h, :k].cpu().long(), c, k,
+                                tie_tol=2 * tol * scale)
+
+
+@pytest.mark.parametrize("kv_dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 6e4])
+def test_small_launches_carry_values_beyond_range_like_the_two_pass_kernels(kv_dtype, value, monkeypatch):
+    """One key element that is not finite, or as large as its type allows in magnitudes beyond half precision: the raw
+    scores keep their kind (finite, infinity and its sign, NaN) and no status is raised."""
+    w = small(kv_dtype=kv_dtype, num_q_heads=8, num_kv_heads=2, num_layers=1, seq_lens=(300,), budget=64, window_size=0, index=92)
+    inp = build_inputs(w)
+    for c in inp["caches"]:
+        c[0, inp["tables"][0][3], 5, 1, 7] = value
+    caches, kv, batch, sc = device_objects(w, inp, DEV)
+    sel = ops.SelectConfig(window_size=0, normalize=False)
+    print(f"beyond range {kv_dtype} {value}", flush=True)
+    _, a, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
+    tune(resident_kernel="off")
+    raw, ws2 = ops.score_paged(kv, batch, sc)
+    _, c = ops.select(kv, batch, sc, sel, raw, ws2, want_scores=True)
+    torch.cuda.synchronize()
+    assert ws.status() == 0
+    a, c = a[:, :300].cpu(), c[:, :300].cpu()
+    assert torch.equal(torch.isnan(a), torch.isnan(c)) and torch.equal(torch.isinf(a), torch.isinf(c))
+    inf = torch.isinf(c)
+    assert torch.equal(a[inf], c[inf])
+    m = torch.isfinite(c)
+    assert float(((a[m] - c[m]).abs() / c[m].abs().clamp_min(1.0)).max()) <= 2e-5
+
+
 def test_fp8_every_code_decodes_like_torch():
     """All 254 finite e4m3 codes through the scorer: with one non-zero coefficient the
     score is code_value * scale * coefficient, which pins the decoder against torch's

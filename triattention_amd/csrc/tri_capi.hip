@@ -281,11 +281,48 @@ bool takes_quarter_tiles(const tri_kv_layout* kv, int B, int Tmax, int A, int ag
                                                Tmax, aggregation);
 }
 
+// A few layers of a few requests, where the resident kernel would be taken for them, go through
+// tri_score_small.hip: a wave per step of 16 tokens, statistics in the selection's workgroups.  Score + select, us, resident
+// / small, by workgroups (128 tokens of a KV head of a layer), four query heads per KV head of 128: 1 layer x 4096
+// tokens (256) 32.1 / 17.5, x 8192 (512) 36.6 / 23.2, 3 x 4096 (768) 32.3 / 22.0, 2 layers x 8192 (1024) 37.8 / 34.5, 3 x 4096 (768)
+// 33.7 / 26.9; beyond 1024 workgroups every one of them evaluates the phases again for too little.  With eight query heads
+// the selection walks a layer in 5 us: 1 layer, 3 x 4096 (768) 25.8 / 23.1, 2 layers x 4096 (512) 26.9 / 23.3, but
+// 2 layers, 3 x 4096 of four KV heads (768) 27.4 / 31.1 and 3 x 4096 (768) 27.0 / 30.9.
+constexpr int64_t kSmallWorkgroups = 1024;
+bool takes_small(const tri::Workspace& w, const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
+                 const tri_select_params* sel) {
+  const int G = sp->num_score_heads / kv->num_kv_heads, L = kv->num_layers;
+  const int64_t wgs = (int64_t)batch->num_seqs * L * kv->num_kv_heads * tri::ceil_div(batch->max_seq_len, 128);
+  return tri::tuning(TRI_TUNE_RESIDENT_KERNEL) == 0 && takes_resident(w, kv, sel) && w.fused.eligible == 2 &&
+         kv->kv_dtype != TRI_KV_FP8_E4M3 && tri::select_small_takes(batch->max_seq_len, G) &&
+         (int64_t)batch->num_seqs * kv->num_kv_heads <= 256 &&
+         (G > 4 ? L <= 2 && wgs * L <= kSmallWorkgroups : L <= 4 && wgs <= kSmallWorkgroups);
+}
+
 // Selection straight from the paged keys: the resident kernel when the shape has one,
 // else score into the workspace and select from there.
 int do_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
                     const tri_select_params* sel, float* fin, int32_t* keep, void* ws, const tri::Workspace& w,
                     hipStream_t s, int pass_nan = 0) {
+  if (takes_small(w, kv, batch, sp, sel)) {
+    tri::SmallScore c{};
+    c.k_layers = kv->k_layers; c.block_table = batch->block_table; c.block_table_pitch = batch->block_table_pitch;
+    c.seq_lens = batch->seq_lens; c.round_start = batch->round_start;
+    c.folded = sp->folded; c.omega = sp->omega; c.offsets = sp->offsets; c.NO = sp->num_offsets;
+    c.raw = at<float>(ws, w.raw); c.raw_pitch = batch->max_seq_len; c.status = at<uint32_t>(ws, w.status);
+    c.stride_block = kv->stride_block; c.stride_token = kv->stride_token; c.stride_head = kv->stride_head;
+    c.L = kv->num_layers; c.A = sp->num_score_heads; c.G = sp->num_score_heads / kv->num_kv_heads;
+    c.Tmax = batch->max_seq_len; c.block_size = kv->block_size;
+    hipError_t e = tri::launch_score_small(c, batch->num_seqs, kv->num_kv_heads, kv->head_dim, kv->kv_dtype, kv->rope_style, s);
+    if (e != hipSuccess) return launch_status(e, "score_small");
+    tri::SmallSelect a{};
+    a.raw = c.raw; a.raw_pitch = c.raw_pitch; a.seq_lens = batch->seq_lens; a.prefill_lens = batch->prefill_lens;
+    a.budgets = batch->budgets; a.fin = fin; a.keep = keep; a.keep_pitch = batch->max_budget; a.status = c.status;
+    a.L = c.L; a.Hkv = kv->num_kv_heads; a.A = c.A; a.G = c.G; a.Tmax = c.Tmax;
+    a.normalize = sel->normalize; a.window_size = sel->window_size; a.protect_prefill = sel->protect_prefill;
+    a.group_reduce = sel->group_reduce; a.layer_reduce = layer_reduce_of(kv, sel); a.pass_nan = 0;
+    return launch_status(tri::launch_select_small(a, batch->num_seqs, s), "select_small");
+  }
   const bool fused = takes_resident(w, kv, sel);
   if (!fused) {
     float* raw = at<float>(ws, w.raw);
@@ -595,6 +632,11 @@ int tri_topk_rows(const float* scores, int64_t row_pitch, int32_t num_rows, cons
 
 namespace {
 
+// Workgroups of 128 tokens and a head up to which a dense call goes through the small launch's kernels (8 heads: 600 tokens
+// 44.5 -> 31.9 us, 4096 45.0 -> 32.0, 12000 60.3 -> 35.5, 16384 53.8 -> 39.0, of 256 elements 73.2 -> 52.9; longer rows
+// do not fit the selection's registers).
+constexpr int64_t kDenseSmallWorkgroups = 2048;
+
 // A dense call as the general layout, batch and parameters, on a workspace whose last part holds what those
 // point to.
 struct DensePlan {
@@ -680,10 +722,32 @@ int tri_dense_compress(const tri_dense_params* p, void* ws, uint64_t ws_bytes, v
   l.folded = at<float>(ws, d.folded); l.arg_key = at<const void*>(ws, d.arg_key); l.arg_words = words;
   l.keep32 = at<int32_t>(ws, d.keep32);
   hipStream_t s = (hipStream_t)stream;
-  rc = launch_status(tri::launch_dense_prologue(l, s), "dense prologue");
-  if (rc) return rc;
   // (NaN scores stay NaN, the largest of a row or, with the sign set, the smallest: torch's normalisation and
   // tri_topk_rows, which this call stands for, treat them so)
+  if (p->aggregation == TRI_REDUCE_MEAN && tri::select_small_takes(p->num_tokens, 1) &&
+      (int64_t)p->num_heads * tri::ceil_div(p->num_tokens, 128) <= kDenseSmallWorkgroups) {
+    // Three launches: the scorer takes the call's arguments by value and folds the statistics itself.
+    tri::SmallScore c{};
+    c.k = p->k; c.round = p->round_start;
+    c.q_mean = p->q_mean_complex; c.q_abs = p->q_abs_mean; c.freq_scale = p->freq_scale_sq;
+    c.disable_mlr = p->disable_mlr; c.disable_trig = p->disable_trig;
+    c.omega = p->omega; c.offsets = p->offsets; c.NO = p->num_offsets;
+    c.raw = at<float>(ws, d.w.raw); c.raw_pitch = p->num_tokens;
+    c.stride_token = d.kv.stride_token; c.stride_head = d.kv.stride_head;
+    c.L = 1; c.A = p->num_heads; c.G = 1; c.Tmax = p->num_tokens; c.block_size = p->num_tokens;
+    rc = launch_status(tri::launch_score_small(c, 1, p->num_heads, p->head_dim, p->kv_dtype, p->rope_style, s), "score_small");
+    if (rc) return rc;
+    tri::SmallSelect a{};
+    a.raw = c.raw; a.raw_pitch = c.raw_pitch; a.keep = at<int32_t>(ws, d.keep32); a.keep_pitch = p->budget;
+    a.L = 1; a.Hkv = p->num_heads; a.A = p->num_heads; a.G = 1; a.Tmax = p->num_tokens;
+    a.normalize = d.sel.normalize; a.window_size = d.sel.window_size;
+    a.group_reduce = TRI_REDUCE_MAX; a.layer_reduce = TRI_REDUCE_MEAN; a.pass_nan = 1;
+    rc = launch_status(tri::launch_select_small(a, 1, s), "select_small");
+    if (rc) return rc;
+    return launch_status(tri::launch_dense_gather(l, s), "dense gather");
+  }
+  rc = launch_status(tri::launch_dense_prologue(l, s), "dense prologue");
+  if (rc) return rc;
   rc = do_select_paged(&d.kv, &d.batch, &d.sp, &d.sel, nullptr, at<int32_t>(ws, d.keep32), ws, d.w, s, 1);
   if (rc) return rc;
   return launch_status(tri::launch_dense_gather(l, s), "dense gather");

@@ -122,6 +122,41 @@ hipError_t launch_prepare(const float* folded, const float* omega, const float* 
 bool score_takes_fine(int B, int L, int Hkv, int D, int G, int Tmax, int aggregation);
 hipError_t launch_score(const ScoreLaunch& a, hipStream_t s);
 
+// Scores of a small launch (tri_score_small.hip): raw[(b * L + l) * A + score head][raw_pitch].
+struct SmallScore {
+  const void* const* k_layers;   // or NULL: one layer at k
+  const void* k;
+  const int32_t* block_table;    // or NULL: dense, physical block = sequence
+  const int32_t* seq_lens;       // or NULL: Tmax
+  const int32_t* round_start;    // or NULL: round
+  const float* folded;           // [L][A][3][F], or NULL: folded from the next three
+  const float* q_mean; const float* q_abs; const float* freq_scale;   // [A][F][2], [A][F], [A][F]
+  const float* omega;
+  const float* offsets;
+  float* raw;
+  uint32_t* status;              // cleared, or NULL
+  int64_t stride_block, stride_token, stride_head, raw_pitch;
+  int L, A, G, NO, Tmax, round, block_size, bs_shift, block_table_pitch, disable_mlr, disable_trig;
+};
+hipError_t launch_score_small(SmallScore a, int B, int Hkv, int D, int kv_dtype, int rope_style, hipStream_t s);
+
+// Statistics, reduction and top-k of what that one leaves (tri_select.hip), a workgroup per (sequence, KV head).
+struct SmallSelect {
+  const float* raw;
+  const int32_t* seq_lens;       // or NULL: Tmax
+  const int32_t* prefill_lens;
+  const int32_t* budgets;        // or NULL: keep_pitch
+  float* fin;                    // [B * Hkv][Tmax], or NULL
+  int32_t* keep;                 // or NULL
+  uint32_t* status;              // 3: a sequence is longer than Tmax (as the resident kernels say it); or NULL
+  int64_t raw_pitch;
+  int L, Hkv, A, G, Tmax, keep_pitch;
+  int normalize, window_size, protect_prefill, group_reduce, layer_reduce, pass_nan;
+};
+hipError_t launch_select_small(const SmallSelect& a, int B, hipStream_t s);
+// Its limits: the row of a KV head in registers.
+bool select_small_takes(int Tmax, int G);
+
 struct SelectLaunch {
   int B, L, Hkv, A, G, Tmax, fine, max_budget;
   int normalize, window_size, protect_prefill, group_reduce, layer_reduce, shared, group_first;

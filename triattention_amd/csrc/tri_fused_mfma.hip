@@ -25,18 +25,12 @@
 #include <vector>
 
 #include "tri_common.h"
+#include "tri_mma_device.h"
 #include "tri_score_device.h"
 #include "tri_fused_device.h"
 
 namespace tri {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kDppRor4 = 0x124;   // row_ror:4
 constexpr int kDppRor8m = 0x128;  // row_ror:8
@@ -59,8 +53,6 @@ __host__ __device__ constexpr int slab_elem(int s, int kb, int e) {
   return DT == TRI_KV_FP8_E4M3 ? (kb + 4 * (s >> 1)) * 16 + (s & 1) * 8 + e : (4 * s + kb) * 8 + e;
 }
 
-__device__ __forceinline__ bf16x8 as_bf16x8(const uint4& v) { return __builtin_bit_cast(bf16x8, v); }
-
 // Largest of three (the instruction returns the other operands' maximum when one is a NaN, as
 // fmaxf does; written out because the compiler canonicalises every operand of fmaxf first).
 __device__ __forceinline__ float max3(float a, float b, float c) {
@@ -71,42 +63,6 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 
 __device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-
-// m[i] = sqrt(x[i].lo^2 + x[i].hi^2) for four packed bf16 pairs, in fp32.  Written out for
-// two reasons: the compiler only selects the accumulating two-operand dot product
-// (v_dot2c_f32_bf16) and spends a v_mov per value on zeroing its destination, and it does
-// not see the opcodes inside an asm statement, so the spacing gfx950 requires between a dot
-// product's write and another vector instruction's read of that register (three
-// instructions) and after a transcendental's write (one) is provided here: four dot
-// products, then the four square roots in the same order, then one idle cycle.
-template <int DT>
-__device__ __forceinline__ void magnitudes4(const uint32_t (&x)[4], float* m) {
-  if constexpr (DT == TRI_KV_FP16) {
-    asm("v_dot2_f32_f16 %0, %4, %4, 0\n\t"
-        "v_dot2_f32_f16 %1, %5, %5, 0\n\t"
-        "v_dot2_f32_f16 %2, %6, %6, 0\n\t"
-        "v_dot2_f32_f16 %3, %7, %7, 0\n\t"
-        "v_sqrt_f32 %0, %0\n\t"
-        "v_sqrt_f32 %1, %1\n\t"
-        "v_sqrt_f32 %2, %2\n\t"
-        "v_sqrt_f32 %3, %3\n\t"
-        "s_nop 0"
-        : "=&v"(m[0]), "=&v"(m[1]), "=&v"(m[2]), "=&v"(m[3])
-        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
-  } else {
-    asm("v_dot2_f32_bf16 %0, %4, %4, 0\n\t"
-        "v_dot2_f32_bf16 %1, %5, %5, 0\n\t"
-        "v_dot2_f32_bf16 %2, %6, %6, 0\n\t"
-        "v_dot2_f32_bf16 %3, %7, %7, 0\n\t"
-        "v_sqrt_f32 %0, %0\n\t"
-        "v_sqrt_f32 %1, %1\n\t"
-        "v_sqrt_f32 %2, %2\n\t"
-        "v_sqrt_f32 %3, %3\n\t"
-        "s_nop 0"
-        : "=&v"(m[0]), "=&v"(m[1]), "=&v"(m[2]), "=&v"(m[3])
-        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]));
-  }
-}
 
 // Eight fp32 values as two packed fp16 pieces each.  The remainders x - hi are exact in fp32 and rounded to fp16 by
 // the same instruction (the mixed-precision fused multiply-add reads and writes halves of packed
@@ -140,15 +96,6 @@ __device__ __forceinline__ void split8_f16(const float (&x)[8], uint4& hi, uint4
 __device__ __forceinline__ f16x2 pk_max_f16(f16x2 a, uint32_t b) {
   asm("v_pk_max_f16 %0, %0, %1" : "+v"(a) : "v"(b));
   return a;
-}
-
-// One 16x16x32 matrix-core step in the operand type of the keys (fp8 keys are converted to bf16).
-template <int DT>
-__device__ __forceinline__ f32x4 mfma_step(const uint4& a, const uint4& b, f32x4 c) {
-  if constexpr (DT == TRI_KV_FP16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
 }
 
 // Piece `pieces` of x in the operand type: what is left of x after `pieces` roundings.
@@ -518,7 +465,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     for (int s = 0; s < NS; ++s) d.c[s] = uint4{w[s][0], w[s][1], w[s][2], w[s][3]};
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int o = 0; o < NK; ++o) acc = mfma_step<DT>(d.c[o % NS], B[o], acc);
+    for (int o = 0; o < NK; ++o) acc = mfma_16x16x32<DT>(d.c[o % NS], B[o], acc);
 #pragma unroll
     for (int set = 0; set < NS / 2; ++set) {
       // |k_f|^2 = k_r^2 + k_i^2 straight from the bf16 pairs (v_dot2_f32_bf16).
@@ -553,8 +500,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       if constexpr (!FP8)   // `which` is the step buffer's number: a constant after unrolling
         mag_seen = pk_max_f16(mag_seen, (&hi.x)[which & 3]);
       constexpr int MT = TRI_KV_FP16;                // operand type of the magnitude MFMAs
-      acc = mfma_step<MT>(hi, B[NK + set], acc);
-      acc = mfma_step<MT>(lo, B[NK + set], acc);
+      acc = mfma_16x16x32<MT>(hi, B[NK + set], acc);
+      acc = mfma_16x16x32<MT>(lo, B[NK + set], acc);
     }
     // The pieces of a head are added across the columns; v[i] is then the score of this lane's i-th token.
     float v[QG];

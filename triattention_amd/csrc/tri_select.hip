@@ -14,6 +14,8 @@
 //                          an ordered compaction that emits the kept token indices ascending;
 //                          ties at the threshold keep the lowest index (replaces torch.topk + chunk merge +
 //                          torch.sort, runtime/selector_hf.py:990-1025).
+#include <type_traits>
+
 #include "tri_common.h"
 
 namespace tri {
@@ -568,76 +570,19 @@ constexpr int kTopkCand = 128;                   // candidates ranked by countin
 // 6.6 / 6.2 (12.5), 288 rows of 2176 7.7 / 9.2 (15.8: two workgroups a CU, 64 registers a thread), 128 rows of 16384
 // 11.3 / 13.5, 8 rows of 32768 19.4 / 23.2 (there the instructions of one CU bound it).  Ranking up to 1024
 // candidates took 30 us at 750, radix passes behind the first histogram 57 and 106 with an outlier.
+// Key 0 is "no element" (the one NaN pattern whose key it would be shares the next key), so the selection
+// never asks for an element's place in the row again.
+__device__ __forceinline__ uint32_t row_key(float f) { return max(float_key(f), 1u); }
+
 template <int VPT>
-__global__ __launch_bounds__(kTopkThreads, VPT <= 4 ? 8 : 4) void topk_rows_reg_kernel(const float* scores, int64_t row_pitch,
-                                                                    const int32_t* row_lens,
-                                                                    const int32_t* row_ks, int rows_per_entry,
-                                                                    int32_t* keep, int keep_pitch, int max_len,
-                                                                    int groups, int64_t group_stride, int group_max) {
+__device__ __forceinline__ void emit_topk(const uint32_t (&key)[VPT], int T, int k, int32_t* out) {
   constexpr int kWaves = kTopkThreads / 64;
   __shared__ uint32_t hist[kTopkBins];
   __shared__ __align__(16) uint32_t cand[kTopkCand];
   __shared__ uint32_t wave_lo[kWaves], wave_hi[kWaves], wave_tot[kWaves];
   __shared__ uint32_t sh_high, sh_ncand, sh_prefix, sh_remaining, sh_count;
-
-  const int row = blockIdx.x;
-  const int entry = row / rows_per_entry;
-  // Lengths and budgets live on the device; the host sized rows for max_len scores and
-  // keep_pitch indices, and neither is ever exceeded whatever the device arrays say.
-  const int T = min(row_lens[entry], max_len);
-  int k = min(row_ks[entry], keep_pitch);
-  if (k > T) k = T;
-  if (k <= 0 || T <= 0) return;
-  const float* x = scores + (int64_t)row * row_pitch;
-  int32_t* out = keep + (int64_t)row * keep_pitch;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-
-  if (k >= T) {
-    for (int i = tid; i < T; i += kTopkThreads) out[i] = i;
-    return;
-  }
-
   const int e0 = wave * (64 * VPT) + lane;        // element i of this thread: e0 + 64 * i
-  const int nvalid = min(max((T - e0 + 63) / 64, 0), VPT);
-  // Key 0 is "no element" (the one NaN pattern whose key it would be shares the next key), so nothing below
-  // asks for an element's place in the row again.
-  auto row_key = [](float f) __attribute__((always_inline)) { return max(float_key(f), 1u); };
-  uint32_t key[VPT];
-  if (groups > 1) {
-    // The row arrives as `groups` partial rows `group_stride` floats apart (a resident launch cut
-    // by layers): they are added (or maximised) in group order, exactly as
-    // fused_layer_reduce_kernel does; the division by the layer count that turns the sum into a
-    // mean does not change the order of the scores and is left out.
-    // The rows of several groups are requested before the first is added (a thread's loads of one
-    // group after the other, each waited for, made 36 groups of a single request take 30 us); the last
-    // round repeats the last group where there is none left and leaves it out of the sum.
-    constexpr int U = VPT >= 32 ? 1 : (VPT >= 16 ? 3 : (VPT >= 8 ? 6 : 12));   // groups in flight per round
-    auto load_row = [&](int g, float (&y)[VPT]) __attribute__((always_inline)) {
-      const float* p = x + (int64_t)g * group_stride;
-#pragma unroll
-      for (int i = 0; i < VPT; ++i) y[i] = p[min(e0 + 64 * i, T - 1)];
-    };
-    float v[VPT];
-    load_row(0, v);
-    for (int g = 1; g < groups; g += U) {
-      float y[U][VPT];
-#pragma unroll
-      for (int u = 0; u < U; ++u) load_row(min(g + u, groups - 1), y[u]);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (g + u >= groups) continue;
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) v[i] = group_max ? fmaxf(v[i], y[u][i]) : __fadd_rn(v[i], y[u][i]);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) key[i] = i < nvalid ? row_key(v[i]) : 0u;
-  } else {
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) key[i] = __float_as_uint(x[min(e0 + 64 * i, T - 1)]);
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) key[i] = i < nvalid ? row_key(__uint_as_float(key[i])) : 0u;
-  }
 
   // ---- range of the finite scores, number of scores at or above +inf.
   uint32_t lo_key = 0xffffffffu, hi_key = 0u;
@@ -849,7 +794,241 @@ __global__ __launch_bounds__(kTopkThreads, VPT <= 4 ? 8 : 4) void topk_rows_reg_
   }
 }
 
+template <int VPT>
+__global__ __launch_bounds__(kTopkThreads, VPT <= 4 ? 8 : 4) void topk_rows_reg_kernel(const float* scores, int64_t row_pitch,
+                                                                    const int32_t* row_lens,
+                                                                    const int32_t* row_ks, int rows_per_entry,
+                                                                    int32_t* keep, int keep_pitch, int max_len,
+                                                                    int groups, int64_t group_stride, int group_max) {
+  const int row = blockIdx.x;
+  const int entry = row / rows_per_entry;
+  // Lengths and budgets live on the device; the host sized rows for max_len scores and
+  // keep_pitch indices, and neither is ever exceeded whatever the device arrays say.
+  const int T = min(row_lens[entry], max_len);
+  int k = min(row_ks[entry], keep_pitch);
+  if (k > T) k = T;
+  if (k <= 0 || T <= 0) return;
+  const float* x = scores + (int64_t)row * row_pitch;
+  int32_t* out = keep + (int64_t)row * keep_pitch;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+
+  if (k >= T) {
+    for (int i = tid; i < T; i += kTopkThreads) out[i] = i;
+    return;
+  }
+
+  const int e0 = wave * (64 * VPT) + lane;        // element i of this thread: e0 + 64 * i
+  const int nvalid = min(max((T - e0 + 63) / 64, 0), VPT);
+  uint32_t key[VPT];
+  if (groups > 1) {
+    // The row arrives as `groups` partial rows `group_stride` floats apart (a resident launch cut
+    // by layers): they are added (or maximised) in group order, exactly as
+    // fused_layer_reduce_kernel does; the division by the layer count that turns the sum into a
+    // mean does not change the order of the scores and is left out.
+    // The rows of several groups are requested before the first is added (a thread's loads of one
+    // group after the other, each waited for, made 36 groups of a single request take 30 us); the last
+    // round repeats the last group where there is none left and leaves it out of the sum.
+    constexpr int U = VPT >= 32 ? 1 : (VPT >= 16 ? 3 : (VPT >= 8 ? 6 : 12));   // groups in flight per round
+    auto load_row = [&](int g, float (&y)[VPT]) __attribute__((always_inline)) {
+      const float* p = x + (int64_t)g * group_stride;
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) y[i] = p[min(e0 + 64 * i, T - 1)];
+    };
+    float v[VPT];
+    load_row(0, v);
+    for (int g = 1; g < groups; g += U) {
+      float y[U][VPT];
+#pragma unroll
+      for (int u = 0; u < U; ++u) load_row(min(g + u, groups - 1), y[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (g + u >= groups) continue;
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) v[i] = group_max ? fmaxf(v[i], y[u][i]) : __fadd_rn(v[i], y[u][i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) key[i] = i < nvalid ? row_key(v[i]) : 0u;
+  } else {
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) key[i] = __float_as_uint(x[min(e0 + 64 * i, T - 1)]);
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) key[i] = i < nvalid ? row_key(__uint_as_float(key[i])) : 0u;
+  }
+  emit_topk<VPT>(key, T, k, out);
+}
+
+// ---- a small launch: statistics, reduction and top-k of the raw scores of one (sequence, KV head) in one workgroup.
+// Sum over the 16 lanes of a row (every lane gets it).
+template <int N>
+__device__ __forceinline__ double row_rotate_f64(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, ((uint64_t)row_rotate<N>((uint32_t)(u >> 32)) << 32) | row_rotate<N>((uint32_t)u));
+}
+__device__ __forceinline__ double row_sum_f64(double v) {
+  v += row_rotate_f64<8>(v);
+  v += row_rotate_f64<4>(v);
+  v += row_rotate_f64<2>(v);
+  return v + row_rotate_f64<1>(v);
+}
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane) << 32) |
+                                        (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane));
+}
+
+__device__ __forceinline__ float row_sum_f32(float v) {
+  v += __uint_as_float(row_rotate<8>(__float_as_uint(v)));
+  v += __uint_as_float(row_rotate<4>(__float_as_uint(v)));
+  v += __uint_as_float(row_rotate<2>(__float_as_uint(v)));
+  return v + __uint_as_float(row_rotate<1>(__float_as_uint(v)));
+}
+
+// The statistics need the whole row, the row is a few thousand scores of a few query heads and the top-k
+// holds it in registers anyway: one launch in place of finalize_stats_kernel (or group_stats_kernel) and
+// combine_kernel, each 4 to 8 us in front of a 6 us top-k for a microsecond's worth of bytes.  Sixteen waves share a
+// CU, so what every wave does counts four times: sums of 64 scores by rows of lanes (fp32, as many as a resident tile's
+// lane adds up; in double where the reduce-first order has them so), the 64 partial sums of a head in double and its
+// statistics in one wave per head.
+// GQ: query heads of a KV head, rounded up to 1, 4 or 8.
+template <int VPT, int GQ>
+__global__ __launch_bounds__(kTopkThreads, 4) void select_small_kernel(SmallSelect a) {
+  constexpr int kWaves = kTopkThreads / 64, NV = 2 * GQ;
+  typedef typename std::conditional<GQ == 1, double, float>::type Sum;
+  __shared__ Sum red[NV][kWaves * 4];
+  __shared__ float2 stats[GQ];               // mean, standard deviation (GQ == 1) or its reciprocal
+  const int row = blockIdx.x, b = row / a.Hkv, h = row % a.Hkv;
+  const int T = a.seq_lens ? min(a.seq_lens[b], a.Tmax) : a.Tmax;
+  if (a.status && a.seq_lens && threadIdx.x == 0 && h == 0 && a.seq_lens[b] > a.Tmax) atomicCAS(a.status, 0u, 3u);
+  if (T <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int e0 = wave * (64 * VPT) + lane;
+  const int nvalid = min(max((T - e0 + 63) / 64, 0), VPT);
+  const int prefill = (a.protect_prefill && a.prefill_lens) ? a.prefill_lens[b] : 0;
+  const int window_from = a.window_size > 0 ? T - min(a.window_size, T) : T;
+  float acc[VPT];
+  for (int l = 0; l < a.L; ++l) {
+    float x[GQ][VPT];
+#pragma unroll
+    for (int g = 0; g < GQ; ++g) {
+      const float* p = a.raw + ((int64_t)(b * a.L + l) * a.A + (int64_t)h * a.G + min(g, a.G - 1)) * a.raw_pitch;
+#pragma unroll
+      for (int i = 0; i < VPT; ++i) x[g][i] = p[min(e0 + 64 * i, T - 1)];
+    }
+    float mean[GQ], sd[GQ];
+#pragma unroll
+    for (int g = 0; g < GQ; ++g) { mean[g] = 0.f; sd[g] = 1.f; }
+    if (a.normalize) {
+#pragma unroll
+      for (int g = 0; g < GQ; ++g) {
+        Sum s = 0, q = 0;
+#pragma unroll
+        for (int i = 0; i < VPT; ++i) {
+          const Sum v = i < nvalid ? (Sum)x[g][i] : (Sum)0;
+          s += v;
+          q = fma(v, v, q);
+        }
+        if constexpr (GQ == 1) { s = row_sum_f64(s); q = row_sum_f64(q); }
+        else { s = row_sum_f32(s); q = row_sum_f32(q); }
+        if ((lane & 15) == 0) {
+          red[2 * g][wave * 4 + (lane >> 4)] = s;
+          red[2 * g + 1][wave * 4 + (lane >> 4)] = q;
+        }
+      }
+      __syncthreads();
+      if (wave < GQ) {
+        double s = row_sum_f64((double)red[2 * wave][lane]), q = row_sum_f64((double)red[2 * wave + 1][lane]);
+        s = ((lane_f64(s, 0) + lane_f64(s, 16)) + lane_f64(s, 32)) + lane_f64(s, 48);
+        q = ((lane_f64(q, 0) + lane_f64(q, 16)) + lane_f64(q, 32)) + lane_f64(q, 48);
+        float m, e;
+        if (a.pass_nan) {                    // (the reduce-first definitions, group_stats_kernel)
+          const double mu = s / (double)T;
+          double var = T > 1 ? (q - (double)T * mu * mu) / (double)(T - 1) : 0.0;
+          if (var < 0.0) var = 0.0;
+          e = (float)sqrt(var);
+          if (e < 1e-8f) e = 1.f;
+          m = (float)mu;
+        } else if (a.normalize == 2) {
+          const double mu = s / (double)T;
+          const double var = q / (double)T - mu * mu;
+          m = (float)mu;
+          e = fmaxf((float)sqrt(var > 0.0 ? var : 0.0), 1e-6f);
+        } else {                             // the reference's formula on fp32 sums (runtime/selector_hf.py:902-909)
+          const float sum = (float)s, sumsq = (float)q, cnt = (float)T;
+          m = __fdiv_rn(sum, cnt);
+          float var = 0.f;
+          if (T > 1) var = __fdiv_rn(__fsub_rn(sumsq, __fmul_rn(cnt, __fmul_rn(m, m))), (float)(T - 1));
+          var = fmaxf(var, 0.f);
+          e = __fsqrt_rn(var);
+          if (e < 1e-8f) e = 1.f;
+        }
+        if (lane == 0) stats[wave] = float2{m, GQ == 1 ? e : __fdiv_rn(1.f, e)};
+      }
+      __syncthreads();
+#pragma unroll
+      for (int g = 0; g < GQ; ++g) { mean[g] = stats[g].x; sd[g] = stats[g].y; }
+    }
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      float v;
+      if constexpr (GQ == 1) {
+        v = a.pass_nan ? passed_zscore(x[0][i], mean[0], sd[0]) : zscore(x[0][i], mean[0], sd[0]);
+      } else {
+        // (times the reciprocal, as the resident kernels do it: a division is ten instructions)
+        v = __fmul_rn(__fsub_rn(x[0][i], mean[0]), sd[0]);
+#pragma unroll
+        for (int g = 1; g < GQ; ++g)
+          if (g < a.G) {
+            const float z = __fmul_rn(__fsub_rn(x[g][i], mean[g]), sd[g]);
+            v = (a.group_reduce == TRI_REDUCE_MAX) ? fmaxf(v, z) : __fadd_rn(v, z);
+          }
+        if (a.group_reduce != TRI_REDUCE_MAX) v = __fdiv_rn(v, (float)a.G);
+      }
+      const int n = e0 + 64 * i;
+      if (n >= window_from || n < prefill) v = INFINITY;
+      if (l == 0) acc[i] = v;
+      else acc[i] = (a.layer_reduce == TRI_REDUCE_MAX) ? fmaxf(acc[i], v) : __fadd_rn(acc[i], v);
+    }
+  }
+  uint32_t key[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    if (a.layer_reduce == TRI_REDUCE_MEAN) acc[i] = __fdiv_rn(acc[i], (float)a.L);
+    if (a.fin && i < nvalid) a.fin[(int64_t)row * a.Tmax + e0 + 64 * i] = acc[i];
+    key[i] = i < nvalid ? row_key(acc[i]) : 0u;
+  }
+  if (!a.keep) return;
+  const int k = min(min(a.budgets ? a.budgets[b] : a.keep_pitch, a.keep_pitch), T);
+  int32_t* keep = a.keep + (int64_t)row * a.keep_pitch;
+  if (k <= 0) return;
+  if (k >= T) {
+    for (int i = tid; i < T; i += kTopkThreads) keep[i] = i;
+    return;
+  }
+  emit_topk<VPT>(key, T, k, keep);
+}
+
 }  // namespace
+
+bool select_small_takes(int Tmax, int G) {
+  return G <= 8 && Tmax <= (G == 1 ? 16 : G <= 4 ? 8 : 4) * kTopkThreads;    // (registers)
+}
+
+hipError_t launch_select_small(const SmallSelect& a, int B, hipStream_t s) {
+  if (!select_small_takes(a.Tmax, a.G) || (a.pass_nan && a.G != 1)) return hipErrorInvalidValue;
+  auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3((unsigned)(B * a.Hkv)), dim3(kTopkThreads), 0, s, a); };
+  const int per = ceil_div(a.Tmax, kTopkThreads);
+  if (a.G > 4) {
+    launch(select_small_kernel<4, 8>);
+  } else if (a.G > 1) {
+    if (per <= 4) launch(select_small_kernel<4, 4>); else launch(select_small_kernel<8, 4>);
+  } else {
+    if (per <= 4) launch(select_small_kernel<4, 1>);
+    else if (per <= 8) launch(select_small_kernel<8, 1>);
+    else launch(select_small_kernel<16, 1>);
+  }
+  return hipGetLastError();
+}
 
 hipError_t launch_topk_rows(const float* scores, int64_t row_pitch, int num_rows,
                             const int32_t* row_lens, const int32_t* row_ks, int rows_per_entry, int max_len,
