@@ -116,7 +116,8 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs a) {
   if (guard_raised(a.guard)) return;
 
   int idx = blockIdx.x;
-  const int col = idx % a.cols; idx /= a.cols;
+  const int chains = gridDim.x / a.cols;
+  const int col = idx / chains; idx %= chains;
   const int head = idx % a.Hkv;
   const Unit unit = unit_of(a, idx / a.Hkv);
   const int kv = unit.kv, l = unit.l, b = unit.b;
@@ -600,13 +601,19 @@ hipError_t launch_compact(const CompactLaunch& a, hipStream_t s) {
   if (takes_one_launch(a, chains, forked)) {
     // The longer the fewer chains there are: up to 256 a tile of 128 KB (one layer x 4096 tokens 9.9 / 19.1 us, called over
     // and over on one cache; 14.3 behind the scorer of a step, the rows not in L2; 16
-    // layers 43.1 / 54.1; up to 128 chains two workgroups take half of every row each, 8 layers
+    // layers 43.1 / 54.1; up to 128 chains several workgroups share every row, 8 layers
     // 24.3 / 37.1), up to 1024 chains 32 KB (36 layers x 2176 tokens 120.6 / 135.8; 36 layers x 1000 ->
     // 600 31.2 / 38.0, where 128 KB overshoot the list: 37.5), beyond that 32 KB in workgroups of 512
     // (16 requests x 2176 tokens 1997 / 2035; 256 threads 2007).
     CompactArgs one = c;
     if (chains <= 256) {
-      if (chains <= 128 && c.chunks_per_row >= 16) one.cols = 2;     // (pieces of 128 bytes: a cache line)
+      // A workgroup takes a CU's rate, so few chains take pieces of a row: of a cache line, or of half a line where a chain's
+      // pieces share an XCD and its L2 (compact_kernel numbers the pieces slowest: workgroups `chains` apart).
+      // One layer x 4096 -> 2048 tokens, rows of 256 bytes, called over and over / behind a flush of the caches, us: two
+      // pieces 10.0 / 22.8, four 8.5 / 20.1, eight 9.7 / 19.8 (four on XCDs as they come 11.0); rows of 512 bytes
+      // 15.1 / 34.5 with two, 10.2 / 23.0 with eight; rows of 128 bytes 9.4 / 20.3 whole, 8.0 / 18.2 in two.
+      const int piece = chains % 8 == 0 ? 64 : 128;
+      while (chains * one.cols * 2 <= 256 && c.chunks_per_row * 16 / (one.cols * 2) >= piece) one.cols *= 2;
       hipLaunchKernelGGL((compact_kernel<1024, 8, true>), dim3(chains * one.cols), dim3(1024), 0, s, one);
     } else if (chains <= 1024) {
       hipLaunchKernelGGL((compact_kernel<256, 8, true>), dim3(chains), dim3(256), 0, s, one);
