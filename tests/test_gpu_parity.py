@@ -1467,6 +1467,34 @@ def test_quarter_tile_scores_give_the_sums_of_whole_tiles(kw, lens):
         assert torch.equal(fin_a[b * h:(b + 1) * h, :t], fin_b[b * h:(b + 1) * h, :t]), (b, t)
 
 
+@pytest.mark.parametrize("offsets", [16, 17, 18, 21])
+@pytest.mark.parametrize("lens,layers,heads", [((1500, 1, 513), 1, (6, 2)), ((3000, 130, 2049, 511), 16, (40, 8))],
+                         ids=["a_tile_a_workgroup", "runs_over_units_and_sequences"])
+def test_max_aggregation_runs_of_tiles(lens, layers, heads, offsets, monkeypatch):
+    """The matrix-core kernel for max aggregation cuts all tiles of a ragged batch into 512 equal runs, which end and begin
+    inside (layer, head) units and sequences, and lays offset 16 out by pieces when it is the only one beyond the
+    first sixteen: raw scores against the vector-unit kernel to 1e-5 of the per-head RMS."""
+    w = small(num_q_heads=heads[0], num_kv_heads=heads[1], num_layers=layers, seq_lens=lens, budget=64, index=93)
+    inp = build_inputs(w)
+    print(f"max runs {offsets} {w}", flush=True)
+    out = {}
+    for kernel in ("mfma", "valu"):
+        tune(max_kernel=kernel)
+        caches, kv, batch, sc = device_objects(w, inp, DEV, aggregation="max")
+        sc = ops.ScoreConfig(sc.folded, sc.omega, torch.arange(offsets, device=DEV, dtype=torch.float32) * 37.0 + 1.0, "max")
+        raw, ws = ops.score_paged(kv, batch, sc)
+        keep, fin = ops.select(kv, batch, sc, ops.SelectConfig(window_size=0), raw, ws, want_scores=True)
+        torch.cuda.synchronize()
+        out[kernel] = (raw.clone(), fin.clone())
+    h = w.num_kv_heads
+    for b, t in enumerate(lens):
+        got, want = out["mfma"][0][b, :, :t], out["valu"][0][b, :, :t]
+        rms = want.pow(2).mean(dim=1, keepdim=True).sqrt().clamp_min(1e-30)
+        assert float(((got - want).abs() / rms).max()) <= 1e-5, b
+        fm, fv = out["mfma"][1][b * h:(b + 1) * h, :t], out["valu"][1][b * h:(b + 1) * h, :t]
+        assert float((fm - fv).abs().max()) <= SELECT_SCORE_TOL * max(float(fv.abs().max()), 1e-30), b
+
+
 @pytest.mark.parametrize("lens", [(1,), (15, 128, 129), (2049,), (4096,), (4097, 16)])
 @pytest.mark.parametrize("kv_dtype,head_dim,heads,layers,rope", [
     ("bf16", 128, (32, 8), 1, "half"), ("bf16", 128, (12, 4), 3, "interleaved"), ("fp16", 128, (8, 8), 4, "half"),

@@ -555,9 +555,18 @@ __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
 // a maximum over the 16 lanes of a row group; offsets from 16 on sit in NX further tiles as
 // column 4 (j - 16) + q, four lanes apart per head.  The magnitude term goes through the
 // matrix cores too: |k_f| in two bf16 pieces times E in three pieces, one piece per column
-// group.  A workgroup builds its operand slabs in LDS from the per-sequence tables (60 KB
-// for 17 offsets), then each wave takes 16 tokens a step.  Outputs as score_max_kernel: raw
+// group.  A workgroup builds its operand slabs in LDS from the per-sequence tables (52 KB
+// for 17 offsets), then each wave takes two steps of 16 tokens at a time.  Outputs as score_max_kernel: raw
 // rows and per-tile sums.
+//
+// What bounds it: matrix and vector instructions, which on this chip hardly overlap (a 16x16x32 product keeps the
+// vector unit from issuing for about 12 of its 16 cycles): 56 products and ~170 vector instructions a step, 33 % and
+// 42 % of the SIMDs' cycles on 2 x 8192 tokens x 36 layers, the rest in barriers, builds and the uneven end.  Selection of
+// that, us: 500 with workgroups of eight tiles (three rounds of 512 for two and a quarter rounds' work) and every
+// operand read waited for before its products, 441 with equal runs of tiles, offset 16 in four operands and one idle
+// cycle pair per stage of the maxima, 415 with the operand reads four ahead, 405 with the keys of the next steps in
+// flight across tiles; ragged, 64 query heads, 2 x 3000 and 900 tokens x 64 layers 526 -> 436, 28 query / 4 KV heads, 3 of 1000
+// to 6000 506 -> 266.  Cutting the pieces off instead of rounding them makes the build cheaper and the case no faster.
 typedef __bf16 mx_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float mx_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kDppRor4 = 0x124;        // row_ror:4
@@ -576,25 +585,30 @@ __device__ __forceinline__ void bf16_pieces(float x, uint32_t (&p)[3]) {
     x -= __uint_as_float(p[i] << 16);
   }
 }
-__device__ __forceinline__ float bf16_elem(const uint4& v, int e) {   // e: compile-time
-  const uint32_t w = e < 2 ? v.x : e < 4 ? v.y : e < 6 ? v.z : v.w;
-  return (e & 1) ? __uint_as_float(w & 0xffff0000u) : __uint_as_float(w << 16);
-}
 
-// max(keep, send of the lane `lane ^ 1` / `^ 2` / `^ 4` / `^ 8` of the row of 16): one instruction (two
+// v[i] = max(keep[i], send[i] of the lane `lane ^ 1` / `^ 2` / `^ 4` / `^ 8` of the row of 16): one instruction each (two
 // for ^ 4, which no single lane pattern of this chip expresses).  Written out because the compiler puts a
 // quieting v_max in front of every operand of fmaxf and moves the other lane's value into a register
 // first; the idle cycles cover the distance this chip requires between a vector instruction's write and a
-// lane-crossing read of that register.
-__device__ __forceinline__ float max_xor1(float keep, float send) {
-  float r;
-  asm("s_nop 1\n\tv_max_f32_dpp %0, %1, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(send), "v"(keep));
-  return r;
+// lane-crossing read of that register, once for all exchanges of a stage.
+__device__ __forceinline__ void max_xor1(float (&v)[8], const float (&send)[8]) {
+  asm("s_nop 1\n\tv_max_f32_dpp %0, %8, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %1, %9, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %2, %10, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %3, %11, %3 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %4, %12, %4 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %5, %13, %5 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %6, %14, %6 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %7, %15, %7 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf"
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+      : "v"(send[0]), "v"(send[1]), "v"(send[2]), "v"(send[3]), "v"(send[4]), "v"(send[5]), "v"(send[6]), "v"(send[7]));
 }
-__device__ __forceinline__ float max_xor2(float keep, float send) {
-  float r;
-  asm("s_nop 1\n\tv_max_f32_dpp %0, %1, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf" : "=v"(r) : "v"(send), "v"(keep));
-  return r;
+__device__ __forceinline__ void max_xor2(float (&v)[4], const float (&send)[4]) {
+  asm("s_nop 1\n\tv_max_f32_dpp %0, %4, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %1, %5, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %2, %6, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_max_f32_dpp %3, %7, %3 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : "v"(send[0]), "v"(send[1]), "v"(send[2]), "v"(send[3]));
 }
 __device__ __forceinline__ float max_xor4(float keep, float send) {
   float r = keep;      // lanes 0..3 and 8..11 of a row take lane + 4, the others lane - 4
@@ -638,42 +652,76 @@ __device__ __forceinline__ void split_pair_bf16(float x0, float x1, uint32_t& hi
 }
 
 constexpr int kMaxMfmaHeads = 4;   // query heads of one KV head per workgroup
-constexpr int kMaxMfmaTilesPerGroup = 8;   // consecutive 512-token tiles per workgroup
+constexpr int kMaxMfmaWorkgroups = 512;    // two per CU: each takes an equal run of tiles of 512 tokens
 // Waves of a workgroup (they share the operand slabs in LDS; two workgroups fit a CU).  Eight waves, four
 // per SIMD in 128 registers, run no faster (6.84 against 6.85 ms on 16 x 16384 tokens x 36 layers).
 constexpr int kMaxMfmaWaves = 4;
 constexpr int kMaxMfmaThreads = kMaxMfmaWaves * 64;
 constexpr int kTrigPitch = 65;     // floats per offset in LDS (odd: 16 offsets read at once fall into 16 banks)
-__host__ __device__ constexpr size_t max_mfma_lds_bytes(int nx, int no) {
-  return (size_t)(kMaxMfmaHeads + nx) * 12 * 64 * 16 + 2 * 64 * 16 + 3 * kMaxMfmaHeads * 64 * 4 +
-         (size_t)2 * no * kTrigPitch * 4 + (kScoreTileTokens + 2) * 4 + kMaxMfmaWaves * kMaxMfmaHeads * 2 * 4;
+// Slabs of 64 x 16 bytes: twelve per column tile (or, one offset beyond the first 16, four for all of its heads' pieces), two of
+// the magnitudes.
+__host__ __device__ constexpr int max_mfma_slabs(int nx, bool pieces) { return (kMaxMfmaHeads + (pieces ? 0 : nx)) * 12 + (pieces ? 4 : 0) + 2; }
+__host__ __device__ constexpr size_t max_mfma_lds_bytes(int nx, bool pieces, int no) {
+  return (size_t)max_mfma_slabs(nx, pieces) * 64 * 16 + 3 * kMaxMfmaHeads * 64 * 4 + (size_t)2 * no * kTrigPitch * 4 +
+         2 * kMaxMfmaWaves * kMaxMfmaHeads * 2 * 4;
 }
 
-template <int NX, bool IL>
+// NX: column tiles for the offsets from 16 on.  PIECES (17 offsets, NX = 1): offset 16 of the four heads takes one operand a
+// key slab, with the three pieces in column groups of their own as the magnitude coefficients have them, in place of
+// three operands a quarter full: 56 matrix instructions a step where there were 64.
+template <int NX, bool PIECES, bool IL>
 __global__ __launch_bounds__(kMaxMfmaThreads) __attribute__((amdgpu_waves_per_eu(kMaxMfmaWaves / 2, kMaxMfmaWaves / 2)))
-void score_max_mfma_kernel(ScoreArgs a) {
+void score_max_mfma_kernel(ScoreArgs a, int B) {
   constexpr int F = 64;
-  constexpr int NT = kMaxMfmaHeads + NX;
+  constexpr int NT = kMaxMfmaHeads + (PIECES ? 0 : NX);        // column tiles whose three pieces share an accumulator
   extern __shared__ __align__(16) char max_mfma_lds[];
   uint4* Bk = reinterpret_cast<uint4*>(max_mfma_lds);          // [NT][4 key slabs][3 pieces][64 lanes]
-  uint4* Bm = Bk + NT * 12 * 64;                               // [2 magnitude slabs][64 lanes]
+  uint4* Bx = Bk + NT * 12 * 64;                               // PIECES: [4 key slabs][64 lanes]
+  uint4* Bm = Bx + (PIECES ? 4 * 64 : 0);                      // [2 magnitude slabs][64 lanes]
   float* cf = reinterpret_cast<float*>(Bm + 2 * 64);           // [A1 | A2 | E][4 query heads][F]
   float* tcos = cf + 3 * kMaxMfmaHeads * F;                    // [NO][kTrigPitch]
   float* tsin = tcos + a.NO * kTrigPitch;                      // [NO][kTrigPitch]
-  int* lds_blk = reinterpret_cast<int*>(tsin + a.NO * kTrigPitch);   // [kScoreTileTokens + 2]
-  float* red = reinterpret_cast<float*>(lds_blk + kScoreTileTokens + 2);   // [waves][4 heads][2]
+  float* red = tsin + a.NO * kTrigPitch;                       // [2][waves][4 heads][2]
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int head = blockIdx.y / a.QC, qc = blockIdx.y % a.QC;
-  const int tile_group = blockIdx.x;
-  const int q0 = qc * kMaxMfmaHeads, nq = min(kMaxMfmaHeads, a.G - q0);
-  const int b = blockIdx.z / a.L, l = blockIdx.z % a.L;
-  const int seq_len = a.seq_lens[b];
-  // The operand slabs depend on (sequence, layer, KV head, group of query heads) only: a workgroup
-  // builds them once (as many vector instructions as scoring 400 tokens) and then takes
-  // kMaxMfmaTilesPerGroup consecutive tiles of 512 tokens.
-  if (tile_group * kMaxMfmaTilesPerGroup * kScoreTileTokens >= seq_len) return;
+  // All tiles of the batch in a row -- sequence, then unit (layer, KV head), then tile -- cut into
+  // equal runs: with eight tiles a workgroup, 2 x 8192 tokens x 36 layers were 1152 workgroups on 512 places, two and a
+  // quarter rounds that took three.  The operand slabs depend on everything but the tile and are built (as many
+  // vector instructions as scoring 400 tokens) where a run enters another unit: a place of their own in front of a
+  // unit's tiles, or the runs over short sequences would be the longer ones.  The groups of four query heads of a run
+  // go to workgroups eight apart, which start together on one XCD and find each other's keys in its L2.
+  const int per_seq = a.L * a.Hkv;
+  const bool apart = gridDim.x % (8 * a.QC) == 0;
+  const int qc = (apart ? blockIdx.x / 8 : blockIdx.x) % a.QC;
+  const int run = apart ? blockIdx.x / (8 * a.QC) * 8 + blockIdx.x % 8 : blockIdx.x / a.QC, runs = gridDim.x / a.QC;
+  auto length = [&](int s) { return min(a.seq_lens[s], a.num_tiles * kScoreTileTokens); };
+  auto places = [&](int s) { const int t = ceil_div(length(s), kScoreTileTokens); return t > 0 ? t + 1 : 0; };
+  int64_t total = 0;
+  for (int s = lane; s < B; s += 64) total += (int64_t)places(s) * per_seq;
+  for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d);
+  int64_t skip = total * run / runs;
+  int64_t left = total * (run + 1) / runs - skip;
+  int b = 0;
+  while (b < B && skip >= (int64_t)places(b) * per_seq) skip -= (int64_t)places(b++) * per_seq;
+  if (left <= 0 || b >= B) return;                     // (the same for the whole workgroup)
+  int seq_len = length(b), tiles = ceil_div(seq_len, kScoreTileTokens);
+  int unit = (int)(skip / (tiles + 1)), tile = (int)(skip % (tiles + 1)) - 1;
+  if (tile < 0) { tile = 0; --left; }
+  if (left <= 0) return;
 
+  const int r16 = lane & 15, kb = lane >> 4;
+  const bool b0 = (r16 & 1) != 0, b1 = (r16 & 2) != 0, b2 = (r16 & 4) != 0, b3 = (r16 & 8) != 0;
+  // After the maxima lane r16 of a row group holds the score of query head r16 % 4 and of the group's
+  // token r16 / 4: every lane stores one score.
+  const int out_q = r16 & 3, out_i = r16 >> 2;
+  const bool far_spread = a.NO > 17;            // more than one offset beyond the first 16: they sit in different lanes
+  constexpr int TW = kScoreTileTokens / kMaxMfmaWaves;
+
+  for (;;) {
+  // ---- the operand slabs of unit (layer, KV head) for this group of query heads
+  const int l = unit / a.Hkv, head = unit % a.Hkv;
+  const int q0 = qc * kMaxMfmaHeads, nq = min(kMaxMfmaHeads, a.G - q0);
+  __syncthreads();                              // (everyone is done with the previous ones)
   for (int i = threadIdx.x; i < 3 * kMaxMfmaHeads * F; i += kMaxMfmaThreads) {
     const int which = i / (kMaxMfmaHeads * F), q = (i / F) % kMaxMfmaHeads, f = i % F;
     const int ah = head * a.G + q0 + min(q, nq - 1);
@@ -719,6 +767,30 @@ void score_max_mfma_kernel(ScoreArgs a) {
 #pragma unroll
     for (int p = 0; p < 3; ++p) Bk[((t * 4 + sl) * 3 + p) * 64 + ln] = uint4{w[p][0], w[p][1], w[p][2], w[p][3]};
   }
+  // Offset 16: column c16 = query head (c16 % 4), piece (c16 / 4).
+  if constexpr (PIECES)
+    for (int i = threadIdx.x; i < 4 * 64; i += kMaxMfmaThreads) {
+      const int ln = i & 63, sl = i >> 6;
+      const int c16 = ln & 15, kb = ln >> 4;
+      const int q = c16 & 3, piece = c16 >> 2;
+      uint32_t w[4];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int d = 32 * sl + 8 * kb + e;
+        const int f = IL ? (d >> 1) : (d & 63);
+        const bool im = IL ? (d & 1) != 0 : d >= 64;
+        const float a1 = cf[(0 * kMaxMfmaHeads + q) * F + f], a2 = cf[(1 * kMaxMfmaHeads + q) * F + f];
+        const float cs = tcos[16 * kTrigPitch + f], sn = tsin[16 * kTrigPitch + f];
+        float x = im ? fmaf(a2, cs, a1 * sn) : fmaf(a1, cs, -(a2 * sn));
+        if (piece > 2 || q >= nq) x = 0.f;
+        uint32_t pc[3];
+        bf16_pieces(x, pc);
+        const uint32_t v = piece == 0 ? pc[0] : piece == 1 ? pc[1] : pc[2];
+        if (e & 1) w[e >> 1] |= v << 16;
+        else w[e >> 1] = v;
+      }
+      Bx[sl * 64 + ln] = uint4{w[0], w[1], w[2], w[3]};
+    }
   // Magnitude slabs: column c16 = query head (c16 % 4), piece (c16 / 4) of E; element e of slab
   // m is the pair whose magnitude the same lane forms from its key registers below.
   for (int i = threadIdx.x; i < 2 * 64; i += kMaxMfmaThreads) {
@@ -739,59 +811,58 @@ void score_max_mfma_kernel(ScoreArgs a) {
     Bm[m * 64 + ln] = uint4{w[0], w[1], w[2], w[3]};
   }
 
-  const int r16 = lane & 15, kb = lane >> 4;
-  const bool b0 = (r16 & 1) != 0, b1 = (r16 & 2) != 0, b2 = (r16 & 4) != 0, b3 = (r16 & 8) != 0;
-  // After the maxima lane r16 of a row group holds the score of query head r16 % 4 and of the group's
-  // token r16 / 4: every lane stores one score.
-  const int out_q = r16 & 3, out_i = r16 >> 2;
-  const bool far_spread = a.NO > 17;            // more than one offset beyond the first 16: they sit in different lanes
   const char* kbase = reinterpret_cast<const char*>(a.k_layers[l]);
-  const int64_t lane_off = (int64_t)head * a.stride_head + 8 * kb;
-  constexpr int TW = kScoreTileTokens / kMaxMfmaWaves;
   const bool out_lane = out_q < nq;
   float* raw_row = a.raw + (int64_t)(b * a.L + l) * a.raw_stride_layer +
                    (int64_t)(head * a.G + q0 + (out_lane ? out_q : 0)) * a.raw_stride_head;
 
-  for (int tile = tile_group * kMaxMfmaTilesPerGroup; tile < (tile_group + 1) * kMaxMfmaTilesPerGroup; ++tile) {
-  const int n0 = tile * kScoreTileTokens;
-  if (n0 >= seq_len) break;                     // (the same for every thread of the workgroup)
-  const int n1 = min(n0 + kScoreTileTokens, seq_len);
-  __syncthreads();                              // slabs built; the previous tile's block ids and sums read
-  int lb0 = 0;
-  if (a.block_table_pitch >= 0) {
-    lb0 = n0 / a.block_size;
-    const int lb1 = (n1 - 1) / a.block_size;
-    for (int i = threadIdx.x; i <= lb1 - lb0; i += kMaxMfmaThreads)
-      lds_blk[i] = a.block_table[(int64_t)b * a.block_table_pitch + lb0 + i];
-    __syncthreads();
-  }
-  const int wstart = n0 + wave * TW;
-  const int wend = min(wstart + TW, n1);
-  float s1 = 0.f, s2 = 0.f;
-
-  // Row lane % 16 of the step that starts at token t0: four 16-byte pieces, one per key slab.
-  // Rows past the tile are clamped to its last token (loaded, never stored).
-  auto load_step = [&](int t0, uint4 (&A)[4]) __attribute__((always_inline)) {
-    const int t = min(t0 + r16, n1 - 1);
-    int64_t phys, in_off;
-    if (a.block_table_pitch < 0) {
-      phys = b; in_off = t;
-    } else {
-      const int lb = a.bs_shift >= 0 ? (t >> a.bs_shift) : (t / a.block_size);
-      phys = lds_blk[lb - lb0];
-      in_off = t - lb * a.block_size;
+  // Byte offsets, from the head's base, of the rows of two of the wave's tokens of a tile, its tokens lane and 64 + lane (past
+  // the tile: its last token; loaded, never stored); two permutes hand them to the lanes of a step.
+  static_assert(TW == 128, "two tokens a lane");
+  struct Rows { int64_t off[2]; };
+  auto rows_of = [&](int tile) __attribute__((always_inline)) {
+    const int n0 = tile * kScoreTileTokens, n1 = min(n0 + kScoreTileTokens, seq_len);
+    Rows r;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int t = min(n0 + wave * TW + 64 * i + lane, n1 - 1);
+      int64_t phys = b;
+      int in_off = t;
+      if (a.block_table_pitch >= 0) {
+        const int lb = a.bs_shift >= 0 ? (t >> a.bs_shift) : (t / a.block_size);
+        phys = a.block_table[(int64_t)b * a.block_table_pitch + lb];
+        in_off = t - lb * a.block_size;
+      }
+      r.off[i] = (phys * a.stride_block + in_off * a.stride_token + (int64_t)head * a.stride_head) * 2;
     }
-    const int64_t e = phys * a.stride_block + in_off * a.stride_token + lane_off;
-    GlobalBytes p = (GlobalBytes)(uintptr_t)kbase + e * 2;
+    return r;
+  };
+  // Row lane % 16 of step s (0 .. 3) of the 64 tokens whose offsets the lanes hold in o: four 16-byte pieces, one per key slab.
+  auto load_step = [&](int64_t o, int s, uint4 (&A)[4]) __attribute__((always_inline)) {
+    const int src = s * 16 + r16;
+    const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)o, src), hi = (uint32_t)__shfl((int)(uint32_t)((uint64_t)o >> 32), src);
+    GlobalBytes p = (GlobalBytes)(uintptr_t)(kbase + (int64_t)(((uint64_t)hi << 32) | lo) + 16 * kb);
 #pragma unroll
     for (int sl = 0; sl < 4; ++sl) {
       const u32x4 v = *(GlobalU4)(p + sl * 64);
       A[sl] = uint4{v.x, v.y, v.z, v.w};
     }
   };
+  uint4 A0[4], A1[4], N0[4], N1[4];
+  Rows rows = rows_of(tile);
+  load_step(rows.off[0], 0, A0);
+  load_step(rows.off[0], 1, A1);
+  __syncthreads();                              // slabs built
+  for (; tile < tiles && left > 0; ++tile, --left) {
+  const int n0 = tile * kScoreTileTokens;
+  const int n1 = min(n0 + kScoreTileTokens, seq_len);
+  const int wstart = n0 + wave * TW;
+  const int wend = min(wstart + TW, n1);
+  float s1 = 0.f, s2 = 0.f;
+  const Rows next = rows_of(min(tile + 1, tiles - 1));     // (a workgroup's last tile of a unit reads a few rows in vain)
 
   // What follows the key products of one 16-token step: magnitude term, maxima, stores.
-  auto finish = [&](const uint4 (&A)[4], mx_f32x4 (&acc)[NT], int t0) __attribute__((always_inline)) {
+  auto finish = [&](const uint4 (&A)[4], mx_f32x4 (&acc)[NT], const mx_f32x4& accx, int t0) __attribute__((always_inline)) {
     // Magnitudes of this lane's 16 pairs (dot product of the bf16 pair with itself, square root) as
     // two bf16 pieces each.
     mx_f32x4 accm = mx_f32x4{0.f, 0.f, 0.f, 0.f};
@@ -827,17 +898,23 @@ void score_max_mfma_kernel(ScoreArgs a) {
     // tokens), each to be maximised over the 16 lanes.  A transposed butterfly: at every stage a lane
     // keeps half of its values and hands the other half to the lane one bit away, so the 16 + 8 + 4 + 2
     // values shrink to the one of (head r16 % 4, token r16 / 4) in 15 exchanges.
-    float u[2][4];
+    float u[8], us[8];                          // [pair of heads][token]
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
+      for (int i = 0; i < 4; ++i) {
         const float x = acc[2 * p][i], y = acc[2 * p + 1][i];
-        u[p][i] = max_xor1(b0 ? y : x, b0 ? x : y);
+        u[4 * p + i] = b0 ? y : x;
+        us[4 * p + i] = b0 ? x : y;
       }
-    float v4[4];
+    max_xor1(u, us);
+    float v4[4], vs[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v4[i] = max_xor2(b1 ? u[1][i] : u[0][i], b1 ? u[0][i] : u[1][i]);
+    for (int i = 0; i < 4; ++i) {
+      v4[i] = b1 ? u[4 + i] : u[i];
+      vs[i] = b1 ? u[i] : u[4 + i];
+    }
+    max_xor2(v4, vs);
     float w2[2];
 #pragma unroll
     for (int p = 0; p < 2; ++p) w2[p] = max_xor4(b2 ? v4[2 * p + 1] : v4[2 * p], b2 ? v4[2 * p] : v4[2 * p + 1]);
@@ -845,7 +922,7 @@ void score_max_mfma_kernel(ScoreArgs a) {
 
     // Offsets from 16 on: the further tiles hold them as column 4 (j - 16) + head, i.e. this lane's head
     // already; the maximum over the tiles, then (more than one such offset) over the four lanes of the head.
-    if constexpr (NX > 0) {
+    if constexpr (NX > 0 && !PIECES) {
       float f[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -876,6 +953,18 @@ void score_max_mfma_kernel(ScoreArgs a) {
       x += dpp<kDppRor8>(x);
       ex[i] = x;
     }
+    if constexpr (PIECES) {
+      // Offset 16: its pieces sit four lanes apart too.
+      float fx[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = accx[i];
+        x += dpp<kDppRor4>(x);
+        x += dpp<kDppRor8>(x);
+        fx[i] = x;
+      }
+      best = max_plain(best, b3 ? (b2 ? fx[3] : fx[2]) : (b2 ? fx[1] : fx[0]));
+    }
     const float v = best + (b3 ? (b2 ? ex[3] : ex[2]) : (b2 ? ex[1] : ex[0]));
     const int tk = t0 + 4 * kb + out_i;
     if (out_lane && tk < wend) {
@@ -889,79 +978,121 @@ void score_max_mfma_kernel(ScoreArgs a) {
   // step, are what the CU runs out of first; the keys of the next two steps are in flight
   // meanwhile.  (A second step that lies beyond the wave's tokens works on clamped rows and
   // stores nothing.)
-  uint4 A0[4] = {}, A1[4] = {}, N0[4] = {}, N1[4] = {};
-  if (wstart < wend) { load_step(wstart, A0); load_step(wstart + 16, A1); }
-  for (int t0 = wstart; t0 < wend; t0 += 32) {
-    if (t0 + 32 < wend) { load_step(t0 + 32, N0); load_step(t0 + 48, N1); }
-
+  auto two_steps = [&](const uint4 (&A0)[4], const uint4 (&A1)[4], int t0) __attribute__((always_inline)) {
     mx_f32x4 acc0[NT], acc1[NT];
+    mx_f32x4 accx0 = {0.f, 0.f, 0.f, 0.f}, accx1 = accx0;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       acc0[t] = mx_f32x4{0.f, 0.f, 0.f, 0.f};
       acc1[t] = mx_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int sl = 0; sl < 4; ++sl)
-#pragma unroll
-        for (int p = 2; p >= 0; --p) {
-          const uint4 bk = Bk[((t * 4 + sl) * 3 + p) * 64 + lane];
-          acc0[t] = mx_mfma(A0[sl], bk, acc0[t]);
-          acc1[t] = mx_mfma(A1[sl], bk, acc1[t]);
-        }
-      // One tile's operands at a time: left to itself the scheduler requests the slabs of all
-      // tiles up front and spills the keys to make room for them.  (Requesting a tile's twelve slabs
-      // one tile ahead, into a second set of registers, changes nothing: 6.84 -> 6.86 ms.)
-      __builtin_amdgcn_sched_barrier(0);
     }
-    finish(A0, acc0, t0);
-    __builtin_amdgcn_sched_barrier(0);
-    finish(A1, acc1, t0 + 16);
+    // Operand slabs in the order of their use -- column tile, key slab, third piece first -- kAhead of them requested
+    // before the first is used: a read that is waited for before the next is requested costs its whole latency, more than
+    // the two products behind it.  The pattern is imposed on the scheduler, which left to itself either requests
+    // a slab right where it is used or all of them up front and spills the keys to make room for them.
+    constexpr int kSlabs = NT * 12 + (PIECES ? 4 : 0), kAhead = 4;
+    auto slab = [&](int i) __attribute__((always_inline)) {
+      const int t = i / 12, sl = i % 12 / 3, p = 2 - i % 3;
+      return i < NT * 12 ? Bk[((t * 4 + sl) * 3 + p) * 64 + lane] : Bx[(i - NT * 12) * 64 + lane];
+    };
+    uint4 q[kAhead];
 #pragma unroll
-    for (int sl = 0; sl < 4; ++sl) { A0[sl] = N0[sl]; A1[sl] = N1[sl]; }
+    for (int i = 0; i < kAhead; ++i) q[i] = slab(i);
+#pragma unroll
+    for (int i = 0; i < kSlabs; ++i) {
+      const uint4 bk = q[i % kAhead];
+      if (i + kAhead < kSlabs) q[i % kAhead] = slab(i + kAhead);
+      const int sl = i < NT * 12 ? i % 12 / 3 : i - NT * 12;
+      mx_f32x4& c0 = i < NT * 12 ? acc0[i / 12 < NT ? i / 12 : 0] : accx0;
+      mx_f32x4& c1 = i < NT * 12 ? acc1[i / 12 < NT ? i / 12 : 0] : accx1;
+      c0 = mx_mfma(A0[sl], bk, c0);
+      c1 = mx_mfma(A1[sl], bk, c1);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);       // LDS reads
+#pragma unroll
+    for (int i = 0; i < kSlabs; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);          // matrix instructions
+      if (i + kAhead < kSlabs) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    finish(A0, acc0, accx0, t0);
+    __builtin_amdgcn_sched_barrier(0);
+    finish(A1, acc1, accx1, t0 + 16);
+  };
+  // Two steps are scored while the next two are on their way, across tiles too.  (The loads are
+  // unconditional: the compiler then counts those in flight instead of waiting for all of them.)
+  for (int s = 0; s < 8; s += 4) {
+    const int64_t here = s == 0 ? rows.off[0] : rows.off[1];
+    load_step(here, 2, N0);
+    load_step(here, 3, N1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (wstart + 16 * s < wend) two_steps(A0, A1, wstart + 16 * s);
+    const int64_t ahead = s == 0 ? rows.off[1] : next.off[0];
+    load_step(ahead, 0, A0);
+    load_step(ahead, 1, A1);
+    __builtin_amdgcn_sched_barrier(0);
+    if (wstart + 16 * (s + 2) < wend) two_steps(N0, N1, wstart + 16 * (s + 2));
   }
+  rows = next;
 
   // Per-tile sums of every query head: over the four row groups of a wave, then the waves.
   // (lane r16 of every row group holds the sums of head r16 % 4 over its token r16 / 4)
   s1 += __shfl_xor(s1, 4); s1 += __shfl_xor(s1, 8); s1 += __shfl_xor(s1, 16); s1 += __shfl_xor(s1, 32);
   s2 += __shfl_xor(s2, 4); s2 += __shfl_xor(s2, 8); s2 += __shfl_xor(s2, 16); s2 += __shfl_xor(s2, 32);
+  float* sums = red + (tile & 1) * (kMaxMfmaWaves * kMaxMfmaHeads * 2);      // (in turn: one barrier a tile)
   if (lane < kMaxMfmaHeads) {
-    red[(wave * kMaxMfmaHeads + lane) * 2 + 0] = s1;
-    red[(wave * kMaxMfmaHeads + lane) * 2 + 1] = s2;
+    sums[(wave * kMaxMfmaHeads + lane) * 2 + 0] = s1;
+    sums[(wave * kMaxMfmaHeads + lane) * 2 + 1] = s2;
   }
   __syncthreads();
   if ((int)threadIdx.x < nq) {
     float t1 = 0.f, t2 = 0.f;
     for (int w = 0; w < kMaxMfmaWaves; ++w) {
-      t1 += red[(w * kMaxMfmaHeads + threadIdx.x) * 2 + 0];
-      t2 += red[(w * kMaxMfmaHeads + threadIdx.x) * 2 + 1];
+      t1 += sums[(w * kMaxMfmaHeads + threadIdx.x) * 2 + 0];
+      t2 += sums[(w * kMaxMfmaHeads + threadIdx.x) * 2 + 1];
     }
     float* out = a.partial + (((int64_t)(b * a.L + l) * a.num_tiles + tile) * a.A + head * a.G + q0 + threadIdx.x) * 2;
     out[0] = t1;
     out[1] = t2;
   }
-  }   // tiles of this workgroup
+  }   // tiles of this unit
+  if (--left <= 0) break;                       // (the next unit's build)
+  tile = 0;
+  if (++unit == per_seq) {
+    unit = 0;
+    do {
+      if (++b >= B) return;
+      seq_len = length(b);
+      tiles = ceil_div(seq_len, kScoreTileTokens);
+    } while (tiles <= 0);
+  }
+  }   // units of this workgroup
 }
 
-template <int NX>
-hipError_t launch_max_mfma_nx(const ScoreArgs& k, dim3 grid, int il, size_t lds, hipStream_t s) {
-  const void* fn = il ? reinterpret_cast<const void*>(&score_max_mfma_kernel<NX, true>)
-                      : reinterpret_cast<const void*>(&score_max_mfma_kernel<NX, false>);
+template <int NX, bool PIECES>
+hipError_t launch_max_mfma_nx(const ScoreArgs& k, int B, int il, hipStream_t s) {
+  const size_t lds = max_mfma_lds_bytes(NX, PIECES, k.NO);
+  const void* fn = il ? reinterpret_cast<const void*>(&score_max_mfma_kernel<NX, PIECES, true>)
+                      : reinterpret_cast<const void*>(&score_max_mfma_kernel<NX, PIECES, false>);
   hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  if (il) hipLaunchKernelGGL((score_max_mfma_kernel<NX, true>), grid, dim3(kMaxMfmaThreads), lds, s, k);
-  else hipLaunchKernelGGL((score_max_mfma_kernel<NX, false>), grid, dim3(kMaxMfmaThreads), lds, s, k);
+  const int64_t tiles = (int64_t)k.num_tiles * B * k.L * k.Hkv;
+  const int runs = max(kMaxMfmaWorkgroups / k.QC, 1);
+  const dim3 grid((unsigned)((tiles < runs ? tiles : runs) * k.QC));
+  if (il) hipLaunchKernelGGL((score_max_mfma_kernel<NX, PIECES, true>), grid, dim3(kMaxMfmaThreads), lds, s, k, B);
+  else hipLaunchKernelGGL((score_max_mfma_kernel<NX, PIECES, false>), grid, dim3(kMaxMfmaThreads), lds, s, k, B);
   return hipGetLastError();
 }
 
 hipError_t launch_max_mfma(const ScoreArgs& k, int B, int il, hipStream_t s) {
   const int nx = k.NO > 16 ? ceil_div(k.NO - 16, 4) : 0;
-  const size_t lds = max_mfma_lds_bytes(nx, k.NO);
-  dim3 grid(ceil_div(k.num_tiles, kMaxMfmaTilesPerGroup), k.Hkv * k.QC, B * k.L);
+  if (k.NO == 17) return launch_max_mfma_nx<1, true>(k, B, il, s);
   switch (nx) {
-    case 0: return launch_max_mfma_nx<0>(k, grid, il, lds, s);
-    case 1: return launch_max_mfma_nx<1>(k, grid, il, lds, s);
-    case 2: return launch_max_mfma_nx<2>(k, grid, il, lds, s);
-    case 3: return launch_max_mfma_nx<3>(k, grid, il, lds, s);
-    case 4: return launch_max_mfma_nx<4>(k, grid, il, lds, s);
+    case 0: return launch_max_mfma_nx<0, false>(k, B, il, s);
+    case 1: return launch_max_mfma_nx<1, false>(k, B, il, s);
+    case 2: return launch_max_mfma_nx<2, false>(k, B, il, s);
+    case 3: return launch_max_mfma_nx<3, false>(k, B, il, s);
+    case 4: return launch_max_mfma_nx<4, false>(k, B, il, s);
     default: return hipErrorInvalidValue;
   }
 }
