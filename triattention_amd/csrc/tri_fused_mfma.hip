@@ -520,10 +520,6 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       v[0] = (upper ? x2 : x0) + dpp<kDppRor8m>(send0);
       v[1] = (upper ? x3 : x1) + dpp<kDppRor8m>(send1);
     }
-    if constexpr (FP8) {
-#pragma unroll
-      for (int i = 0; i < QG; ++i) v[i] *= raw.scale[i];
-    }
     // first ring slot of the step (scalar; a step never straddles the wrap: t and RING are
     // multiples of 16).  The ring has a place for every row of the step and every head slot: rows past the
     // tile's last token and slots beyond the last query head (zero columns) are written too and never read.
@@ -536,9 +532,11 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     }
 #pragma unroll
     for (int i = 0; i < QG; ++i) {
-      ring[slot0 * 4 + lane_ring + 4 * i] = v[i];
-      s1 += v[i];
-      s2 = fmaf(v[i], v[i], s2);
+      // (one-byte keys: the row's scale multiplies the finished score)
+      const float score = FP8 ? v[i] * raw.scale[i] : v[i];
+      ring[slot0 * 4 + lane_ring + 4 * i] = score;
+      s1 = FP8 ? fmaf(v[i], raw.scale[i], s1) : s1 + v[i];
+      s2 = fmaf(score, score, s2);
     }
   };
 
