@@ -198,8 +198,9 @@ class TriAttentionCompressor:
             return None
         if self.omega.numel() != f or self.offsets.numel() > 32 or not -2**31 <= self.state.get_round_start() < 2**31:
             return None
-        return tuple(x.to(device=keys.device, dtype=torch.float32).contiguous()
-                     for x in (*stats, self.omega, self.offsets))
+        dev = keys.device
+        return tuple(x if x.dtype is torch.float32 and x.device == dev and x.is_contiguous()
+                     else x.to(device=dev, dtype=torch.float32).contiguous() for x in (*stats, self.omega, self.offsets))
 
     def compress(self, key_states: torch.Tensor, value_states: torch.Tensor,
                  cache_positions: Optional[torch.Tensor] = None, layer_idx: int = 0

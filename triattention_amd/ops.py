@@ -35,7 +35,7 @@ if hasattr(torch, "float8_e4m3fn"):
 
 
 def _stream() -> int:
-    return int(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -548,15 +548,13 @@ def dense_compress(keys: torch.Tensor, values: torch.Tensor, q_mean_complex: tor
     out_k = torch.empty((1, h, budget, d), dtype=keys.dtype, device=keys.device)
     out_v = torch.empty((1, h, budget, values.shape[3]), dtype=values.dtype, device=values.device)
     keep = torch.empty((1, h, budget), dtype=torch.int64, device=keys.device)
+    # (in the order of the fields: by name they cost 3 us of a call whose kernels take 20)
     p = _lib.DenseParams(
-        num_heads=h, num_tokens=t, head_dim=d, kv_dtype=_DTYPES[keys.dtype],
-        rope_style=ROPE_INTERLEAVED if rope_style == "interleaved" else ROPE_HALF, budget=budget,
-        window_size=window_size, normalize=int(normalize), round_start=round_start, num_offsets=offsets.numel(),
-        aggregation=REDUCE_MAX if aggregation == "max" else REDUCE_MEAN, disable_mlr=int(disable_mlr),
-        disable_trig=int(disable_trig), v_row_bytes=values.shape[3] * v_es, k=_ptr(keys), v=_ptr(values),
-        k_stride_head=ks[1] * k_es, k_stride_token=ks[2] * k_es, v_stride_head=vs[1] * v_es, v_stride_token=vs[2] * v_es,
-        q_mean_complex=_ptr(q_mean_complex), q_abs_mean=_ptr(q_abs_mean), freq_scale_sq=_ptr(freq_scale_sq),
-        omega=_ptr(omega), offsets=_ptr(offsets), out_k=_ptr(out_k), out_v=_ptr(out_v), out_keep=_ptr(keep))
+        h, t, d, _DTYPES[keys.dtype], ROPE_INTERLEAVED if rope_style == "interleaved" else ROPE_HALF, budget, window_size,
+        normalize, round_start, offsets.numel(), REDUCE_MAX if aggregation == "max" else REDUCE_MEAN, disable_mlr,
+        disable_trig, values.shape[3] * v_es, keys.data_ptr(), values.data_ptr(), ks[1] * k_es, ks[2] * k_es, vs[1] * v_es,
+        vs[2] * v_es, q_mean_complex.data_ptr(), q_abs_mean.data_ptr(), freq_scale_sq.data_ptr(), omega.data_ptr(),
+        offsets.data_ptr(), out_k.data_ptr(), out_v.data_ptr(), keep.data_ptr())
     need = int(lib.tri_dense_workspace_bytes(C.byref(p)))
     if need == 0:
         raise ValueError("invalid dense call: " + lib.tri_last_error().decode("utf-8", "replace"))
