@@ -68,9 +68,9 @@ struct Workspace {
   FusedPlan fused;
 };
 
-// Coefficient operands of a KV head in the matrix-core resident kernel: key slabs (head_dim / 32; once more for the
-// third pieces of five to eight query heads) and magnitude slabs (head_dim / 64).  F = head_dim / 2.
-__host__ __device__ inline int mfma_operands(int F, int G) { return (G > 4 ? 2 : 1) * (F / 16) + F / 32; }
+// Coefficient operands of a KV head in the matrix-core resident kernel: key slabs (head_dim / 32) and magnitude slabs
+// (head_dim / 64), each once more for the third pieces of five to eight query heads.  F = head_dim / 2.
+__host__ __device__ inline int mfma_operands(int F, int G) { return (G > 4 ? 2 : 1) * (F / 16 + F / 32); }
 
 inline Workspace plan_workspace(int B, int L, int A, int F, int NO, int Hkv, int Tmax, const FusedPlan& fused) {
   Workspace w{};

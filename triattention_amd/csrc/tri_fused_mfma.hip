@@ -121,7 +121,7 @@ __device__ __forceinline__ float coefficient_piece(float x, int pieces) {
 // column j, k indices kb*8 .. + 7 of its slab.  Up to four query heads per KV head: operands 0..NS-1 are the
 // key slabs, NS/2 magnitude slabs follow; column j = (query head j % 4, piece j / 4).  Five to eight: NS key
 // operands with column j = (query head j % 8, piece j / 8), NS more with the third piece in columns 0..7 and
-// zeros beside it, NS/2 magnitude operands (query head j % 8, piece j / 8).  Piece p of a coefficient x is
+// zeros beside it, then the magnitude operands the same way.  Piece p of a coefficient x is
 // what is left of x after p roundings to the operand type (x = x1 + x2 + x3).
 constexpr int kPrepThreads = 1024;
 // Query heads whose coefficients are staged at a time, and the pitch of a staged head
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
   constexpr int F = HD / 2;              // frequency pairs
   constexpr int NS = HD / 32;            // key slabs
   const int NSO = mfma_operands(F, G);   // operands of a KV head
-  const int NK = NSO - NS / 2;           // of them key operands, the magnitude operands follow
+  const int NK = G > 4 ? 2 * NS : NS;    // of them key operands, the magnitude operands follow
   constexpr int kPrepHeads = prep_heads<HD>(), kPrepPitch = prep_pitch<HD>();
   __shared__ float buf[kPrepHeads * kPrepPitch];
   __shared__ float mean_cs[2][F];
@@ -199,11 +199,11 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
       const int head = idx / (64 * NSO);
       const int j = lane & 15, kb = lane >> 4;
       const bool mag = o >= NK;
-      const int slab = mag ? o - NK : o % NS;
+      const int slab = mag ? (o - NK) % (NS / 2) : o % NS;
       int q, sp;                                            // query head and piece of column j (piece 3: a zero column)
       if (G > 4) {
         q = j & 7;
-        sp = !mag && o >= NS ? (j < 8 ? 2 : 3) : j >> 3;
+        sp = (mag ? o - NK >= NS / 2 : o >= NS) ? (j < 8 ? 2 : 3) : j >> 3;
       } else {
         q = j & 3;
         sp = j >> 2;
@@ -253,12 +253,15 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
 // Two groups (five to eight query heads): a second operand set per group of four would leave a quarter of the
 // matrix columns empty twice and every step with two column reductions (three columns per head, four
 // values each, both groups: 34 of its 84 vector instructions at a head dimension of 64).  Instead the
-// columns are (query head, piece 1 | piece 2) and a second operand holds the third pieces beside zeros: one
-// accumulator for all eight heads, one exchange between column halves at the end, and the magnitude
-// coefficients, whose two fp16 pieces carry 24 bits, take one operand in place of two.  Vector / matrix
-// instructions a step: 84 / 8 -> 56 / 6 at a head dimension of 64, 166 / 16 -> 97 / 12 at 128.  24 requests of 1500 to
-// 12001 tokens x 36 layers x 64 query heads of 64: 1316 -> 1166 us; 1 x 32768 x 64 layers x 64 of 128: 824 -> 815 (there
-// the layers' statistics are waited for, not the instructions).
+// columns are (query head, piece 1 | piece 2) and a second operand holds the third pieces beside zeros: two
+// accumulators for all eight heads, added before the one exchange between column halves at the end -- (piece 1 +
+// piece 3) + piece 2, every sum in the order in which the column reduction took it, so the scores and the
+// statistics are the bits that two operand sets give.  Vector instructions a step: 84 -> 60 at a head dimension of
+// 64, 166 -> 101 at 128; matrix instructions 8 and 16 as before.  With the lane-parallel statistics
+// (gather_head_stats) 24 requests of 1500 to 12001 tokens x 36 layers x 64 query heads of 64 take 1114 us in place of
+// 1314, 1 x 32768 x 64 layers x 64 of 128 802 in place of 827 (there the layers' statistics are waited for, not the
+// instructions).  One accumulator and two pieces of the magnitude coefficients (6 and 12 matrix instructions) give
+// 1081 and 796, with the same error, but round differently: a near-tie then shifts a kept list of 12000.
 __device__ __forceinline__ int nsteps_of(int ntok) { return (ntok + 15) >> 4; }
 
 // W: waves per workgroup.  Eight (one workgroup per CU), or four for models with at most four
@@ -271,7 +274,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   static_assert(HD == 128 || ((HD == 64 || HD == 256) && DT != TRI_KV_FP8_E4M3), "head dimensions with a kernel");
   constexpr int NS = HD / 32;            // key slabs per step
   constexpr int NK = QG * NS;            // key operands (MFMAs) of a KV head
-  constexpr int NSO = NK + NS / 2;       // all operands
+  constexpr int NSO = QG * (NS + NS / 2);   // all operands
   static_assert(SL % (16 * NB) == 0, "the slack must hold whole rotations of the step buffers");
   // Token t of layer l sits at (l * ring_stride + t) % RING, ring_stride the tokens of this launch's tiles (at
   // most TW): what a tile leaves free of the ring is slack, down to SL for a whole tile.
@@ -301,10 +304,10 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int heads_here = min(8, a.Hkv - chunk * 8);
 
   float* ring = lds + wave * (RING * RQ);                      // [QG][RING][4 query heads]
-  float* part = lds + W * (RING * RQ);                         // [waves][64][2]
-  float* stats = part + W * 128;                          // [2][32*QG score heads][2]
+  float* part = lds + W * (RING * RQ);                         // [waves][64][QG][2]
+  float* stats = part + W * 128 * QG;                          // [2][32*QG score heads][2]
   uint32_t* ctl = reinterpret_cast<uint32_t*>(stats + 128 * QG);  // arrive count, claimed, ready; [8..15]: how far each wave is
-  for (int i = threadIdx.x; i < W * 128; i += W * kWave) part[i] = 0.f;
+  for (int i = threadIdx.x; i < W * 128 * QG; i += W * kWave) part[i] = 0.f;
   if (threadIdx.x < 16) ctl[threadIdx.x] = 0;
   __syncthreads();
   // From here on the waves of the workgroup run independently.
@@ -414,7 +417,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // consecutive tokens are 16 bytes apart, whatever the number of groups (with [RING][8] the stores of
   // one group fell on half the banks; it does not show in the kernel's time).
   const uint32_t lane_ring = (uint32_t)(q >> 2) * (RING * 4) + (uint32_t)(4 * kb + rsel) * 4 + (q & 3);
-  float s1 = 0.f, s2 = 0.f;
+  float s1[QG] = {}, s2[QG] = {};       // sums of this lane's i-th token of every step
   // Largest of a sample of the layer's magnitudes (their first fp16 pieces), per lane; see the check
   // after every layer.
   f16x2 mag_seen = {(_Float16)0.f, (_Float16)0.f};
@@ -465,7 +468,12 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     for (int s = 0; s < NS; ++s) d.c[s] = uint4{w[s][0], w[s][1], w[s][2], w[s][3]};
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int o = 0; o < NK; ++o) acc = mfma_16x16x32<DT>(d.c[o % NS], B[o], acc);
+    for (int s = 0; s < NS; ++s) acc = mfma_16x16x32<DT>(d.c[s], B[s], acc);
+    f32x4 acc3 = {0.f, 0.f, 0.f, 0.f};
+    if constexpr (QG == 2) {
+#pragma unroll
+      for (int s = 0; s < NS; ++s) acc3 = mfma_16x16x32<DT>(d.c[s], B[NS + s], acc3);
+    }
 #pragma unroll
     for (int set = 0; set < NS / 2; ++set) {
       // |k_f|^2 = k_r^2 + k_i^2 straight from the bf16 pairs (v_dot2_f32_bf16).
@@ -502,6 +510,10 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       constexpr int MT = TRI_KV_FP16;                // operand type of the magnitude MFMAs
       acc = mfma_16x16x32<MT>(hi, B[NK + set], acc);
       acc = mfma_16x16x32<MT>(lo, B[NK + set], acc);
+      if constexpr (QG == 2) {
+        acc3 = mfma_16x16x32<MT>(hi, B[NK + NS / 2 + set], acc3);
+        acc3 = mfma_16x16x32<MT>(lo, B[NK + NS / 2 + set], acc3);
+      }
     }
     // The pieces of a head are added across the columns; v[i] is then the score of this lane's i-th token.
     float v[QG];
@@ -515,7 +527,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
         v[0] = (rsel == r) ? x : v[0];
       }
     } else {
-      const float x0 = acc[0], x1 = acc[1], x2 = acc[2], x3 = acc[3];
+      const float x0 = acc[0] + acc3[0], x1 = acc[1] + acc3[1], x2 = acc[2] + acc3[2], x3 = acc[3] + acc3[3];
       const float send0 = upper ? x0 : x2, send1 = upper ? x1 : x3;
       v[0] = (upper ? x2 : x0) + dpp<kDppRor8m>(send0);
       v[1] = (upper ? x3 : x1) + dpp<kDppRor8m>(send1);
@@ -535,8 +547,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       // (one-byte keys: the row's scale multiplies the finished score)
       const float score = FP8 ? v[i] * raw.scale[i] : v[i];
       ring[slot0 * 4 + lane_ring + 4 * i] = score;
-      s1 = FP8 ? fmaf(v[i], raw.scale[i], s1) : s1 + v[i];
-      s2 = fmaf(score, score, s2);
+      s1[i] = FP8 ? fmaf(v[i], raw.scale[i], s1[i]) : s1[i] + v[i];
+      s2[i] = fmaf(score, score, s2[i]);
     }
   };
 
@@ -552,10 +564,13 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // before any wave deposits layer l + 1 (a wave consumes layer l, which needs every
   // deposit of layer l, before it finishes layer l + 1), so the counter never mixes layers.
   auto arrive = [&](int l) __attribute__((always_inline)) {
-    part[(wave * 64 + lane) * 2] = s1;
-    part[(wave * 64 + lane) * 2 + 1] = s2;
-    s1 = 0.f;
-    s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < QG; ++i) {
+      part[((wave * 64 + lane) * QG + i) * 2] = s1[i];
+      part[((wave * 64 + lane) * QG + i) * 2 + 1] = s2[i];
+      s1[i] = 0.f;
+      s2[i] = 0.f;
+    }
     uint32_t prev = 0;
     if (lane == 0) prev = __hip_atomic_fetch_add(arrive_cnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
     prev = __builtin_amdgcn_readfirstlane(prev);
@@ -567,7 +582,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       const int w = ahl / a.G, qq = ahl - w * a.G;
       constexpr int kLanes = 16 / QG;                // lanes that hold scores of one query head
       float t = 0.f;
-      for (int i = 0; i < kLanes; ++i) t += part[(w * 64 + i * (4 * QG) + qq) * 2 + which];
+      for (int i = 0; i < kLanes; ++i)               // in token order
+        for (int u = 0; u < QG; ++u) t += part[((w * 64 + i * (4 * QG) + qq) * QG + u) * 2 + which];
       xchg_store(out + item, ((unsigned long long)(uint32_t)(l + 1) << 32) | __float_as_uint(t));
     }
   };
@@ -766,7 +782,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       // A magnitude beyond fp16's range (or a key that is not finite) has left an infinity or a NaN
       // in this layer's sums.
       bool bad = false;
-      bad = !(s2 < INFINITY);
+#pragma unroll
+      for (int i = 0; i < QG; ++i) bad = bad || !(s2[i] < INFINITY);
       // The other end of fp16's range: below 2^-14 the first piece is a subnormal and below 2^-3 the
       // second one is, so magnitudes carry an absolute error of up to 2^-25 whatever their size.
       // Against keys of ordinary size that is nothing (scaled by 2^-10, magnitudes around 2^-9, the
@@ -812,7 +829,7 @@ struct LaunchShape {
 
 template <int TW, int SL, int QG, int W>
 constexpr size_t mfma_lds_bytes() {
-  return ((size_t)W * (TW + SL) * 4 * QG + W * 128 + 128 * QG + 16) * 4;
+  return ((size_t)W * (TW + SL) * 4 * QG + W * 128 * QG + 128 * QG + 16) * 4;
 }
 
 template <int DT, bool IL, int TW, int SL, int QG, int NB, int W = kFusedWaves, int HD = 128>
