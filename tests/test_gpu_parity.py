@@ -1559,6 +1559,45 @@ def test_small_launches_carry_values_beyond_range_like_the_two_pass_kernels(kv_d
     assert float(((a[m] - c[m]).abs() / c[m].abs().clamp_min(1.0)).max()) <= 2e-5
 
 
+@pytest.mark.parametrize("g", [1, 2, 3, 4, 7, 8])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("layers", [1, 2])
+def test_small_launches_rank_values_that_are_no_numbers_like_the_two_pass_kernels(layers, value, g, monkeypatch):
+    """One key element that is a NaN or an infinity, with and without normalisation (where it reaches every token of its
+    row through the mean), with a guarded window and prefill: the small launches keep what the score-then-select
+    kernels keep, token for token where the row holds no finite score, and their scores are of the same kind."""
+    w = small(num_q_heads=2 * g, num_kv_heads=2, num_layers=layers, seq_lens=(300,), budget=64, index=94)
+    inp = build_inputs(w)
+    inp["caches"][0][0, inp["tables"][0][3], 5, 1, 7] = value
+    caches, kv, batch, sc = device_objects(w, inp, DEV, prefill_lens=[5])
+    print(f"not a number {value} {w}", flush=True)
+    for kw in (dict(), dict(normalize=False), dict(group_reduce="mean"), dict(normalize="population"),
+               dict(normalize=False, layer_reduce="max", group_reduce="mean")):
+        sel = ops.SelectConfig(window_size=w.window_size, protect_prefill=True, **kw)
+        tune(resident_kernel="auto")
+        keep_s, fin_s, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
+        tune(resident_kernel="off")
+        raw, ws2 = ops.score_paged(kv, batch, sc)
+        keep_t, fin_t = ops.select(kv, batch, sc, sel, raw, ws2, want_scores=True)
+        torch.cuda.synchronize()
+        assert ws.status() == 0
+        for h in range(2):
+            a, c = fin_s[h, :300].cpu(), fin_t[h, :300].cpu()
+            got, want = keep_s[h:h + 1, :64].cpu().long(), keep_t[h:h + 1, :64].cpu().long()
+            assert torch.equal(torch.isnan(a), torch.isnan(c)) and torch.equal(torch.isinf(a), torch.isinf(c)), (kw, h)
+            inf, m = torch.isinf(c), torch.isfinite(c)
+            assert torch.equal(a[inf], c[inf]), (kw, h)
+            if bool(m.any()):
+                scale = float(c[m].abs().max())
+                finite = raw[0, :, :300].transpose(-1, -2).cpu()[:, h * g:(h + 1) * g]
+                tol = selection_score_tol(finite[torch.isfinite(finite).all(-1).all(-1)]) if sel.normalize else 5e-6
+                assert float((a[m] - c[m]).abs().max()) <= tol * scale, (kw, h)
+                assert_keep_matches(got, want, c.clone().masked_fill_(torch.isnan(c), float("inf"))[None], 64,
+                                    tie_tol=2 * tol * scale)
+            else:
+                assert torch.equal(got, want), (kw, h, a, c)
+
+
 def test_fp8_every_code_decodes_like_torch():
     """All 254 finite e4m3 codes through the scorer: with one non-zero coefficient the
     score is code_value * scale * coefficient, which pins the decoder against torch's

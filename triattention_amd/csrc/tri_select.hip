@@ -891,6 +891,9 @@ __device__ __forceinline__ float row_sum_f32(float v) {
 // lane adds up; in double where the reduce-first order has them so), the 64 partial sums of a head in double and its
 // statistics in one wave per head.
 // GQ: query heads of a KV head, rounded up to 1, 4 or 8.
+// A token whose z-scores are NaN ranks as combine_kernel ranks it: below every other (its general form starts each
+// maximum from -inf, which drops a NaN), but with four or eight query heads, whose form starts from the first head, as
+// the NaN that it is; one score per KV head of a dense call (pass_nan) keeps it too.
 template <int VPT, int GQ>
 __global__ __launch_bounds__(kTopkThreads, 4) void select_small_kernel(SmallSelect a) {
   constexpr int kWaves = kTopkThreads / 64, NV = 2 * GQ;
@@ -972,7 +975,7 @@ __global__ __launch_bounds__(kTopkThreads, 4) void select_small_kernel(SmallSele
     for (int i = 0; i < VPT; ++i) {
       float v;
       if constexpr (GQ == 1) {
-        v = a.pass_nan ? passed_zscore(x[0][i], mean[0], sd[0]) : zscore(x[0][i], mean[0], sd[0]);
+        v = a.pass_nan ? passed_zscore(x[0][i], mean[0], sd[0]) : fmaxf(-INFINITY, zscore(x[0][i], mean[0], sd[0]));
       } else {
         // (times the reciprocal, as the resident kernels do it: a division is ten instructions)
         v = __fmul_rn(__fsub_rn(x[0][i], mean[0]), sd[0]);
@@ -983,6 +986,7 @@ __global__ __launch_bounds__(kTopkThreads, 4) void select_small_kernel(SmallSele
             v = (a.group_reduce == TRI_REDUCE_MAX) ? fmaxf(v, z) : __fadd_rn(v, z);
           }
         if (a.group_reduce != TRI_REDUCE_MAX) v = __fdiv_rn(v, (float)a.G);
+        if (a.G != GQ) v = fmaxf(-INFINITY, v);
       }
       const int n = e0 + 64 * i;
       if (n >= window_from || n < prefill) v = INFINITY;
