@@ -1598,6 +1598,30 @@ def test_small_launches_rank_values_that_are_no_numbers_like_the_two_pass_kernel
                 assert torch.equal(got, want), (kw, h, a, c)
 
 
+@pytest.mark.parametrize("kv_dtype,head_dim,g", [("fp16", 128, 4), ("fp16", 64, 7), ("fp16", 256, 1), ("bf16", 128, 4)])
+@pytest.mark.parametrize("what,factor", [("all", 1e-30), ("all", 1e-25), ("all", 1e-20), ("all", 1e-15), ("all", 1e15), ("all", 1e25),
+                                         ("trig", 1e-20), ("trig", 1e15), ("norm", 1e-20), ("norm", 1e15)])
+def test_small_launches_take_coefficients_of_any_size(what, factor, kv_dtype, head_dim, g, monkeypatch):
+    """Statistics far below and above the range of half precision, in both terms of the score or in one of them: the
+    scores agree with the two-pass kernels' fp32 arithmetic to 5e-6 of the largest, as with statistics of ordinary size."""
+    w = small(kv_dtype=kv_dtype, head_dim=head_dim, num_q_heads=2 * g, num_kv_heads=2, num_layers=1, seq_lens=(300,),
+              budget=64, window_size=0, index=95)
+    inp = build_inputs(w)
+    caches, kv, batch, sc = device_objects(w, inp, DEV)
+    sc.folded[:, :, {"all": slice(0, 3), "trig": slice(0, 2), "norm": slice(2, 3)}[what]] *= factor
+    sel = ops.SelectConfig(window_size=0, normalize=False)
+    print(f"coefficients {what} x {factor} {w}", flush=True)
+    _, a, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
+    tune(resident_kernel="off")
+    raw, ws2 = ops.score_paged(kv, batch, sc)
+    _, c = ops.select(kv, batch, sc, sel, raw, ws2, want_scores=True)
+    torch.cuda.synchronize()
+    assert ws.status() == 0
+    a, c = a[:, :300].double().cpu(), c[:, :300].double().cpu()
+    assert bool(torch.isfinite(c).all())
+    assert float((a - c).abs().max()) <= 5e-6 * float(c.abs().max())
+
+
 def test_fp8_every_code_decodes_like_torch():
     """All 254 finite e4m3 codes through the scorer: with one non-zero coefficient the
     score is code_value * scale * coefficient, which pins the decoder against torch's

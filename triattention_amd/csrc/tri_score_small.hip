@@ -17,7 +17,8 @@
 //  - the magnitudes enter as three bf16 pieces of eight bits, cut off and not rounded, which is the whole
 //    fp32 value, and so do the magnitude coefficients;
 //  - fp16 keys: the coefficients of a query head are scaled by a power of two into fp16's range, and the
-//    scores scaled back;
+//    scores scaled back; with bf16 keys the pieces have fp32's range as they are (below 2^-109 the third one is a
+//    subnormal, and a coefficient keeps the bits above 2^-133);
 //  - a step in which any score is not finite (keys that are not, products beyond fp32) is evaluated again
 //    pair by pair in fp32, so infinities and NaNs come out as a sum of products gives them.
 #include "tri_common.h"
@@ -93,7 +94,9 @@ __device__ __forceinline__ uint4 mma_operand(const float* cf, const float* scale
   return uint4{w[0], w[1], w[2], w[3]};
 }
 
-// Power of two that takes the largest of |P|, |R| of a query head to about 2^13 (fp16 keys).  Called by a whole wave.
+// Power of two that takes the largest of |P|, |R| of a query head to about 2^13 (fp16 keys), the second and third
+// pieces then lie in fp16's range too.  Upwards as far as fp32 goes: beyond 2^126 a coefficient is a subnormal of fp32
+// itself.  Down to 2^-40: a larger coefficient overflows, and its steps are evaluated pair by pair.  Called by a whole wave.
 template <int F>
 __device__ __forceinline__ float fp16_scale(const float* c, int lane) {
   float m = 0.f;
@@ -102,7 +105,7 @@ __device__ __forceinline__ float fp16_scale(const float* c, int lane) {
   int e = 0;
   if (m > 0.f && m < INFINITY) (void)frexpf(m, &e);
   else e = 13;
-  return ldexpf(1.f, min(max(13 - e, -40), 40));
+  return ldexpf(1.f, min(max(13 - e, -40), 126));
 }
 
 // Means over the offsets of cos and sin of the phases, the way prepare_kernel evaluates them (summed in offset order
