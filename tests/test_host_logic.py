@@ -904,3 +904,28 @@ def test_quarter_tiles_are_for_launches_that_leave_most_of_the_chip_idle():
     assert tile(3, 32, 8, 128, 2176, dtype=2) == 128
     assert tile(3, 64, 8, 128, 29) == 512 and tile(3, 64, 8, 128, 30) == 128             # room for the sums
     assert tile(3, 31, 8, 128, 2176) == 0 and tile(3, 32, 8, 100, 2176) == 0 and tile(3, 32, 8, 128, 0) == 0
+
+
+def test_matrix_instructions_wait_for_what_inline_asm_wrote(tmp_path):
+    """The second pieces of the magnitudes come out of inline asm, which the compiler's spacing of vector writes and
+    matrix reads does not look into: the library's code holds two idle cycles after the last of them, whatever the
+    scheduler puts behind."""
+    import shutil
+    import subprocess
+    objdump = Path("/opt/rocm/llvm/bin/llvm-objdump")
+    if not objdump.exists():
+        pytest.skip("no llvm-objdump")
+    _lib.load()
+    lib = tmp_path / "lib.so"
+    shutil.copy(tri_build.LIB_PATH, lib)
+    subprocess.run([str(objdump), "--offloading", str(lib)], check=True, capture_output=True, timeout=120)
+    runs = 0
+    for code in sorted(tmp_path.glob("lib.so.*gfx950*")):
+        text = subprocess.run([str(objdump), "-d", "--no-show-raw-insn", str(code)], check=True, capture_output=True, text=True,
+                              timeout=120).stdout
+        lines = [x.split("//")[0].strip() for x in text.splitlines() if x.startswith("\t")]
+        for here, behind in zip(lines, lines[1:]):
+            if here.startswith("v_fma_mixhi_f16") and not behind.startswith("v_fma_mixhi_f16"):
+                runs += 1
+                assert re.fullmatch(r"s_nop [1-9]", behind), behind
+    assert runs > 0

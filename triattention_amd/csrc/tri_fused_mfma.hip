@@ -67,7 +67,9 @@ __device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w 
 // Eight fp32 values as two packed fp16 pieces each.  The remainders x - hi are exact in fp32 and rounded to fp16 by
 // the same instruction (the mixed-precision fused multiply-add reads and writes halves of packed
 // registers): three instructions per two values, which used to be four (no case got measurably faster by it alone).  A half written by one instruction is read by the next but three at
-// the earliest: this chip wants one between.
+// the earliest: this chip wants one between.  The two idle cycles at the end are what it wants between a vector
+// instruction and a matrix instruction that reads its result (the compiler, which keeps that distance elsewhere, does not
+// see the instructions of an asm statement).
 __device__ __forceinline__ void split8_f16(const float (&x)[8], uint4& hi, uint4& lo) {
   uint32_t h[4], l[4];
 #pragma unroll
@@ -85,7 +87,7 @@ __device__ __forceinline__ void split8_f16(const float (&x)[8], uint4& hi, uint4
       "v_fma_mixhi_f16 %1, %5, -1.0, %9 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
       "v_fma_mixhi_f16 %2, %6, -1.0, %10 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
       "v_fma_mixhi_f16 %3, %7, -1.0, %11 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
-      "s_nop 0"
+      "s_nop 1"
       : "+&v"(l[0]), "+&v"(l[1]), "+&v"(l[2]), "+&v"(l[3])
       : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(x[1]), "v"(x[3]), "v"(x[5]), "v"(x[7]));
   hi = uint4{h[0], h[1], h[2], h[3]};
