@@ -729,7 +729,8 @@ def main() -> int:
         "path": path,
         "plan": m["plan"],
         "roofline": {"kernel": {"two_pass": two_pass_kernel, "resident_valu": "fused_select_kernel",
-                                "resident_mfma": "fused_mfma_kernel"}[path], "bound": "hbm",
+                                "resident_mfma": "score_small_kernel" if (m["plan"] or {}).get("small_launches")
+                                                 else "fused_mfma_kernel"}[path], "bound": "hbm",
                      "achieved": score_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": score_gbs / HBM_PEAK_GBS,
                      "traffic": traffic[0] if traffic else None,
                      "traffic_source": (traffic[1] + " (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of this command, scaled by "

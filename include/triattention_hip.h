@@ -231,8 +231,8 @@ int tri_select_paged(const tri_kv_layout* kv, const tri_batch* batch, const tri_
                      uint64_t workspace_bytes, void* stream);
 
 /* Which path tri_select_paged / tri_compress_step take for these arguments on the
- * current device: 2 = resident kernel scoring on the matrix cores (bf16, fp16 and fp8 keys; a few layers of a few
- * requests take two short matrix-core launches in its place, which wait for nothing), 1 = resident
+ * current device: 2 = resident kernel scoring on the matrix cores (bf16, fp16 and fp8 keys), or the two short
+ * launches that take its place for a few layers of a few requests (tri_small_launches), 1 = resident
  * kernel scoring on the vector unit, 0 = score then select, -1 = invalid arguments.
  * Host-only.  No counterpart in the reference (it has a single path). */
 int tri_select_path(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
@@ -245,7 +245,9 @@ int tri_select_path(const tri_kv_layout* kv, const tri_batch* batch, const tri_s
  * at most ceil(num_seqs / sequences per launch)).  assume_resident_workgroups > 0 answers for a
  * device that holds that many resident workgroups at once (a dry run that touches no device:
  * capacity planning, tests of the planner on a host without a GPU; 256 is an MI355X with 8-wave
- * workgroups); 0 answers for the current device.  Host-only.  No counterpart in the reference. */
+ * workgroups); 0 answers for the current device.  Where tri_small_launches says 1 this is the resident plan that
+ * the workspace is sized for and that TRI_TUNE_RESIDENT_KERNEL = 1 would run, not what runs.  Host-only.  No
+ * counterpart in the reference. */
 typedef struct tri_plan_info {
   int32_t path;                 /* 0 two-pass, 1 resident on the vector unit, 2 resident on the matrix cores */
   int32_t tile_tokens;          /* tokens a workgroup scores per layer (0 on the two-pass path) */
@@ -259,6 +261,14 @@ typedef struct tri_plan_info {
 } tri_plan_info;
 int tri_describe_plan(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
                       const tri_select_params* sel, int32_t assume_resident_workgroups, tri_plan_info* out);
+
+/* 1 where tri_select_paged / tri_compress_step take two short launches in place of the resident matrix-core kernel: a
+ * wave per 16 tokens of a KV head of a layer with the preparation inside, then statistics, reduction and top-k in one
+ * workgroup per (sequence, KV head).  They wait for nothing; the status word then only reports a device-side length
+ * beyond max_seq_len (3).  0: they are not taken, -1: invalid arguments.  assume_resident_workgroups as for
+ * tri_describe_plan.  Host-only.  No counterpart in the reference. */
+int tri_small_launches(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
+                       const tri_select_params* sel, int32_t assume_resident_workgroups);
 
 /* Tokens a workgroup of the score-then-select kernels takes in one call that scores and selects: 512, or 128
  * (quarter tiles, the same bits) for a launch that would leave most CUs idle; 0 for invalid arguments.

@@ -451,7 +451,8 @@ def test_layer_selection_matches_reference_golden(tag, kw, fixture):
 def test_one_layer_of_a_per_layer_selection_takes_the_resident_kernel(tag, kw, fixture):
     """The reference's per-layer modes call the selector once per layer (runtime/selector_hf.py:473-747
     from the layer loop): a keep set per layer of a one-layer call is the group selection of that layer,
-    so the call takes the resident kernel and still gives the reference's rows for layer 1."""
+    so the call takes the resident kernel, or the two short launches that take its place for so little, and still gives the
+    reference's rows for layer 1."""
     gold = load_golden(fixture)
     layers, hkv, t, d = gold["keys"].shape
     hq = gold["q_mean_complex"].shape[1]
@@ -468,19 +469,23 @@ def test_one_layer_of_a_per_layer_selection_takes_the_resident_kernel(tag, kw, f
                             torch.ones(1, hq, d // 2, device=DEV))
     sc = ops.ScoreConfig(folded, gold["omega"].to(DEV), synth.geometric_offsets(device=DEV))
     sel = ops.SelectConfig(normalize=kw.get("normalize", True), window_size=int(gold["window"]), layer_reduce=None)
-    assert ops.select_path(kv, batch, sc, sel) == "resident_mfma"
-    keep, fin, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
-    sel.allow_resident = False
-    assert ops.select_path(kv, batch, sc, sel) == "two_pass"
-    keep_t, fin_t, _ = ops.select_paged(kv, batch, sc, sel, want_scores=True)
-    torch.cuda.synchronize()
-    assert ws.status() == 0
-    assert torch.equal(keep.cpu().long().view(hkv, -1), gold[f"layer1_{tag}_keep"])
-    assert torch.equal(keep_t.cpu().long().view(hkv, -1), gold[f"layer1_{tag}_keep"])
-    a, b = fin.cpu().view(hkv, -1)[:, :t], fin_t.cpu().view(hkv, -1)[:, :t]
-    m = torch.isfinite(b)
-    assert torch.equal(torch.isfinite(a), m)
-    assert float((a[m] - b[m]).abs().max()) <= 1e-4 * float(b[m].abs().max())
+    for kernel, small_launches in (("auto", 1), ("mfma", 0)):
+        tune(resident_kernel=kernel)
+        sel.allow_resident = True
+        assert ops.describe_plan(kv, batch, sc, sel)["small_launches"] == small_launches
+        assert ops.select_path(kv, batch, sc, sel) == "resident_mfma"
+        keep, fin, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
+        sel.allow_resident = False
+        assert ops.select_path(kv, batch, sc, sel) == "two_pass"
+        keep_t, fin_t, _ = ops.select_paged(kv, batch, sc, sel, want_scores=True)
+        torch.cuda.synchronize()
+        assert ws.status() == 0
+        assert torch.equal(keep.cpu().long().view(hkv, -1), gold[f"layer1_{tag}_keep"])
+        assert torch.equal(keep_t.cpu().long().view(hkv, -1), gold[f"layer1_{tag}_keep"])
+        a, b = fin.cpu().view(hkv, -1)[:, :t], fin_t.cpu().view(hkv, -1)[:, :t]
+        m = torch.isfinite(b)
+        assert torch.equal(torch.isfinite(a), m)
+        assert float((a[m] - b[m]).abs().max()) <= 1e-4 * float(b[m].abs().max())
 
 
 @pytest.mark.parametrize("width", [3000, 8192, 16384, 20001, 32768, 40000])
@@ -1123,7 +1128,8 @@ def test_resident_selection_on_dense_keys(kernel, monkeypatch):
 
 def test_resident_path_is_taken_unless_multi_layer_workgroups_would_underfill_the_chip():
     """Workgroups that run one layer make a short launch however few they are; workgroups that run
-    several layers must fill most of the chip, or the two-pass kernels take the batch."""
+    several layers must fill most of the chip, or the two-pass kernels take the batch.  Of the short ones the smallest
+    are two launches of their own under the automatic choice; the plan says so beside the resident one's cut."""
     sel = ops.SelectConfig(window_size=12)
     cases = ((1, None, (300,), "resident_mfma"),             # 3 tiles of 128, one layer
              (1, None, (16384,), "resident_mfma"),           # 64 tiles, a quarter of the chip, one layer
@@ -1148,6 +1154,8 @@ def test_resident_path_is_taken_unless_multi_layer_workgroups_would_underfill_th
         info = ops.describe_plan(kv, batch, sc, sel)
         assert info["path"] == want
         if want != "two_pass":
+            assert info["small_launches"] == (layers * len(seq_lens) * 8 * -(-max(seq_lens) // 128) <= 1024
+                                              and max(seq_lens) <= 8192)
             # the dry run for a device of this one's size gives this device's plan, and a launch fits the device
             assert ops.describe_plan(kv, batch, sc, sel, assume_resident_workgroups=info["resident_workgroups"]) == info
             assert info["launches"] == 1 and info["layer_groups"] * info["layers_per_group"] >= layers
@@ -1503,7 +1511,8 @@ def test_max_aggregation_runs_of_tiles(lens, layers, heads, offsets, monkeypatch
 def test_small_launches_match_the_two_pass_kernels(kv_dtype, head_dim, heads, layers, rope, lens, monkeypatch):
     """A few layers of a few requests go through kernels of their own (a wave per step, statistics in the selection's
     workgroups): selection scores and kept sets against the score-then-select kernels, and without
-    normalisation, where the raw scores show, to 5e-6 of the largest (two fp32 evaluations of one sum)."""
+    normalisation, where the raw scores show, to 5e-6 of the largest (two fp32 evaluations of one sum).  The longest
+    batch is too much for some shapes, which then take the resident or the two-pass kernels."""
     w = small(kv_dtype=kv_dtype, head_dim=head_dim, num_q_heads=heads[0], num_kv_heads=heads[1], num_layers=layers, rope_style=rope,
               seq_lens=lens, budget=96, index=91)
     print(f"small {w}", flush=True)
@@ -1513,6 +1522,8 @@ def test_small_launches_match_the_two_pass_kernels(kv_dtype, head_dim, heads, la
     for kw in (dict(), dict(normalize=False, layer_reduce="max"), dict(group_reduce="mean", protect_prefill=True)):
         sel = ops.SelectConfig(window_size=w.window_size, **kw)
         tune(resident_kernel="auto")
+        too_much = lens == (4097, 16) and heads in ((8, 8), (24, 3), (14, 2))
+        assert ops.describe_plan(kv, batch, sc, sel)["small_launches"] == (0 if too_much else 1)
         keep_s, fin_s, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
         keep_only, _, _ = ops.select_paged(kv, batch, sc, sel)
         tune(resident_kernel="off")
@@ -1545,6 +1556,7 @@ def test_small_launches_carry_values_beyond_range_like_the_two_pass_kernels(kv_d
     caches, kv, batch, sc = device_objects(w, inp, DEV)
     sel = ops.SelectConfig(window_size=0, normalize=False)
     print(f"beyond range {kv_dtype} {value}", flush=True)
+    assert ops.describe_plan(kv, batch, sc, sel)["small_launches"] == 1
     _, a, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
     tune(resident_kernel="off")
     raw, ws2 = ops.score_paged(kv, batch, sc)
@@ -1575,6 +1587,7 @@ def test_small_launches_rank_values_that_are_no_numbers_like_the_two_pass_kernel
                dict(normalize=False, layer_reduce="max", group_reduce="mean")):
         sel = ops.SelectConfig(window_size=w.window_size, protect_prefill=True, **kw)
         tune(resident_kernel="auto")
+        assert ops.describe_plan(kv, batch, sc, sel)["small_launches"] == 1
         keep_s, fin_s, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
         tune(resident_kernel="off")
         raw, ws2 = ops.score_paged(kv, batch, sc)
@@ -1611,6 +1624,7 @@ def test_small_launches_take_coefficients_of_any_size(what, factor, kv_dtype, he
     sc.folded[:, :, {"all": slice(0, 3), "trig": slice(0, 2), "norm": slice(2, 3)}[what]] *= factor
     sel = ops.SelectConfig(window_size=0, normalize=False)
     print(f"coefficients {what} x {factor} {w}", flush=True)
+    assert ops.describe_plan(kv, batch, sc, sel)["small_launches"] == 1
     _, a, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
     tune(resident_kernel="off")
     raw, ws2 = ops.score_paged(kv, batch, sc)

@@ -846,6 +846,38 @@ def _describe(layers, q_heads, kv_heads, head_dim, lens, assume=256, kv_dtype=0,
     return (info.path, info.tile_tokens, info.tiles_per_seq, info.layer_groups, info.layers_per_group, info.launches)
 
 
+def _small_launches(layers, q_heads, kv_heads, head_dim, lens, kv_dtype=0, assume=256, **select):
+    import ctypes as C
+    lib = _lib.load()
+    kv = _lib.KvLayout(num_layers=layers, num_kv_heads=kv_heads, head_dim=head_dim, block_size=16, kv_dtype=kv_dtype,
+                       stride_block=16 * kv_heads * head_dim, stride_token=kv_heads * head_dim, stride_head=head_dim,
+                       k_layers=8, v_layers=8, k_scale_layers=8 if kv_dtype == 2 else None)
+    batch = _lib.Batch(num_seqs=len(lens), max_seq_len=max(lens), max_budget=64, block_table_pitch=4096, block_table=8,
+                       seq_lens=8, round_start=8, budgets=8)
+    sp = _lib.ScoreParams(num_score_heads=q_heads, num_offsets=17, folded=16, omega=8, offsets=8)
+    kw = dict(normalize=1, window_size=128, group_reduce=1)
+    kw.update(select)
+    sel = _lib.SelectParams(**kw)
+    return lib.tri_small_launches(C.byref(kv), C.byref(batch), C.byref(sp), C.byref(sel), assume)
+
+
+def test_small_launches_are_reported():
+    """``tri_small_launches`` for a device that holds 256 resident workgroups: the calls whose place in the plan
+    (``tri_describe_plan`` still gives the resident one) two short launches take, and what keeps a call off them."""
+    one = (1, 32, 8, 128, [4096])
+    assert _small_launches(*one) == 1 and _describe(*one)[0] == 2
+    assert _small_launches(1, 32, 8, 128, [4096], layer_reduce=-1) == 1      # a keep set of the one layer
+    assert _small_launches(1, 14, 2, 256, [300, 16]) == 1 and _small_launches(1, 8, 8, 64, [16384], kv_dtype=1) == 1
+    assert _small_launches(36, 32, 8, 128, [2176]) == 0                      # many layers
+    assert _small_launches(*one, kv_dtype=2) == 0                            # one-byte keys
+    assert _small_launches(1, 32, 8, 128, [8193]) == 0                       # a row that does not fit the registers
+    assert _small_launches(*one, shared=1) == 0 and _small_launches(*one, group_first=1) == 0
+    assert _small_launches(*one, no_resident=1) == 0
+    with _lib.tuning(resident_kernel="mfma"):
+        assert _small_launches(*one) == 0
+    assert _small_launches(1, 31, 8, 128, [4096]) == -1 and _small_launches(*one, assume=-1) == -1
+
+
 def test_planner_cuts_the_benchmarked_shapes_as_documented():
     """``tri_describe_plan`` for a device that holds 256 resident workgroups (an MI355X), without one:
     (path, tile tokens, tiles of the longest sequence, layer groups, layers per group, launches)."""

@@ -33,7 +33,7 @@ EXPORTS = (
     "tri_abi_version", "tri_last_error", "tri_source_digest", "tri_set_tuning", "tri_get_tuning", "tri_resident_gate_enter",
     "tri_resident_gate_leave", "tri_fold_stats", "tri_workspace_bytes", "tri_workspace_status_offset",
     "tri_score_paged",
-    "tri_select", "tri_select_paged", "tri_select_path", "tri_describe_plan", "tri_score_tile_tokens", "tri_topk_rows",
+    "tri_select", "tri_select_paged", "tri_select_path", "tri_describe_plan", "tri_small_launches", "tri_score_tile_tokens", "tri_topk_rows",
     "tri_dense_workspace_bytes", "tri_dense_compress",
     "tri_compact_paged", "tri_compact_full_staging_bytes",
     "tri_compact_paged_full", "tri_compress_step", "tri_compress_step_static", "tri_qstats_workspace_bytes", "tri_qstats",
@@ -139,6 +139,8 @@ def load() -> C.CDLL:
                                     C.POINTER(SelectParams)]
     lib.tri_describe_plan.argtypes = [C.POINTER(KvLayout), C.POINTER(Batch), C.POINTER(ScoreParams),
                                       C.POINTER(SelectParams), I32, C.POINTER(PlanInfo)]
+    lib.tri_small_launches.argtypes = [C.POINTER(KvLayout), C.POINTER(Batch), C.POINTER(ScoreParams),
+                                       C.POINTER(SelectParams), I32]
     lib.tri_score_tile_tokens.argtypes = [C.POINTER(KvLayout), I32, I32, I32, I32]
     lib.tri_topk_rows.argtypes = [P, I64, I32, P, P, I32, I32, P, I32, P]
     lib.tri_compact_paged.argtypes = [C.POINTER(KvLayout), C.POINTER(Batch), P, I32, I32, P]

@@ -610,6 +610,16 @@ int tri_describe_plan(const tri_kv_layout* kv, const tri_batch* batch, const tri
   return TRI_OK;
 }
 
+int tri_small_launches(const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
+                       const tri_select_params* sel, int32_t assume_resident_workgroups) {
+  if (check_layout(kv, false) || check_batch(batch, false) || check_score(kv, sp) || check_select(sel)) return -1;
+  if (assume_resident_workgroups < 0) {
+    fail(TRI_ERR_INVALID_ARGUMENT, "assume_resident_workgroups %d", assume_resident_workgroups);
+    return -1;
+  }
+  return takes_small(plan(kv, batch, sp, assume_resident_workgroups), kv, batch, sp, sel) ? 1 : 0;
+}
+
 int32_t tri_score_tile_tokens(const tri_kv_layout* kv, int32_t num_seqs, int32_t max_seq_len, int32_t num_score_heads,
                               int32_t aggregation) {
   if (check_layout(kv, false) || num_seqs <= 0 || max_seq_len <= 0 || num_score_heads <= 0 ||

@@ -489,7 +489,9 @@ def select_paged(kv: PagedKV, batch: StepBatch, sc: ScoreConfig, sel: SelectConf
 def select_path(kv: PagedKV, batch: StepBatch, sc: ScoreConfig, sel: SelectConfig) -> str:
     """'resident_mfma' / 'resident_valu' when select_paged / compress_step run the single
     resident kernel (scoring on the matrix cores / on the vector unit) for these arguments
-    on the current device, else 'two_pass'."""
+    on the current device, else 'two_pass'.  A few layers of a few requests count as
+    'resident_mfma' too, though two short launches take that kernel's place
+    (describe_plan's "small_launches")."""
     sp, ss = sc.struct(), sel.struct()
     rc = int(_lib.load().tri_select_path(C.byref(kv.struct), C.byref(batch.struct), C.byref(sp), C.byref(ss)))
     if rc < 0:
@@ -508,12 +510,16 @@ def describe_plan(kv: PagedKV, batch: StepBatch, sc: ScoreConfig, sel: SelectCon
                   assume_resident_workgroups: int = 0) -> dict:
     """How select_paged / compress_step would cut these arguments into workgroups (``tri_describe_plan``):
     path, tile length, tiles of the longest sequence, layer groups, launches, workspace bytes --
-    for the current device, or for one that holds ``assume_resident_workgroups`` at once."""
+    for the current device, or for one that holds ``assume_resident_workgroups`` at once.  "small_launches"
+    is 1 where two short launches run in place of the resident kernel (``tri_small_launches``); the rest is then
+    the resident plan that the workspace is sized for."""
     sp, ss, info = sc.struct(), sel.struct(), _lib.PlanInfo()
     _lib.check(_lib.load().tri_describe_plan(C.byref(kv.struct), C.byref(batch.struct), C.byref(sp), C.byref(ss),
                                              int(assume_resident_workgroups), C.byref(info)))
     out = {name: int(getattr(info, name)) for name, _ in _lib.PlanInfo._fields_}
     out["path"] = {2: "resident_mfma", 1: "resident_valu"}.get(out["path"], "two_pass")
+    out["small_launches"] = int(_lib.load().tri_small_launches(C.byref(kv.struct), C.byref(batch.struct), C.byref(sp),
+                                                               C.byref(ss), int(assume_resident_workgroups)))
     return out
 
 
