@@ -1522,7 +1522,7 @@ def test_small_launches_match_the_two_pass_kernels(kv_dtype, head_dim, heads, la
     for kw in (dict(), dict(normalize=False, layer_reduce="max"), dict(group_reduce="mean", protect_prefill=True)):
         sel = ops.SelectConfig(window_size=w.window_size, **kw)
         tune(resident_kernel="auto")
-        too_much = lens == (4097, 16) and heads in ((8, 8), (24, 3), (14, 2))
+        too_much = lens == (4097, 16) and heads in ((8, 8), (24, 3), (14, 2), (12, 4))
         assert ops.describe_plan(kv, batch, sc, sel)["small_launches"] == (0 if too_much else 1)
         keep_s, fin_s, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
         keep_only, _, _ = ops.select_paged(kv, batch, sc, sel)

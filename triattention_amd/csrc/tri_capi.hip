@@ -4,6 +4,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <algorithm>
 #include <atomic>
 #include <climits>
 #include <mutex>
@@ -282,13 +283,31 @@ bool takes_quarter_tiles(const tri_kv_layout* kv, int B, int Tmax, int A, int ag
 }
 
 // A few layers of a few requests, where the resident kernel would be taken for them, go through
-// tri_score_small.hip: a wave per step of 16 tokens, statistics in the selection's workgroups.  Score + select, us, resident
-// / small, by workgroups (128 tokens of a KV head of a layer), four query heads per KV head of 128: 1 layer x 4096
-// tokens (256) 32.1 / 17.5, x 8192 (512) 36.6 / 23.2, 3 x 4096 (768) 32.3 / 22.0, 2 layers x 8192 (1024) 37.8 / 34.5, 3 x 4096 (768)
-// 33.7 / 26.9; beyond 1024 workgroups every one of them evaluates the phases again for too little.  With eight query heads
-// the selection walks a layer in 5 us: 1 layer, 3 x 4096 (768) 25.8 / 23.1, 2 layers x 4096 (512) 26.9 / 23.3, but
-// 2 layers, 3 x 4096 of four KV heads (768) 27.4 / 31.1 and 3 x 4096 (768) 27.0 / 30.9.
-constexpr int64_t kSmallWorkgroups = 1024;
+// tri_score_small.hip: a wave per step of 16 tokens, statistics in the selection's workgroups.  Which of the two is faster goes by
+//  - the scorer's workgroups (128 tokens of a KV head of a layer), each of which evaluates the phases again: one round
+//    of the chip is 1024 of them, 512 at a head dimension of 256;
+//  - the layers, which the selection walks one after the other, the longer the more tokens a thread holds of a row: up to
+//    4096 tokens four (one query head per KV head 8192, eight), beyond that twice as many;
+//  - what the resident kernel costs: with at most four KV heads its workgroups have four waves and it is about 5 us faster.
+// Score + select on the GPU, us, resident / small, `layers x requests x tokens, KV heads x head dimension, workgroups`.  Three
+// or four query heads per KV head: 1 x 1 x 4096, 8 x 128, 256: 29.7 / 14.5; 1 x 3 x 5376, 8 x 256, 1008: 40.7 / 39.7;
+// 2 x 1 x 4096, 16 x 128, 1024: 31.5 / 27.3; 3 x 1 x 4096, 8 x 128, 768: 30.6 / 26.7; 4 x 1 x 2412, 8 x 128, 608: 29.7 / 28.0,
+// but 4 x 2 x 2048, 8 x 128, 1024: 29.7 / 31.4.  Four KV heads: 3 x 4 x 1554, 4 x 64, 624: 23.0 / 22.5, but 3 x 4 x 2688,
+// 4 x 128, 1008: 25.9 / 29.7; 2 x 2 x 3239, 4 x 256, 416: 30.3 / 25.4, but 2 x 8 x 1220, 4 x 256, 640: 28.8 / 31.9.  Long rows:
+// 2 x 1 x 6784, 8 x 128, 848: 33.9 / 33.9, 2 x 1 x 7678, 4 x 64, 480: 28.4 / 24.9, but 2 x 3 x 5038, 4 x 128, 960: 27.5 / 33.2,
+// 3 x 1 x 5376, 8 x 128, 1008: 33.7 / 36.2, 4 x 1 x 8192, 4 x 128, 1024: 31.4 / 42.8, 4 x 1 x 4170, 1 x 64, 132: 25.1 / 30.7.
+// One query head: 4 x 2 x 2048, 8 x 128, 1024: 29.6 / 27.2; 2 x 1 x 14202, 4 x 128, 888: 36.6 / 35.5, but 4 x 1 x 16384, 2 x 128,
+// 1024: 39.3 / 43.1.  Eight: 1 x 1 x 4096, 8 x 128, 256: 30.3 / 18.9; 2 x 1 x 4096, 8 x 128, 512: 31.9 / 25.9, but 1 x 8 x 4096,
+// 4 x 128, 1024: 26.5 / 30.8, 2 x 4 x 2555, 2 x 128, 320: 22.6 / 24.8.  Of 830 shapes drawn over 1 to 4 layers, 1 to 8 query heads,
+// 1 to 16 KV heads of 64 to 256 and 64 to 1024 workgroups 690 go this way, six of them more than 2 % slower (at most 1.1 x).
+int64_t small_workgroups(int L, int G, int D, int Tmax, bool four_waves) {
+  const bool wide = D == 256, long_rows = Tmax > (G == 1 ? 8192 : 4096);
+  if (G > 4) return L > 2 ? 0 : four_waves ? (wide ? 256 : 512) / L : L == 1 ? 768 : 512;
+  if (L > 4 || (long_rows && L > 2)) return 0;
+  if (long_rows) return four_waves ? (L == 2 || wide ? 512 : 1024) : (L == 2 && wide ? 768 : 1024);
+  const int layers_times = (G == 1 ? 4096 : 3072) / (four_waves ? 2 : 1);
+  return std::min(four_waves && wide ? 512 : 1024, layers_times / L);
+}
 bool takes_small(const tri::Workspace& w, const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
                  const tri_select_params* sel) {
   const int G = sp->num_score_heads / kv->num_kv_heads, L = kv->num_layers;
@@ -296,7 +315,7 @@ bool takes_small(const tri::Workspace& w, const tri_kv_layout* kv, const tri_bat
   return tri::tuning(TRI_TUNE_RESIDENT_KERNEL) == 0 && takes_resident(w, kv, sel) && w.fused.eligible == 2 &&
          kv->kv_dtype != TRI_KV_FP8_E4M3 && tri::select_small_takes(batch->max_seq_len, G) &&
          (int64_t)batch->num_seqs * kv->num_kv_heads <= 256 &&
-         (G > 4 ? L <= 2 && wgs * L <= kSmallWorkgroups : L <= 4 && wgs <= kSmallWorkgroups);
+         wgs <= small_workgroups(L, G, kv->head_dim, batch->max_seq_len, w.fused.waves == 4);
 }
 
 // Selection straight from the paged keys: the resident kernel when the shape has one,
