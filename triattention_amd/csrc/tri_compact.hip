@@ -116,8 +116,7 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs a) {
   if (guard_raised(a.guard)) return;
 
   int idx = blockIdx.x;
-  const int chains = gridDim.x / a.cols;
-  const int col = idx / chains; idx %= chains;
+  const int col = blockIdx.y;
   const int head = idx % a.Hkv;
   const Unit unit = unit_of(a, idx / a.Hkv);
   const int kv = unit.kv, l = unit.l, b = unit.b;
@@ -608,13 +607,13 @@ hipError_t launch_compact(const CompactLaunch& a, hipStream_t s) {
     CompactArgs one = c;
     if (chains <= 256) {
       // A workgroup takes a CU's rate, so few chains take pieces of a row: of a cache line, or of half a line where a chain's
-      // pieces share an XCD and its L2 (compact_kernel numbers the pieces slowest: workgroups `chains` apart).
+      // pieces share an XCD and its L2 (the grid numbers the pieces slowest: workgroups `chains` apart).
       // One layer x 4096 -> 2048 tokens, rows of 256 bytes, called over and over / behind a flush of the caches, us: two
       // pieces 10.0 / 22.8, four 8.5 / 20.1, eight 9.7 / 19.8 (four on XCDs as they come 11.0); rows of 512 bytes
       // 15.1 / 34.5 with two, 10.2 / 23.0 with eight; rows of 128 bytes 9.4 / 20.3 whole, 8.0 / 18.2 in two.
       const int piece = chains % 8 == 0 ? 64 : 128;
       while (chains * one.cols * 2 <= 256 && c.chunks_per_row * 16 / (one.cols * 2) >= piece) one.cols *= 2;
-      hipLaunchKernelGGL((compact_kernel<1024, 8, true>), dim3(chains * one.cols), dim3(1024), 0, s, one);
+      hipLaunchKernelGGL((compact_kernel<1024, 8, true>), dim3(chains, one.cols), dim3(1024), 0, s, one);
     } else if (chains <= 1024) {
       hipLaunchKernelGGL((compact_kernel<256, 8, true>), dim3(chains), dim3(256), 0, s, one);
     } else {
