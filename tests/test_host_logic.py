@@ -979,3 +979,29 @@ def test_matrix_instructions_wait_for_what_inline_asm_wrote(tmp_path):
                 runs += 1
                 assert re.fullmatch(r"s_nop [1-9]", behind), behind
     assert runs > 0
+
+
+def test_dense_call_takes_switches_of_any_kind_that_has_a_truth_value(monkeypatch):
+    """The switches of ``ops.dense_compress`` are converted to C integers whatever they came as: a numpy bool, a tensor
+    of one element, a float.  (The library is replaced by a recorder: there is no GPU here.)"""
+    import ctypes as C
+    import types
+
+    import numpy as np
+    import torch
+    from triattention_amd import ops
+    seen = []
+
+    def workspace_bytes(ref):
+        p = C.cast(ref, C.POINTER(_lib.DenseParams)).contents
+        seen.append((p.num_heads, p.num_tokens, p.head_dim, p.budget, p.window_size, p.normalize, p.round_start, p.disable_mlr,
+                     p.disable_trig))
+        return 256
+    monkeypatch.setattr(_lib, "load", lambda: types.SimpleNamespace(tri_dense_workspace_bytes=workspace_bytes,
+                                                                    tri_dense_compress=lambda *a: 0))
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    k = torch.zeros(1, 2, 8, 64, dtype=torch.bfloat16)
+    stats = [torch.zeros(2, 32, 2), torch.zeros(2, 32), torch.zeros(2, 32), torch.zeros(32), torch.zeros(17)]
+    for yes, no in ((True, False), (np.bool_(True), np.bool_(False)), (torch.tensor(True), torch.tensor(False)), (1.0, 0.0)):
+        ops.dense_compress(k, k, *stats, budget=4, round_start=8, window_size=2, normalize=yes, disable_mlr=no, disable_trig=yes)
+        assert seen.pop() == (2, 8, 64, 4, 2, 1, 8, 0, 1)

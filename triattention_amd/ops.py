@@ -557,8 +557,8 @@ def dense_compress(keys: torch.Tensor, values: torch.Tensor, q_mean_complex: tor
     # (in the order of the fields: by name they cost 3 us of a call whose kernels take 20)
     p = _lib.DenseParams(
         h, t, d, _DTYPES[keys.dtype], ROPE_INTERLEAVED if rope_style == "interleaved" else ROPE_HALF, budget, window_size,
-        normalize, round_start, offsets.numel(), REDUCE_MAX if aggregation == "max" else REDUCE_MEAN, disable_mlr,
-        disable_trig, values.shape[3] * v_es, keys.data_ptr(), values.data_ptr(), ks[1] * k_es, ks[2] * k_es, vs[1] * v_es,
+        int(normalize), round_start, offsets.numel(), REDUCE_MAX if aggregation == "max" else REDUCE_MEAN, int(disable_mlr),
+        int(disable_trig), values.shape[3] * v_es, keys.data_ptr(), values.data_ptr(), ks[1] * k_es, ks[2] * k_es, vs[1] * v_es,
         vs[2] * v_es, q_mean_complex.data_ptr(), q_abs_mean.data_ptr(), freq_scale_sq.data_ptr(), omega.data_ptr(),
         offsets.data_ptr(), out_k.data_ptr(), out_v.data_ptr(), keep.data_ptr())
     need = int(lib.tri_dense_workspace_bytes(C.byref(p)))
