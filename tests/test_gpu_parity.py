@@ -1064,7 +1064,7 @@ def test_matrix_core_scores_carry_every_piece(kv_dtype, head_dim, monkeypatch):
                                                  ("fp16", 64, 6), ("fp8", 128, 8)])
 def test_every_piece_of_five_to_eight_query_heads(kv_dtype, head_dim, g, monkeypatch):
     """The operand layout of five to eight query heads per KV head (two pieces side by side, the third in an
-    operand of its own; two pieces of the magnitude coefficients): same bound as with four.  Tiles that end
+    operand of its own, of the magnitude coefficients too): same bound as with four.  Tiles that end
     inside a step, one token into it and at its end."""
     w = small(kv_dtype=kv_dtype, head_dim=head_dim, num_q_heads=3 * g, num_kv_heads=3, seq_lens=(1201, 1000, 33), index=78)
     _assert_scores_carry_every_piece(w)
@@ -1475,7 +1475,7 @@ def test_quarter_tile_scores_give_the_sums_of_whole_tiles(kw, lens):
         assert torch.equal(fin_a[b * h:(b + 1) * h, :t], fin_b[b * h:(b + 1) * h, :t]), (b, t)
 
 
-@pytest.mark.parametrize("offsets", [16, 17, 18, 21])
+@pytest.mark.parametrize("offsets", [16, 17, 18, 21, 25, 32])
 @pytest.mark.parametrize("lens,layers,heads", [((1500, 1, 513), 1, (6, 2)), ((3000, 130, 2049, 511), 16, (40, 8))],
                          ids=["a_tile_a_workgroup", "runs_over_units_and_sequences"])
 def test_max_aggregation_runs_of_tiles(lens, layers, heads, offsets, monkeypatch):
@@ -1806,8 +1806,8 @@ def test_research_path_selection_matches_oracle(hq, hkv, decode_start, keep_coun
     """``hf_selection.select_keep_indices_per_head`` (decode tokens only, population std clamped at 1e-6,
     group max, layer mean, no window) against ``oracle.selection.hf_keep_per_head``, whose selection is
     pinned by the reference's own ``_select_per_head_independent`` (tests/golden/hf_select.pt); on the
-    kernels the library picks for so small a step (two-pass) and on either resident kernel, which
-    evaluate the same population statistics in their gather."""
+    kernels the library picks for so small a step (the two short launches with up to four query heads, else the
+    resident kernel by layers) and on either resident kernel, which evaluate the same population statistics in their gather."""
     from triattention_amd import hf_selection
     if kernel == "valu" and hq // hkv > 4:
         pytest.skip("the vector-unit resident kernel takes up to four query heads per KV head")

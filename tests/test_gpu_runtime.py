@@ -420,7 +420,7 @@ def test_batch_hook_on_the_resident_kernel(tmp_path, monkeypatch):
 @pytest.mark.parametrize("tokens,kv_heads,two_pass", [(1185, 8, True), (3072, 6, True), (3072, 2, False)])
 def test_hook_call_for_one_small_request_takes_the_kernels_that_do_not_wait(tmp_path, monkeypatch, tokens, kv_heads, two_pass):
     """A single request below the selector's limit takes the score-then-select kernels (and gives their bits); a
-    shape without quarter tiles keeps the library's own choice, the resident kernel."""
+    shape without quarter tiles keeps the library's own choice, here the short launches in the resident kernel's place."""
     from helpers import build_inputs
     from triattention_amd import ops, synth
     paths, select_path = [], ops.select_path
@@ -448,8 +448,9 @@ def test_hook_call_for_one_small_request_takes_the_kernels_that_do_not_wait(tmp_
                                                         (None, "auto", 2, True)],
                          ids=["small", "whole_tiles", "kernel_by_name", "two_requests"])
 def test_hook_waits_for_the_status_word_only_where_it_takes_a_resident_kernel(tmp_path, monkeypatch, tile, kernel, requests, waits):
-    """The rule for one small request: the library's quarter tiles (where its answer is whole tiles, the resident
-    kernel), no kernel asked for by name, one request.  Eager, captured and replayed calls alike."""
+    """The rule for one small request: the library's quarter tiles (where its answer is whole tiles, the library's own
+    choice: the resident kernel or the short launches in its place), no kernel asked for by name, one request.  Eager,
+    captured and replayed calls alike."""
     from helpers import build_inputs
     from triattention_amd import ops, synth
     if kernel != "auto":
@@ -534,18 +535,19 @@ def test_hook_calls_on_two_streams_do_not_share_what_is_in_flight(tmp_path, monk
             assert not torch.equal(a.view(torch.int16), c0.view(torch.int16))
 
 
-@pytest.mark.parametrize("resident", [False, True])
+@pytest.mark.parametrize("resident", [False, True, "mfma"])
 def test_repeated_shape_replays_a_graph_with_the_same_results(tmp_path, monkeypatch, resident):
     """A decoding request comes back to the hook with the same lengths every ``divide_length``
     tokens: from the second visit on the selector replays a captured launch sequence.  Eight steps
     with fresh cache contents, other block lists, other round starts and a prefill guard that comes
     and goes, next to a selector that never replays: equal results, bit-identical caches after every
-    step (the program's own eager work and synchronisations lie between the replays)."""
+    step (the program's own eager work and synchronisations lie between the replays).  On the two-pass kernels, on what the
+    library picks for so little (the two short launches) and on the resident kernel."""
     from helpers import build_inputs
     from triattention_amd import synth
     from triattention_amd.runtime import selector as selector_mod
-    if not resident:
-        tune(resident_kernel="off")
+    if resident is not True:
+        tune(resident_kernel=resident or "off")
     w = synth.Workload(name="t", num_layers=3, num_q_heads=8, num_kv_heads=2, head_dim=128,
                        seq_lens=(1184,) * (16 if resident else 1), budget=160, block_size=16, window_size=12,
                        rope_theta=1e6, index=41)
