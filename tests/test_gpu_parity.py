@@ -1476,11 +1476,12 @@ def test_quarter_tile_scores_give_the_sums_of_whole_tiles(kw, lens):
 
 
 @pytest.mark.parametrize("offsets", [16, 17, 18, 21, 25, 32])
-@pytest.mark.parametrize("lens,layers,heads", [((1500, 1, 513), 1, (6, 2)), ((3000, 130, 2049, 511), 16, (40, 8))],
-                         ids=["a_tile_a_workgroup", "runs_over_units_and_sequences"])
+@pytest.mark.parametrize("lens,layers,heads", [((1500, 1, 513), 1, (6, 2)), ((3000, 130, 2049, 511), 16, (40, 8)),
+                                               ((2600, 90, 513, 1537), 11, (35, 5)), ((700, 1100), 9, (80, 80))],
+                         ids=["a_tile_a_workgroup", "runs_over_units_and_sequences", "runs_not_a_multiple_of_eight", "few_runs_a_head"])
 def test_max_aggregation_runs_of_tiles(lens, layers, heads, offsets, monkeypatch):
-    """The matrix-core kernel for max aggregation cuts all tiles of a ragged batch into 512 equal runs, which end and begin
-    inside (layer, head) units and sequences, and lays offset 16 out by pieces when it is the only one beyond the
+    """The matrix-core kernel for max aggregation cuts a head's tiles of a ragged batch into equal runs, up to 512 over
+    all heads, which end and begin inside layers and sequences, and lays offset 16 out by pieces when it is the only one beyond the
     first sixteen: raw scores against the vector-unit kernel to 1e-5 of the per-head RMS."""
     w = small(num_q_heads=heads[0], num_kv_heads=heads[1], num_layers=layers, seq_lens=lens, budget=64, index=93)
     inp = build_inputs(w)

@@ -19,6 +19,8 @@
 // two exchange steps each lane of a quad owns one query head, a half-row mirror
 // adds the two quads, so lanes 0-3 / 4-7 of a row hold duplicates; those two quads
 // store two different tokens with a single instruction.
+#include <algorithm>
+
 #include "tri_common.h"
 #include "tri_score_device.h"
 #include <cstdlib>
@@ -684,28 +686,33 @@ void score_max_mfma_kernel(ScoreArgs a, int B) {
   float* red = tsin + a.NO * kTrigPitch;                       // [2][waves][4 heads][2]
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // All tiles of the batch in a row -- sequence, then unit (layer, KV head), then tile -- cut into
-  // equal runs: with eight tiles a workgroup, 2 x 8192 tokens x 36 layers were 1152 workgroups on 512 places, two and a
-  // quarter rounds that took three.  The operand slabs depend on everything but the tile and are built (as many
-  // vector instructions as scoring 400 tokens) where a run enters another unit: a place of their own in front of a
-  // unit's tiles, or the runs over short sequences would be the longer ones.  The groups of four query heads of a run
-  // go to workgroups eight apart, which start together on one XCD and find each other's keys in its L2.
-  const int per_seq = a.L * a.Hkv;
-  const bool apart = gridDim.x % (8 * a.QC) == 0;
-  const int qc = (apart ? blockIdx.x / 8 : blockIdx.x) % a.QC;
-  const int run = apart ? blockIdx.x / (8 * a.QC) * 8 + blockIdx.x % 8 : blockIdx.x / a.QC, runs = gridDim.x / a.QC;
+  // All tiles of a KV head in a row -- sequence, then layer, then tile -- cut into equal runs: with eight tiles a
+  // workgroup, 2 x 8192 tokens x 36 layers were 1152 workgroups on 512 places, two and a quarter rounds that took
+  // three.  The operand slabs depend on everything but the tile and are built (as many vector instructions as scoring
+  // 400 tokens) where a run enters another layer: a place of their own in front of a layer's tiles, or the runs
+  // over short sequences would be the longer ones.  The same run of every KV head and group of four query heads
+  // goes to workgroups eight apart, which start together on one XCD: groups find each other's keys in its L2, and the
+  // 16 bytes that every head writes of a token's raw row come in at about the same time.  (Runs through the heads of a
+  // layer one after the other wrote the eight pieces of a line a millisecond apart: of 75.6 M write requests none was of
+  // 64 bytes, of 74.2 M 14.4 M are now.  Selection of 16 x 16384 tokens x 36 layers, 32 query heads to a line, 7.6 -> 6.2 ms, 6.6 with
+  // the workgroups of eight tiles; 2 x 8192 410 -> 385 us.)
+  const int columns = a.Hkv * a.QC;
+  const bool apart = gridDim.x % (8 * columns) == 0;
+  const int column = (apart ? blockIdx.x / 8 : blockIdx.x) % columns;
+  const int head = column / a.QC, qc = column % a.QC;
+  const int run = apart ? blockIdx.x / (8 * columns) * 8 + blockIdx.x % 8 : blockIdx.x / columns, runs = gridDim.x / columns;
   auto length = [&](int s) { return min(a.seq_lens[s], a.num_tiles * kScoreTileTokens); };
   auto places = [&](int s) { const int t = ceil_div(length(s), kScoreTileTokens); return t > 0 ? t + 1 : 0; };
   int64_t total = 0;
-  for (int s = lane; s < B; s += 64) total += (int64_t)places(s) * per_seq;
+  for (int s = lane; s < B; s += 64) total += (int64_t)places(s) * a.L;
   for (int d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d);
   int64_t skip = total * run / runs;
   int64_t left = total * (run + 1) / runs - skip;
   int b = 0;
-  while (b < B && skip >= (int64_t)places(b) * per_seq) skip -= (int64_t)places(b++) * per_seq;
+  while (b < B && skip >= (int64_t)places(b) * a.L) skip -= (int64_t)places(b++) * a.L;
   if (left <= 0 || b >= B) return;                     // (the same for the whole workgroup)
   int seq_len = length(b), tiles = ceil_div(seq_len, kScoreTileTokens);
-  int unit = (int)(skip / (tiles + 1)), tile = (int)(skip % (tiles + 1)) - 1;
+  int l = (int)(skip / (tiles + 1)), tile = (int)(skip % (tiles + 1)) - 1;
   if (tile < 0) { tile = 0; --left; }
   if (left <= 0) return;
 
@@ -718,8 +725,7 @@ void score_max_mfma_kernel(ScoreArgs a, int B) {
   constexpr int TW = kScoreTileTokens / kMaxMfmaWaves;
 
   for (;;) {
-  // ---- the operand slabs of unit (layer, KV head) for this group of query heads
-  const int l = unit / a.Hkv, head = unit % a.Hkv;
+  // ---- the operand slabs of this layer for this group of query heads
   const int q0 = qc * kMaxMfmaHeads, nq = min(kMaxMfmaHeads, a.G - q0);
   __syncthreads();                              // (everyone is done with the previous ones)
   for (int i = threadIdx.x; i < 3 * kMaxMfmaHeads * F; i += kMaxMfmaThreads) {
@@ -859,7 +865,7 @@ void score_max_mfma_kernel(ScoreArgs a, int B) {
   const int wstart = n0 + wave * TW;
   const int wend = min(wstart + TW, n1);
   float s1 = 0.f, s2 = 0.f;
-  const Rows next = rows_of(min(tile + 1, tiles - 1));     // (a workgroup's last tile of a unit reads a few rows in vain)
+  const Rows next = rows_of(min(tile + 1, tiles - 1));     // (a workgroup's last tile of a layer reads a few rows in vain)
 
   // What follows the key products of one 16-token step: magnitude term, maxima, stores.
   auto finish = [&](const uint4 (&A)[4], mx_f32x4 (&acc)[NT], const mx_f32x4& accx, int t0) __attribute__((always_inline)) {
@@ -1055,18 +1061,18 @@ void score_max_mfma_kernel(ScoreArgs a, int B) {
     out[0] = t1;
     out[1] = t2;
   }
-  }   // tiles of this unit
-  if (--left <= 0) break;                       // (the next unit's build)
+  }   // tiles of this layer
+  if (--left <= 0) break;                       // (the next layer's build)
   tile = 0;
-  if (++unit == per_seq) {
-    unit = 0;
+  if (++l == a.L) {
+    l = 0;
     do {
       if (++b >= B) return;
       seq_len = length(b);
       tiles = ceil_div(seq_len, kScoreTileTokens);
     } while (tiles <= 0);
   }
-  }   // units of this workgroup
+  }   // layers of this workgroup
 }
 
 template <int NX, bool PIECES>
@@ -1076,9 +1082,13 @@ hipError_t launch_max_mfma_nx(const ScoreArgs& k, int B, int il, hipStream_t s) 
                       : reinterpret_cast<const void*>(&score_max_mfma_kernel<NX, PIECES, false>);
   hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  const int64_t tiles = (int64_t)k.num_tiles * B * k.L * k.Hkv;
-  const int runs = max(kMaxMfmaWorkgroups / k.QC, 1);
-  const dim3 grid((unsigned)((tiles < runs ? tiles : runs) * k.QC));
+  // Runs of every (KV head, group of four query heads): a multiple of eight, which puts a run's workgroups on one XCD,
+  // where that leaves hardly a place of the chip empty.
+  const int columns = k.Hkv * k.QC;
+  const int64_t tiles = (int64_t)k.num_tiles * B * k.L;
+  int64_t runs = std::min<int64_t>(std::max(kMaxMfmaWorkgroups / columns, 1), tiles);
+  if (runs / 8 * 8 * 16 >= runs * 15) runs = runs / 8 * 8;
+  const dim3 grid((unsigned)(runs * columns));
   if (il) hipLaunchKernelGGL((score_max_mfma_kernel<NX, PIECES, true>), grid, dim3(kMaxMfmaThreads), lds, s, k, B);
   else hipLaunchKernelGGL((score_max_mfma_kernel<NX, PIECES, false>), grid, dim3(kMaxMfmaThreads), lds, s, k, B);
   return hipGetLastError();
