@@ -662,7 +662,7 @@ int tri_topk_rows(const float* scores, int64_t row_pitch, int32_t num_rows, cons
 namespace {
 
 // Workgroups of 128 tokens and a head up to which a dense call goes through the small launch's kernels (8 heads: 600 tokens
-// 44.5 -> 31.9 us, 4096 45.0 -> 32.0, 12000 60.3 -> 35.5, 16384 53.8 -> 39.0, of 256 elements 73.2 -> 52.9; longer rows
+// 38 -> 21 us, 4096 44 -> 21, 9000 56 -> 35, 16384 52 -> 37, of 256 elements 57 -> 49; 128 heads of 256 x 2048 tokens 100 -> 98; longer rows
 // do not fit the selection's registers).
 constexpr int64_t kDenseSmallWorkgroups = 2048;
 

@@ -1,8 +1,8 @@
 // In-place, order-preserving paged K/V compaction for gfx950.
 //
 // keep[] is strictly ascending, so keep[j] >= j: destination slot j always lies at
-// or below its source.  One workgroup owns one (sequence, layer, K or V, head), or half of such a
-// head's row, and walks the destination slots in ascending tiles.  Every tile is read completely
+// or below its source.  One workgroup owns one (sequence, layer, K or V, head), or a piece (a half to an
+// eighth) of such a head's row, and walks the destination slots in ascending tiles.  Every tile is read completely
 // into registers, the workgroup synchronises, then the tile is written: a tile's writes
 // land below the next tile's first slot while every later source lies at or above
 // it, so nothing that is still to be read is ever overwritten and no staging copy

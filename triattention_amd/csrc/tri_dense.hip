@@ -8,7 +8,7 @@
 // A layer of 4096 tokens is 4 us of memory traffic; the step was host work: four host-to-device copies of a few
 // numbers, twenty launches of ten libraries' operators around the scorer, 268 us a call.  One library call with seven
 // launches (these two, preparation, scorer, statistics, combination, top-k) and no copy: 45 us.  Up to 16384 tokens three
-// (tri_score_small.hip, which folds for itself, select_small_kernel and the gather): 32 us, of which the GPU works 20.
+// (tri_score_small.hip, which folds for itself, select_small_kernel and the gather): 28 us, of which the GPU works 20.
 #include "tri_common.h"
 
 namespace tri {

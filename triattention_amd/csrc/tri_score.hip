@@ -562,13 +562,13 @@ __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
 // rows and per-tile sums.
 //
 // What bounds it: matrix and vector instructions, which on this chip hardly overlap (a 16x16x32 product keeps the
-// vector unit from issuing for about 12 of its 16 cycles): 56 products and ~170 vector instructions a step, 33 % and
-// 42 % of the SIMDs' cycles on 2 x 8192 tokens x 36 layers, the rest in barriers, builds and the uneven end.  Selection of
-// that, us: 500 with workgroups of eight tiles (three rounds of 512 for two and a quarter rounds' work) and every
+// vector unit from issuing for about 12 of its 16 cycles): 56 products and ~170 vector instructions a step, with the builds 34 % and
+// 44 % of the SIMDs' cycles on 2 x 8192 tokens x 36 layers, the rest in barriers, builds and the uneven end.  The whole selection of
+// that (five launches, of which the scorer alone takes 357 to 480 in a trace of 20 passes), us: 500 with workgroups of eight tiles (three rounds of 512 for two and a quarter rounds' work) and every
 // operand read waited for before its products, 441 with equal runs of tiles, offset 16 in four operands and one idle
 // cycle pair per stage of the maxima, 415 with the operand reads four ahead, 405 with the keys of the next steps in
-// flight across tiles; ragged, 64 query heads, 2 x 3000 and 900 tokens x 64 layers 526 -> 436, 28 query / 4 KV heads, 3 of 1000
-// to 6000 506 -> 266.  Cutting the pieces off instead of rounding them makes the build cheaper and the case no faster.
+// flight across tiles, 385 with a run's heads side by side; ragged, 64 query heads, 2 x 3000 and 900 tokens x 64 layers
+// 526 -> 436, 28 query / 4 KV heads, 3 of 1000 to 6000 506 -> 266.  Cutting the pieces off instead of rounding them makes the build cheaper and the case no faster.
 typedef __bf16 mx_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float mx_f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kDppRor4 = 0x124;        // row_ror:4

@@ -887,8 +887,8 @@ __device__ __forceinline__ float row_sum_f32(float v) {
 // The statistics need the whole row, the row is a few thousand scores of a few query heads and the top-k
 // holds it in registers anyway: one launch in place of finalize_stats_kernel (or group_stats_kernel) and
 // combine_kernel, each 4 to 8 us in front of a 6 us top-k for a microsecond's worth of bytes.  Sixteen waves share a
-// CU, so what every wave does counts four times: sums of 64 scores by rows of lanes (fp32, as many as a resident tile's
-// lane adds up; in double where the reduce-first order has them so), the 64 partial sums of a head in double and its
+// CU, so what every wave does counts four times: sums of 64 scores, 128 of rows beyond 4096 tokens, by rows of lanes (fp32, at most as
+// many as a resident tile's lanes add up; in double where the reduce-first order has them so), the 64 partial sums of a head in double and its
 // statistics in one wave per head.
 // GQ: query heads of a KV head, rounded up to 1, 4 or 8.
 // A token whose z-scores are NaN ranks as combine_kernel ranks it: below every other (its general form starts each
