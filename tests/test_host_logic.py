@@ -870,22 +870,23 @@ def test_small_launches_are_reported():
     assert _small_launches(1, 14, 2, 256, [300, 16]) == 1 and _small_launches(1, 8, 8, 64, [16384], kv_dtype=1) == 1
     assert _small_launches(36, 32, 8, 128, [2176]) == 0                      # many layers
     # ... and where the resident kernel is the faster one: many workgroups in layers that the selection walks in turn
-    assert _small_launches(3, 32, 8, 128, [4096]) == 1 and _small_launches(4, 32, 8, 128, [3072]) == 1     # 768 workgroups
-    assert _small_launches(4, 32, 8, 128, [3073]) == 0 and _small_launches(4, 8, 8, 128, [4096]) == 1
+    assert _small_launches(4, 32, 8, 128, [4096]) == 1 and _small_launches(4, 40, 10, 128, [4096]) == 0    # 1024, 1280 workgroups
     assert _small_launches(5, 32, 8, 128, [128]) == 0
-    assert _small_launches(2, 32, 8, 128, [8192]) == 1 and _small_launches(3, 32, 8, 128, [4097]) == 0     # long rows
-    assert _small_launches(2, 32, 8, 256, [6144]) == 1 and _small_launches(2, 32, 8, 256, [6145]) == 0
-    assert _small_launches(4, 8, 8, 128, [4097]) == 0 and _small_launches(3, 1, 1, 128, [8193]) == 0
-    assert _small_launches(2, 4, 4, 128, [16384]) == 0 and _small_launches(2, 2, 2, 128, [16384]) == 1
+    assert _small_launches(2, 32, 8, 128, [8192]) == 1 and _small_launches(2, 8, 8, 128, [8193]) == 0      # long rows
+    assert _small_launches(3, 20, 5, 128, [6528]) == 1 and _small_launches(3, 20, 5, 128, [6529]) == 0     # 765, 780
+    assert _small_launches(4, 4, 1, 128, [4096]) == 1 and _small_launches(4, 4, 1, 128, [4097]) == 0
+    assert _small_launches(4, 1, 1, 128, [16384]) == 1 and _small_launches(4, 2, 2, 128, [8193]) == 0
     # ... whose workgroups of up to four KV heads are cheaper
-    assert _small_launches(3, 16, 4, 128, [5376 // 4] * 3) == 1 and _small_launches(3, 16, 4, 128, [1409] * 4) == 0
-    assert _small_launches(1, 16, 4, 128, [4096] * 8) == 1 and _small_launches(1, 16, 4, 256, [2048] * 8) == 1
-    assert _small_launches(1, 16, 4, 256, [2049] * 8) == 0
+    assert _small_launches(2, 16, 4, 128, [4097] * 2) == 1 and _small_launches(2, 16, 4, 128, [4097] * 3) == 0
+    assert _small_launches(3, 8, 2, 128, [4097] * 2) == 1 and _small_launches(3, 16, 4, 128, [5505]) == 0
+    assert _small_launches(4, 16, 4, 128, [1408] * 4) == 1 and _small_launches(4, 16, 4, 128, [1409] * 4) == 0
+    assert _small_launches(4, 4, 4, 128, [2048] * 4) == 1 and _small_launches(3, 16, 4, 128, [2688] * 4) == 1
+    assert _small_launches(3, 16, 4, 256, [640] * 8) == 1 and _small_launches(3, 16, 4, 256, [769] * 8) == 0
     # ... and with five to eight query heads
-    assert _small_launches(1, 64, 8, 128, [4096] * 3) == 1 and _small_launches(1, 64, 8, 128, [4096] * 4) == 0
+    assert _small_launches(1, 64, 8, 128, [4096] * 4) == 1 and _small_launches(1, 64, 8, 128, [4096] * 5) == 0
     assert _small_launches(2, 64, 8, 128, [4096]) == 1 and _small_launches(2, 64, 8, 128, [2049] * 2) == 0
-    assert _small_launches(1, 32, 4, 128, [4096] * 4) == 1 and _small_launches(1, 32, 4, 128, [4096] * 5) == 0
-    assert _small_launches(1, 32, 4, 256, [2048] * 4) == 1 and _small_launches(1, 32, 4, 256, [2049] * 4) == 0
+    assert _small_launches(1, 32, 4, 128, [4096] * 6) == 1 and _small_launches(1, 32, 4, 128, [4096] * 7) == 0
+    assert _small_launches(1, 32, 4, 256, [4096] * 4) == 1 and _small_launches(1, 32, 4, 256, [4096] * 5) == 0
     assert _small_launches(3, 64, 8, 128, [128]) == 0
     assert _small_launches(*one, kv_dtype=2) == 0                            # one-byte keys
     assert _small_launches(1, 32, 8, 128, [8193]) == 0                       # a row that does not fit the registers

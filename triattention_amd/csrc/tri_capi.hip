@@ -289,24 +289,25 @@ bool takes_quarter_tiles(const tri_kv_layout* kv, int B, int Tmax, int A, int ag
 //  - the layers, which the selection walks one after the other, the longer the more tokens a thread holds of a row: up to
 //    4096 tokens four (one query head per KV head 8192, eight), beyond that twice as many;
 //  - what the resident kernel costs: with at most four KV heads its workgroups have four waves and it is about 5 us faster.
-// Score + select on the GPU, us, resident / small, `layers x requests x tokens, KV heads x head dimension, workgroups`.  Three
-// or four query heads per KV head: 1 x 1 x 4096, 8 x 128, 256: 29.7 / 14.5; 1 x 3 x 5376, 8 x 256, 1008: 40.7 / 39.7;
-// 2 x 1 x 4096, 16 x 128, 1024: 31.5 / 27.3; 3 x 1 x 4096, 8 x 128, 768: 30.6 / 26.7; 4 x 1 x 2412, 8 x 128, 608: 29.7 / 28.0,
-// but 4 x 2 x 2048, 8 x 128, 1024: 29.7 / 31.4.  Four KV heads: 3 x 4 x 1554, 4 x 64, 624: 23.0 / 22.5, but 3 x 4 x 2688,
-// 4 x 128, 1008: 25.9 / 29.7; 2 x 2 x 3239, 4 x 256, 416: 30.3 / 25.4, but 2 x 8 x 1220, 4 x 256, 640: 28.8 / 31.9.  Long rows:
-// 2 x 1 x 6784, 8 x 128, 848: 33.9 / 33.9, 2 x 1 x 7678, 4 x 64, 480: 28.4 / 24.9, but 2 x 3 x 5038, 4 x 128, 960: 27.5 / 33.2,
-// 3 x 1 x 5376, 8 x 128, 1008: 33.7 / 36.2, 4 x 1 x 8192, 4 x 128, 1024: 31.4 / 42.8, 4 x 1 x 4170, 1 x 64, 132: 25.1 / 30.7.
-// One query head: 4 x 2 x 2048, 8 x 128, 1024: 29.6 / 27.2; 2 x 1 x 14202, 4 x 128, 888: 36.6 / 35.5, but 4 x 1 x 16384, 2 x 128,
-// 1024: 39.3 / 43.1.  Eight: 1 x 1 x 4096, 8 x 128, 256: 30.3 / 18.9; 2 x 1 x 4096, 8 x 128, 512: 31.9 / 25.9, but 1 x 8 x 4096,
-// 4 x 128, 1024: 26.5 / 30.8, 2 x 4 x 2555, 2 x 128, 320: 22.6 / 24.8.  Of 830 shapes drawn over 1 to 4 layers, 1 to 8 query heads,
-// 1 to 16 KV heads of 64 to 256 and 64 to 1024 workgroups 690 go this way, six of them more than 2 % slower (at most 1.1 x).
+// Score + select, called eagerly (the event that chains resident launches is 3 us of theirs; a captured launch has none), us,
+// resident / small, `layers x requests x tokens, KV heads x head dimension, workgroups`.  Two to four query heads per KV
+// head: 1 x 8 x 1987, 8 x 128, 1024: 31.0 / 24.9; 1 x 4 x 3923, 8 x 256, 992: 41.5 / 34.9; 2 x 1 x 3771, 16 x 128, 960:
+// 33.9 / 27.3; 3 x 3 x 1663, 8 x 64, 936: 29.6 / 25.1; 4 x 8 x 415, 8 x 128, 1024: 33.7 / 33.0.  Four KV heads: 2 x 4 x 3495, 4 x 64, 896:
+// 27.3 / 22.2; 3 x 8 x 1057, 4 x 128, 864: 28.0 / 26.4, but 3 x 8 x 1075, 4 x 256, 864: 32.1 / 36.4 and 4 x 3 x 2596, 4 x 64, 1008:
+// 27.0 / 28.2.  Long rows: 1 x 4 x 7782, 4 x 64, 976: 31.0 / 25.8; 2 x 1 x 7139, 8 x 128, 896: 36.7 / 32.2, but 2 x 3 x 5038, 4 x 128, 960:
+// 31.1 / 32.7, 3 x 1 x 5052, 8 x 128, 960: 35.7 / 37.7, 3 x 2 x 5036, 4 x 128, 960: 31.5 / 37.8, 4 x 1 x 4170, 1 x 64, 132: 27.9 / 30.9 and
+// 4 x 1 x 7652, 4 x 256, 960: 39.5 / 51.0.  One query head: 4 x 1 x 7964, 4 x 64, 1008: 33.2 / 28.7; 2 x 1 x 14202, 4 x 128, 888:
+// 38.7 / 35.4, but 3 x 1 x 8914, 4 x 128, 840: 36.4 / 37.3, 4 x 1 x 14881, 2 x 128, 936: 40.4 / 42.7.  Eight: 1 x 4 x 3821, 8 x 128, 960:
+// 32.7 / 30.4; 2 x 2 x 3534, 4 x 128, 448: 27.4 / 25.6, but 1 x 8 x 3770, 4 x 128, 960: 26.7 / 29.9.  Of 830 shapes drawn over 1 to
+// 4 layers, 1 to 8 query heads, 1 to 16 KV heads of 64 to 256 and 64 to 1024 workgroups 760 go this way, two of them more than
+// 2 % slower (1.04 x), and seven of the others would be more than 2 % faster.
 int64_t small_workgroups(int L, int G, int D, int Tmax, bool four_waves) {
   const bool wide = D == 256, long_rows = Tmax > (G == 1 ? 8192 : 4096);
-  if (G > 4) return L > 2 ? 0 : four_waves ? (wide ? 256 : 512) / L : L == 1 ? 768 : 512;
-  if (L > 4 || (long_rows && L > 2)) return 0;
-  if (long_rows) return four_waves ? (L == 2 || wide ? 512 : 1024) : (L == 2 && wide ? 768 : 1024);
-  const int layers_times = (G == 1 ? 4096 : 3072) / (four_waves ? 2 : 1);
-  return std::min(four_waves && wide ? 512 : 1024, layers_times / L);
+  if (L > (G > 4 ? 2 : 4)) return 0;
+  if (G > 4) return std::min(1024 / L, four_waves ? (wide ? 512 : 768) : 1024);
+  if (long_rows) return L == 1 ? 1024 : L == 2 ? (four_waves && G > 1 ? 768 : 1024) : L == 3 ? (four_waves ? 512 : 768) : G == 1 ? 512 : 0;
+  if (four_waves && G > 1 && L >= 3) return wide ? 512 : L == 4 ? 704 : 1024;
+  return 1024;
 }
 bool takes_small(const tri::Workspace& w, const tri_kv_layout* kv, const tri_batch* batch, const tri_score_params* sp,
                  const tri_select_params* sel) {
