@@ -7,15 +7,15 @@
 //
 // with k[n][.] the 128 cached elements of one KV head of token n (bf16, exact), C the P / R
 // coefficients laid out per element, E the magnitude coefficients.  One wave owns one KV
-// head.  An MFMA multiplies a 16-token x 32-element slab of keys, taken straight from the
-// 16-byte loads (no unpacking), with a 32 x 16 coefficient slab whose columns are
-// (query head, split): every fp32 coefficient is carried as three bf16 pieces
+// head.  An MFMA multiplies a 16 x 32 coefficient slab whose rows are (query head, split) with a
+// 32-element x 16-token slab of keys, taken straight from the 16-byte loads (no
+// unpacking): every fp32 coefficient is carried as three bf16 pieces
 // c = c1 + c2 + c3, so the products are exact and the sum is an fp32 accumulation of the
 // same terms the vector-unit kernel adds.  The magnitudes are evaluated on the vector unit
 // in fp32 (sqrt(k_r^2 + k_i^2)), cut into two fp16 pieces and contracted the same way
 // (v_mfma_f32_16x16x32_f16 against fp16 pieces of the magnitude coefficients).
-// The three column groups of a query head are added with row rotations, which leaves every
-// token's four scores spread over the lanes exactly as the ring in LDS wants them.
+// The pieces of a query head are rows of one lane's accumulator and add up there; every
+// token's four scores are then spread over the lanes exactly as the ring in LDS wants them.
 //
 // Per 16 tokens of a head: 8 MFMAs, and vector work only for the magnitudes (about a third
 // of the vector-unit kernel's instruction count), so bf16 keys run at the key stream's pace.
@@ -32,8 +32,6 @@
 namespace tri {
 namespace {
 
-constexpr int kDppRor4 = 0x124;   // row_ror:4
-constexpr int kDppRor8m = 0x128;  // row_ror:8
 
 // What a lane loads of one (token, head) row per step; the token is lane % 16 of the step,
 // kb = lane / 16.  Two-byte keys: the 16-byte chunks 4*s + kb, s = 0..3 (8 elements each,
@@ -41,10 +39,10 @@ constexpr int kDppRor8m = 0x128;  // row_ror:8
 // MFMA s takes half s % 2 of chunk s / 2) and the dequantisation scale of the token this
 // lane will store.
 // HD: head dimension, 128 or (two-byte keys only) 64: half the chunks, MFMAs and pairs.
-template <int DT, int HD, int QG>
+template <int DT, int HD>
 struct StepData {
   uint4 c[DT == TRI_KV_FP8_E4M3 ? 2 : HD / 32];
-  float scale[QG];      // fp8 only
+  float scale;          // fp8 only
 };
 
 // Index, inside the 128 elements of a head row, of element e of lane block kb in MFMA s.
@@ -118,12 +116,12 @@ __device__ __forceinline__ float coefficient_piece(float x, int pieces) {
 //    means over the offsets, the way prepare_kernel does (phase_cos_sin, means summed in offset
 //    order in double);
 //  - combines the means with the folded statistics of its KV heads of layer l (heads z * heads_per_wg
-//    and up) into P = a1*C - a2*S, R = a2*C + a1*S, E and writes them as MFMA B operands:
+//    and up) into P = a1*C - a2*S, R = a2*C + a1*S, E and writes them as MFMA A operands:
 // bmat[((b*L + l)*Hkv + head)*NSO + o][lane][8] of two bytes.  Lane (j = lane % 16, kb) of an operand holds
-// column j, k indices kb*8 .. + 7 of its slab.  Up to four query heads per KV head: operands 0..NS-1 are the
-// key slabs, NS/2 magnitude slabs follow; column j = (query head j % 4, piece j / 4).  Five to eight: NS key
-// operands with column j = (query head j % 8, piece j / 8), NS more with the third piece in columns 0..7 and
-// zeros beside it, then the magnitude operands the same way.  Piece p of a coefficient x is
+// row j, k indices kb*8 .. + 7 of its slab.  Up to four query heads per KV head: operands 0..NS-1 are the
+// key slabs, NS/2 magnitude slabs follow; row j = (query head j / 4, piece j % 4).  Five to eight: NS key
+// operands with row j = (query head j / 2, piece j % 2), NS more with the third piece in the even rows and
+// zeros between, then the magnitude operands the same way.  Piece p of a coefficient x is
 // what is left of x after p roundings to the operand type (x = x1 + x2 + x3).
 constexpr int kPrepThreads = 1024;
 // Query heads whose coefficients are staged at a time, and the pitch of a staged head
@@ -202,13 +200,13 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
       const int j = lane & 15, kb = lane >> 4;
       const bool mag = o >= NK;
       const int slab = mag ? (o - NK) % (NS / 2) : o % NS;
-      int q, sp;                                            // query head and piece of column j (piece 3: a zero column)
+      int q, sp;                                            // query head and piece of row j (piece 3: a zero row)
       if (G > 4) {
-        q = j & 7;
-        sp = (mag ? o - NK >= NS / 2 : o >= NS) ? (j < 8 ? 2 : 3) : j >> 3;
+        q = j >> 1;
+        sp = (mag ? o - NK >= NS / 2 : o >= NS) ? ((j & 1) ? 3 : 2) : j & 1;
       } else {
-        q = j & 3;
-        sp = j >> 2;
+        q = j >> 2;
+        sp = j & 3;
       }
       uint32_t out[4] = {0, 0, 0, 0};
       if (q < G && sp < 3) {
@@ -252,18 +250,17 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
 
 // QG: groups of four query heads per KV head (1 or 2).
 //
-// Two groups (five to eight query heads): a second operand set per group of four would leave a quarter of the
-// matrix columns empty twice and every step with two column reductions (three columns per head, four
-// values each, both groups: 34 of its 84 vector instructions at a head dimension of 64).  Instead the
-// columns are (query head, piece 1 | piece 2) and a second operand holds the third pieces beside zeros: two
-// accumulators for all eight heads, added before the one exchange between column halves at the end -- (piece 1 +
-// piece 3) + piece 2, every sum in the order in which the column reduction took it, so the scores and the
-// statistics are the bits that two operand sets give.  Vector instructions a step: 84 -> 60 at a head dimension of
-// 64, 166 -> 101 at 128; matrix instructions 8 and 16 as before.  With the lane-parallel statistics
-// (gather_head_stats) 24 requests of 1500 to 12001 tokens x 36 layers x 64 query heads of 64 take 1114 us in place of
-// 1314, 1 x 32768 x 64 layers x 64 of 128 802 in place of 827 (there the layers' statistics are waited for, not the
-// instructions).  One accumulator and two pieces of the magnitude coefficients (6 and 12 matrix instructions) give
-// 1081 and 796, with the same error, but round differently: a near-tie then shifts a kept list of 12000.
+// Rows of an operand are ordered so that one lane's four accumulator values are the pieces of its own head (one group) or
+// heads (two): they add up in two or four instructions.  With the tokens as rows and (query head, piece) as columns the
+// pieces sat in other lanes, 16 and 14 instructions of row rotations and selections a step; the sums are the same bits.
+// By itself that is worth 1.4 % at a head dimension of 64 (24 requests of 1500 to 12001 tokens x 36 layers x 64 query heads
+// of 64: 1116 -> 1097 us) and nothing where the key stream or the other tiles are waited for.
+//
+// Two groups (five to eight query heads): a second operand set per group of four would leave a quarter of the rows
+// empty twice.  Instead the rows are (query head, piece 1 | piece 2) and a second operand holds the third pieces beside
+// zeros: two accumulators for all eight heads, added at the end -- (piece 1 + piece 3) + piece 2, every sum in the
+// order of one group's.  One accumulator and two pieces of the magnitude coefficients (6 and 12 matrix instructions for 8 and
+// 16) have the same error, but round differently: a near-tie then shifts a kept list of 12000.
 __device__ __forceinline__ int nsteps_of(int ntok) { return (ntok + 15) >> 4; }
 
 // W: waves per workgroup.  Eight (one workgroup per CU), or four for models with at most four
@@ -306,7 +303,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int heads_here = min(8, a.Hkv - chunk * 8);
 
   float* ring = lds + wave * (RING * RQ);                      // [QG][RING][4 query heads]
-  float* part = lds + W * (RING * RQ);                         // [waves][64][QG][2]
+  float* part = lds + W * (RING * RQ);                         // [waves][16 tokens of a step][4*QG query heads][2]
   float* stats = part + W * 128 * QG;                          // [2][32*QG score heads][2]
   uint32_t* ctl = reinterpret_cast<uint32_t*>(stats + 128 * QG);  // arrive count, claimed, ready; [8..15]: how far each wave is
   for (int i = threadIdx.x; i < W * 128 * QG; i += W * kWave) part[i] = 0.f;
@@ -316,12 +313,9 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   if (wave >= heads_here) return;
   const int head = chunk * 8 + wave;
 
-  const int j = lane & 15, kb = lane >> 4;       // MFMA column / k block; also output row block
-  // What this lane ends up with of a step: one group: the score of query head q = j % 4 for the step's token
-  // 4 kb + j / 4; two: of query head q = j % 8 for the tokens 4 kb + 2 (j / 8) and the one after.
-  const int q = QG == 1 ? j & 3 : j & 7;
-  const int rsel = QG == 1 ? j >> 2 : 2 * (j >> 3);
-  const bool upper = j >= 8;
+  // MFMA column (token of the step) and k block; kb is the output's row block too: this lane ends up with the step's
+  // token j, its score of query head kb (one group) or of the heads 2 kb and 2 kb + 1 (two).
+  const int j = lane & 15, kb = lane >> 4;
 
   // Coefficient slabs of the current layer.
   uint4 B[NSO];
@@ -367,7 +361,10 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const uint32_t tok_bytes = (uint32_t)(a.stride_token * ES);
   const uint32_t lane_row = (uint32_t)j * tok_bytes;
   const uint32_t lane_col = (uint32_t)kb * 16u;
-  const uint32_t lane_scale_row = (uint32_t)(4 * kb + rsel) * (uint32_t)a.Hkv * 4u;   // fp8: token this lane stores
+  // fp8: four lanes side by side load the scale of one token, so that sixteen lanes touch one line and not four (every
+  // lane its own token's: 8 x 16384 tokens x 32 layers 850 -> 900 us); scale_lane is where the scale of this lane's token is.
+  const uint32_t lane_scale_row = (uint32_t)(lane >> 2) * (uint32_t)a.Hkv * 4u;
+  const int scale_lane = 16 * j;
   struct LayerBase { const char* k; const char* scale; };   // of this wave's head (scalar registers)
   auto layer_base = [&](int l) __attribute__((always_inline)) {
     LayerBase lb;
@@ -391,7 +388,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     step_off_hi = (uint32_t)((uint64_t)off >> 32);
     if constexpr (FP8) step_slot = step_blk * a.block_size + in_blk;
   }
-  auto load_step = [&](StepData<DT, HD, QG>& d, const LayerBase& lb, int t) __attribute__((always_inline)) {
+  auto load_step = [&](StepData<DT, HD>& d, const LayerBase& lb, int t) __attribute__((always_inline)) {
     const int step = t >> 4;
     const uint32_t rows_left = (uint32_t)(last_tok - (n0 + t));
     const uint64_t row_off = ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)step_off_hi, step) << 32) |
@@ -408,24 +405,22 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       const uint32_t hkv4 = (uint32_t)a.Hkv * 4u;
       const uint64_t slot_off = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(step_slot, step) * hkv4;
       const char* sc = reinterpret_cast<const char*>(uniform_ptr(lb.scale + slot_off));
-#pragma unroll
-      for (int i = 0; i < QG; ++i)
-        d.scale[i] = *(GlobalF32)((GlobalBytes)(uintptr_t)sc + min(lane_scale_row + (uint32_t)i * hkv4, rows_left * hkv4));
+      d.scale = *(GlobalF32)((GlobalBytes)(uintptr_t)sc + min(lane_scale_row, rows_left * hkv4));
     }
   };
 
   // Ring of this wave: [group of four query heads][RING tokens][4], so that the 16-byte reads of consecutive
   // tokens are 16 bytes apart, whatever the number of groups.  With one group the 64 lanes of a store (16 tokens x
-  // 4 heads) cover 64 consecutive words; with two a store takes every second token of both groups, whose words fall
-  // on the same half of the banks (1.1 % of the cycles of 8 x 32768 tokens x 64 layers).
-  const uint32_t lane_ring = (uint32_t)(q >> 2) * (RING * 4) + (uint32_t)(4 * kb + rsel) * 4 + (q & 3);
-  float s1[QG] = {}, s2[QG] = {};       // sums of this lane's i-th token of every step
+  // 4 heads) cover 64 consecutive words; with two a lane's pair of heads is one 8-byte store, and either half of the
+  // wave covers 64 consecutive words of its group.
+  const uint32_t lane_ring = QG == 1 ? (uint32_t)(4 * j + kb) : (uint32_t)(kb >> 1) * (RING * 4) + (uint32_t)(4 * j + 2 * (kb & 1));
+  float s1[QG] = {}, s2[QG] = {};       // sums of this lane's i-th head over the steps
   // Largest of a sample of the layer's magnitudes (their first fp16 pieces), per lane; see the check
   // after every layer.
   f16x2 mag_seen = {(_Float16)0.f, (_Float16)0.f};
-  // Scores of the 16 tokens of a step: MFMAs over keys and magnitudes, split columns added
-  // by row rotations; lane (j, kb) ends up with the score of token 4*kb + j/4, query head j%4.
-  auto compute_step = [&](const StepData<DT, HD, QG>& raw, int l, int t, int which) __attribute__((always_inline)) {
+  // Scores of the 16 tokens of a step: MFMAs over keys and magnitudes, then the pieces of a head, which are rows of
+  // one lane's accumulator, are added.
+  auto compute_step = [&](const StepData<DT, HD>& raw, float scale, int l, int t, int which) __attribute__((always_inline)) {
     // The four bf16 A operands of the step as dwords (two elements each): the loaded
     // registers for bf16 keys, one conversion per dword (exact) for fp8 keys.
     uint32_t w[NS][4];
@@ -470,11 +465,11 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     for (int s = 0; s < NS; ++s) d.c[s] = uint4{w[s][0], w[s][1], w[s][2], w[s][3]};
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < NS; ++s) acc = mfma_16x16x32<DT>(d.c[s], B[s], acc);
+    for (int s = 0; s < NS; ++s) acc = mfma_16x16x32<DT>(B[s], d.c[s], acc);
     f32x4 acc3 = {0.f, 0.f, 0.f, 0.f};
     if constexpr (QG == 2) {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) acc3 = mfma_16x16x32<DT>(d.c[s], B[NS + s], acc3);
+      for (int s = 0; s < NS; ++s) acc3 = mfma_16x16x32<DT>(B[NS + s], d.c[s], acc3);
     }
 #pragma unroll
     for (int set = 0; set < NS / 2; ++set) {
@@ -510,48 +505,41 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       if constexpr (!FP8)   // `which` is the step buffer's number: a constant after unrolling
         mag_seen = pk_max_f16(mag_seen, (&hi.x)[which & 3]);
       constexpr int MT = TRI_KV_FP16;                // operand type of the magnitude MFMAs
-      acc = mfma_16x16x32<MT>(hi, B[NK + set], acc);
-      acc = mfma_16x16x32<MT>(lo, B[NK + set], acc);
+      acc = mfma_16x16x32<MT>(B[NK + set], hi, acc);
+      acc = mfma_16x16x32<MT>(B[NK + set], lo, acc);
       if constexpr (QG == 2) {
-        acc3 = mfma_16x16x32<MT>(hi, B[NK + NS / 2 + set], acc3);
-        acc3 = mfma_16x16x32<MT>(lo, B[NK + NS / 2 + set], acc3);
+        acc3 = mfma_16x16x32<MT>(B[NK + NS / 2 + set], hi, acc3);
+        acc3 = mfma_16x16x32<MT>(B[NK + NS / 2 + set], lo, acc3);
       }
     }
-    // The pieces of a head are added across the columns; v[i] is then the score of this lane's i-th token.
+    // v[i]: the score of this lane's token and its i-th head.
     float v[QG];
     if constexpr (QG == 1) {
-      v[0] = 0.f;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float x = acc[r];
-        x += dpp<kDppRor8m>(x);
-        x += dpp<kDppRor4>(x);
-        v[0] = (rsel == r) ? x : v[0];
-      }
+      v[0] = (acc[0] + acc[2]) + acc[1];
     } else {
-      const float x0 = acc[0] + acc3[0], x1 = acc[1] + acc3[1], x2 = acc[2] + acc3[2], x3 = acc[3] + acc3[3];
-      const float send0 = upper ? x0 : x2, send1 = upper ? x1 : x3;
-      v[0] = (upper ? x2 : x0) + dpp<kDppRor8m>(send0);
-      v[1] = (upper ? x3 : x1) + dpp<kDppRor8m>(send1);
+      v[0] = (acc[0] + acc3[0]) + acc[1];
+      v[1] = (acc[2] + acc3[2]) + acc[3];
     }
     // first ring slot of the step (scalar; a step never straddles the wrap: t and RING are
     // multiples of 16).  The ring has a place for every row of the step and every head slot: rows past the
-    // tile's last token and slots beyond the last query head (zero columns) are written too and never read.
+    // tile's last token and slots beyond the last query head (zero rows) are written too and never read.
     const uint32_t slot0 = (uint32_t)(l * a.ring_stride + t) % RING;
     if (t + 16 > ntok) {                              // (wave-uniform: the last step of a tile)
       asm volatile("");
 #pragma unroll
       for (int i = 0; i < QG; ++i)
-        if (t + 4 * kb + rsel + i >= ntok) v[i] = 0.f;
+        if (t + j >= ntok) v[i] = 0.f;
     }
+    float score[QG];
 #pragma unroll
     for (int i = 0; i < QG; ++i) {
-      // (one-byte keys: the row's scale multiplies the finished score)
-      const float score = FP8 ? v[i] * raw.scale[i] : v[i];
-      ring[slot0 * 4 + lane_ring + 4 * i] = score;
-      s1[i] = FP8 ? fmaf(v[i], raw.scale[i], s1[i]) : s1[i] + v[i];
-      s2[i] = fmaf(score, score, s2[i]);
+      score[i] = FP8 ? v[i] * scale : v[i];
+      s1[i] = FP8 ? fmaf(v[i], scale, s1[i]) : s1[i] + v[i];
+      s2[i] = fmaf(score[i], score[i], s2[i]);
     }
+    float* entry = ring + slot0 * 4 + lane_ring;
+    if constexpr (QG == 1) *entry = score[0];
+    else *reinterpret_cast<float2*>(entry) = float2{score[0], score[1]};
   };
 
   bool aborted = false;
@@ -568,8 +556,9 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   auto arrive = [&](int l) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < QG; ++i) {
-      part[((wave * 64 + lane) * QG + i) * 2] = s1[i];
-      part[((wave * 64 + lane) * QG + i) * 2 + 1] = s2[i];
+      float* p = part + ((wave * 16 + j) * (4 * QG) + QG * kb + i) * 2;
+      p[0] = s1[i];
+      p[1] = s2[i];
       s1[i] = 0.f;
       s2[i] = 0.f;
     }
@@ -582,10 +571,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     for (int item = lane; item < items; item += 64) {
       const int ahl = item >> 1, which = item & 1;
       const int w = ahl / a.G, qq = ahl - w * a.G;
-      constexpr int kLanes = 16 / QG;                // lanes that hold scores of one query head
       float t = 0.f;
-      for (int i = 0; i < kLanes; ++i)               // in token order
-        for (int u = 0; u < QG; ++u) t += part[((w * 64 + i * (4 * QG) + qq) * QG + u) * 2 + which];
+      for (int i = 0; i < 16; ++i) t += part[((w * 16 + i) * (4 * QG) + qq) * 2 + which];   // in token order
       xchg_store(out + item, ((unsigned long long)(uint32_t)(l + 1) << 32) | __float_as_uint(t));
     }
   };
@@ -736,10 +723,14 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int nsteps = (ntok + 15) >> 4;
   const int rotations = (nsteps + NB - 1) / NB;
   const int rot_before_consume = min((RING - a.ring_stride) / (16 * NB), rotations);
-  auto score = [&](const StepData<DT, HD, QG>& d, int l, int slot, int which) __attribute__((always_inline)) {
-    if (slot < nsteps) compute_step(d, l, slot * 16, which);
+  auto score = [&](const StepData<DT, HD>& d, int l, int slot, int which) __attribute__((always_inline)) {
+    // One-byte keys: the scale of this lane's token, from the lane that loaded it (requested in front of the branch, or
+    // the compiler asks for it where it is used and waits there).
+    float scale = 1.f;
+    if constexpr (FP8) scale = __int_as_float(__builtin_amdgcn_ds_bpermute(scale_lane, __float_as_int(d.scale)));
+    if (slot < nsteps) compute_step(d, scale, l, slot * 16, which);
   };
-  StepData<DT, HD, QG> buf[NB];
+  StepData<DT, HD> buf[NB];
   LayerBase base_cur = layer_base(l_begin), base_next = base_cur;
   // The two waves of a SIMD (waves i and i + 4 of a workgroup of eight) compete for its issue slots and
   // the arbiter prefers the older one: left alone, waves 0..3 of every workgroup run ahead, then wait at
