@@ -892,6 +892,18 @@ RESIDENT_CASES.update({
 })
 
 
+# Five to eight query heads: the slack ends inside a rotation of the step buffers, and a wave's sums pass through the
+# ring slots behind its tile.  Whole tiles, last tiles of one step, of the slack's seven and of one more, both rings.
+RESIDENT_CASES.update({
+    "g8_slack_whole_tiles_small_chip": dict(w=small(num_q_heads=64, num_kv_heads=8, budget=128, num_layers=3,
+                                                    seq_lens=(12288, 10241, 5232, 4721, 113, 16)), workgroups=24),
+    "g8_slack_short_ring": dict(w=small(num_q_heads=48, num_kv_heads=8, budget=128, num_layers=3,
+                                        seq_lens=(256, 272, 369, 129, 1))),
+    "g5_slack_hkv3": dict(w=small(num_q_heads=15, num_kv_heads=3, budget=128, num_layers=3,
+                                  seq_lens=(6144, 5121, 640, 17)), workgroups=12),
+})
+
+
 @pytest.mark.parametrize("case", ["one_request_36_layers", "one_request_split_by_layer", "one_request_uneven_layer_groups",
                                   "three_requests_split", "sixteen_requests"])
 def test_steady_state_step_matches_oracle(case, monkeypatch):

@@ -22,6 +22,7 @@
 // fp8 e4m3 keys are widened to bf16 (exact) in registers and take the same route; the
 // per-(token, head) scale multiplies the finished score.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "tri_common.h"
@@ -254,7 +255,8 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
 // heads (two): they add up in two or four instructions.  With the tokens as rows and (query head, piece) as columns the
 // pieces sat in other lanes, 16 and 14 instructions of row rotations and selections a step; the sums are the same bits.
 // By itself that is worth 1.4 % at a head dimension of 64 (24 requests of 1500 to 12001 tokens x 36 layers x 64 query heads
-// of 64: 1116 -> 1097 us) and nothing where the key stream or the other tiles are waited for.
+// of 64: 1116 -> 1097 us) and nothing where the key stream or the other tiles are waited for; the other 1 % of that shape and the
+// 7 % of 1 x 32768 tokens x 64 layers x 64 heads of 128 (802 -> 747) are `publish` and the longer ring.
 //
 // Two groups (five to eight query heads): a second operand set per group of four would leave a quarter of the rows
 // empty twice.  Instead the rows are (query head, piece 1 | piece 2) and a second operand holds the third pieces beside
@@ -274,7 +276,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   constexpr int NS = HD / 32;            // key slabs per step
   constexpr int NK = QG * NS;            // key operands (MFMAs) of a KV head
   constexpr int NSO = QG * (NS + NS / 2);   // all operands
-  static_assert(SL % (16 * NB) == 0, "the slack must hold whole rotations of the step buffers");
+  static_assert(SL % 16 == 0, "the slack must hold whole steps");
+  constexpr int kPart = SL / 16 % NB;    // steps by which the slack of a whole tile exceeds whole rotations
   // Token t of layer l sits at (l * ring_stride + t) % RING, ring_stride the tokens of this launch's tiles (at
   // most TW): what a tile leaves free of the ring is slack, down to SL for a whole tile.
   constexpr int RING = TW + SL;
@@ -303,10 +306,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int heads_here = min(8, a.Hkv - chunk * 8);
 
   float* ring = lds + wave * (RING * RQ);                      // [QG][RING][4 query heads]
-  float* part = lds + W * (RING * RQ);                         // [waves][16 tokens of a step][4*QG query heads][2]
-  float* stats = part + W * 128 * QG;                          // [2][32*QG score heads][2]
-  uint32_t* ctl = reinterpret_cast<uint32_t*>(stats + 128 * QG);  // arrive count, claimed, ready; [8..15]: how far each wave is
-  for (int i = threadIdx.x; i < W * 128 * QG; i += W * kWave) part[i] = 0.f;
+  float* stats = lds + W * (RING * RQ);                        // one group: [2][32 score heads][2]
+  uint32_t* ctl = reinterpret_cast<uint32_t*>(stats + (QG == 1 ? 128 : 0));  // claimed, ready; [8..15]: how far each wave is
   if (threadIdx.x < 16) ctl[threadIdx.x] = 0;
   __syncthreads();
   // From here on the waves of the workgroup run independently.
@@ -543,37 +544,36 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   };
 
   bool aborted = false;
-  uint32_t* arrive_cnt = ctl;
-  uint32_t* claimed = ctl + 1;
-  uint32_t* ready = ctl + 2;
+  uint32_t* claimed = ctl;
+  uint32_t* ready = ctl + 1;
   const int items = heads_here * a.G * 2;        // (score head, sum | sum of squares) of this workgroup
   const int ah0 = chunk * 8 * a.G;
 
-  // Deposit this wave's sums of layer l; the last wave of the workgroup to do so adds the
-  // lanes in a fixed order and publishes the tile's sums.  Every wave deposits layer l
-  // before any wave deposits layer l + 1 (a wave consumes layer l, which needs every
-  // deposit of layer l, before it finishes layer l + 1), so the counter never mixes layers.
-  auto arrive = [&](int l) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < QG; ++i) {
-      float* p = part + ((wave * 16 + j) * (4 * QG) + QG * kb + i) * 2;
-      p[0] = s1[i];
-      p[1] = s2[i];
-      s1[i] = 0.f;
-      s2[i] = 0.f;
+  // Publish this wave's sums of layer l.  The sixteen lanes of a row group hold a head's sums over the tokens that share
+  // a place in the step.  They are added in token order by the lane of each of the head's two words, through the ring
+  // slots of the next layer's first two steps (free: of the layer before nothing is left in the ring), which the sums are
+  // stored to as scores are.  So every wave has its own head's words on their way as soon as it is through; they used to
+  // meet in LDS, where the last wave of the workgroup added and published all of them: every head waited for the slowest
+  // one of every tile, and the 8 KB (two groups) are slack now.
+  auto publish = [&](int l) __attribute__((always_inline)) {
+    const uint32_t slot1 = (uint32_t)((l + 1) * a.ring_stride) % RING, slot2 = (uint32_t)((l + 1) * a.ring_stride + 16) % RING;
+    if constexpr (QG == 1) {
+      ring[slot1 * 4 + lane_ring] = s1[0];
+      ring[slot2 * 4 + lane_ring] = s2[0];
+    } else {
+      *reinterpret_cast<float2*>(ring + slot1 * 4 + lane_ring) = float2{s1[0], s1[1]};
+      *reinterpret_cast<float2*>(ring + slot2 * 4 + lane_ring) = float2{s2[0], s2[1]};
     }
-    uint32_t prev = 0;
-    if (lane == 0) prev = __hip_atomic_fetch_add(arrive_cnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-    prev = __builtin_amdgcn_readfirstlane(prev);
-    if (prev + 1 != (uint32_t)(l - l_begin + 1) * (uint32_t)heads_here) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    unsigned long long* out = a.xchg + (((int64_t)(b * a.L + l) * a.tiles_per_seq + tile) * a.A + ah0) * 2;
-    for (int item = lane; item < items; item += 64) {
-      const int ahl = item >> 1, which = item & 1;
-      const int w = ahl / a.G, qq = ahl - w * a.G;
+#pragma unroll
+    for (int i = 0; i < QG; ++i) { s1[i] = 0.f; s2[i] = 0.f; }
+    const int qq = lane >> 1, which = lane & 1;                 // lane: (query head, sum | sum of squares)
+    if (qq < a.G) {
+      const float* p = ring + (qq >> 2) * (RING * 4) + (which ? slot2 : slot1) * 4 + (qq & 3);
       float t = 0.f;
-      for (int i = 0; i < 16; ++i) t += part[((w * 16 + i) * (4 * QG) + qq) * 2 + which];   // in token order
-      xchg_store(out + item, ((unsigned long long)(uint32_t)(l + 1) << 32) | __float_as_uint(t));
+#pragma unroll
+      for (int i = 0; i < 16; ++i) t += p[4 * i];
+      xchg_store(a.xchg + (((int64_t)(b * a.L + l) * a.tiles_per_seq + tile) * a.A + ah0 + wave * a.G) * 2 + lane,
+                 ((unsigned long long)(uint32_t)(l + 1) << 32) | __float_as_uint(t));
     }
   };
 
@@ -605,7 +605,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       }
       won = __builtin_amdgcn_readfirstlane(won);
       if (won) {
-        gather_layer_stats(a, b, l, seq_tiles, T, ah0, items, stats + (l & 1) * 64 * QG, lane, aborted);
+        gather_layer_stats(a, b, l, seq_tiles, T, ah0, items, stats + (l & 1) * 64, lane, aborted);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         if (lane == 0)
           __hip_atomic_store(ready, (uint32_t)(l - l_begin + 1), __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -615,7 +615,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
           __builtin_amdgcn_s_sleep(2);
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-      const float* st = stats + (l & 1) * 64 * QG;
+      const float* st = stats + (l & 1) * 64;
 #pragma unroll
       for (int qq = 0; qq < RQ; ++qq)
         if (qq < a.G) {
@@ -722,7 +722,10 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // but key loads and scoring, and the work at layer boundaries sits between them.
   const int nsteps = (ntok + 15) >> 4;
   const int rotations = (nsteps + NB - 1) / NB;
-  const int rot_before_consume = min((RING - a.ring_stride) / (16 * NB), rotations);
+  // How far a layer is scored before the layer before it is turned into contributions (a part of a rotation can only lie
+  // inside one).
+  const int rot_before_consume = kPart ? min(((RING - a.ring_stride) / 16 - kPart) / NB, rotations - 1)
+                                       : min((RING - a.ring_stride) / (16 * NB), rotations);
   auto score = [&](const StepData<DT, HD>& d, int l, int slot, int which) __attribute__((always_inline)) {
     // One-byte keys: the scale of this lane's token, from the lane that loaded it (requested in front of the branch, or
     // the compiler asks for it where it is used and waits there).
@@ -739,24 +742,34 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // So each wave posts how far it is at every rotation and takes the higher priority while it is behind
   // its neighbour (8 x 32768 tokens x 64 layers 6.55 -> 6.48 ms, one-byte keys 1.70 -> 1.63 ms).
   uint32_t* progress = ctl + 8;
+  auto balance = [&](int l, int r) __attribute__((always_inline)) {
+    if constexpr (W == 8) {
+      const uint32_t mine = (uint32_t)((l - l_begin) * rotations + r);
+      if (lane == 0) __hip_atomic_store(progress + wave, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const uint32_t other = (uint32_t)__builtin_amdgcn_readfirstlane(
+          (int)__hip_atomic_load(progress + (wave ^ 4), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+      if (mine < other) __builtin_amdgcn_s_setprio(2);
+      else __builtin_amdgcn_s_setprio(0);
+    }
+  };
+  // Steps from .. to - 1 of rotation r (constants: every buffer has its registers).
+  auto steps = [&](int l, int r, auto from, auto to) __attribute__((always_inline)) {
+    const bool wrap = r + 1 >= rotations;
+    const LayerBase lb = {wrap ? base_next.k : base_cur.k, wrap ? base_next.scale : base_cur.scale};
+    const int s0 = wrap ? 0 : (r + 1) * NB;
+#pragma unroll
+    for (int i = decltype(from)::value; i < decltype(to)::value; ++i) {
+      score(buf[i], l, r * NB + i, i);
+      load_step(buf[i], lb, min(s0 + i, nsteps - 1) * 16);
+    }
+  };
+  constexpr std::integral_constant<int, 0> kFirst{};
+  constexpr std::integral_constant<int, kPart> kMiddle{};
+  constexpr std::integral_constant<int, NB> kLast{};
   auto rotate = [&](int l, int r0, int r1) __attribute__((always_inline)) {
     for (int r = r0; r < r1; ++r) {
-      if constexpr (W == 8) {
-        const uint32_t mine = (uint32_t)((l - l_begin) * rotations + r);
-        if (lane == 0) __hip_atomic_store(progress + wave, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        const uint32_t other = (uint32_t)__builtin_amdgcn_readfirstlane(
-            (int)__hip_atomic_load(progress + (wave ^ 4), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-        if (mine < other) __builtin_amdgcn_s_setprio(2);
-        else __builtin_amdgcn_s_setprio(0);
-      }
-      const bool wrap = r + 1 >= rotations;
-      const LayerBase lb = {wrap ? base_next.k : base_cur.k, wrap ? base_next.scale : base_cur.scale};
-      const int s0 = wrap ? 0 : (r + 1) * NB;
-#pragma unroll
-      for (int i = 0; i < NB; ++i) {
-        score(buf[i], l, r * NB + i, i);
-        load_step(buf[i], lb, min(s0 + i, nsteps - 1) * 16);
-      }
+      balance(l, r);
+      steps(l, r, kFirst, kLast);
     }
   };
   auto settle = [&]() __attribute__((always_inline)) { __builtin_amdgcn_s_waitcnt(0x0F70); };
@@ -769,8 +782,13 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     base_next = layer_base(min(l + 1, l_end - 1));
     settle();
     rotate(l, 0, rot_before_consume);
+    if constexpr (kPart != 0) {
+      balance(l, rot_before_consume);
+      steps(l, rot_before_consume, kFirst, kMiddle);
+    }
     if (l > l_begin) consume(l - 1);
-    rotate(l, rot_before_consume, rotations);
+    if constexpr (kPart != 0) steps(l, rot_before_consume, kMiddle, kLast);
+    rotate(l, rot_before_consume + (kPart != 0), rotations);
     if constexpr (!FP8) {
       // A magnitude beyond fp16's range (or a key that is not finite) has left an infinity or a NaN
       // in this layer's sums.
@@ -788,7 +806,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       mag_seen = f16x2{(_Float16)0.f, (_Float16)0.f};
       if ((__any(bad) || !__any(seen)) && lane == 0) atomicExch(a.status, 2u);
     }
-    if (a.normalize) arrive(l);
+    if (a.normalize) publish(l);
     if (l + 1 < l_end) load_coefs(l + 1);
   }
   consume(l_end - 1);
@@ -822,7 +840,7 @@ struct LaunchShape {
 
 template <int TW, int SL, int QG, int W>
 constexpr size_t mfma_lds_bytes() {
-  return ((size_t)W * (TW + SL) * 4 * QG + W * 128 * QG + 128 * QG + 16) * 4;
+  return ((size_t)W * (TW + SL) * 4 * QG + (QG == 1 ? 128 : 0) + 16) * 4;
 }
 
 template <int DT, bool IL, int TW, int SL, int QG, int NB, int W = kFusedWaves, int HD = 128>
@@ -923,15 +941,18 @@ hipError_t launch_mfma_tw(FusedArgs& k, const uint4* bmat, int tw, int waves, in
     // Two workgroups per CU: the ring of the largest tile with one rotation of slack less
     // (a smaller tile is a run-time argument inside it).
     constexpr int NB4 = DT == TRI_KV_FP8_E4M3 ? 8 : 4;
-    if (k.G > 4) return tw == 512 ? launch_mfma_t<DT, IL, 512, 64, 2, 4, 4>(k, bmat, shape, s)
+    if (k.G > 4) return tw == 512 ? launch_mfma_t<DT, IL, 512, 112, 2, 4, 4>(k, bmat, shape, s)
                                   : hipErrorInvalidValue;
     return tw == 1024 ? launch_mfma_t<DT, IL, 1024, 128, 1, NB4, 4>(k, bmat, shape, s)
                       : hipErrorInvalidValue;
   }
   if (k.G > 4) {
-    switch (tw) {   // eight query heads per KV head: 32 bytes of ring per token
-      case 512: return launch_mfma_t<DT, IL, 512, 64, 2, 4>(k, bmat, shape, s);
-      case 256: return launch_mfma_t<DT, IL, 256, 320, 2, 4>(k, bmat, shape, s);
+    // Eight query heads per KV head: 32 bytes of ring per token, and slack is what LDS has least of: 112 tokens, all
+    // there is, in place of 64 (1 x 32768 tokens x 64 layers 802 -> 747 us, with `publish`).  Head dimension 64 keeps 64, whole rotations:
+    // 1087 against 1103 us with 112 (24 requests of 1500 to 12001 tokens x 36 layers; a third copy of the steps for nothing).
+    switch (tw) {
+      case 512: return launch_mfma_t<DT, IL, 512, 112, 2, 4>(k, bmat, shape, s);
+      case 256: return launch_mfma_t<DT, IL, 256, 368, 2, 4>(k, bmat, shape, s);
       default: return hipErrorInvalidValue;
     }
   }
