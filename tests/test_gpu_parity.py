@@ -326,7 +326,7 @@ def test_group_selection_matches_reference_golden(tag, kw, path, fixture, monkey
     ("selector_c1_shape.pt", "resident_mfma", 3, 10),   # ... and in two launches (two sequences, then one)
     ("selector_c1_shape.pt", "resident_valu", 1, 5),
     # eight query heads per KV head (Qwen3-32B attention), 37 % kept: tiles of 512 tokens on the instance the
-    # 8 x 32768-token configuration runs (two column groups, slack of 64)
+    # 8 x 32768-token configuration runs (two groups of query heads)
     ("selector_c2_shape.pt", "two_pass", 1, None),
     ("selector_c2_shape.pt", "resident_mfma", 1, 10),
     ("selector_c2_shape.pt", "resident_mfma", 2, 10),   # two requests, one launch each

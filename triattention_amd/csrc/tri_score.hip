@@ -561,9 +561,9 @@ __global__ __launch_bounds__(kScoreThreads) void score_max_kernel(ScoreArgs a) {
 // for 17 offsets), then each wave takes two steps of 16 tokens at a time.  Outputs as score_max_kernel: raw
 // rows and per-tile sums.
 //
-// What bounds it: matrix and vector instructions, which on this chip hardly overlap (a 16x16x32 product keeps the
-// vector unit from issuing for about 12 of its 16 cycles): 56 products and ~170 vector instructions a step, with the builds 34 % and
-// 44 % of the SIMDs' cycles on 2 x 8192 tokens x 36 layers, the rest in barriers, builds and the uneven end.  The whole selection of
+// What bounds it: its key loads, 256-byte slices of token rows.  On 2 x 8192 tokens x 36 layers the selection takes 386 us; copies
+// for timing only took 225 without the key loads, 388 without the magnitudes, 385 with a quarter of the 56 products a step, 343
+// without the stores, 384 with one build of the slabs.  The whole selection of
 // that (five launches, of which the scorer alone takes 357 to 480 in a trace of 20 passes), us: 500 with workgroups of eight tiles (three rounds of 512 for two and a quarter rounds' work) and every
 // operand read waited for before its products, 441 with equal runs of tiles, offset 16 in four operands and one idle
 // cycle pair per stage of the maxima, 415 with the operand reads four ahead, 405 with the keys of the next steps in
