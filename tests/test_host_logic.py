@@ -982,6 +982,22 @@ def test_matrix_instructions_wait_for_what_inline_asm_wrote(tmp_path):
     assert runs > 0
 
 
+def test_lanes_that_read_each_others_words_are_ordered_for_the_compiler():
+    """Matrix-core scorer: a wave's lanes pass sums through the ring in LDS, and read scores that other lanes stored.
+    The hardware keeps the order; that the compiler has to keep it too is said between the stores and the reads, and
+    again before the slots are reused.  (Checked in the source: what one compiler makes of it shows nothing about the next.)"""
+    src = (tri_build.CSRC / "tri_fused_mfma.hip").read_text()
+    publish = src[src.index("auto publish = "):src.index("float fin[TW / 64];")]
+    order = "order_lds_of_wave();"
+    stores, reads = publish.index("s2[0], s2[QG - 1]};"), publish.index("t += p[4 * i];")
+    assert stores < publish.index(order) < reads < publish.rindex(order)
+    calls = [m.start() for m in re.finditer(r"\bconsume\(l", src)]
+    assert len(calls) == 2
+    for at in calls:
+        assert order in src[at - 60:at]
+    assert order in src[calls[0]:calls[0] + 60]
+
+
 def test_dense_call_takes_switches_of_any_kind_that_has_a_truth_value(monkeypatch):
     """The switches of ``ops.dense_compress`` are converted to C integers whatever they came as: a numpy bool, a tensor
     of one element, a float.  (The library is replaced by a recorder: there is no GPU here.)"""

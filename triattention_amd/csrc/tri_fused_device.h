@@ -157,6 +157,11 @@ __device__ __forceinline__ void xchg_store(unsigned long long* p, unsigned long 
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Between LDS stores of a wave and loads by which its lanes read each other's words, and between such loads and the stores
+// that reuse the words.  The hardware takes a wave's LDS operations in order, so this costs no instruction; the compiler
+// knows the addresses of one lane only and may otherwise move the one across the other.
+__device__ __forceinline__ void order_lds_of_wave() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
 // Entry l of a device-resident table of pointers, read through the constant address space:
 // a scalar load (tracked by its own counter), where a vector load would make the wave
 // wait for every key load issued before it.  The tables are never written by a kernel.

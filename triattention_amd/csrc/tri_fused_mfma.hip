@@ -585,6 +585,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     *reinterpret_cast<float2*>(ring + slot2 * 4 + lane_ring) = float2{s2[0], s2[QG - 1]};
 #pragma unroll
     for (int i = 0; i < QG; ++i) { s1[i] = 0.f; s2[i] = 0.f; }
+    order_lds_of_wave();
     const int qq = lane >> 1, which = lane & 1;                 // lane: (query head, sum | sum of squares)
     if (qq < a.G) {
       const float* p = ring + (qq >> 2) * (RING * 4) + (which ? slot2 : slot1) * 4 + (qq & 3);
@@ -594,6 +595,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       xchg_store(a.xchg + (((int64_t)(b * a.L + l) * a.tiles_per_seq + tile) * a.A + ah0 + wave * a.G) * 2 + lane,
                  ((unsigned long long)(uint32_t)(l + 1) << 32) | __float_as_uint(t));
     }
+    order_lds_of_wave();      // (the next layer's first steps go to the same slots)
   };
 
   float fin[TW / 64];
@@ -805,7 +807,11 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       balance(l, rot_before_consume);
       steps(l, rot_before_consume, kFirst, kMiddle);
     }
-    if (l > l_begin) consume(l - 1);
+    if (l > l_begin) {
+      order_lds_of_wave();
+      consume(l - 1);
+      order_lds_of_wave();
+    }
     if constexpr (kPart != 0) steps(l, rot_before_consume, kMiddle, kLast);
     rotate(l, rot_before_consume + (kPart != 0), rotations);
     if constexpr (!FP8) {
@@ -828,6 +834,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     if (a.normalize) publish(l);
     if (l + 1 < l_end) load_coefs(l + 1);
   }
+  order_lds_of_wave();
   consume(l_end - 1);
 
   if (a.layer_groups > 1) {
