@@ -904,6 +904,19 @@ RESIDENT_CASES.update({
 })
 
 
+# The same with at most four KV heads (workgroups of four waves, a device that holds 24 of them): sums that meet in LDS up to
+# seven query heads, every wave's own with eight.  Tiles of 512, as "plan" says: the longest sequence leaves room for no other.
+# Whole tiles, behind which the slack is four or five steps, and last tiles of 1, 4, 5 and 6 steps.
+FOUR_WAVES = dict(budget=128, num_layers=3, seq_lens=(12288, 10241, 5200, 4689, 4672, 1088, 16))
+for tag, heads, more in [("g5_hkv3", (15, 3), {}), ("g6_hkv4", (24, 4), dict(rope_style="interleaved")), ("g7_hkv4", (28, 4), {}),
+                         ("g8_hkv2", (16, 2), {}), ("g7_hkv2_fp16", (14, 2), dict(kv_dtype="fp16")),
+                         ("g7_hkv4_fp8", (28, 4), dict(kv_dtype="fp8")), ("g8_hkv1_fp8", (8, 1), dict(kv_dtype="fp8")),
+                         ("d64_g7_hkv4", (28, 4), dict(head_dim=64)), ("d64_g8_hkv2", (16, 2), dict(head_dim=64)),
+                         ("d256_g5_hkv2", (10, 2), dict(head_dim=256))]:
+    RESIDENT_CASES["four_waves_" + tag] = dict(w=small(num_q_heads=heads[0], num_kv_heads=heads[1], **FOUR_WAVES, **more),
+                                               workgroups=12, plan=dict(tile_tokens=512))
+
+
 @pytest.mark.parametrize("case", ["one_request_36_layers", "one_request_split_by_layer", "one_request_uneven_layer_groups",
                                   "three_requests_split", "sixteen_requests"])
 def test_steady_state_step_matches_oracle(case, monkeypatch):
@@ -956,7 +969,9 @@ def test_steady_state_step_matches_oracle(case, monkeypatch):
 # Named cases in which the two paths keep different indices at near-ties (scores within
 # KEEP_TIE_TOL of the threshold), and how many of the case's kept indices: 16 sequences x heads x
 # 256 kept indices each, two of which sit that close to their threshold.  Everywhere else: none.
-NEAR_TIES = {("fp16_tile192", "mfma"): 2, ("d64_tile_refined", "mfma"): 2}
+# (four_waves_d256_g5_hkv2: one pair of its 1568 kept indices, within the exact bound asserted below, and the same pair whichever
+# way the sums of a layer are published: the bits do not depend on that.)
+NEAR_TIES = {("fp16_tile192", "mfma"): 2, ("d64_tile_refined", "mfma"): 2, ("four_waves_d256_g5_hkv2", "mfma"): 2}
 
 
 @pytest.mark.parametrize("kernel", ["mfma", "valu"])
@@ -986,6 +1001,9 @@ def test_resident_selection_matches_two_pass(name, kernel, monkeypatch):
     selkw.update(case.get("sel", {}))
     sel = ops.SelectConfig(**selkw)
     assert ops.select_path(kv, batch, sc, sel) == "resident_" + kernel
+    if "plan" in case:                # what the case is there for
+        plan = ops.describe_plan(kv, batch, sc, sel)
+        assert {key: plan[key] for key in case["plan"]} == case["plan"], plan
     keep_r, fin_r, ws = ops.select_paged(kv, batch, sc, sel, want_scores=True)
     raw, ws2 = ops.score_paged(kv, batch, sc)
     keep_t, fin_t = ops.select(kv, batch, sc, sel, raw, ws2, want_scores=True)

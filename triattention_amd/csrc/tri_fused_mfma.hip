@@ -265,6 +265,9 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
 // 16) have the same error, but round differently: a near-tie then shifts a kept list of 12000.
 __device__ __forceinline__ int nsteps_of(int ntok) { return (ntok + 15) >> 4; }
 
+// LDS floats in which the sums of a layer meet (`publish`); none where every wave always publishes its own.
+constexpr int meeting_floats(int QG, int W) { return QG == 1 || W == 4 ? W * 128 * QG : 0; }
+
 // W: waves per workgroup.  Eight (one workgroup per CU), or four for models with at most four
 // KV heads: a workgroup of eight would leave half its waves without a head and the CU with half
 // the loads in flight, so two workgroups of four share a CU (half the LDS each; two waves per
@@ -306,8 +309,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int heads_here = min(8, a.Hkv - chunk * 8);
 
   float* ring = lds + wave * (RING * RQ);                      // [QG][RING][4 query heads]
-  float* part = lds + W * (RING * RQ);                         // one group: [waves][16 tokens of a step][4 query heads][2]
-  float* stats = part + (QG == 1 ? W * 128 : 0);               // one group: [2][32 score heads][2]
+  float* part = lds + W * (RING * RQ);                         // [waves][16 tokens of a step][RQ query heads][2], where sums meet
+  float* stats = part + meeting_floats(QG, W);                 // one group: [2][32 score heads][2]
   uint32_t* ctl = reinterpret_cast<uint32_t*>(stats + (QG == 1 ? 128 : 0));  // claimed, ready, arrived; [8..15]: how far each wave is
   if (threadIdx.x < 16) ctl[threadIdx.x] = 0;
   __syncthreads();
@@ -552,30 +555,43 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   const int ah0 = chunk * 8 * a.G;
 
   // Publish this wave's sums of layer l.  The sixteen lanes of a row group hold a head's sums over the tokens that share
-  // a place in the step.  They are added in token order by the lane of each of the head's two words, through the ring
-  // slots of the next layer's first two steps (free: of the layer before nothing is left in the ring), which the sums are
-  // stored to as scores are.  So every wave has its own head's words on their way as soon as it is through; they used to
-  // meet in LDS, where the last wave of the workgroup added and published all of them: every head waited for the slowest
-  // one of every tile, and the 8 KB (two groups) are slack now.
-  // One group: one wave fetches the statistics of all heads, so nothing is won by a head that comes early, and the sums
-  // still meet in LDS (16 x 16384 tokens x 36 layers 3135 us, 3142 with a publication per wave).  Every wave deposits
-  // layer l before any deposits layer l + 1 (it consumes layer l first), so the counter never mixes layers.
+  // a place in the step; the lane of each of the head's two words adds them in token order.
+  //
+  // Two groups, eight waves: every wave publishes its own, through the ring slots of the next layer's first two steps (free:
+  // of the layer before nothing is left in the ring), which the sums are stored to as scores are.  So a head's words are on
+  // their way as soon as its wave is through, where meeting in LDS lets every head wait for the slowest wave of every tile.
+  // 1 x 32768 tokens x 64 layers, 64 / 8 heads of 128, both with 64 tokens of slack: 829 -> 783 us; 40, 48, 56 / 8 heads gain
+  // as much (with 112: 849 -> 800, 849 -> 793, 854 -> 804).
+  //
+  // Meeting in LDS, where the last wave of the workgroup adds and publishes all of them:
+  //  - One group: one wave fetches the statistics of all heads, so nothing is won by a head that comes early (16 x 16384
+  //    tokens x 36 layers 3135 us, 3142 with a publication per wave).
+  //  - Two groups, four waves, fewer than eight query heads: a wave's words end inside a 128-byte line that the next
+  //    head's wave, and the next tile's workgroup, write too.  24 requests of 2500 to 11000 tokens x 28 layers, us with a
+  //    publication per wave | meeting: 898 | 856 for 20 / 4 heads of 128, 923 | 886 for 24 / 4, 935 | 896 for 28 / 4, but
+  //    684 | 691 for 32 / 4 (8 x 16384 tokens), whose waves publish whole lines; heads of 64 (16 x 16384 x 36) 1000 | 943 for
+  //    20 / 4, 896 | 915 for 32 / 4.  Padding every wave's words to a line takes 934 to 908 only, and scratch.
+  // Every wave deposits layer l before any deposits layer l + 1 (the last one to arrive has added by the time any wave gets
+  // past consuming layer l), so the counter never mixes layers.
   auto publish = [&](int l) __attribute__((always_inline)) {
-    if constexpr (QG == 1) {
-      float* mine = part + ((wave * 16 + j) * 4 + kb) * 2;
-      mine[0] = s1[0];
-      mine[1] = s2[0];
-      s1[0] = s2[0] = 0.f;
+    if (QG == 1 || (W == 4 && a.G < RQ)) {
+      float* mine = part + ((wave * 16 + j) * RQ + kb * QG) * 2;
+#pragma unroll
+      for (int i = 0; i < QG; ++i) {
+        mine[2 * i] = s1[i];
+        mine[2 * i + 1] = s2[i];
+        s1[i] = s2[i] = 0.f;
+      }
       uint32_t prev = 0;
       if (lane == 0) prev = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
       prev = __builtin_amdgcn_readfirstlane(prev);
       if (prev + 1 != (uint32_t)(l - l_begin + 1) * (uint32_t)heads_here) return;
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
       unsigned long long* out = a.xchg + (((int64_t)(b * a.L + l) * a.tiles_per_seq + tile) * a.A + ah0) * 2;
-      if (lane < items) {
+      if (lane < items) {                            // (at most 64: eight waves of four heads, four of seven)
         const int ahl = lane >> 1, w = ahl / a.G, qq = ahl - w * a.G;
         float t = 0.f;
-        for (int i = 0; i < 16; ++i) t += part[((w * 16 + i) * 4 + qq) * 2 + (lane & 1)];     // in token order
+        for (int i = 0; i < 16; ++i) t += part[((w * 16 + i) * RQ + qq) * 2 + (lane & 1)];     // in token order
         xchg_store(out + lane, ((unsigned long long)(uint32_t)(l + 1) << 32) | __float_as_uint(t));
       }
       return;
@@ -866,7 +882,7 @@ struct LaunchShape {
 
 template <int TW, int SL, int QG, int W>
 constexpr size_t mfma_lds_bytes() {
-  return ((size_t)W * (TW + SL) * 4 * QG + (QG == 1 ? W * 128 + 128 : 0) + 16) * 4;
+  return ((size_t)W * (TW + SL) * 4 * QG + meeting_floats(QG, W) + (QG == 1 ? 128 : 0) + 16) * 4;
 }
 
 template <int DT, bool IL, int TW, int SL, int QG, int NB, int W = kFusedWaves, int HD = 128>
@@ -965,9 +981,11 @@ hipError_t launch_mfma_tw(FusedArgs& k, const uint4* bmat, int tw, int waves, in
   }
   if (waves == 4) {
     // Two workgroups per CU: the ring of the largest tile with one rotation of slack less
-    // (a smaller tile is a run-time argument inside it).
+    // (a smaller tile is a run-time argument inside it).  Five to eight query heads: the 80 tokens that LDS has
+    // beside the ring and the sums (28 / 4 heads, 8 x 16384 tokens x 28 layers, bf16: 685 us, with 64 691; 1 x 32768
+    // 235 and 236; 3 x 5001 116.0 and 117.5).
     constexpr int NB4 = DT == TRI_KV_FP8_E4M3 ? 8 : 4;
-    if (k.G > 4) return tw == 512 ? launch_mfma_t<DT, IL, 512, 112, 2, 4, 4>(k, bmat, shape, s)
+    if (k.G > 4) return tw == 512 ? launch_mfma_t<DT, IL, 512, 80, 2, 4, 4>(k, bmat, shape, s)
                                   : hipErrorInvalidValue;
     return tw == 1024 ? launch_mfma_t<DT, IL, 1024, 128, 1, NB4, 4>(k, bmat, shape, s)
                       : hipErrorInvalidValue;
