@@ -991,12 +991,16 @@ hipError_t launch_mfma_tw(FusedArgs& k, const uint4* bmat, int tw, int waves, in
                       : hipErrorInvalidValue;
   }
   if (k.G > 4) {
-    // Eight query heads per KV head: 32 bytes of ring per token, and slack is what LDS has least of: 112 tokens, all
-    // there is, in place of 64 (1 x 32768 tokens x 64 layers 802 -> 747 us, with `publish`).  Head dimension 64 keeps 64, whole rotations:
-    // 1087 against 1103 us with 112 (24 requests of 1500 to 12001 tokens x 36 layers; a third copy of the steps for nothing).
+    // Five to eight query heads per KV head: 32 bytes of ring per token, and slack is what LDS has least of.  Tiles of up to 512:
+    // 112 tokens, all there is, in place of 64 (both with `publish` per wave, 64 layers, 64 / 8 heads: 1 x 32768 tokens 783 ->
+    // 770 us, 4 x 16384 1460 -> 1445, 13 of 2100 to 8000 2035 -> 2026; one-byte keys the same within 0.6 %: 8 x 16384 1913 and
+    // 1925, 1 x 32768 505 and 507).  Tiles of up to 256: 320 tokens, whole rotations and more than a tile; with 368, all there
+    // is, a layer would be consumed a step before its end and the code hold a third copy of the steps (5 x 13056 tokens x 64
+    // layers 1517 us with 368, 1513 with 320, one-byte keys 1150 and 1121; 17 x 3840 x 64 one-byte keys 1126 and 1113).  Head dimension 64 has whole rotations too: 1087 us with 64 tokens, 1103 with 112 (24 requests of
+    // 1500 to 12001 x 36 layers).
     switch (tw) {
       case 512: return launch_mfma_t<DT, IL, 512, 112, 2, 4>(k, bmat, shape, s);
-      case 256: return launch_mfma_t<DT, IL, 256, 368, 2, 4>(k, bmat, shape, s);
+      case 256: return launch_mfma_t<DT, IL, 256, 320, 2, 4>(k, bmat, shape, s);
       default: return hipErrorInvalidValue;
     }
   }
