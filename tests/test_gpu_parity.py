@@ -892,15 +892,20 @@ RESIDENT_CASES.update({
 })
 
 
-# Five to eight query heads: the slack ends inside a rotation of the step buffers, and a wave's sums pass through the
-# ring slots behind its tile.  Whole tiles, last tiles of one step, of the slack's seven and of one more, both rings.
+# Five to eight query heads, eight waves: the slack of a tile of 512 ends inside a rotation of the step buffers (seven steps), and a
+# wave's sums pass through the ring slots behind its tile.  Whole tiles of 512, last tiles of one step, of the slack's seven and of
+# one more.  Shorter tiles have more slack than a layer has steps: 128 on the short ring (below: 256), 320 with four waves.
 RESIDENT_CASES.update({
     "g8_slack_whole_tiles_small_chip": dict(w=small(num_q_heads=64, num_kv_heads=8, budget=128, num_layers=3,
-                                                    seq_lens=(12288, 10241, 5232, 4721, 113, 16)), workgroups=24),
+                                                    seq_lens=(12288, 10241, 5232, 4721, 113, 16)), workgroups=24,
+                                            plan=dict(tile_tokens=512)),
+    "g8_fp8_whole_tiles_small_chip": dict(w=small(num_q_heads=64, num_kv_heads=8, budget=128, num_layers=3, kv_dtype="fp8",
+                                                  seq_lens=(12288, 10241, 5232, 4721, 113, 16)), workgroups=24,
+                                          plan=dict(tile_tokens=512)),
     "g8_slack_short_ring": dict(w=small(num_q_heads=48, num_kv_heads=8, budget=128, num_layers=3,
-                                        seq_lens=(256, 272, 369, 129, 1))),
+                                        seq_lens=(256, 272, 369, 129, 1)), plan=dict(tile_tokens=128)),
     "g5_slack_hkv3": dict(w=small(num_q_heads=15, num_kv_heads=3, budget=128, num_layers=3,
-                                  seq_lens=(6144, 5121, 640, 17)), workgroups=12),
+                                  seq_lens=(6144, 5121, 640, 17)), workgroups=12, plan=dict(tile_tokens=320)),
 })
 
 
