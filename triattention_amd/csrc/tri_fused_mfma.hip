@@ -37,13 +37,13 @@ namespace {
 // What a lane loads of one (token, head) row per step; the token is lane % 16 of the step,
 // kb = lane / 16.  Two-byte keys: the 16-byte chunks 4*s + kb, s = 0..3 (8 elements each,
 // MFMA s takes chunk s).  fp8 keys: the 16-byte chunks kb and 4 + kb (16 elements each;
-// MFMA s takes half s % 2 of chunk s / 2) and the dequantisation scale of the token this
-// lane will store.
-// HD: head dimension, 128 or (two-byte keys only) 64: half the chunks, MFMAs and pairs.
+// MFMA s takes half s % 2 of chunk s / 2) and a dequantisation scale: that of token lane / 4 of the
+// step; the lane's own token's comes from lane `scale_lane` when the step is scored.
+// HD: head dimension, 128 or (two-byte keys only) 64 or 256: half or twice the chunks, MFMAs and pairs.
 template <int DT, int HD>
 struct StepData {
   uint4 c[DT == TRI_KV_FP8_E4M3 ? 2 : HD / 32];
-  float scale;          // fp8 only
+  float scale;          // fp8 only; of token lane / 4
 };
 
 // Index, inside the 128 elements of a head row, of element e of lane block kb in MFMA s.
@@ -255,8 +255,8 @@ __global__ __launch_bounds__(kPrepThreads) void prep_mfma_kernel(const float* fo
 // heads (two): they add up in two or four instructions.  With the tokens as rows and (query head, piece) as columns the
 // pieces sat in other lanes, 16 and 14 instructions of row rotations and selections a step; the sums are the same bits.
 // By itself that is worth 1.4 % at a head dimension of 64 (24 requests of 1500 to 12001 tokens x 36 layers x 64 query heads
-// of 64: 1116 -> 1097 us) and nothing where the key stream or the other tiles are waited for; the other 1 % of that shape and the
-// 7 % of 1 x 32768 tokens x 64 layers x 64 heads of 128 (802 -> 747) are `publish` and the longer ring.
+// of 64: 1116 -> 1097 us) and nothing where the key stream or the other tiles are waited for (1 x 32768 tokens x 64 layers x 64
+// heads of 128: 832 -> 829; what `publish` and the slack give there stands beside them).
 //
 // Two groups (five to eight query heads): a second operand set per group of four would leave a quarter of the rows
 // empty twice.  Instead the rows are (query head, piece 1 | piece 2) and a second operand holds the third pieces beside
@@ -322,12 +322,12 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // token j, its score of query head kb (one group) or of the heads 2 kb and 2 kb + 1 (two).
   const int j = lane & 15, kb = lane >> 4;
 
-  // Coefficient slabs of the current layer.
-  uint4 B[NSO];
+  // Coefficient slabs of the current layer, the A operands.
+  uint4 coef[NSO];
   auto load_coefs = [&](int l) __attribute__((always_inline)) {
     const uint4* p = bmat + (((int64_t)(b * a.L + l) * a.Hkv + head) * NSO) * 64 + lane;
 #pragma unroll
-    for (int o = 0; o < NSO; ++o) B[o] = p[o * 64];
+    for (int o = 0; o < NSO; ++o) coef[o] = p[o * 64];
     {
       // A coefficient beyond fp16's range (65504) arrives as an infinity: the scores of this
       // launch would be meaningless, so the status word is raised (the caller repeats the
@@ -336,7 +336,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       uint32_t bad = 0;
 #pragma unroll
       for (int o = (DT == TRI_KV_FP16 ? 0 : NK); o < NSO; ++o) {
-        const uint32_t w4[4] = {B[o].x, B[o].y, B[o].z, B[o].w};
+        const uint32_t w4[4] = {coef[o].x, coef[o].y, coef[o].z, coef[o].w};
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           bad |= (uint32_t)((w4[i] & 0x7c00u) == 0x7c00u) | (uint32_t)((w4[i] & 0x7c000000u) == 0x7c000000u);
@@ -426,7 +426,7 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // Scores of the 16 tokens of a step: MFMAs over keys and magnitudes, then the pieces of a head, which are rows of
   // one lane's accumulator, are added.
   auto compute_step = [&](const StepData<DT, HD>& raw, float scale, int l, int t, int which) __attribute__((always_inline)) {
-    // The four bf16 A operands of the step as dwords (two elements each): the loaded
+    // The keys of the step, the B operands of its MFMAs, as dwords (two elements each): the loaded
     // registers for bf16 keys, one conversion per dword (exact) for fp8 keys.
     uint32_t w[NS][4];
     // One-byte keys in the half-split layout: lane block kb holds the real parts of pairs
@@ -470,11 +470,11 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
     for (int s = 0; s < NS; ++s) d.c[s] = uint4{w[s][0], w[s][1], w[s][2], w[s][3]};
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < NS; ++s) acc = mfma_16x16x32<DT>(B[s], d.c[s], acc);
+    for (int s = 0; s < NS; ++s) acc = mfma_16x16x32<DT>(coef[s], d.c[s], acc);
     f32x4 acc3 = {0.f, 0.f, 0.f, 0.f};
     if constexpr (QG == 2) {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) acc3 = mfma_16x16x32<DT>(B[NS + s], d.c[s], acc3);
+      for (int s = 0; s < NS; ++s) acc3 = mfma_16x16x32<DT>(coef[NS + s], d.c[s], acc3);
     }
 #pragma unroll
     for (int set = 0; set < NS / 2; ++set) {
@@ -510,11 +510,11 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
       if constexpr (!FP8)   // `which` is the step buffer's number: a constant after unrolling
         mag_seen = pk_max_f16(mag_seen, (&hi.x)[which & 3]);
       constexpr int MT = TRI_KV_FP16;                // operand type of the magnitude MFMAs
-      acc = mfma_16x16x32<MT>(B[NK + set], hi, acc);
-      acc = mfma_16x16x32<MT>(B[NK + set], lo, acc);
+      acc = mfma_16x16x32<MT>(coef[NK + set], hi, acc);
+      acc = mfma_16x16x32<MT>(coef[NK + set], lo, acc);
       if constexpr (QG == 2) {
-        acc3 = mfma_16x16x32<MT>(B[NK + NS / 2 + set], hi, acc3);
-        acc3 = mfma_16x16x32<MT>(B[NK + NS / 2 + set], lo, acc3);
+        acc3 = mfma_16x16x32<MT>(coef[NK + NS / 2 + set], hi, acc3);
+        acc3 = mfma_16x16x32<MT>(coef[NK + NS / 2 + set], lo, acc3);
       }
     }
     // v[i]: the score of this lane's token and its i-th head.
@@ -756,7 +756,8 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   // with the step NB ahead.  A layer is padded to whole rotations (padding steps re-read the
   // last row and are not scored), so the loads of a layer's last rotation are exactly the
   // first NB steps of the next layer; the rotations form inner loops that contain nothing
-  // but key loads and scoring, and the work at layer boundaries sits between them.
+  // but key loads and scoring, and the work at layer boundaries sits between them (where the slack is no whole number of
+  // rotations, one of them is cut in two around the consumption of the layer before).
   const int nsteps = (ntok + 15) >> 4;
   const int rotations = (nsteps + NB - 1) / NB;
   // How far a layer is scored before the layer before it is turned into contributions (a part of a rotation can only lie
@@ -965,8 +966,8 @@ hipError_t launch_mfma_tw(FusedArgs& k, const uint4* bmat, int tw, int waves, in
   }
   if (head_dim == 64) {
     // Half the bytes per row: eight step buffers keep as many bytes in flight (four query heads
-    // per KV head; with eight the LDS has no room for the slack that eight buffers need).  One
-    // instance per shape, with the largest ring.
+    // per KV head; with eight, eight buffers are slower: 24 requests of 1500 to 12001 tokens x 36 layers 1181 us, with four
+    // 1087).  One instance per shape, with the largest ring.
     if constexpr (DT != TRI_KV_FP8_E4M3) {
       if (k.G > 4) {
         if (tw != 512) return hipErrorInvalidValue;
