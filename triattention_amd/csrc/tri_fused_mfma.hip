@@ -568,9 +568,10 @@ void fused_mfma_kernel(FusedArgs a, const uint4* bmat) {
   //    tokens x 36 layers 3135 us, 3142 with a publication per wave).
   //  - Two groups, four waves, fewer than eight query heads: a wave's words end inside a 128-byte line that the next
   //    head's wave, and the next tile's workgroup, write too.  24 requests of 2500 to 11000 tokens x 28 layers, us with a
-  //    publication per wave | meeting: 898 | 856 for 20 / 4 heads of 128, 923 | 886 for 24 / 4, 935 | 896 for 28 / 4, but
-  //    684 | 691 for 32 / 4 (8 x 16384 tokens), whose waves publish whole lines; heads of 64 (16 x 16384 x 36) 1000 | 943 for
-  //    20 / 4, 896 | 915 for 32 / 4.  Padding every wave's words to a line takes 934 to 908 only, and scratch.
+  //    publication per wave | meeting: 898 | 856 for 20 / 4 heads of 128, 923 | 886 for 24 / 4, 935 | 896 for 28 / 4 (the former
+  //    with 112 tokens of slack; with 64 no better), but 688 | 691 for 32 / 4 (8 x 16384 tokens, both with 64), whose waves
+  //    publish whole lines; heads of 64 (16 x 16384 x 36) 1000 | 943 for 20 / 4, 896 | 916 for 32 / 4.  Padding every wave's
+  //    words to a line takes 934 to 908 only, and scratch.
   // Every wave deposits layer l before any deposits layer l + 1 (the last one to arrive has added by the time any wave gets
   // past consuming layer l), so the counter never mixes layers.
   auto publish = [&](int l) __attribute__((always_inline)) {
